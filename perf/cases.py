@@ -192,6 +192,15 @@ def _values(n, width, dtype, gen):
     return x.to(dtype)
 
 
+def _cached_groups(case, past):
+    """The sequences with a cached part, some at a time (the order in which the cached tokens are drawn)."""
+    group = max(1, int(2 ** 27 // max(1, int(past.max()) * case["Hkv"] * case["D"])))
+    for b0 in range(0, len(past), group):
+        idx = np.array([b for b in range(b0, min(len(past), b0 + group)) if past[b] > 0], np.int64)
+        if len(idx):
+            yield idx
+
+
 def prepare(case, seed):
     pkg = _package()
     gen = torch.Generator(device="cuda").manual_seed(int(seed))
@@ -222,12 +231,7 @@ def prepare(case, seed):
             k[s:s + n] += (0.85 * m[:, None] * lean.reshape(1, -1)).to(dtype)
         return k
 
-    # the cached part of every sequence, some sequences at a time
-    group = max(1, int(2 ** 27 // max(1, int(past.max()) * Hkv * D)))
-    for b0 in range(0, B, group):
-        idx = np.array([b for b in range(b0, min(B, b0 + group)) if past[b] > 0], np.int64)
-        if not len(idx):
-            continue
+    for idx in _cached_groups(case, past):
         begins = np.concatenate([[0], np.cumsum(past[idx])]).astype(np.int32)
         op.step_begin(np.zeros(len(idx), np.int32), begins, np.concatenate([[0], np.cumsum(nblk[idx])]).astype(np.int32))
         op.set_block_indices(np.concatenate([table[bib[b]:bib[b + 1]] for b in idx]), pool)
@@ -285,3 +289,63 @@ def run(state):
     for l in range(case["layers"]):
         op.forward(q[l], k[l], v[l], kc[l], vc[l], out[l], None if scores is None else scores[l], layer=l)
     return {"out": out, "scores": scores, "key_cache": kc, "value_cache": vc}
+
+
+def _cached(x, case):
+    """What a cache of the case's type holds of rows x [n, Hkv, D], in 64 bits.  Quantised rows: scale = (max - min) / levels
+    and zero-point = -min / scale in binary32, codes rounded to nearest."""
+    levels = {"u8": 255.0, "u4": 15.0}.get(case["kv"])
+    if levels is None:
+        return x.double()
+    x = x.float()
+    mn, mx = x.amin(-1, keepdim=True), x.amax(-1, keepdim=True)
+    scale = (mx - mn) / torch.tensor(levels, device=x.device)  # (by a tensor: a Python number would become a reciprocal)
+    scale = torch.where(scale == 0, torch.full_like(scale, 1e-4), scale)
+    zp, inv = -mn / scale, 1.0 / scale
+    codes = (x.double() * inv.double() + zp.double()).float().round().clamp(0, levels)  # one rounding, as a fused multiply-add
+    return (codes.double() - zp.double()) * scale.double()
+
+
+def exact(case, seed):
+    """Outputs and scores in 64 bits; cache contents are bytes and have no such value.  None for eviction (block numbers) and for
+    block-sparse prefill, where the blocks that are kept hang on comparisons of computed sums."""
+    if case["kind"] != "step" or work(case)["flops"] > 4e12:
+        return None
+    gen = torch.Generator(device="cuda").manual_seed(int(seed))
+    past, new = _lengths(case)
+    L, Hq, Hkv, D, w = case["layers"], case["Hq"], case["Hkv"], case["D"], case["window"]
+    dtype, B, T = DTYPES[case["q"]], len(past), int(new.sum())
+    rows = [[[None] * L for _ in range(B)] for _ in range(2)]  # [K | V][sequence][layer]: the cached rows as drawn
+    for idx in _cached_groups(case, past):
+        begins = np.concatenate([[0], np.cumsum(past[idx])])
+        for l in range(L):
+            for which in range(2):
+                x = _values(int(begins[-1]), Hkv * D, dtype, gen)
+                for i, b in enumerate(idx):
+                    rows[which][b][l] = x[begins[i]:begins[i + 1]]
+    sb = np.concatenate([[0], np.cumsum(new)])
+    q = torch.randn(L, T, Hq * D, generator=gen, device="cuda").to(dtype)
+    kv_new = [_values(L * T, Hkv * D, dtype, gen).view(L, T, -1) for _ in range(2)]
+    out = torch.zeros(L, T, Hq * D, dtype=torch.float64, device="cuda")
+    scores = torch.zeros(L, int((past + new).sum()), dtype=torch.float64, device="cuda") if case["scores"] else None
+    so = np.concatenate([[0], np.cumsum(past + new)])
+    for l in range(L):
+        for b in range(B):
+            parts = [[rows[j][b][l]] if past[b] else [] for j in range(2)]
+            k, v = (_cached(torch.cat(parts[j] + [kv_new[j][l, sb[b]:sb[b + 1]]]).view(-1, Hkv, D), case).transpose(0, 1).contiguous()
+                    for j in range(2))
+            n_kv, kt = k.shape[1], k.transpose(1, 2).contiguous()
+            pos = torch.arange(n_kv, device="cuda")
+            step = max(1, int(2 ** 28 // (n_kv * Hq)))  # query tokens at a time
+            for t0 in range(0, int(new[b]), step):
+                t1 = min(int(new[b]), t0 + step)
+                x = q[l, sb[b] + t0:sb[b] + t1].double().view(t1 - t0, Hkv, Hq // Hkv, D).permute(1, 2, 0, 3).reshape(Hkv, -1, D).contiguous()
+                p = torch.bmm(x, kt).view(Hkv, Hq // Hkv, t1 - t0, n_kv) / D ** 0.5
+                last = int(past[b]) + torch.arange(t0, t1, device="cuda")[:, None]
+                p.masked_fill_((pos > last) | ((pos <= last - w) if w else (pos < 0)), float("-inf"))
+                p = torch.softmax(p, -1)
+                o = torch.bmm(p.view(Hkv, -1, n_kv), v).view(Hkv, Hq // Hkv, t1 - t0, D)
+                out[l, sb[b] + t0:sb[b] + t1] = o.permute(2, 0, 1, 3).reshape(t1 - t0, Hq * D)
+                if scores is not None and t1 == int(new[b]):  # the default window: the last query token, summed over the heads
+                    scores[l, so[b]:so[b + 1]] = p[:, :, -1].sum((0, 1))
+    return {"out": out, "scores": scores, "key_cache": None, "value_cache": None}
