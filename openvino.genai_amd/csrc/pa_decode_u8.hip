@@ -43,6 +43,25 @@ __device__ inline void bytes_to_half_pairs(uint32_t w, uint32_t& p01, uint32_t& 
     p23 = perm(0u, w, 0x0c030c02u);
 }
 
+// the eight nibbles of `w` -> four dwords of fp16 pairs, zero-extended: with byte i holding element 2 i in its high nibble,
+// the pairs are the elements (1, 5), (3, 7), (0, 4), (2, 6)
+__device__ inline u4v nibbles_to_half_pairs(uint32_t w) {
+    return u4v{w & 0x000f000fu, (w >> 8) & 0x000f000fu, (w >> 4) & 0x000f000fu, (w >> 12) & 0x000f000fu};
+}
+
+// The largest power of two not above `v` and its reciprocal, both kept within 2^+-100 (zero, subnormal and non-finite
+// values included).
+constexpr float VUNIT_MIN = 0x1p-100f;
+__device__ inline void power_of_two_below(float v, float& unit, float& inv) {
+    const uint32_t e = min(max(__builtin_bit_cast(uint32_t, v) & 0x7f800000u, 27u << 23), 227u << 23);
+    unit = __builtin_bit_cast(float, e);
+    inv = __builtin_bit_cast(float, (254u << 23) - e);
+}
+
+// bytes of a wave's staging slot: a tile of K or V, or (u4, whose tiles are smaller) its share of the merge's
+// accumulators, eight heads' rows
+__host__ __device__ constexpr int decode_slot_bytes(int D, bool u4) { return u4 ? 8 * D * 4 : TOK * (D + 8); }
+
 // Reductions over the four 16-lane groups with the gfx950 lane-swap instructions (no LDS round trip):
 // v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of the second,
 // v_permlane32_swap the upper half of the first with the lower half of the second; with both operands holding the
@@ -102,7 +121,22 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
     }
 }
 
-template <int D, int QDT, int WAVES, int BS>
+// U4: rows of `f32 scale | f32 zero-point | D / 2 bytes` (element 2 i in the high nibble of byte i).  Everything up to the
+// operands is the u8 kernel's; what differs:
+//   * QK: four masks of a 32-bit word give four pairs of f16 subnormals (elements 1,5 | 3,7 | 0,4 | 2,6 of the eight), and
+//     the query operand is permuted to match.  bf16 queries are brought below 2 by a power of two per head before they
+//     become f16 operands, so that nothing of their range is lost.
+//   * PV: the weights are relative to the largest V scale seen so far (a power of two, `vunit`), so that small or large
+//     values of V neither underflow nor overflow f16; a tile's products are formed from zero and added to the running
+//     sums in f32 with one rounding per tile (the matrix pipe truncates as it accumulates, and with sixteen levels
+//     the zero-point term is of the size of the code sums themselves).
+//   * scores: the scaled logits go to `logits` in f32 and become scores in a kernel of their own, as for the
+//     shape-generic path that serves the other u4 steps; no probability is rounded to 16 bits on the way.
+// Bound by vector instructions (at 186 registers two waves a SIMD; capped at 168 for three the kernel spills and takes 56
+// instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 28 us + 4 us
+// of merge, where the shape-generic kernel, one lane to a row, took 149 + 17 us and an append launch of 5; 64 sequences of
+// 4096 tokens in 65 us = 4.6 TB/s.
+template <int D, int QDT, int WAVES, int BS, bool U4>
 // (head size 256: one workgroup per CU, whose waves may then use the accumulation registers as well -- 16 KB blocks,
 // two of them in flight, 64 accumulators and 32 query registers do not fit 256 registers)
 __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kernel(DecodeArgs a) {
@@ -114,15 +148,15 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     const int sub_shift = BS == 32 ? 31 - __builtin_clz(a.sh.bs >> 5) : 0;
     const int bsz = BS == 32 ? a.sh.bs : BS;
     constexpr int NT = 64 * WAVES;
-    constexpr int ROW = D + 8;
+    constexpr int ROW = (U4 ? D / 2 : D) + 8;
     constexpr int TILE = TOK * ROW;        // bytes of one (block, head) of K or V
     constexpr int FULL = TILE / 1024;      // whole-wave 16-byte passes; 16 chunks remain
     constexpr int KS = D / 32;             // k-steps of the QK contraction
     constexpr int RT = D / 16;             // 16-row output tiles of PV
-    constexpr int VB = D / 16;             // V bytes per lane per token row
+    constexpr int VB = D / 16;             // V channels per lane per token row
     constexpr int NW = (VB + 3) / 4;       // ... held in this many 32-bit words
-    constexpr int SLOT = TILE;             // a wave's LDS staging slot: a K block, then a V block
-    constexpr int EPL = (D + 63) / 64;     // elements per lane of a new K / V row
+    constexpr int SLOT = decode_slot_bytes(D, U4);  // a wave's LDS staging slot: a K block, then a V block
+    constexpr int EPL = U4 && D == 64 ? 2 : (D + 63) / 64;  // elements per lane of a new K / V row
     constexpr int ROW_LANES = D / EPL;     // lanes a new row spreads over (D = 96: 48, the others repeat lanes 32 - 47)
     constexpr int DEPTH = 2;               // blocks a wave keeps in flight
     // Channel of row m of output tile r (the lane with n = m reads that channel's byte of each of its token rows): a
@@ -153,7 +187,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     uint8_t* slot = smem + wv * SLOT;                                  // wave-private staging
     float* wave_mlz = reinterpret_cast<float*>(smem + WAVES * SLOT);   // [WAVES][16][4]
     float* msnap = wave_mlz + WAVES * 16 * 4;                          // [max_tiles][16]
-    _Float16* ptile = reinterpret_cast<_Float16*>(msnap + (a.want_scores ? a.max_tiles * 16 : 0));  // [G][max_tiles*TOK]
+    _Float16* ptile = reinterpret_cast<_Float16*>(msnap + (a.want_scores ? a.max_tiles * 16 : 0));  // (u4: neither)  // [G][max_tiles*TOK]
     const int pstride = a.max_tiles * TOK;
 
     // The step's new K / V row of this (sequence, kv head) goes into the caches here when the step's append is fused
@@ -170,8 +204,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         uint16_t kr[EPL], vr[EPL];
         load_row16<EPL>(a.key + src, kr);
         load_row16<EPL>(a.value + src, vr);
-        quantize_row_u8<QDT, EPL>(kr, const_cast<uint8_t*>(a.key_cache) + dst, rl, lane < ROW_LANES);
-        quantize_row_u8<QDT, EPL>(vr, const_cast<uint8_t*>(a.value_cache) + dst, rl, lane < ROW_LANES);
+        quantize_row<QDT, EPL, U4>(kr, const_cast<uint8_t*>(a.key_cache) + dst, rl, lane < ROW_LANES);
+        quantize_row<QDT, EPL, U4>(vr, const_cast<uint8_t*>(a.value_cache) + dst, rl, lane < ROW_LANES);
     };
     if (append_first) {
         append_rows();
@@ -199,7 +233,44 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // query operand (B of QK): lane (n, g) holds q[head n][32 s + 8 g + e]
     h8 qreg[KS];
     float qsum = 0.0f;
-    {
+    float qunit = 1.0f;  // u4, bf16 queries: the power of two the head's operands were divided by
+    if constexpr (U4) {
+        // step 2 i + h of the contraction takes, on lanes of group g, the elements 64 i + 16 g + 8 h + {1, 5, 3, 7, 0, 4, 2, 6}
+        const uint16_t* qp = a.query + ((long)t * Hq + hkv * G + n) * D + 16 * g;
+        uint4 raw[KS];
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            raw[s] = n < G ? *reinterpret_cast<const uint4*>(qp + 64 * (s >> 1) + 8 * (s & 1)) : make_uint4(0, 0, 0, 0);
+        float inv_unit = 1.0f;
+        if (QDT == DT_BF16) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    mx = fmaxf(mx, fmaxf(fabsf(__builtin_bit_cast(float, w[e] << 16)), fabsf(__builtin_bit_cast(float, w[e] & 0xffff0000u))));
+            }
+            power_of_two_below(xor_reduce_max_g(mx), qunit, inv_unit);
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
+            constexpr int first_of[4] = {1, 3, 0, 2};  // pair e: elements first_of[e] and first_of[e] + 4
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    const int el = first_of[e] + 4 * half;
+                    const uint16_t bits = (uint16_t)(w[el >> 1] >> (16 * (el & 1)));
+                    qreg[s][2 * e + half] = QDT == DT_F16 ? __builtin_bit_cast(_Float16, bits)
+                                                          : (_Float16)(bf16_bits_to_float(bits) * inv_unit);
+                }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qsum += (float)qreg[s][e];
+        }
+        qsum = xor_reduce_sum_g(qsum);
+    } else {
         const uint16_t* qp = a.query + ((long)t * Hq + hkv * G + n) * D + 8 * g;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -224,10 +295,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         }
         qsum = xor_reduce_sum_g(qsum);
     }
-    const float scl24 = st.scale * LOG2E * TWO24;  // logits are kept in the log2 domain
+    const float scl24 = st.scale * LOG2E * TWO24 * qunit;  // logits are kept in the log2 domain
     const float qsum24 = qsum * (1.0f / TWO24);
 
     float m_run = -INFINITY, l_part = 0.0f, z_part = 0.0f;
+    float vunit = VUNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
     f4 acc[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r] = f4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -246,14 +318,21 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         f4 sc0 = f4{0.0f, 0.0f, 0.0f, 0.0f}, sc1 = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            const uint2 w0 = *reinterpret_cast<const uint2*>(slot + ROW * n + 8 + 32 * s + 8 * g);
-            const uint2 w1 = *reinterpret_cast<const uint2*>(slot + ROW * (16 + n) + 8 + 32 * s + 8 * g);
             u4v a0, a1;
-            uint32_t x0, x1;
-            bytes_to_half_pairs(w0.x, x0, x1); a0[0] = x0; a0[1] = x1;
-            bytes_to_half_pairs(w0.y, x0, x1); a0[2] = x0; a0[3] = x1;
-            bytes_to_half_pairs(w1.x, x0, x1); a1[0] = x0; a1[1] = x1;
-            bytes_to_half_pairs(w1.y, x0, x1); a1[2] = x0; a1[3] = x1;
+            if constexpr (U4) {
+                const uint32_t w0 = *reinterpret_cast<const uint32_t*>(slot + ROW * n + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
+                const uint32_t w1 = *reinterpret_cast<const uint32_t*>(slot + ROW * (16 + n) + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
+                a0 = nibbles_to_half_pairs(w0);
+                a1 = nibbles_to_half_pairs(w1);
+            } else {
+                const uint2 w0 = *reinterpret_cast<const uint2*>(slot + ROW * n + 8 + 32 * s + 8 * g);
+                const uint2 w1 = *reinterpret_cast<const uint2*>(slot + ROW * (16 + n) + 8 + 32 * s + 8 * g);
+                uint32_t x0, x1;
+                bytes_to_half_pairs(w0.x, x0, x1); a0[0] = x0; a0[1] = x1;
+                bytes_to_half_pairs(w0.y, x0, x1); a0[2] = x0; a0[3] = x1;
+                bytes_to_half_pairs(w1.x, x0, x1); a1[0] = x0; a1[1] = x1;
+                bytes_to_half_pairs(w1.y, x0, x1); a1[2] = x0; a1[3] = x1;
+            }
             sc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a0), qreg[s], sc0, 0, 0, 0);
             sc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a1), qreg[s], sc1, 0, 0, 0);
         }
@@ -279,6 +358,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         // Rows outside [first, kv_len) may hold anything, headers included: blocks that reach beyond either end
         // mask them (EDGE); the blocks in between, nearly all of a long context, skip the tests and selects.
         h8 pb, pl;
+        float acc_corr = 1.0f;  // u4: what the running sums are multiplied by when the tile's are added
         auto softmax = [&](auto edge_tag) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge_tag)::value;
             float x[8];
@@ -306,11 +386,24 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             float psum = 0.0f, zsum = 0.0f;
             _Float16 ph[8];
             float wf[8];
+            float inv_vunit = 1.0f;
+            if constexpr (U4) {
+                float top = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) top = fmaxf(top, seen[j] ? hv[j].x : 0.0f);
+                float unit, inv;
+                power_of_two_below(fmaxf(xor_reduce_max_g(top), vunit), unit, inv);
+                acc_corr = corr * (vunit * inv);
+                vunit = unit;
+                inv_vunit = inv;
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float p = __builtin_amdgcn_exp2f(x[j] - m_new);
                 wf[j] = seen[j] ? p * hv[j].x : 0.0f;
                 psum += p;
+                if constexpr (U4) zsum += seen[j] ? wf[j] * hv[j].y : 0.0f;
+                if constexpr (U4) wf[j] *= inv_vunit;  // (a power of two)
                 pb[j] = (_Float16)wf[j];
                 ph[j] = (_Float16)p;
             }
@@ -325,15 +418,25 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             // the zero-point term must see the weight the matrix product sees, or the rounding error is scaled by the
             // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
 #pragma unroll
-            for (int j = 0; j < 8; ++j) zsum += seen[j] ? wf[j] * hv[j].y : 0.0f;
+            for (int j = 0; j < 8; ++j)
+                if constexpr (!U4) zsum += seen[j] ? wf[j] * hv[j].y : 0.0f;
             l_part = l_part * corr + psum;
             z_part = z_part * corr + zsum;
             m_run = m_new;
-            if (__any(corr != 1.0f)) {
+            if constexpr (!U4) {
+                if (__any(corr != 1.0f)) {
 #pragma unroll
-                for (int r = 0; r < RT; ++r) acc[r] *= corr;
+                    for (int r = 0; r < RT; ++r) acc[r] *= corr;
+                }
             }
-            if (a.want_scores) {
+            if constexpr (U4) {
+                if (a.want_scores && n < G) {
+                    float* dst = a.logits + (long)(hkv * G + n) * a.total_scores + dsc->score_off + pos0 + 4 * g;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (seen[j]) dst[16 * (j >> 2) + (j & 3)] = x[j];
+                }
+            } else if (a.want_scores) {
                 const int lt = tile - tb;
                 if (n < G) {
                     _Float16* dst = ptile + n * pstride + lt * TOK + 4 * g;
@@ -353,10 +456,22 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint8_t* p = slot + ROW * (16 * (j >> 2) + 4 * g + (j & 3)) + 8;
-            if constexpr (VB == 16) {  // (rows start on 8-byte boundaries)
+            if constexpr (VB == 16 && !U4) {  // (rows start on 8-byte boundaries)
                 const uint2 w0 = *reinterpret_cast<const uint2*>(p + 16 * n);
                 const uint2 w1 = *reinterpret_cast<const uint2*>(p + 16 * n + 8);
                 vw[0][j] = w0.x, vw[1][j] = w0.y, vw[2][j] = w1.x, vw[3][j] = w1.y;
+            } else if constexpr (U4) {  // VB channels in VB / 2 bytes: channel VB n + r in nibble r, the even ones the high nibbles
+                if constexpr (VB == 16) {
+                    const uint2 w = *reinterpret_cast<const uint2*>(p + 8 * n);
+                    vw[0][j] = (w.x >> 4) & 0x0f0f0f0fu, vw[1][j] = w.x & 0x0f0f0f0fu;
+                    vw[2][j] = (w.y >> 4) & 0x0f0f0f0fu, vw[3][j] = w.y & 0x0f0f0f0fu;
+                } else if constexpr (VB == 8) {
+                    const uint32_t w = *reinterpret_cast<const uint32_t*>(p + 4 * n);
+                    vw[0][j] = (w >> 4) & 0x0f0f0f0fu, vw[1][j] = w & 0x0f0f0f0fu;
+                } else {  // two bytes: both nibble sets in one word
+                    const uint32_t w = *reinterpret_cast<const uint16_t*>(p + 2 * n);
+                    vw[0][j] = ((w >> 4) & 0x0f0fu) | ((w & 0x0f0fu) << 16);
+                }
             } else if constexpr (VB == 8) {
                 const uint2 w = *reinterpret_cast<const uint2*>(p + 8 * n);
                 vw[0][j] = w.x, vw[1][j] = w.y;
@@ -369,12 +484,22 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            const uint32_t sel = 0x0c000c00u | (uint32_t)(r & 3) | ((uint32_t)(4 + (r & 3)) << 16);
+            // the word and the byte within it that hold channel chan(., r): u4 words hold four channels of one parity
+            const int word = U4 ? (VB == 4 ? 0 : 2 * (r >> 3) + (r & 1)) : r >> 2;
+            const int byte = U4 ? (VB == 4 ? 2 * (r & 1) + (r >> 1) : (r >> 1) & 3) : r & 3;
+            const uint32_t sel = 0x0c000c00u | (uint32_t)byte | ((uint32_t)(4 + byte) << 16);
             u4v av;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) av[p] = perm(vw[r >> 2][2 * p + 1], vw[r >> 2][2 * p], sel);
-            acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb, acc[r], 0, 0, 0);
-            acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl, acc[r], 0, 0, 0);
+            for (int p = 0; p < 4; ++p) av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
+            if constexpr (U4) {
+                f4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb, part, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[r][i] = __builtin_fmaf(acc[r][i], acc_corr, part[i]);
+            } else {
+                acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb, acc[r], 0, 0, 0);
+                acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl, acc[r], 0, 0, 0);
+            }
         }
         __builtin_amdgcn_wave_barrier();
     };
@@ -386,6 +511,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // ---- merge the waves ---------------------------------------------------------------------------
     // Every wave leaves (max, denominator, zero-point sum) per head and its raw accumulators of the group's heads
     // (lanes n < G) in LDS; after one barrier each thread folds the waves for two channels of one head.
+    if constexpr (U4) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r] *= vunit;
+    }
     const float l_w = xor_reduce_sum_g(l_part);
     const float z_w = xor_reduce_sum_g(z_part);
     __syncthreads();  // staging slots are dead from here on
@@ -424,7 +553,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 for (int i = 0; i < 4; ++i) dst[chan(4 * g + i, r)] = acc[r][i];  // lane (n, g), register i of tile r: row 4 g + i
         }
         __syncthreads();
-        if (n0 == 0 && a.want_scores) {
+        if (!U4 && n0 == 0 && a.want_scores) {
             // one factor per (block, head): exp2(snapshot - M) (/ L when this workgroup saw the whole context), written
             // over the snapshot.  Entry e belongs to head e % 16 = this thread's n; the barrier before the score
             // phase publishes the factors
@@ -465,7 +594,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     }
 
     // ---- scores: the factors were formed in place of the block maxima during the merge ---------------
-    if (!a.want_scores) return;
+    if (U4 || !a.want_scores) return;
     __syncthreads();
     const float* fac = msnap;
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -707,8 +836,9 @@ __global__ __launch_bounds__(256) void pa_decode_post_kernel(DecodeArgs a, float
 }  // namespace
 
 // LDS layout: staging | per-wave (m, l, z) | [scores: block maxima | probabilities] | block-table slice
-size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size) {
-    size_t bytes = (size_t)waves * TOK * (D + 8) + waves * 16 * 4 * sizeof(float);
+size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4) {
+    size_t bytes = (size_t)waves * decode_slot_bytes(D, u4) + waves * 16 * 4 * sizeof(float);
+    if (u4) want_scores = false;  // (u4 keeps logits in global memory instead)
     if (want_scores) bytes += (size_t)max_tiles * 16 * sizeof(float) + (size_t)G * max_tiles * TOK * sizeof(uint16_t);
     bytes = (bytes + 15) & ~(size_t)15;
     *table_off = (int32_t)bytes;
@@ -716,18 +846,19 @@ size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int wa
     return (bytes + 15) & ~(size_t)15;
 }
 
-template <int D, int QDT, int WAVES, int BS>
+template <int D, int QDT, int WAVES, int BS, bool U4 = false>
 static hipError_t launch_decode_typed(hipStream_t s, const DecodeArgs& a_in, float* scores, int max_kv_len,
                                       hipEvent_t ev0, hipEvent_t ev1) {
     DecodeArgs a = a_in;
-    const size_t lds = decode_u8_lds_bytes(D, a.G, a.max_tiles, a.want_scores != 0, WAVES, &a.table_off, BS);
-    auto kern = pa_decode_u8_kernel<D, QDT, WAVES, BS>;
+    const size_t lds = decode_u8_lds_bytes(D, a.G, a.max_tiles, a.want_scores != 0, WAVES, &a.table_off, BS, U4);
+    auto kern = pa_decode_u8_kernel<D, QDT, WAVES, BS, U4>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     if (a.n_seqs > 65535) return hipErrorInvalidValue;  // grid z
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(kern, dim3((unsigned)a.nsplit, (unsigned)a.sh.Hkv, (unsigned)a.n_seqs), dim3(64 * WAVES), lds, s, a);
     if (ev1) (void)hipEventRecord(ev1, s);
+    if constexpr (U4) return a.nsplit > 1 ? launch_decode_merge(s, a, QDT) : hipGetLastError();  // (scores: from the logits, by the caller)
     return launch_decode_post(s, a, QDT, scores, max_kv_len);
 }
 
@@ -803,7 +934,22 @@ hipError_t launch_decode_post(hipStream_t s, const DecodeArgs& a, int q_dtype, f
 // a context is created, keeps that allocation out of the first attention call.
 hipError_t preload_decode_u8() {
     hipFuncAttributes at;
-    return hipFuncGetAttributes(&at, reinterpret_cast<const void*>(pa_decode_u8_kernel<128, DT_F16, 4, 32>));
+    return hipFuncGetAttributes(&at, reinterpret_cast<const void*>(pa_decode_u8_kernel<128, DT_F16, 4, 32, false>));
+}
+
+hipError_t launch_decode_u4(hipStream_t s, const DecodeArgs& a, int q_dtype, hipEvent_t ev0, hipEvent_t ev1) {
+    if (a.waves != 4 || a.sh.bs < 16 || a.sh.bs > 256 || (a.sh.bs & (a.sh.bs - 1))) return hipErrorInvalidValue;
+#define PA_U4(D_, BS_)                                                                                        \
+    if (a.sh.D == D_ && (a.sh.bs == 16) == (BS_ == 16))                                                       \
+        return q_dtype == DT_F16 ? launch_decode_typed<D_, DT_F16, 4, BS_, true>(s, a, nullptr, 0, ev0, ev1) \
+                                 : launch_decode_typed<D_, DT_BF16, 4, BS_, true>(s, a, nullptr, 0, ev0, ev1);
+    PA_U4(128, 32)
+    PA_U4(128, 16)
+    PA_U4(64, 32)
+    PA_U4(64, 16)
+    PA_U4(256, 32)
+#undef PA_U4
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_decode_u8(hipStream_t s, const DecodeArgs& a, int q_dtype, float* scores, int max_kv_len,

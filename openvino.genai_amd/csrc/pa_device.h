@@ -101,8 +101,10 @@ __device__ __forceinline__ float row16_sum(float v) {
 // `raw` holds the lane's EPL consecutive elements (bit patterns of QDT), elements lane * EPL ..; `dst` is the row's
 // first byte.  A row shorter than 64 * EPL elements: the surplus lanes hold copies of other lanes' elements (which
 // leaves minimum and maximum alone), pass those lanes' numbers and `store` = false.
-template <int QDT, int EPL>
-__device__ __forceinline__ void quantize_row_u8(const uint16_t (&raw)[EPL], uint8_t* dst, const int lane, const bool store = true) {
+// U4: two codes per byte, scale = (max - min) / 15, codes clamped to 15, the lane's even elements in the high nibbles (EPL
+// is 2 or 4).
+template <int QDT, int EPL, bool U4>
+__device__ __forceinline__ void quantize_row(const uint16_t (&raw)[EPL], uint8_t* dst, const int lane, const bool store = true) {
 #pragma clang fp contract(off)
     float x[EPL];
 #pragma unroll
@@ -112,7 +114,8 @@ __device__ __forceinline__ void quantize_row_u8(const uint16_t (&raw)[EPL], uint
     for (int e = 1; e < EPL; ++e) { mn = fminf(mn, x[e]); mx = fmaxf(mx, x[e]); }
     mn = wave_min(mn);
     mx = wave_max(mx);
-    float scale = (mx - mn) / 255.0f;
+    constexpr float LEVELS = U4 ? 15.0f : 255.0f;
+    float scale = (mx - mn) / LEVELS;
     if (scale == 0.0f) scale = 0.0001f;
     const float zp = -mn / scale;
     const float inv = 1.0f / scale;
@@ -120,15 +123,23 @@ __device__ __forceinline__ void quantize_row_u8(const uint16_t (&raw)[EPL], uint
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
         float v = rintf(__fmaf_rn(x[e], inv, zp));
-        v = fminf(fmaxf(v, 0.0f), 255.0f);
-        packed |= (uint32_t)(int)v << (8 * e);
+        v = fminf(fmaxf(v, 0.0f), LEVELS);
+        packed |= (uint32_t)(int)v << (U4 ? 8 * (e >> 1) + 4 * (1 - (e & 1)) : 8 * e);
     }
     if (!store) return;
     if (lane == 0) *reinterpret_cast<float2*>(dst) = make_float2(scale, zp);
-    uint8_t* c = dst + 8 + lane * EPL;
-    if constexpr (EPL == 4) *reinterpret_cast<uint32_t*>(c) = packed;
+    uint8_t* c = dst + 8 + lane * (U4 ? EPL / 2 : EPL);
+    if constexpr (U4) {
+        static_assert(EPL == 2 || EPL == 4, "whole bytes per lane");
+        if constexpr (EPL == 4) *reinterpret_cast<uint16_t*>(c) = (uint16_t)packed;
+        else *c = (uint8_t)packed;
+    } else if constexpr (EPL == 4) *reinterpret_cast<uint32_t*>(c) = packed;
     else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(c) = (uint16_t)packed;
     else *c = (uint8_t)packed;
+}
+template <int QDT, int EPL>
+__device__ __forceinline__ void quantize_row_u8(const uint16_t (&raw)[EPL], uint8_t* dst, const int lane, const bool store = true) {
+    quantize_row<QDT, EPL, false>(raw, dst, lane, store);
 }
 // The lane's EPL consecutive elements of a row of 16-bit values.
 template <int EPL>
@@ -257,6 +268,7 @@ struct DecodeArgs {
     float* part_ml;               // nsplit > 1: [T*Hq*nsplit, 2] (max in the log2 domain, denominator)
     float* final_ml;              // [T*Hq, 2]
     _Float16* group_scores;       // nsplit == 1: [Hkv, total_scores] per-kv-head score sums on their way to the score kernel
+    float* logits;                // u4 with scores: [Hq, total_scores] scaled logits in the log2 domain
     _Float16* p_split;            // nsplit > 1: [Hq, p_split_stride(total_scores, B)] probabilities relative to the
                                   // split maximum; a sequence's run starts at p_split_offset (16-byte aligned)
 };
@@ -264,10 +276,17 @@ struct DecodeArgs {
 __host__ __device__ inline long p_split_offset(long score_offset, int b) { return ((score_offset + 7) & ~7L) + 8L * b; }
 __host__ __device__ inline long p_split_stride(long total_scores, int B) { return total_scores + 8L * B + 8; }
 
-size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size);
+size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4 = false);
 // ev0 / ev1 (may be null) are recorded right before and after the main kernel.
 hipError_t launch_decode_u8(hipStream_t s, const DecodeArgs& a, int q_dtype, float* scores, int max_kv_len,
                             hipEvent_t ev0, hipEvent_t ev1);
+
+// The same kernel over u4 rows (head sizes 64, 128 and -- 32-token blocks and up -- 256; four waves); with scores it leaves
+// logits and final (max, denominator) pairs for `launch_scores_from_logits`.
+hipError_t launch_decode_u4(hipStream_t s, const DecodeArgs& a, int q_dtype, hipEvent_t ev0, hipEvent_t ev1);
+// Scores of the step's single-token sequences from logits and final (max, denominator) pairs in the log2 domain.
+hipError_t launch_scores_from_logits(hipStream_t s, const StepDev& st, int Hq, float* logits, int total_scores, float* final_ml,
+                                     float* scores, int max_kv_len);
 
 // ---- block-sparse prefill (XAttention) -----------------------------------------------------------
 // Blocks and strided groups are counted by absolute position: query / key block I covers positions

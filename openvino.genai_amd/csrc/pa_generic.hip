@@ -312,6 +312,8 @@ __global__ __launch_bounds__(256) void pa_merge_kernel(StepDev st, GenericShape 
 }
 
 // Single-token sequences: score_j = sum over heads of exp(logit - M) / L, heads in ascending order.
+// LOG2: logits and maxima are in the log2 domain (the u4 decode kernel's).
+template <bool LOG2>
 __global__ __launch_bounds__(256) void pa_scores_single_kernel(StepDev st, GenericShape sh, AttnWorkspace ws,
                                                                float* __restrict__ scores) {
     const int b = blockIdx.y;
@@ -327,7 +329,8 @@ __global__ __launch_bounds__(256) void pa_scores_single_kernel(StepDev st, Gener
             for (int h = 0; h < sh.Hq; ++h) {
                 const float M = ws.final_ml[2 * ((long)t * sh.Hq + h)];
                 const float L = ws.final_ml[2 * ((long)t * sh.Hq + h) + 1];
-                sum += __expf(ws.logits[(long)h * ws.total_scores + st.score_offsets[b] + j] - M) / L;
+                const float x = ws.logits[(long)h * ws.total_scores + st.score_offsets[b] + j] - M;
+                sum += (LOG2 ? __builtin_amdgcn_exp2f(x) : __expf(x)) / L;
             }
         }
         scores[st.score_offsets[b] + j] = sum;
@@ -478,7 +481,7 @@ hipError_t launch_typed(hipStream_t s, const StepDev& st, const GenericShape& sh
                        reinterpret_cast<uint16_t*>(out));
     if (scores) {
         dim3 grid((unsigned)min(ceil_div(max_kv_len, 256), 1024), (unsigned)st.B);
-        hipLaunchKernelGGL(pa_scores_single_kernel, grid, dim3(256), 0, s, st, sh, ws, scores);
+        hipLaunchKernelGGL((pa_scores_single_kernel<false>), grid, dim3(256), 0, s, st, sh, ws, scores);
         if (st.T > st.B)
             hipLaunchKernelGGL((pa_scores_window_kernel<QDT>), grid, dim3(256), 0, s, st, sh, ws, q, k, bi, scores, 0);
     }
@@ -492,6 +495,19 @@ bool generic_shape_ok(const GenericShape& sh) {
 }
 
 }  // namespace
+
+hipError_t launch_scores_from_logits(hipStream_t s, const StepDev& st, int Hq, float* logits, int total_scores, float* final_ml,
+                                     float* scores, int max_kv_len) {
+    GenericShape sh{};
+    sh.Hq = Hq;
+    AttnWorkspace ws{};
+    ws.final_ml = final_ml;
+    ws.logits = logits;
+    ws.total_scores = total_scores;
+    const dim3 grid((unsigned)min(ceil_div(max_kv_len, 256), 1024), (unsigned)st.B);
+    hipLaunchKernelGGL((pa_scores_single_kernel<true>), grid, dim3(256), 0, s, st, sh, ws, scores);
+    return hipGetLastError();
+}
 
 hipError_t launch_attention_generic(hipStream_t s, const StepDev& st, const GenericShape& sh, int q_dtype,
                                     const void* query, const void* key_cache, const void* value_cache,

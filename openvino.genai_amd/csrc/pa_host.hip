@@ -363,6 +363,14 @@ bool decode_u8_shape(const pa_config& c) {
            c.num_heads / c.num_kv_heads <= 16;
 }
 
+// Shapes the u4 variant of the decode kernel is built for.  (Head size 96: a tile of such rows is no whole number of the
+// kernel's passes; they stay on the shape-generic kernel.)
+bool decode_u4_shape(const pa_config& c) {
+    return c.kv_cache_dtype == PA_U4 && v_dtype(c) == PA_U4 && v_head(c) == c.head_size && tuned_block_size(c.block_size) &&
+           (c.head_size == 64 || c.head_size == 128 || (c.head_size == 256 && c.block_size >= 32)) &&
+           c.num_heads / c.num_kv_heads <= 16;
+}
+
 // Shapes the MFMA kernel is built for: 16-bit caches of the query's type, or u8 caches (dequantised on the way to
 // LDS).  It takes every sequence the decode kernel does not.
 // (head sizes 96 and 256: its one-row-group variants only -- at 256 one workgroup per CU, two blocks of LDS slots fill
@@ -383,6 +391,7 @@ bool decode16_shape(const pa_config& c) {
 
 // The same questions asked of a context: one with ALiBi slopes has no tuned attention kernel.
 bool decode_u8_shape(const pa_ctx* ctx) { return !ctx->has_alibi && decode_u8_shape(ctx->cfg); }
+bool decode_u4_shape(const pa_ctx* ctx) { return !ctx->has_alibi && decode_u4_shape(ctx->cfg); }
 bool mfma_shape(const pa_ctx* ctx) { return !ctx->has_alibi && mfma_shape(ctx->cfg); }
 bool decode16_shape(const pa_ctx* ctx) { return !ctx->has_alibi && decode16_shape(ctx->cfg); }
 // Whether the planned step runs on the matrix kernel (or, a step of single-token sequences over a 16-bit cache, on the
@@ -400,6 +409,13 @@ bool decode_u8_step(const pa_ctx* ctx) {
     return decode_u8_shape(ctx) && !ctx->h_dec.empty() && (mfma_shape(ctx) || (int32_t)ctx->h_dec.size() == ctx->B);
 }
 
+// Whether the planned step runs on the u4 variant of that kernel: single-token sequences alone (there is no matrix kernel
+// over u4 rows to take others), as many as the launch grid's z axis holds.  A step with a multi-token sequence stays on the
+// shape-generic kernel.
+bool decode_u4_step(const pa_ctx* ctx) {
+    return decode_u4_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B && ctx->B <= 65535;
+}
+
 // Split-K plan of the decode kernels: workgroups per (sequence, kv head) and the most blocks one walks.
 void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, int32_t* max_tiles_out,
                     const std::vector<int32_t>* seqs = nullptr, int32_t* waves_out = nullptr) {
@@ -413,21 +429,23 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
         most = std::max(most, (kv + 31) / 32 - first / 32);
         all_tiles += (kv + 31) / 32 - first / 32;
     }
-    const bool u8 = c.kv_cache_dtype == PA_U8;
+    const bool u4 = c.kv_cache_dtype == PA_U4, u8 = c.kv_cache_dtype == PA_U8 || u4;
     const int64_t pairs = (int64_t)(seqs ? seqs->size() : ctx->h_dec.size()) * c.num_kv_heads;
     // `slots` workgroups of `waves` waves run at once (a CU's 160 KB of LDS shared between them, allocated in
     // granules: one granule of margin each)
     auto plan = [&](int32_t waves, int32_t slots, int32_t* cap_out) {
         auto lds_of = [&](int32_t tiles) {
             int32_t off;
-            return u8 ? pa::decode_u8_lds_bytes(c.head_size, G, tiles, want_scores, waves, &off, c.block_size)
+            return u8 ? pa::decode_u8_lds_bytes(c.head_size, G, tiles, want_scores, waves, &off, c.block_size, u4)
                       : pa::decode16_lds_bytes(c.head_size, G, tiles, want_scores) + pa::decode16_table_bytes(tiles, c.block_size);
         };
         // the score path keeps a split's probabilities in LDS: that bounds the blocks per workgroup
         const size_t budget = (size_t)(160 * 1024 / (slots / 256));
         auto fits = [&](int32_t tiles) { return (lds_of(tiles) + 1279) / 1280 * 1280 <= budget; };
         int32_t cap = most;
-        if (want_scores) {
+        if (u4) {  // (no probabilities in LDS; the table slice of a workgroup stays within 64 KB)
+            cap = std::min<int32_t>(most, 8192);
+        } else if (want_scores) {
             cap = std::min<int32_t>(most, (int32_t)(budget / (64 * G)));
             while (cap > 1 && !fits(cap)) --cap;
         }
@@ -447,10 +465,14 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             // workgroups sharing a CU take t2 for)
             const bool sc = want_scores;
             const double dscale = c.head_size / 128.0;
-            const double t2 = (u8 ? (sc ? 0.525 : 0.468) : (sc ? 1.104 : 1.064)) * dscale;
-            const double t1 = slots == 256 ? t2 / 2 : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
-            const double tile_bytes = 2.0 * 32 * (u8 ? c.head_size + 8 : 2 * c.head_size), bw = sc ? 5.9e6 : 6.97e6;
-            const double post_a = u8 ? (sc ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
+            // (u4 rows, counts of 1 - 32 forced over batches of 1 - 128 sequences and contexts of 512 - 32768 tokens: 0.33 and
+            // 0.49 us per tile -- vector instructions, whatever the bytes -- and 0.0105 us per further workgroup; the counts
+            // these give are within 5 % of the best forced one, 14 % for 128 sequences of 128 - 8000 tokens.  With the u8
+            // figures 32 sequences of 256 - 4096 tokens were cut in 2 instead of 4: 49.3 against 41.9 us per layer)
+            const double t2 = u4 ? 0.49 * dscale : (u8 ? (sc ? 0.525 : 0.468) : (sc ? 1.104 : 1.064)) * dscale;
+            const double t1 = slots == 256 ? t2 / 2 : u4 ? 0.33 * dscale : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
+            const double tile_bytes = 2.0 * 32 * pa::row_bytes(c.head_size, c.kv_cache_dtype), bw = sc && !u4 ? 5.9e6 : 6.97e6;
+            const double post_a = u8 ? (sc && !u4 ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = u4 ? 0.0105 : u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
             auto t_tile = [&](int64_t w) {  // per tile, with w workgroups running at once
                 return std::max(w <= slots / 2 || slots == 256 ? t1 : t2, (double)w * tile_bytes / bw);
             };
@@ -499,7 +521,7 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
     // A context whose probabilities do not fit half a CU's LDS is cut into splits that send every head's
     // probabilities through HBM and add a merge.  With enough (sequence, kv head) pairs to give every CU a workgroup
     // of its own, one workgroup of eight waves per CU (the same waves per CU, the whole LDS) needs fewer of them.
-    if (u8 && c.block_size >= 32 && c.head_size != 96 && c.head_size <= 128 && most > cap4 && pairs >= 256) {
+    if (u8 && !u4 && c.block_size >= 32 && c.head_size != 96 && c.head_size <= 128 && most > cap4 && pairs >= 256) {
         int32_t cap8 = 0;
         const int32_t s8 = plan(8, 256, &cap8);
         if (s8 < s) {
@@ -569,7 +591,7 @@ void plan_items(pa_ctx* ctx) {
     int32_t n_single_seqs = 0;
     std::vector<Tile> tiles;
     int64_t total_blocks = 0;
-    const bool split_off_decode = decode_u8_shape(ctx);
+    const bool split_off_decode = decode_u8_shape(ctx) || decode_u4_shape(ctx);
     ctx->h_dec.clear();
     ctx->h_dec16.clear();
     // A mixed step over a 16-bit cache with the 16-bit decode kernel available: chunk items and single-token
@@ -803,7 +825,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     const int32_t* table = table_for(ctx, layer);
     const pa_config& c = ctx->cfg;
     const size_t rows = (size_t)ctx->T * c.num_heads;
-    const bool use_decode = decode_u8_step(ctx);
+    const bool use_u4 = decode_u4_step(ctx), use_decode = decode_u8_step(ctx) || use_u4;
     const bool use_mfma = matrix_step(ctx);
     // 16-bit caches, no dense chunk in the step: the single-token sequences go to their own decode kernel.  (Next to
     // dense chunks they stay work items of the matrix kernel: bandwidth-bound and matrix-bound items share the CUs
@@ -813,7 +835,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
                               (ctx->n_single + ctx->n_sparse == ctx->n_items || side_by_side);
     const bool mfma_left = use_mfma && !(use_decode16 && ctx->n_single == ctx->n_items);
     if (static_ws)
-        PA_REQUIRE((use_decode && (int32_t)ctx->h_dec.size() == ctx->B) || (use_decode16 && !mfma_left && !use_decode),
+        PA_REQUIRE((use_decode && !use_u4 && (int32_t)ctx->h_dec.size() == ctx->B) || (use_decode16 && !mfma_left && !use_decode),
                    PA_NOT_IMPLEMENTED,
                    "pa_attention_static serves steps in which every sequence schedules one token, over a u8 cache or a "
                    "16-bit cache of the query's type (block size 16 to 256, a power of two; head size 64, 96, 128 or 256 -- over u8 with 16-token blocks not 256 --, K and V alike; at most 16 heads per kv head)");
@@ -853,7 +875,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.n_seqs = (int32_t)ctx->h_dec.size();
         a.seq_list = ctx->dec_in_order ? nullptr : ctx->dec_list.as<int32_t>();
         ctx->nsplit = a.nsplit;
-        const DecodeWs ws = decode_workspace(ctx, rows, a.nsplit, io->scores != nullptr, static_ws);
+        const DecodeWs ws = decode_workspace(ctx, rows, a.nsplit, io->scores != nullptr && !use_u4, static_ws);
         a.query = static_cast<const uint16_t*>(io->query);
         a.key_cache = static_cast<const uint8_t*>(io->key_cache);
         a.value_cache = static_cast<const uint8_t*>(io->value_cache);
@@ -864,6 +886,18 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.final_ml = ws.final_ml;
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
+        if (use_u4) {
+            if (io->scores) {
+                ctx->logits.reserve((size_t)c.num_heads * ctx->total_scores * sizeof(float));
+                a.logits = ctx->logits.as<float>();
+            }
+            HIP_CHECK(pa::launch_decode_u4(ctx->stream, a, c.query_dtype, ev0, ev1));
+            if (io->scores)
+                HIP_CHECK(pa::launch_scores_from_logits(ctx->stream, ctx->dev, c.num_heads, a.logits, ctx->total_scores,
+                                                        a.final_ml, io->scores, ctx->max_kv));
+            ctx->timed = ctx->profiling;
+            return;
+        }
         // (next to the matrix kernel of a mixed step: on the second stream, like the 16-bit decode kernel below)
         HIP_CHECK(pa::launch_decode_u8(use_mfma && !static_ws ? fork_side() : ctx->stream, a, c.query_dtype, io->scores,
                                        ctx->max_kv, use_mfma ? nullptr : ev0, use_mfma ? nullptr : ev1));
@@ -1229,7 +1263,7 @@ void shape_tables(pa_ctx* ctx, bool shared) {
 size_t table_upload_bytes(pa_ctx* ctx, int32_t count, size_t* id_bytes, bool* with_descs) {
     *id_bytes = std::max<size_t>(((size_t)count * sizeof(int32_t) + 127) & ~(size_t)127, 128);
     size_t total = *id_bytes;
-    *with_descs = decode_u8_step(ctx);
+    *with_descs = decode_u8_step(ctx) || decode_u4_step(ctx);
     if (*with_descs)
         for (int w = 0; w < 2; ++w) {
             ctx->desc_off[w] = total;
@@ -1503,7 +1537,7 @@ int32_t pa_forward(pa_ctx* ctx, int32_t layer, const pa_layer_io* io) {
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
         // a step of single-token sequences that all go to one of the decode kernels: it appends the new rows itself
         const bool fuse = ctx->step_ready &&
-                          ((decode_u8_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B) ||
+                          ((decode_u8_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B) || decode_u4_step(ctx) ||
                            (mfma_shape(ctx) && decode16_shape(ctx) && (int32_t)ctx->h_dec16.size() == ctx->B &&
                             ctx->n_sparse == 0 && ctx->n_single == ctx->n_items));
         if (fuse) check_io(ctx, layer, io, true, false);
