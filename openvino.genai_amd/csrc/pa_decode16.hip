@@ -335,15 +335,25 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
                     uint16_t* o = a.out + ((long)t * Hq + hq) * D + 16 * rr + 4 * g;
                     *reinterpret_cast<uint2*>(o) = make_uint2(pack2<DT>(v[0] * inv_l, v[1] * inv_l), pack2<DT>(v[2] * inv_l, v[3] * inv_l));
                 } else {
-                    *reinterpret_cast<f4*>(a.part_acc + prow * D + 16 * rr + 4 * g) = f4{v[0], v[1], v[2], v[3]};
+                    float* dst = a.part_acc + prow * D + 16 * rr + 4 * g;
+                    if (a.arrived) {
+                        store_partial(dst, v[0], v[1], true);
+                        store_partial(dst + 2, v[2], v[3], true);
+                    } else {
+                        *reinterpret_cast<f4*>(dst) = f4{v[0], v[1], v[2], v[3]};
+                    }
                 }
             }
         }
     }
     if (wv == 0 && g == 0 && n < G) {
-        float* ml = final_out ? a.final_ml + 2 * ((long)t * Hq + hq) : a.part_ml + 2 * prow;
-        ml[0] = M;
-        ml[1] = L;
+        if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * ((long)t * Hq + hq)) = make_float2(M, L);
+        else store_partial(a.part_ml + 2 * prow, M, L, a.arrived != nullptr);
+    }
+    if (a.arrived) {  // (only in launches without scores)
+        static_assert(WAVES * SLOT >= FOLD_MAX_PAIRS * 8, "the fold's table fits the V slots");
+        fold_if_last<D, DT, 64 * WAVES>(a, t, hkv, (long)(blockIdx.x / nsplit), reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_ml));
+        return;
     }
 
     // ---- scores: the factors were formed in place of the block maxima before the merge --------------

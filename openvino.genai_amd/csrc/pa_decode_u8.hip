@@ -583,14 +583,19 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 *reinterpret_cast<uint32_t*>(a.out + ((long)t * Hq + hq) * D + d) =
                     (uint32_t)store16<QDT>(o0 * inv_l) | ((uint32_t)store16<QDT>(o1 * inv_l) << 16);
             } else {
-                *reinterpret_cast<float2*>(a.part_acc + prow * D + d) = make_float2(o0, o1);
+                store_partial(a.part_acc + prow * D + d, o0, o1, a.arrived != nullptr);
             }
             if (d == 0) {  // maxima stay in the log2 domain within this kernel family
-                float* ml = final_out ? a.final_ml + 2 * ((long)t * Hq + hq) : a.part_ml + 2 * prow;
-                ml[0] = M;
-                ml[1] = L;
+                if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * ((long)t * Hq + hq)) = make_float2(M, L);
+                else store_partial(a.part_ml + 2 * prow, M, L, a.arrived != nullptr);
             }
         }
+    }
+
+    if (a.arrived) {  // (only in launches without scores of this kernel's own)
+        static_assert(WAVES * SLOT >= FOLD_MAX_PAIRS * 8, "the fold's table fits the staging area");
+        fold_if_last<D, QDT, NT>(a, t, hkv, (long)blockIdx.z * Hkv + hkv, reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_mlz));
+        return;
     }
 
     // ---- scores: the factors were formed in place of the block maxima during the merge ---------------
@@ -858,7 +863,7 @@ static hipError_t launch_decode_typed(hipStream_t s, const DecodeArgs& a_in, flo
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(kern, dim3((unsigned)a.nsplit, (unsigned)a.sh.Hkv, (unsigned)a.n_seqs), dim3(64 * WAVES), lds, s, a);
     if (ev1) (void)hipEventRecord(ev1, s);
-    if constexpr (U4) return a.nsplit > 1 ? launch_decode_merge(s, a, QDT) : hipGetLastError();  // (scores: from the logits, by the caller)
+    if constexpr (U4) return a.nsplit > 1 && !a.arrived ? launch_decode_merge(s, a, QDT) : hipGetLastError();  // (scores: from the logits, by the caller)
     return launch_decode_post(s, a, QDT, scores, max_kv_len);
 }
 
@@ -926,7 +931,7 @@ hipError_t launch_decode_post(hipStream_t s, const DecodeArgs& a, int q_dtype, f
 #undef PA_POST
     }
     hipError_t e;
-    if (a.nsplit > 1 && (e = launch_decode_merge(s, a, q_dtype)) != hipSuccess) return e;
+    if (a.nsplit > 1 && !a.arrived && (e = launch_decode_merge(s, a, q_dtype)) != hipSuccess) return e;
     return scores ? launch_decode_scores(s, a, scores, max_kv_len) : hipSuccess;
 }
 

@@ -168,6 +168,7 @@ struct pa_ctx {
     DevBuf dec16_list;
     std::vector<int32_t> h_multi;     // sequences that schedule more than one token
     DevBuf multi_list;
+    DevBuf arrived;    // decode launches that fold their own splits: per (listed sequence, kv head) a count, zero between launches
     DevBuf tile_max;   // per (head, 32-token tile) maxima of single-token sequences handled by the matrix kernel
     bool dec_in_order = false, dec16_in_order = false;  // the lists hold 0 .. B-1 in order: every sequence, none moved
     bool stash_ok = false;  // the step's single-token items are short enough to keep their probabilities in LDS
@@ -761,6 +762,12 @@ void plan_items(pa_ctx* ctx) {
         ctx->dec_list.reserve(ctx->h_dec.size() * sizeof(int32_t));
         stage_upload(ctx, ctx->dec_list.p, ctx->h_dec.data(), ctx->h_dec.size() * sizeof(int32_t));
     }
+    // (the launches leave the counters at zero; an enlarged buffer starts there)
+    const size_t counters = std::max(ctx->h_dec.size(), ctx->h_dec16.size()) * (size_t)ctx->cfg.num_kv_heads * sizeof(int32_t);
+    if (counters > ctx->arrived.cap) {
+        ctx->arrived.reserve(counters);
+        HIP_CHECK(hipMemsetAsync(ctx->arrived.p, 0, ctx->arrived.cap, ctx->stream));
+    }
     ctx->tok_nsplit_off = item_bytes;
     if (split_off_decode && !ctx->h_dec.empty())
         for (int w = 0; w < 2; ++w)
@@ -816,6 +823,14 @@ DecodeWs decode_workspace(pa_ctx* ctx, size_t rows, int32_t nsplit, bool want_sc
     w.group_scores = ctx->group_scores.as<_Float16>();
     w.p_split = ctx->p_split.as<_Float16>();
     return w;
+}
+
+// The counters with which a decode launch of several splits folds its own partials (null: it does not).  With scores the
+// merge is part of the score launch, which needs the splits' factors anyway (u4: its scores come from logits and final
+// values).  Contexts cut into more (head, split) pairs than the fold stages keep the merge launch.
+int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, bool u4) {
+    if (a.nsplit <= 1 || (a.want_scores && !u4) || a.G * a.nsplit > pa::FOLD_MAX_PAIRS) return nullptr;
+    return ctx->arrived.as<int32_t>();
 }
 
 // fuse_append: the call is the attention half of pa_forward in a step whose sequences all go to one decode kernel (the
@@ -886,6 +901,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.final_ml = ws.final_ml;
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
+        a.arrived = fold_counters(ctx, a, use_u4);
         if (use_u4) {
             if (io->scores) {
                 ctx->logits.reserve((size_t)c.num_heads * ctx->total_scores * sizeof(float));
@@ -929,6 +945,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.final_ml = ws.final_ml;
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
+        a.arrived = fold_counters(ctx, a, false);
         HIP_CHECK(pa::launch_decode16(side_by_side ? fork_side() : ctx->stream, a, c.query_dtype, io->scores, ctx->max_kv,
                                       mfma_left ? nullptr : ev0, mfma_left ? nullptr : ev1));
         ctx->timed = ctx->profiling;
@@ -1098,6 +1115,7 @@ void pa_destroy(pa_ctx* ctx) {
     ctx->dec16_list.release();
     ctx->multi_list.release();
     ctx->tile_max.release();
+    ctx->arrived.release();
     ctx->trig_lut.release();
     ctx->rot_args.release();
     ctx->div_seqs.release();
