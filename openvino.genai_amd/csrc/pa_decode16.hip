@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
     }
     if (a.arrived) {  // (only in launches without scores)
         static_assert(WAVES * SLOT >= FOLD_MAX_PAIRS * 8, "the fold's table fits the V slots");
-        fold_if_last<D, DT, 64 * WAVES>(a, t, hkv, (long)(blockIdx.x / nsplit), reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_ml));
+        fold_if_last<D, DT, 64 * WAVES>(a, t, hkv, G, (long)(blockIdx.x / nsplit), reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_ml));
         return;
     }
 

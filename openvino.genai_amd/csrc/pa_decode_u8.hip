@@ -136,7 +136,14 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
 // instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 28 us + 4 us
 // of merge, where the shape-generic kernel, one lane to a row, took 149 + 17 us and an append launch of 5; 64 sequences of
 // 4096 tokens in 65 us = 4.6 TB/s.
-template <int D, int QDT, int WAVES, int BS, bool U4>
+// COLS: 0 for sequences of one token each, whose group's heads are the columns of the matrix products.  1 or 2: sequences of a
+// few tokens (the validation step of speculative decoding or prompt lookup), up to 16 * COLS (token, head) columns that share
+// every cache byte; a column sees the positions up to its own token.  The append has run before, there are no scores.  A tile's
+// products are formed from zero and added to the running sums in f32: the matrix kernel, which takes these sequences when
+// scores are wanted, centres the codes for the same reason (the matrix pipe truncates as it accumulates).
+// 16 sequences of 500 - 4000 tokens x 5 new ones (32 / 8 heads, D = 128): 31.7 us in
+// 4 parts (78 MB: 2.5 TB/s, bound by the vector instructions of two softmaxes per tile); the matrix kernel took 51 + 5 us of merge.
+template <int D, int QDT, int WAVES, int BS, bool U4, int COLS>
 // (head size 256: one workgroup per CU, whose waves may then use the accumulation registers as well -- 16 KB blocks,
 // two of them in flight, 64 accumulators and 32 query registers do not fit 256 registers)
 __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kernel(DecodeArgs a) {
@@ -158,7 +165,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     constexpr int SLOT = decode_slot_bytes(D, U4);  // a wave's LDS staging slot: a K block, then a V block
     constexpr int EPL = U4 && D == 64 ? 2 : (D + 63) / 64;  // elements per lane of a new K / V row
     constexpr int ROW_LANES = D / EPL;     // lanes a new row spreads over (D = 96: 48, the others repeat lanes 32 - 47)
-    constexpr int DEPTH = 2;               // blocks a wave keeps in flight
+    constexpr int DEPTH = COLS == 2 && D == 128 ? 1 : 2;  // tiles a wave keeps in flight (the second of 32 columns would spill)
+    constexpr int NG = COLS ? COLS : 1;    // groups of 16 columns
+    constexpr bool FRESH = U4 || COLS > 0; // a tile's products start from zero
+    static_assert(COLS == 0 || !U4, "sequences of several tokens over u4 rows are the shape-generic kernel's");
     // Channel of row m of output tile r (the lane with n = m reads that channel's byte of each of its token rows): a
     // lane's VB consecutive channels, except that with 6 bytes per lane (D = 96) the lanes take four consecutive
     // channels of the first 64 and two of the last 32, so that their reads stay aligned.
@@ -186,7 +196,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // LDS carve-up
     uint8_t* slot = smem + wv * SLOT;                                  // wave-private staging
     float* wave_mlz = reinterpret_cast<float*>(smem + WAVES * SLOT);   // [WAVES][16][4]
-    float* msnap = wave_mlz + WAVES * 16 * 4;                          // [max_tiles][16]
+    float* msnap = wave_mlz + WAVES * 16 * NG * 4;                          // [max_tiles][16]
     _Float16* ptile = reinterpret_cast<_Float16*>(msnap + (a.want_scores ? a.max_tiles * 16 : 0));  // (u4: neither)  // [G][max_tiles*TOK]
     const int pstride = a.max_tiles * TOK;
 
@@ -195,7 +205,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // see the row, and loads and stores of a wave may complete out of order with respect to each other, so the wave
     // waits for its stores explicitly (vmcnt(0)) before it issues the fetch of that block: at once when the block is
     // among its first ones, else (the stores then follow its first fetches) right in front of that fetch.
-    const bool appends = a.fuse_append && te == tile_hi && te > tb && (tile_hi - 1 - tb) % WAVES == wv;
+    const bool appends = COLS == 0 && a.fuse_append && te == tile_hi && te > tb && (tile_hi - 1 - tb) % WAVES == wv;
     const bool append_first = appends && tile_hi - 1 - tb < 4 * WAVES;
     auto append_rows = [&]() __attribute__((always_inline)) {
         const int rl = lane < ROW_LANES ? lane : lane - (64 - ROW_LANES);
@@ -231,8 +241,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     }
 
     // query operand (B of QK): lane (n, g) holds q[head n][32 s + 8 g + e]
-    h8 qreg[KS];
-    float qsum = 0.0f;
+    // column c = 16 gi + n: head c of the group, or (COLS) token c / G of the sequence, head c % G
+    const int R = COLS ? dsc->nq * G : G;
+    h8 qreg[NG][KS];
+    float qsum[NG];
     float qunit = 1.0f;  // u4, bf16 queries: the power of two the head's operands were divided by
     if constexpr (U4) {
         // step 2 i + h of the contraction takes, on lanes of group g, the elements 64 i + 16 g + 8 h + {1, 5, 3, 7, 0, 4, 2, 6}
@@ -263,46 +275,64 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 for (int half = 0; half < 2; ++half) {
                     const int el = first_of[e] + 4 * half;
                     const uint16_t bits = (uint16_t)(w[el >> 1] >> (16 * (el & 1)));
-                    qreg[s][2 * e + half] = QDT == DT_F16 ? __builtin_bit_cast(_Float16, bits)
-                                                          : (_Float16)(bf16_bits_to_float(bits) * inv_unit);
+                    qreg[0][s][2 * e + half] = QDT == DT_F16 ? __builtin_bit_cast(_Float16, bits)
+                                                             : (_Float16)(bf16_bits_to_float(bits) * inv_unit);
                 }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qsum += (float)qreg[s][e];
         }
-        qsum = xor_reduce_sum_g(qsum);
     } else {
-        const uint16_t* qp = a.query + ((long)t * Hq + hkv * G + n) * D + 8 * g;
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) {
+        const int c = 16 * gi + n;
+        const uint16_t* qp = a.query + ((long)(COLS ? t + c / G : t) * Hq + hkv * G + (COLS ? c % G : n)) * D + 8 * g;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            if (n < G) {
+            if (c < R) {
                 const uint4 v = *reinterpret_cast<const uint4*>(qp + 32 * s);
                 if (QDT == DT_F16) {
-                    qreg[s] = __builtin_bit_cast(h8, v);
+                    qreg[gi][s] = __builtin_bit_cast(h8, v);
                 } else {
                     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        qreg[s][2 * e] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] & 0xffff));
-                        qreg[s][2 * e + 1] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] >> 16));
+                        qreg[gi][s][2 * e] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] & 0xffff));
+                        qreg[gi][s][2 * e + 1] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] >> 16));
                     }
                 }
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qreg[s][e] = (_Float16)0.0f;
+                for (int e = 0; e < 8; ++e) qreg[gi][s][e] = (_Float16)0.0f;
             }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qsum += (float)qreg[s][e];
         }
-        qsum = xor_reduce_sum_g(qsum);
+        }
+    }
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+        qsum[gi] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qsum[gi] += (float)qreg[gi][s][e];
+        qsum[gi] = xor_reduce_sum_g(qsum[gi]);
     }
     const float scl24 = st.scale * LOG2E * TWO24 * qunit;  // logits are kept in the log2 domain
-    const float qsum24 = qsum * (1.0f / TWO24);
-
-    float m_run = -INFINITY, l_part = 0.0f, z_part = 0.0f;
-    float vunit = VUNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
-    f4 acc[RT];
+    float qsum24[NG], m_run[NG], l_part[NG], z_part[NG];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) acc[r] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int gi = 0; gi < NG; ++gi) {
+        qsum24[gi] = qsum[gi] * (1.0f / TWO24);
+        m_run[gi] = -INFINITY;
+        l_part[gi] = 0.0f;
+        z_part[gi] = 0.0f;
+    }
+    // the positions every column sees: tiles inside need no mask (COLS: those between the last token's window and the first
+    // token)
+    const int free_lo = COLS && st.sliding_window > 0 ? max(0, kv_len - st.sliding_window) : first;
+    const int free_hi = COLS ? kv_len - dsc->nq + 1 : kv_len;
+    float vunit = VUNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
+    f4 acc[NG][RT];
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi)
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[gi][r] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 
     __syncthreads();  // block-table slice is in LDS
     // one block of this wave's share: the block sits in (kr, vr, tr); once both halves are staged in LDS the same
@@ -315,7 +345,9 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         __builtin_amdgcn_wave_barrier();
 
         // ---- S^T[token][head] = K . Q^T ---------------------------------------------------------
-        f4 sc0 = f4{0.0f, 0.0f, 0.0f, 0.0f}, sc1 = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        f4 sc0[NG], sc1[NG];
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) sc0[gi] = sc1[gi] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             u4v a0, a1;
@@ -333,8 +365,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 bytes_to_half_pairs(w1.x, x0, x1); a1[0] = x0; a1[1] = x1;
                 bytes_to_half_pairs(w1.y, x0, x1); a1[2] = x0; a1[3] = x1;
             }
-            sc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a0), qreg[s], sc0, 0, 0, 0);
-            sc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a1), qreg[s], sc1, 0, 0, 0);
+#pragma unroll
+            for (int gi = 0; gi < NG; ++gi) {
+                sc0[gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a0), qreg[gi][s], sc0[gi], 0, 0, 0);
+                sc1[gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a1), qreg[gi][s], sc1[gi], 0, 0, 0);
+            }
         }
         // headers of this lane's eight tokens: token(u, i) = 16 u + 4 g + i
         float2 hk[8];
@@ -357,32 +392,42 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         // ---- online softmax (log2 domain) -------------------------------------------------------
         // Rows outside [first, kv_len) may hold anything, headers included: blocks that reach beyond either end
         // mask them (EDGE); the blocks in between, nearly all of a long context, skip the tests and selects.
-        h8 pb, pl;
-        float acc_corr = 1.0f;  // u4: what the running sums are multiplied by when the tile's are added
+        h8 pb[NG], pl[NG];
+        float acc_corr[NG];  // FRESH: what the running sums are multiplied by when the tile's are added
         auto softmax = [&](auto edge_tag) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge_tag)::value;
-            float x[8];
-            bool seen[8];
-            float mx = -INFINITY;
+            float x[NG][8], m_new[NG], corr[NG];
+            bool seen[NG][8];
             const int pos0 = tile * TOK;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float raw = (j < 4) ? sc0[j & 3] : sc1[j & 3];
-                const int pos = pos0 + 16 * (j >> 2) + 4 * g + (j & 3);
-                // scale * sc_k * (q . codes - zp_k * sum(q)), the code products still carrying their 2^-24
-                float v = (hk[j].x * scl24) * __builtin_fmaf(-hk[j].y, qsum24, raw);
-                seen[j] = !EDGE || (pos < kv_len && pos >= first);
-                v = seen[j] ? v : -INFINITY;
-                x[j] = v;
-                mx = fmaxf(mx, v);
+            for (int gi = 0; gi < NG; ++gi) {
+                const int vis_hi = COLS ? min(kv_len, kv_len - dsc->nq + (16 * gi + n) / G + 1) : kv_len;
+                const int vis_lo = COLS && st.sliding_window > 0 ? max(0, vis_hi - st.sliding_window) : first;
+                float mx = -INFINITY;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float raw = (j < 4) ? sc0[gi][j & 3] : sc1[gi][j & 3];
+                    const int pos = pos0 + 16 * (j >> 2) + 4 * g + (j & 3);
+                    // scale * sc_k * (q . codes - zp_k * sum(q)), the code products still carrying their 2^-24
+                    float v = (hk[j].x * scl24) * __builtin_fmaf(-hk[j].y, qsum24[gi], raw);
+                    seen[gi][j] = !EDGE || (pos < vis_hi && pos >= vis_lo);
+                    v = seen[gi][j] ? v : -INFINITY;
+                    x[gi][j] = v;
+                    mx = fmaxf(mx, v);
+                }
+                mx = xor_reduce_max_g(mx);
+                const float m_top = fmaxf(m_run[gi], mx);
+                // (COLS: a column may see nothing of a tile, and nothing yet)
+                m_new[gi] = COLS && EDGE && m_top == -INFINITY ? 0.0f : m_top;
+                corr[gi] = __builtin_amdgcn_exp2f(m_run[gi] - m_new[gi]);
+                m_run[gi] = m_top;
             }
-            mx = xor_reduce_max_g(mx);
-            const float m_new = fmaxf(m_run, mx);
-            const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
             float2 hv[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 hv[j] = *reinterpret_cast<const float2*>(slot + ROW * (16 * (j >> 2) + 4 * g + (j & 3)));
+#pragma unroll
+            for (int gi = 0; gi < NG; ++gi) {
             float psum = 0.0f, zsum = 0.0f;
             _Float16 ph[8];
             float wf[8];
@@ -390,51 +435,52 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             if constexpr (U4) {
                 float top = 0.0f;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) top = fmaxf(top, seen[j] ? hv[j].x : 0.0f);
+                for (int j = 0; j < 8; ++j) top = fmaxf(top, seen[gi][j] ? hv[j].x : 0.0f);
                 float unit, inv;
                 power_of_two_below(fmaxf(xor_reduce_max_g(top), vunit), unit, inv);
-                acc_corr = corr * (vunit * inv);
+                acc_corr[gi] = corr[gi] * (vunit * inv);
                 vunit = unit;
                 inv_vunit = inv;
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const float p = __builtin_amdgcn_exp2f(x[j] - m_new);
-                wf[j] = seen[j] ? p * hv[j].x : 0.0f;
+                const float p = __builtin_amdgcn_exp2f(x[gi][j] - m_new[gi]);
+                wf[j] = seen[gi][j] ? p * hv[j].x : 0.0f;
                 psum += p;
-                if constexpr (U4) zsum += seen[j] ? wf[j] * hv[j].y : 0.0f;
+                if constexpr (U4) zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
                 if constexpr (U4) wf[j] *= inv_vunit;  // (a power of two)
-                pb[j] = (_Float16)wf[j];
+                pb[gi][j] = (_Float16)wf[j];
                 ph[j] = (_Float16)p;
             }
             // The weights are pinned in their registers: the compiler may otherwise form the f16 value twice (from the
             // f32 product, and with a mixed-precision multiply), and the two differ by one f16 step at a tie
-            asm volatile("" : "+v"(pb));
+            asm volatile("" : "+v"(pb[gi]));
             // what the rounding to f16 dropped goes through the matrix pipe as a second operand: with 11 bits alone a
             // row that leans on a few tokens with large V values of opposite sign can miss the tolerance
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pl[j] = (_Float16)(wf[j] - (float)pb[j]);
-            asm volatile("" : "+v"(pl));
+            for (int j = 0; j < 8; ++j) pl[gi][j] = (_Float16)(wf[j] - (float)pb[gi][j]);
+            asm volatile("" : "+v"(pl[gi]));
             // the zero-point term must see the weight the matrix product sees, or the rounding error is scaled by the
             // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if constexpr (!U4) zsum += seen[j] ? wf[j] * hv[j].y : 0.0f;
-            l_part = l_part * corr + psum;
-            z_part = z_part * corr + zsum;
-            m_run = m_new;
-            if constexpr (!U4) {
-                if (__any(corr != 1.0f)) {
+                if constexpr (!U4) zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
+            l_part[gi] = l_part[gi] * corr[gi] + psum;
+            z_part[gi] = z_part[gi] * corr[gi] + zsum;
+            if constexpr (COLS > 0) acc_corr[gi] = corr[gi];
+            if constexpr (!FRESH) {
+                if (__any(corr[gi] != 1.0f)) {
 #pragma unroll
-                    for (int r = 0; r < RT; ++r) acc[r] *= corr;
+                    for (int r = 0; r < RT; ++r) acc[gi][r] *= corr[gi];
                 }
             }
-            if constexpr (U4) {
+            if constexpr (COLS > 0) {  // no scores
+            } else if constexpr (U4) {
                 if (a.want_scores && n < G) {
                     float* dst = a.logits + (long)(hkv * G + n) * a.total_scores + dsc->score_off + pos0 + 4 * g;
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        if (seen[j]) dst[16 * (j >> 2) + (j & 3)] = x[j];
+                        if (seen[gi][j]) dst[16 * (j >> 2) + (j & 3)] = x[gi][j];
                 }
             } else if (a.want_scores) {
                 const int lt = tile - tb;
@@ -443,11 +489,12 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
                     *reinterpret_cast<h4*>(dst) = h4{ph[0], ph[1], ph[2], ph[3]};
                     *reinterpret_cast<h4*>(dst + 16) = h4{ph[4], ph[5], ph[6], ph[7]};
-                    if (g == 0) msnap[lt * 16 + n] = m_new;
+                    if (g == 0) msnap[lt * 16 + n] = m_new[gi];
                 }
             }
+            }
         };
-        if (tile * TOK < first || tile * TOK + TOK > kv_len) softmax(std::true_type{});
+        if (tile * TOK < free_lo || tile * TOK + TOK > free_hi) softmax(std::true_type{});
         else softmax(std::false_type{});
 
         // ---- O^T[d][head] += V^T . P^T ----------------------------------------------------------
@@ -491,14 +538,17 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             u4v av;
 #pragma unroll
             for (int p = 0; p < 4; ++p) av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
-            if constexpr (U4) {
-                f4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb, part, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[r][i] = __builtin_fmaf(acc[r][i], acc_corr, part[i]);
-            } else {
-                acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb, acc[r], 0, 0, 0);
-                acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl, acc[r], 0, 0, 0);
+            for (int gi = 0; gi < NG; ++gi) {
+                if constexpr (FRESH) {
+                    f4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl[gi], f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                    part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb[gi], part, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[gi][r][i] = __builtin_fmaf(acc[gi][r][i], acc_corr[gi], part[i]);
+                } else {
+                    acc[gi][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pb[gi], acc[gi][r], 0, 0, 0);
+                    acc[gi][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, av), pl[gi], acc[gi][r], 0, 0, 0);
+                }
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -513,29 +563,33 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // (lanes n < G) in LDS; after one barrier each thread folds the waves for two channels of one head.
     if constexpr (U4) {
 #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[r] *= vunit;
+        for (int r = 0; r < RT; ++r) acc[0][r] *= vunit;
     }
-    const float l_w = xor_reduce_sum_g(l_part);
-    const float z_w = xor_reduce_sum_g(z_part);
+    constexpr int NCOL = 16 * NG;
     __syncthreads();  // staging slots are dead from here on
-    if (g == 0) {
-        wave_mlz[(wv * 16 + n) * 4 + 0] = m_run;
-        wave_mlz[(wv * 16 + n) * 4 + 1] = l_w;
-        wave_mlz[(wv * 16 + n) * 4 + 2] = z_w;
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+        const float l_w = xor_reduce_sum_g(l_part[gi]);
+        const float z_w = xor_reduce_sum_g(z_part[gi]);
+        if (g == 0) {
+            wave_mlz[(wv * NCOL + 16 * gi + n) * 4 + 0] = m_run[gi];
+            wave_mlz[(wv * NCOL + 16 * gi + n) * 4 + 1] = l_w;
+            wave_mlz[(wv * NCOL + 16 * gi + n) * 4 + 2] = z_w;
+        }
     }
     // folds the waves' (m, l, z) of one head: the maximum, each wave's factor, denominator and zero-point sum
     auto fold_head = [&](const int head, float (&f)[WAVES], float& M, float& L, float& Z) __attribute__((always_inline)) {
         M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wave_mlz[(w * 16 + head) * 4]);
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wave_mlz[(w * NCOL + head) * 4]);
         L = 0.0f;
         Z = 0.0f;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            const float mw = wave_mlz[(w * 16 + head) * 4];
+            const float mw = wave_mlz[(w * NCOL + head) * 4];
             f[w] = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
-            L += wave_mlz[(w * 16 + head) * 4 + 1] * f[w];
-            Z += wave_mlz[(w * 16 + head) * 4 + 2] * f[w];
+            L += wave_mlz[(w * NCOL + head) * 4 + 1] * f[w];
+            Z += wave_mlz[(w * NCOL + head) * 4 + 2] * f[w];
         }
     };
     // accumulators: [WAVES][HC][D] floats in the dead staging area, HC heads at a time
@@ -543,17 +597,19 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     static_assert((size_t)WAVES * HC * D * sizeof(float) <= (size_t)WAVES * SLOT, "accumulators of a pass fit the staging area");
     float* red = reinterpret_cast<float*>(smem);
     const bool final_out = nsplit == 1;
-    for (int n0 = 0; n0 < G; n0 += HC) {
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi)
+    for (int n0 = 16 * gi; n0 < min(R, 16 * gi + 16); n0 += HC) {  // (n0, like `head` below: a column)
         if (n0) __syncthreads();
-        if (n >= n0 && n < min(G, n0 + HC)) {
-            float* dst = red + ((wv * HC + n - n0) * D);
+        if (16 * gi + n >= n0 && 16 * gi + n < min(R, n0 + HC)) {
+            float* dst = red + ((wv * HC + 16 * gi + n - n0) * D);
 #pragma unroll
             for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) dst[chan(4 * g + i, r)] = acc[r][i];  // lane (n, g), register i of tile r: row 4 g + i
+                for (int i = 0; i < 4; ++i) dst[chan(4 * g + i, r)] = acc[gi][r][i];  // lane (n, g), register i of tile r: row 4 g + i
         }
         __syncthreads();
-        if (!U4 && n0 == 0 && a.want_scores) {
+        if (!U4 && COLS == 0 && n0 == 0 && a.want_scores) {
             // one factor per (block, head): exp2(snapshot - M) (/ L when this workgroup saw the whole context), written
             // over the snapshot.  Entry e belongs to head e % 16 = this thread's n; the barrier before the score
             // phase publishes the factors
@@ -563,10 +619,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             for (int e = tid; e < max(te - tb, 0) * 16; e += NT)
                 msnap[e] = n < G ? __builtin_amdgcn_exp2f(msnap[e] - M) * fl : 0.0f;
         }
-        const int heads = min(G, n0 + HC) - n0;
+        const int heads = min(R, n0 + HC) - n0;
         for (int idx = tid; idx < heads * (D / 2); idx += NT) {
             const int hl = idx / (D / 2), d = 2 * (idx % (D / 2));
-            const int head = n0 + hl, hq = hkv * G + head;
+            const int head = n0 + hl;
+            const long orow = COLS ? (long)(t + head / G) * Hq + hkv * G + head % G : (long)t * Hq + hkv * G + head;
             float f[WAVES], M, L, Z;
             fold_head(head, f, M, L, Z);
             float v0 = 0.0f, v1 = 0.0f;
@@ -577,16 +634,16 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 v1 += v.y * f[w];
             }
             const float o0 = v0 * TWO24 - Z, o1 = v1 * TWO24 - Z;
-            const long prow = ((long)t * Hq + hq) * nsplit + split;
+            const long prow = orow * nsplit + split;
             if (final_out) {
                 const float inv_l = L > 0.0f ? 1.0f / L : 0.0f;
-                *reinterpret_cast<uint32_t*>(a.out + ((long)t * Hq + hq) * D + d) =
+                *reinterpret_cast<uint32_t*>(a.out + orow * D + d) =
                     (uint32_t)store16<QDT>(o0 * inv_l) | ((uint32_t)store16<QDT>(o1 * inv_l) << 16);
             } else {
                 store_partial(a.part_acc + prow * D + d, o0, o1, a.arrived != nullptr);
             }
             if (d == 0) {  // maxima stay in the log2 domain within this kernel family
-                if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * ((long)t * Hq + hq)) = make_float2(M, L);
+                if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * orow) = make_float2(M, L);
                 else store_partial(a.part_ml + 2 * prow, M, L, a.arrived != nullptr);
             }
         }
@@ -594,12 +651,12 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
 
     if (a.arrived) {  // (only in launches without scores of this kernel's own)
         static_assert(WAVES * SLOT >= FOLD_MAX_PAIRS * 8, "the fold's table fits the staging area");
-        fold_if_last<D, QDT, NT>(a, t, hkv, (long)blockIdx.z * Hkv + hkv, reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_mlz));
+        fold_if_last<D, QDT, NT>(a, t, hkv, R, (long)blockIdx.z * Hkv + hkv, reinterpret_cast<float2*>(smem), reinterpret_cast<int32_t*>(wave_mlz));
         return;
     }
 
     // ---- scores: the factors were formed in place of the block maxima during the merge ---------------
-    if (U4 || !a.want_scores) return;
+    if (U4 || COLS > 0 || !a.want_scores) return;
     __syncthreads();
     const float* fac = msnap;
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -841,8 +898,8 @@ __global__ __launch_bounds__(256) void pa_decode_post_kernel(DecodeArgs a, float
 }  // namespace
 
 // LDS layout: staging | per-wave (m, l, z) | [scores: block maxima | probabilities] | block-table slice
-size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4) {
-    size_t bytes = (size_t)waves * decode_slot_bytes(D, u4) + waves * 16 * 4 * sizeof(float);
+size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4, int cols) {
+    size_t bytes = (size_t)waves * decode_slot_bytes(D, u4) + waves * 16 * (cols > 1 ? cols : 1) * 4 * sizeof(float);
     if (u4) want_scores = false;  // (u4 keeps logits in global memory instead)
     if (want_scores) bytes += (size_t)max_tiles * 16 * sizeof(float) + (size_t)G * max_tiles * TOK * sizeof(uint16_t);
     bytes = (bytes + 15) & ~(size_t)15;
@@ -851,19 +908,19 @@ size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int wa
     return (bytes + 15) & ~(size_t)15;
 }
 
-template <int D, int QDT, int WAVES, int BS, bool U4 = false>
+template <int D, int QDT, int WAVES, int BS, bool U4 = false, int COLS = 0>
 static hipError_t launch_decode_typed(hipStream_t s, const DecodeArgs& a_in, float* scores, int max_kv_len,
                                       hipEvent_t ev0, hipEvent_t ev1) {
     DecodeArgs a = a_in;
-    const size_t lds = decode_u8_lds_bytes(D, a.G, a.max_tiles, a.want_scores != 0, WAVES, &a.table_off, BS, U4);
-    auto kern = pa_decode_u8_kernel<D, QDT, WAVES, BS, U4>;
+    const size_t lds = decode_u8_lds_bytes(D, a.G, a.max_tiles, a.want_scores != 0, WAVES, &a.table_off, BS, U4, COLS);
+    auto kern = pa_decode_u8_kernel<D, QDT, WAVES, BS, U4, COLS>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     if (a.n_seqs > 65535) return hipErrorInvalidValue;  // grid z
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(kern, dim3((unsigned)a.nsplit, (unsigned)a.sh.Hkv, (unsigned)a.n_seqs), dim3(64 * WAVES), lds, s, a);
     if (ev1) (void)hipEventRecord(ev1, s);
-    if constexpr (U4) return a.nsplit > 1 && !a.arrived ? launch_decode_merge(s, a, QDT) : hipGetLastError();  // (scores: from the logits, by the caller)
+    if constexpr (U4 || COLS > 0) return a.nsplit > 1 && !a.arrived ? launch_decode_merge(s, a, QDT) : hipGetLastError();  // (scores: from the logits, by the caller)
     return launch_decode_post(s, a, QDT, scores, max_kv_len);
 }
 
@@ -939,7 +996,25 @@ hipError_t launch_decode_post(hipStream_t s, const DecodeArgs& a, int q_dtype, f
 // a context is created, keeps that allocation out of the first attention call.
 hipError_t preload_decode_u8() {
     hipFuncAttributes at;
-    return hipFuncGetAttributes(&at, reinterpret_cast<const void*>(pa_decode_u8_kernel<128, DT_F16, 4, 32, false>));
+    return hipFuncGetAttributes(&at, reinterpret_cast<const void*>(pa_decode_u8_kernel<128, DT_F16, 4, 32, false, 0>));
+}
+
+hipError_t launch_decode_few(hipStream_t s, const DecodeArgs& a, int q_dtype, int cols, hipEvent_t ev0, hipEvent_t ev1) {
+    if (a.waves != 4 || a.want_scores || a.fuse_append || a.sh.bs < 16 || a.sh.bs > 256 || (a.sh.bs & (a.sh.bs - 1))) return hipErrorInvalidValue;
+#define PA_FEW(D_, BS_, COLS_)                                                                                          \
+    if (a.sh.D == D_ && (a.sh.bs == 16) == (BS_ == 16) && cols == COLS_)                                                \
+        return q_dtype == DT_F16 ? launch_decode_typed<D_, DT_F16, 4, BS_, false, COLS_>(s, a, nullptr, 0, ev0, ev1)    \
+                                 : launch_decode_typed<D_, DT_BF16, 4, BS_, false, COLS_>(s, a, nullptr, 0, ev0, ev1);
+    PA_FEW(128, 32, 1)
+    PA_FEW(128, 32, 2)
+    PA_FEW(128, 16, 1)
+    PA_FEW(128, 16, 2)
+    PA_FEW(64, 32, 1)
+    PA_FEW(64, 32, 2)
+    PA_FEW(64, 16, 1)
+    PA_FEW(64, 16, 2)
+#undef PA_FEW
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_decode_u4(hipStream_t s, const DecodeArgs& a, int q_dtype, hipEvent_t ev0, hipEvent_t ev1) {

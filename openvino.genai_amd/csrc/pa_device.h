@@ -237,7 +237,8 @@ struct DecodeDesc {
     int32_t table_off;      // first entry of the sequence's block table
     int32_t score_off;      // first entry of the sequence in `scores`
     int32_t last_id;        // physical id of the block that holds position kv_len - 1
-    int32_t pad[7];
+    int32_t nq;             // tokens the sequence schedules, rows t .. t + nq - 1 (few-token launches; else 1)
+    int32_t pad[6];
     int32_t ids[16];        // physical ids of the split's first 16 blocks (0 beyond te)
 };
 static_assert(sizeof(DecodeDesc) == 128, "one descriptor = 128 bytes");
@@ -302,9 +303,11 @@ __device__ __forceinline__ float2 load_partial(const float* p) {
 // as a launch of its own (kernels 6.7 + 4.1 us), and 2.2 us less on the host; 32 such layers through the Python binding, which the
 // host bounds, 482 -> 386 us; 16 sequences of 64 - 2048 tokens over f16 (D = 64, 22 layers) 373 -> 308 us.
 template <int D, int QDT, int NT>
-__device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, const int hkv, const long counter, float2* lds,
-                                             int32_t* flag) {
+__device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, const int hkv, const int rows, const long counter,
+                                             float2* lds, int32_t* flag) {
     const int tid = threadIdx.x, ns = a.nsplit, G = a.G;
+    // `rows` (token, head) rows of the group: i = head i % G of token t + i / G
+    auto row_of = [&](const int i) __attribute__((always_inline)) { return (long)(t + i / G) * a.sh.Hq + hkv * G + i % G; };
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
@@ -314,14 +317,14 @@ __device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, c
     }
     __syncthreads();
     if (!*flag) return;  // (uniform)
-    const long row0 = (long)t * a.sh.Hq + (long)hkv * G;
-    for (int i = tid; i < G * ns; i += NT) lds[i] = load_partial(a.part_ml + 2 * (row0 * ns + i));
+    for (int i = tid; i < rows * ns; i += NT) lds[i] = load_partial(a.part_ml + 2 * (row_of(i / ns) * ns + i % ns));
     bool staged = false;
-    for (int i0 = 0; i0 < G * (D / 2); i0 += NT) {
-        const bool mine = i0 + tid < G * (D / 2);
+    for (int i0 = 0; i0 < rows * (D / 2); i0 += NT) {
+        const bool mine = i0 + tid < rows * (D / 2);
         const int idx = mine ? i0 + tid : 0;
         const int head = idx / (D / 2), d = 2 * (idx % (D / 2));
-        const float* pa = a.part_acc + (row0 + head) * ns * D + d;
+        const long row = row_of(head);
+        const float* pa = a.part_acc + row * ns * D + d;
         float M = -INFINITY, L = 0.0f, o0 = 0.0f, o1 = 0.0f;
         for (int s0 = 0; s0 < ns; s0 += 8) {
             float2 v[8];  // eight splits' loads in flight (the first round's while the maxima are on their way)
@@ -344,11 +347,11 @@ __device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, c
         }
         if (!mine) continue;
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        *reinterpret_cast<uint32_t*>(a.out + (row0 + head) * D + d) =
+        *reinterpret_cast<uint32_t*>(a.out + row * D + d) =
             (uint32_t)store16<QDT>(o0 * inv) | ((uint32_t)store16<QDT>(o1 * inv) << 16);
         if (d == 0) {
-            a.final_ml[2 * (row0 + head)] = M;
-            a.final_ml[2 * (row0 + head) + 1] = L;
+            a.final_ml[2 * row] = M;
+            a.final_ml[2 * row + 1] = L;
         }
     }
 }
@@ -357,11 +360,14 @@ __device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, c
 __host__ __device__ inline long p_split_offset(long score_offset, int b) { return ((score_offset + 7) & ~7L) + 8L * b; }
 __host__ __device__ inline long p_split_stride(long total_scores, int B) { return total_scores + 8L * B + 8; }
 
-size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4 = false);
+size_t decode_u8_lds_bytes(int D, int G, int max_tiles, bool want_scores, int waves, int32_t* table_off, int block_size, bool u4 = false, int cols = 0);
 // ev0 / ev1 (may be null) are recorded right before and after the main kernel.
 hipError_t launch_decode_u8(hipStream_t s, const DecodeArgs& a, int q_dtype, float* scores, int max_kv_len,
                             hipEvent_t ev0, hipEvent_t ev1);
 
+// The same kernel for sequences of a few tokens each over u8 rows (head sizes 64 and 128, four waves, the append done before,
+// no scores): at most 16 * cols (token, head) rows per kv head, cols = 1 or 2.
+hipError_t launch_decode_few(hipStream_t s, const DecodeArgs& a, int q_dtype, int cols, hipEvent_t ev0, hipEvent_t ev1);
 // The same kernel over u4 rows (head sizes 64, 128 and -- 32-token blocks and up -- 256; four waves); with scores it leaves
 // logits and final (max, denominator) pairs for `launch_scores_from_logits`.
 hipError_t launch_decode_u4(hipStream_t s, const DecodeArgs& a, int q_dtype, hipEvent_t ev0, hipEvent_t ev1);

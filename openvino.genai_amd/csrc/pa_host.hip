@@ -191,6 +191,11 @@ struct pa_ctx {
     // per-(sequence, split) descriptors of both plans
     struct DecPlan { int32_t nsplit = 1, max_tiles = 1, waves = 4; } dec_plan[2];
     size_t desc_off[2] = {0, 0};       // byte offsets of the two descriptor arrays in a table's buffer
+    std::vector<int32_t> h_few;  // every sequence of a step of few-token sequences, longest context first (else empty)
+    DecPlan few_plan;
+    int32_t few_cols = 1;        // 16-column groups of the decode kernel's few-token variant
+    size_t few_off = 0;          // its descriptors within a table's buffer
+    std::vector<char> table_few; // per table: whether they are in there
     // the step's host arrays (packed metadata, work items, lists, block tables with their descriptors) pass through
     // this pinned area on their way to the device: pieces are handed out front to back, their copies are queued and not
     // waited for, and pa_step_begin starts over at the front once it has waited for the stream
@@ -302,19 +307,22 @@ void check_io(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool need_kv, b
                            "query/out must start at a multiple of 16 bytes, scores at a multiple of 4");
 }
 
-// Descriptors of the u8 decode kernel's workgroups for one block table (host ids), both plans, into the staging copy
+bool decode_u8_step(const pa_ctx* ctx);
+bool decode_u4_step(const pa_ctx* ctx);
+
+// Descriptors of the u8 decode kernel's workgroups for one block table (host ids), both plans (and those of a step of
+// few-token sequences), into the staging copy
 // of the table's buffer.
 void fill_decode_descs(const pa_ctx* ctx, const int32_t* ids, uint8_t* stage) {
     const int32_t sw = ctx->sliding_window;
     std::vector<int32_t> soff(ctx->B + 1, 0);
     for (int32_t b = 0; b < ctx->B; ++b) soff[b + 1] = soff[b] + ctx->h_past[b] + (ctx->h_sb[b + 1] - ctx->h_sb[b]);
-    for (int w = 0; w < 2; ++w) {
-        const int32_t nsplit = ctx->dec_plan[w].nsplit;
-        pa::DecodeDesc* out = reinterpret_cast<pa::DecodeDesc*>(stage + ctx->desc_off[w]);
-        for (size_t i = 0; i < ctx->h_dec.size(); ++i) {
-            const int32_t b = ctx->h_dec[i];
-            const int32_t kv_len = ctx->h_past[b] + 1;
-            const int32_t first = sw > 0 ? std::max(0, kv_len - sw) : 0;
+    auto fill = [&](const std::vector<int32_t>& seqs, const int32_t nsplit, pa::DecodeDesc* out) {
+        for (size_t i = 0; i < seqs.size(); ++i) {
+            const int32_t b = seqs[i];
+            const int32_t nq = ctx->h_sb[b + 1] - ctx->h_sb[b];
+            const int32_t kv_len = ctx->h_past[b] + nq;
+            const int32_t first = sw > 0 ? std::max(0, ctx->h_past[b] + 1 - sw) : 0;
             const int32_t lo = first / 32, hi = (kv_len + 31) / 32;
             const int32_t per = (hi - lo + nsplit - 1) / nsplit;
             const int32_t* tab = ids + ctx->h_bib[b];
@@ -327,6 +335,7 @@ void fill_decode_descs(const pa_ctx* ctx, const int32_t* ids, uint8_t* stage) {
                 std::memset(d.pad, 0, sizeof(d.pad));
                 d.b = b;
                 d.t = ctx->h_sb[b];
+                d.nq = nq;
                 d.kv_len = kv_len;
                 d.first = first;
                 d.tb = lo + s * per;
@@ -338,7 +347,11 @@ void fill_decode_descs(const pa_ctx* ctx, const int32_t* ids, uint8_t* stage) {
                     d.ids[j] = bpt * d.tb + j < bpt * d.te ? tab[std::min((bpt * d.tb + j) >> sub_shift, last_block)] : 0;
             }
         }
-    }
+    };
+    if (decode_u8_step(ctx) || decode_u4_step(ctx))
+        for (int w = 0; w < 2; ++w)
+            fill(ctx->h_dec, ctx->dec_plan[w].nsplit, reinterpret_cast<pa::DecodeDesc*>(stage + ctx->desc_off[w]));
+    if (!ctx->h_few.empty()) fill(ctx->h_few, ctx->few_plan.nsplit, reinterpret_cast<pa::DecodeDesc*>(stage + ctx->few_off));
 }
 
 void do_kv_append(pa_ctx* ctx, int32_t layer, const pa_layer_io* io) {
@@ -421,12 +434,13 @@ bool decode_u4_step(const pa_ctx* ctx) {
 void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, int32_t* max_tiles_out,
                     const std::vector<int32_t>* seqs = nullptr, int32_t* waves_out = nullptr) {
     const pa_config& c = ctx->cfg;
+    const bool few = seqs == &ctx->h_few;
     const int32_t G = c.num_heads / c.num_kv_heads;
     int32_t most = 1;
     int64_t all_tiles = 0;
     for (int32_t b : seqs ? *seqs : ctx->h_dec) {
-        const int32_t kv = ctx->h_past[b] + 1;
-        const int32_t first = ctx->sliding_window > 0 ? std::max(0, kv - ctx->sliding_window) : 0;
+        const int32_t kv = ctx->h_past[b] + ctx->h_sb[b + 1] - ctx->h_sb[b];
+        const int32_t first = ctx->sliding_window > 0 ? std::max(0, ctx->h_past[b] + 1 - ctx->sliding_window) : 0;
         most = std::max(most, (kv + 31) / 32 - first / 32);
         all_tiles += (kv + 31) / 32 - first / 32;
     }
@@ -444,7 +458,7 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
         const size_t budget = (size_t)(160 * 1024 / (slots / 256));
         auto fits = [&](int32_t tiles) { return (lds_of(tiles) + 1279) / 1280 * 1280 <= budget; };
         int32_t cap = most;
-        if (u4) {  // (no probabilities in LDS; the table slice of a workgroup stays within 64 KB)
+        if (u4 || few) {  // (no probabilities in LDS; the table slice of a workgroup stays within 64 KB)
             cap = std::min<int32_t>(most, 8192);
         } else if (want_scores) {
             cap = std::min<int32_t>(most, (int32_t)(budget / (64 * G)));
@@ -470,10 +484,14 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             // 0.49 us per tile -- vector instructions, whatever the bytes -- and 0.0105 us per further workgroup; the counts
             // these give are within 5 % of the best forced one, 14 % for 128 sequences of 128 - 8000 tokens.  With the u8
             // figures 32 sequences of 256 - 4096 tokens were cut in 2 instead of 4: 49.3 against 41.9 us per layer)
-            const double t2 = u4 ? 0.49 * dscale : (u8 ? (sc ? 0.525 : 0.468) : (sc ? 1.104 : 1.064)) * dscale;
-            const double t1 = slots == 256 ? t2 / 2 : u4 ? 0.33 * dscale : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
+            // (few-token sequences, counts of 1 - 24 forced over batches of 1 - 64 sequences: the partial rows of up to 32 columns
+            // make a further workgroup as dear as three of the single-token kernel, and a second round of them never
+            // paid: 16 sequences of 500 - 4000 tokens x 5 in 1 / 2 / 3 / 4 / 5 / 8 parts 61.0 / 47.4 / 48.2 / 41.7 / 51.5 /
+            // 55.0 us per layer, 64 of 4096 x 4 in 1 / 2 / 3 parts 110 / 127 / 142)
+            const double t2 = few ? 0.40 * dscale : u4 ? 0.49 * dscale : (u8 ? (sc ? 0.525 : 0.468) : (sc ? 1.104 : 1.064)) * dscale;
+            const double t1 = slots == 256 ? t2 / 2 : few ? 0.38 * dscale : u4 ? 0.33 * dscale : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
             const double tile_bytes = 2.0 * 32 * pa::row_bytes(c.head_size, c.kv_cache_dtype), bw = sc && !u4 ? 5.9e6 : 6.97e6;
-            const double post_a = u8 ? (sc && !u4 ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = u4 ? 0.0105 : u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
+            const double post_a = u8 ? (sc && !u4 ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = few ? 0.02 : u4 ? 0.0105 : u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
             auto t_tile = [&](int64_t w) {  // per tile, with w workgroups running at once
                 return std::max(w <= slots / 2 || slots == 256 ? t1 : t2, (double)w * tile_bytes / bw);
             };
@@ -486,7 +504,7 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             double best_t = 0.0;
             for (int32_t n = 1; n <= std::min(most, 64); ++n) {
                 const int32_t per = (most + n - 1) / n;
-                if (per > cap) continue;
+                if (per > cap || (few && n > 1 && pairs * n > slots && best_n > 0)) continue;
                 const int64_t w = pairs * n, w_run = std::max<int64_t>(1, std::llround((double)w * fill));
                 const int64_t full = w_run / slots, rem = w_run % slots;
                 // (a cut that fills its rounds exactly is preferred over one that does not at equal estimates: the
@@ -728,6 +746,20 @@ void plan_items(pa_ctx* ctx) {
         ctx->dec_in_order = identity(ctx->h_dec);
         ctx->dec16_in_order = identity(ctx->h_dec16);
     }
+    // Steps whose sequences schedule a few tokens each (the validation step of speculative decoding): with at most 32 (token,
+    // head) rows per kv head they are the decode kernel's work, not the matrix kernel's, whose workgroups hold 128 rows and
+    // all widen codes for the one wave that has any.  Taken by calls without scores; the items above serve the others.
+    ctx->h_few.clear();
+    if (T > B && B <= 65535 && decode_u8_shape(ctx) && (ctx->cfg.head_size == 64 || ctx->cfg.head_size == 128) && ctx->n_sparse == 0) {
+        int32_t rows = 0;
+        for (int32_t b = 0; b < B; ++b) rows = std::max(rows, std::min(sb[b + 1] - sb[b], 33) * G);
+        if (rows <= 32) {
+            for (int32_t b = 0; b < B; ++b) ctx->h_few.push_back(b);
+            std::stable_sort(ctx->h_few.begin(), ctx->h_few.end(), [&](int32_t x, int32_t y) { return past[x] > past[y]; });
+            ctx->few_cols = rows <= 16 ? 1 : 2;
+            plan_decode_u8(ctx, false, &ctx->few_plan.nsplit, &ctx->few_plan.max_tiles, &ctx->h_few);
+        }
+    }
     ctx->x_keep_words = 1 + longest_sparse;  // entries of a work item's block list
     ctx->n_items = (int32_t)items.size();
     ctx->max_split = max_split;
@@ -763,7 +795,7 @@ void plan_items(pa_ctx* ctx) {
         stage_upload(ctx, ctx->dec_list.p, ctx->h_dec.data(), ctx->h_dec.size() * sizeof(int32_t));
     }
     // (the launches leave the counters at zero; an enlarged buffer starts there)
-    const size_t counters = std::max(ctx->h_dec.size(), ctx->h_dec16.size()) * (size_t)ctx->cfg.num_kv_heads * sizeof(int32_t);
+    const size_t counters = std::max({ctx->h_dec.size(), ctx->h_dec16.size(), ctx->h_few.size()}) * (size_t)ctx->cfg.num_kv_heads * sizeof(int32_t);
     if (counters > ctx->arrived.cap) {
         ctx->arrived.reserve(counters);
         HIP_CHECK(hipMemsetAsync(ctx->arrived.p, 0, ctx->arrived.cap, ctx->stream));
@@ -872,6 +904,31 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         }
         return ctx->side;
     };
+    if (!ctx->h_few.empty() && !io->scores && !static_ws && ctx->table_few[ctx->shared_table ? 0 : (size_t)layer]) {
+        pa::DecodeArgs a{};
+        a.st = ctx->dev;
+        a.sh = shape_of(c);
+        a.G = c.num_heads / c.num_kv_heads;
+        a.nsplit = ctx->few_plan.nsplit;
+        a.max_tiles = ctx->few_plan.max_tiles;
+        a.waves = 4;
+        a.descs = reinterpret_cast<const pa::DecodeDesc*>(reinterpret_cast<const uint8_t*>(table) + ctx->few_off);
+        a.n_seqs = (int32_t)ctx->h_few.size();
+        ctx->nsplit = a.nsplit;
+        const DecodeWs ws = decode_workspace(ctx, rows, a.nsplit, false, false);
+        a.query = static_cast<const uint16_t*>(io->query);
+        a.key_cache = static_cast<const uint8_t*>(io->key_cache);
+        a.value_cache = static_cast<const uint8_t*>(io->value_cache);
+        a.block_indices = table;
+        a.out = static_cast<uint16_t*>(io->out);
+        a.part_acc = ws.part_acc;
+        a.part_ml = ws.part_ml;
+        a.final_ml = ws.final_ml;
+        if (a.nsplit > 1 && 16 * ctx->few_cols * a.nsplit <= pa::FOLD_MAX_PAIRS) a.arrived = ctx->arrived.as<int32_t>();
+        HIP_CHECK(pa::launch_decode_few(ctx->stream, a, c.query_dtype, ctx->few_cols, ev0, ev1));
+        ctx->timed = ctx->profiling;
+        return;
+    }
     if (use_decode) {
         pa::DecodeArgs a{};
         a.st = ctx->dev;
@@ -1273,6 +1330,7 @@ void shape_tables(pa_ctx* ctx, bool shared) {
         ctx->table_ptr.assign(n, nullptr);
         ctx->table_count.assign(n, -1);
         ctx->table_bound.assign(n, 0);
+        ctx->table_few.assign(n, 0);
     }
 }
 
@@ -1281,12 +1339,17 @@ void shape_tables(pa_ctx* ctx, bool shared) {
 size_t table_upload_bytes(pa_ctx* ctx, int32_t count, size_t* id_bytes, bool* with_descs) {
     *id_bytes = std::max<size_t>(((size_t)count * sizeof(int32_t) + 127) & ~(size_t)127, 128);
     size_t total = *id_bytes;
-    *with_descs = decode_u8_step(ctx) || decode_u4_step(ctx);
-    if (*with_descs)
+    const bool single = decode_u8_step(ctx) || decode_u4_step(ctx), few = !ctx->h_few.empty();
+    *with_descs = single || few;
+    if (single)
         for (int w = 0; w < 2; ++w) {
             ctx->desc_off[w] = total;
             total += ctx->h_dec.size() * ctx->dec_plan[w].nsplit * sizeof(pa::DecodeDesc);
         }
+    if (few) {
+        ctx->few_off = total;
+        total += ctx->h_few.size() * ctx->few_plan.nsplit * sizeof(pa::DecodeDesc);
+    }
     return total;
 }
 
@@ -1322,6 +1385,7 @@ int32_t pa_set_block_indices(pa_ctx* ctx, int32_t layer, const int32_t* ids, int
         ctx->table_ptr[idx] = ctx->tables[idx].p;
         ctx->table_count[idx] = count;
         ctx->table_bound[idx] = bound;
+        ctx->table_few[idx] = !ctx->h_few.empty();
     });
 }
 
@@ -1370,6 +1434,7 @@ int32_t pa_set_block_indices_layers(pa_ctx* ctx, int32_t first_layer, int32_t nu
             ctx->table_ptr[idx] = dst + (size_t)l * stride;
             ctx->table_count[idx] = count;
             ctx->table_bound[idx] = bound[(size_t)l];
+            ctx->table_few[idx] = !ctx->h_few.empty();
         }
     });
 }

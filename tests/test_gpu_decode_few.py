@@ -1,0 +1,57 @@
+"""Steps whose sequences schedule a few tokens each over a u8 cache (the decode kernel's few-token variant) against the CPU checker,
+with the calls beside them that stay on the matrix kernel: scores wanted, one row too many, block-sparse sequences."""
+import numpy as np
+import pytest
+
+import harness as H
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (query type, block size, Hq, Hkv, D, past lengths, new tokens, window): one and two column groups, tile edges between a
+    # sequence's tokens (a wave whose first tile the early tokens do not see), single tokens beside, one split and several
+    ("f16", 32, 32, 8, 128, [500, 31, 0, 1290], [5, 5, 5, 5], 0), ("bf16", 16, 8, 2, 128, [30, 31, 63, 15, 2200], [4, 3, 2, 4, 1], 0),
+    ("f16", 64, 4, 4, 64, [29, 4000], [32, 17], 0), ("bf16", 256, 16, 1, 64, [255, 700], [2, 1], 40), ("f16", 32, 8, 8, 128, [124], [16], 0),
+    ("f16", 32, 6, 2, 64, [95, 300, 64], [5, 5, 1], 33), ("bf16", 32, 40, 8, 128, [64] * 40, [6] * 40, 0), ("f16", 16, 7, 1, 128, [9000], [4], 0),
+    # 33 rows and more: the matrix kernel's
+    ("f16", 32, 3, 1, 128, [100, 40], [11, 2], 0), ("f16", 32, 4, 2, 96, [70, 40], [3, 2], 0),
+]
+
+
+@pytest.mark.parametrize("qd,bs,Hq,Hkv,D,past,new,sw", CASES)
+def test_decode_few(pkg, qd, bs, Hq, Hkv, D, past, new, sw):
+    import torch
+    dev = torch.device("cuda:0")
+    print(f"case decode few {qd} bs{bs} {Hq}/{Hkv} D{D} past {past[:5]} new {new[:5]} window {sw}", flush=True)
+    case = H.build_case(H.case_from_lens("few", Hq, Hkv, D, bs, qd, "u8", past, new, sw), seed=D + bs + len(past), outliers=True)
+    ref = H.run_case_on_checker(case)
+    got = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
+    assert np.array_equal(got["key_cache"], ref["key_cache"]) and np.array_equal(got["value_cache"], ref["value_cache"])
+    H.assert_close(got["out"], ref["out"], qd)
+    scored = H.run_case_on_gpu(pkg, case, dev, op=got["op"])
+    H.assert_close(scored["out"], ref["out"], qd)
+    H.assert_close(scored["scores"], ref["scores"], "f16", "scores")
+    again = H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=got["op"])
+    assert np.array_equal(again["out16"], got["out16"])
+
+
+def test_decode_few_beside_xattention(pkg):
+    """Thresholds set and taken back between the table's upload and the layer calls: every order gives the step's result."""
+    import torch
+    dev = torch.device("cuda:0")
+    case = H.build_case(H.case_from_lens("few", 8, 2, 128, 32, "f16", "u8", [300, 70], [4, 3]), seed=2)
+    ref = H.run_case_on_checker(case, want_scores=False)
+    op = pkg.PagedAttention(8, 2, 128, 32, "f16", "u8", 1, 0, torch.cuda.current_stream(dev))
+    q, k, v = (H.to_device_16(torch, case[n], "f16", dev) for n in ("query", "key", "value"))
+    for order in ("table", "set table", "set table back", "table set", "table set back"):
+        kc, vc = (torch.from_numpy(case[n]).to(dev) for n in ("key_cache0", "value_cache0"))
+        out = torch.zeros_like(q)
+        op.step_begin(case["past_lens"], case["subsequence_begins"], case["block_indices_begins"], 304, None, 0, case["scale"])
+        for what in order.split():
+            if what == "table":
+                op.set_block_indices(case["block_indices"], case["num_blocks"])
+            else:  # (a threshold of 1 keeps every block)
+                op.set_xattention(np.ones(2, np.float32) if what == "set" else None, 64, 8)
+        op.forward(q, k, v, kc, vc, out)
+        op.synchronize()
+        H.assert_close(out.float().cpu().numpy(), ref["out"], "f16", order)
