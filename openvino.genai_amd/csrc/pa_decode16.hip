@@ -411,8 +411,10 @@ hipError_t launch_decode16_sized(hipStream_t s, const DecodeArgs& a_in, hipEvent
     a.table_off = (int32_t)lds;
     lds += decode16_table_bytes(a.max_tiles, BS);
     auto kern = pa_decode16_kernel<D, DT, BS>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
+    if (lds > 64 * 1024) {  // (what a launch may ask for without)
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(kern, dim3((unsigned)a.n_seqs * a.sh.Hkv * a.nsplit), dim3(256), lds, s, a);
     if (ev1) (void)hipEventRecord(ev1, s);

@@ -914,8 +914,10 @@ static hipError_t launch_decode_typed(hipStream_t s, const DecodeArgs& a_in, flo
     DecodeArgs a = a_in;
     const size_t lds = decode_u8_lds_bytes(D, a.G, a.max_tiles, a.want_scores != 0, WAVES, &a.table_off, BS, U4, COLS);
     auto kern = pa_decode_u8_kernel<D, QDT, WAVES, BS, U4, COLS>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
+    if (lds > 64 * 1024) {  // (what a launch may ask for without)
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
     if (a.n_seqs > 65535) return hipErrorInvalidValue;  // grid z
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(kern, dim3((unsigned)a.nsplit, (unsigned)a.sh.Hkv, (unsigned)a.n_seqs), dim3(64 * WAVES), lds, s, a);

@@ -91,12 +91,11 @@ class PagedAttention:
         self._ck(L.lib().pa_set_block_indices_layers(self._h, int(first_layer), len(arrs), ptrs, n, int(num_blocks)))
 
     def _io(self, query, key, value, key_cache, value_cache, out, scores):
-        io = L.pa_layer_io()
-        ptr = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None
-        io.query, io.key, io.value = ptr(query), ptr(key), ptr(value)
-        io.key_cache, io.value_cache, io.num_blocks = ptr(key_cache), ptr(value_cache), key_cache.shape[0]
-        io.out, io.scores = ptr(out), ptr(scores)
-        return io
+        # (one per layer call, and a small step's time is this host's: built in one go rather than field by field)
+        return L.pa_layer_io(None if query is None else query.data_ptr(), None if key is None else key.data_ptr(),
+                             None if value is None else value.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
+                             key_cache.shape[0], None if out is None else out.data_ptr(),
+                             None if scores is None else scores.data_ptr())
 
     def kv_append(self, key, value, key_cache, value_cache, layer=0):
         io = self._io(None, key, value, key_cache, value_cache, None, None)
@@ -114,7 +113,9 @@ class PagedAttention:
 
     def forward(self, query, key, value, key_cache, value_cache, out, scores=None, layer=0):
         io = self._io(query, key, value, key_cache, value_cache, out, scores)
-        self._ck(L.lib().pa_forward(self._h, layer, C.byref(io)))
+        status = L.lib().pa_forward(self._h, layer, C.byref(io))
+        if status:
+            self._ck(status)
 
     def synchronize(self):
         self._ck(L.lib().pa_synchronize(self._h))
