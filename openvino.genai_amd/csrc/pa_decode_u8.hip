@@ -457,9 +457,16 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             asm volatile("" : "+v"(pb[gi]));
             // what the rounding to f16 dropped goes through the matrix pipe as a second operand: with 11 bits alone a
             // row that leans on a few tokens with large V values of opposite sign can miss the tolerance
+            {
+                const u4v hi = __builtin_bit_cast(u4v, pb[gi]);
+                u4v lo;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pl[gi][j] = (_Float16)(wf[j] - (float)pb[gi][j]);
-            asm volatile("" : "+v"(pl[gi]));
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t h = hi[j];
+                    lo[j] = residual_f16x2(h, wf[2 * j], wf[2 * j + 1]);
+                }
+                pl[gi] = __builtin_bit_cast(h8, lo);
+            }
             // the zero-point term must see the weight the matrix product sees, or the rounding error is scaled by the
             // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
 #pragma unroll

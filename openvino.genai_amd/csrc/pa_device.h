@@ -40,6 +40,17 @@ __device__ inline uint16_t store16(float f) {
     return DT == DT_F16 ? float_to_half_bits(f) : float_to_bf16_bits(f);
 }
 
+#if defined(__HIPCC__)
+// What rounding two f32 values to the f16 pair `hi` dropped, as an f16 pair: f16(w - hi), one mixed-precision multiply-add each
+// (left to itself the compiler takes three instructions: a conversion back, a subtraction and half a packed conversion).
+__device__ __forceinline__ uint32_t residual_f16x2(const uint32_t hi, const float w0, const float w1) {
+    uint32_t lo;
+    asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(w0));
+    asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(w1));
+    return lo;
+}
+#endif
+
 // ---- wave-wide reductions (64 lanes) ----------------------------------------------------------
 __device__ inline float wave_max(float v) {
 #pragma unroll

@@ -203,7 +203,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
     constexpr int RT = D / 16;
     constexpr int CPR = ROWB / 16;         // 16-byte chunks per row
     static_assert(DMA || NCH <= NT * UPT, "one chunk per load unit");
-    constexpr int HDRB = U8 ? 4 * TOK * 4 : 0;  // per buffer: sc_k | zp_k * sc_k | sc_v | zp_v, one f32 per token each
+    constexpr int HDRB = U8 ? 4 * TOK * 4 : 0;  // per buffer: sc_k * scl | zp_k * sc_k | sc_v | zp_v, one f32 per token each
     constexpr float CODE_UNIT = 16777216.0f;    // a code byte read as f16 is code * 2^-24
     // Block t+1 is read while block t+2 is written: two K slots; the V and header slots are indexed modulo four.
     constexpr int OFF_V = NKS * TILEK, OFF_H = NKS * TILEK + NVS * TILEV;
@@ -287,7 +287,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
         }
     }
     const float scl = st.scale * LOG2E;
-    float qsum[2] = {0.0f, 0.0f};  // u8: sum of the row's query elements (for the zero-point term), times scl
+    float qsum[2] = {0.0f, 0.0f};  // u8: sum of the row's query elements (for the zero-point term), times scl / CODE_UNIT
     if (U8) {
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
@@ -298,7 +298,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) part += (float)qh[e];
             }
-            qsum[gi] = xor_sum_g(part) * scl;
+            qsum[gi] = xor_sum_g(part) * (scl / CODE_UNIT);
         }
     }
     // positions every row of this wave can see: blocks inside [free_lo, free_hi] need no mask
@@ -417,7 +417,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
                 if (lt % CPR == 0) {  // the table holds what is left of the zero-points
                     float* hdr = reinterpret_cast<float*>(smem + OFF_H + (j & 3) * HDRB) + lt / CPR;
                     const float sck = __builtin_bit_cast(float, ksb);
-                    hdr[0] = live ? sck : 0.0f;
+                    hdr[0] = live ? sck * scl : 0.0f;
                     hdr[TOK] = live ? (kzf - kc) * sck : 0.0f;
                     hdr[2 * TOK] = live ? __builtin_bit_cast(float, vsb) : 0.0f;
                     hdr[3 * TOK] = live ? vzf - vc : 0.0f;
@@ -517,14 +517,14 @@ void pa_prefill16_kernel(PrefillArgs a) {
         }
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
-            float x[8];
+            float x[8];  // logits (log2 domain) over CODE_UNIT, which the exponent's multiply-add puts back
             float mx = -INFINITY;
             if (U8) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        x[4 * u + i] = fmaf(sc[gi][u][i] * (scl * CODE_UNIT), h_sck[u][i], -h_zpk[u][i] * qsum[gi]);
+                        x[4 * u + i] = fmaf(sc[gi][u][i], h_sck[u][i], -h_zpk[u][i] * qsum[gi]);
             }
             if (MASKED) {
                 const int lim = row_pos[gi];
@@ -537,7 +537,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
             }
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) mx = fmaxf(mx, x[jj]);
-            mx = xor_max_g(mx);
+            mx = xor_max_g(mx) * CODE_UNIT;
             const float m_new = mx > m_run[gi] + 4.0f ? mx : m_run[gi];
             const float m_safe = m_new == -INFINITY ? 0.0f : m_new;
             corr[gi] = __builtin_amdgcn_exp2f(m_run[gi] - m_safe);
@@ -545,7 +545,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
             float psum = 0.0f;
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) {
-                p[jj] = __builtin_amdgcn_exp2f(x[jj] - m_safe);
+                p[jj] = __builtin_amdgcn_exp2f(fmaf(x[jj], CODE_UNIT, -m_safe));
                 psum += p[jj];
             }
             if (U8) {
@@ -565,8 +565,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
                     // a tie the two differ by one f16 step, and the low half would belong to another high half
                     asm volatile("" : "+v"(wb));
                     pb[gi][jj] = wb;
-                    const h2 hi = __builtin_bit_cast(h2, wb);
-                    pl[gi][jj] = __builtin_bit_cast(uint32_t, h2{(_Float16)(w0 - (float)hi[0]), (_Float16)(w1 - (float)hi[1])});
+                    pl[gi][jj] = residual_f16x2(wb, w0, w1);
                     zs = fmaf(w0, h_zpv[jj >> 1][(2 * jj) & 3], zs);
                     zs = fmaf(w1, h_zpv[jj >> 1][(2 * jj + 1) & 3], zs);
                 }
@@ -688,9 +687,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
                     lo = pack2<DT>(p[gi][2 * jj] - __builtin_bit_cast(float, hi << 16),
                                    p[gi][2 * jj + 1] - __builtin_bit_cast(float, hi & 0xffff0000u));
                 } else {
-                    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-                    const h2 h = __builtin_bit_cast(h2, hi);
-                    lo = pack2<DT>(p[gi][2 * jj] - (float)h[0], p[gi][2 * jj + 1] - (float)h[1]);
+                    lo = residual_f16x2(hi, p[gi][2 * jj], p[gi][2 * jj + 1]);
                 }
                 pl[gi][jj] = lo;
                 l_part[gi] = add_pair<DT>(lo, l_part[gi]);
