@@ -191,6 +191,7 @@ struct pa_ctx {
     // per-(sequence, split) descriptors of both plans
     struct DecPlan { int32_t nsplit = 1, max_tiles = 1, waves = 4; } dec_plan[2];
     size_t desc_off[2] = {0, 0};       // byte offsets of the two descriptor arrays in a table's buffer
+    bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams (else one after the other)
     std::vector<int32_t> h_few;  // every sequence of a step of few-token sequences, longest context first (else empty)
     DecPlan few_plan;
     int32_t few_cols = 1;        // 16-column groups of the decode kernel's few-token variant
@@ -628,6 +629,19 @@ void plan_items(pa_ctx* ctx) {
         }
         ctx->split16 = narrow_all && any_single && any_chunk && decode16_shape(ctx) && ctx->cfg.head_size != 256;
     }
+    // Fork and join cost four runtime calls and two waits between queues, 10 - 25 us per layer.  Sixteen mixed steps (4 to 60
+    // single tokens beside 250 - 4096 chunk tokens), us per layer one after the other / side by side -- 16-bit caches: 68 / 72
+    // at 4 GFLOP of chunk work, 141 / 169 at 9, 162 / 190 and (D = 64) 108 / 120 at 25, 211 / 209 at 63, 355 / 349 at 125:
+    // side by side from 45 GFLOP on.  Over u8, whose decode kernel leaves more of a CU to its neighbour, 75 / 75 at 4 GFLOP
+    // beside 55 MB of single tokens' rows, 126 / 119 at 10 beside 187 MB, 274 / 270 at 84: always.
+    {
+        double flops = 0;
+        for (int32_t b = 0; b < B; ++b) {
+            const int32_t q_len = sb[b + 1] - sb[b], kv = past[b] + q_len, vis = sw > 0 ? std::min(kv, sw) : kv;
+            if (q_len > 1) flops += 4.0 * ctx->cfg.num_heads * ctx->cfg.head_size * (double)q_len * std::max(vis - q_len / 2, 1);
+        }
+        ctx->fork_pays = !narrow_all || flops >= 45e9;
+    }
     size_t planned_tiles = 0;
     for (int32_t b = 0; b < B; ++b) {
         const int32_t q_len = sb[b + 1] - sb[b];
@@ -890,8 +904,10 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     hipEvent_t ev0 = ctx->profiling ? ctx->ev0 : nullptr, ev1 = ctx->profiling ? ctx->ev1 : nullptr;
     // fork: what is launched on the returned stream starts behind what the context's stream holds so far and runs
     // next to what follows on it, until the join at the end of this call
+    // (a step whose two kernels are too short for that, see plan_items: the same kernels one after the other)
     bool forked = false;
     auto fork_side = [&]() -> hipStream_t {
+        if (!ctx->fork_pays) return ctx->stream;
         if (!ctx->side) {
             HIP_CHECK(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
             HIP_CHECK(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));
