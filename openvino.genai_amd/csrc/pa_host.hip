@@ -493,6 +493,7 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             const double t1 = slots == 256 ? t2 / 2 : few ? 0.38 * dscale : u4 ? 0.33 * dscale : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
             const double tile_bytes = 2.0 * 32 * pa::row_bytes(c.head_size, c.kv_cache_dtype), bw = sc && !u4 ? 5.9e6 : 6.97e6;
             const double post_a = u8 ? (sc && !u4 ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = few ? 0.02 : u4 ? 0.0105 : u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
+            const double fill = (double)all_tiles / ((double)most * (double)(pairs / c.num_kv_heads));
             auto t_tile = [&](int64_t w) {  // per tile, with w workgroups running at once
                 return std::max(w <= slots / 2 || slots == 256 ? t1 : t2, (double)w * tile_bytes / bw);
             };
@@ -500,7 +501,6 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             // as much shorter than the longest one's as its context is; the launch then behaves like one of fewer
             // workgroups of the longest kind (16 sequences x 64 - 2048 positions, D = 64: 6 parts instead of 3, the step
             // 17.2 -> 16.4 us, 12.5 -> 11.2 us without scores; equal contexts are not touched).
-            const double fill = (double)all_tiles / ((double)most * (double)(pairs / c.num_kv_heads));
             int32_t best_n = 0;
             double best_t = 0.0;
             for (int32_t n = 1; n <= std::min(most, 64); ++n) {
@@ -510,7 +510,11 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
                 const int64_t full = w_run / slots, rem = w_run % slots;
                 // (a cut that fills its rounds exactly is preferred over one that does not at equal estimates: the
                 // estimate of a partly filled round is the less certain one -- 8 x 32769 runs 2 % faster in 8 than in 7)
-                const double t = ((double)full * per * t_tile(slots) + (rem > 0 ? per * t_tile(rem) : 0.0)) *
+                // (launches that fold their own splits: what counts of a short workgroup are its waves' rounds -- nine tiles
+                // take four waves as long as twelve.  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17
+                // 12.6; of 1117 over f16 in 18 parts 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3)
+                const double steps = sc ? per : (per + 3) / 4 * 4;
+                const double t = ((double)full * steps * t_tile(slots) + (rem > 0 ? steps * t_tile(rem) : 0.0)) *
                                      (n > 1 && rem > 0 ? 1.02 : 1.0) +
                                  (n > 1 ? post_a + post_b * (double)w : 0.0);
                 if (best_n == 0 || t < best_t) {
