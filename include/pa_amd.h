@@ -153,7 +153,8 @@ typedef struct pa_layer_io {
  * kernels serve block_size 16, 32, 64, 128 and 256 with head size 64 or 128, K and V alike, over a u8 cache or an f16 /
  * bf16 cache of the query's type; every other combination pa_create accepts (other head sizes, a value head size or
  * value precision of its own, u4 rows, a 16-bit cache of the other 16-bit type, other block sizes) runs on shape-generic
- * kernels, correct but far from the tuned ones' speed.  In a step whose sequences all schedule one token, over a cache
+ * kernels, correct but far from the tuned ones' speed -- except steps of single-token sequences over u4 K and V rows of head
+ * size 64, 128 or (block size 32 up) 256 with at most 16 heads per kv head, which have a tuned kernel too.  In a step whose sequences all schedule one token, over a cache
  * the tuned kernels serve, the append is done by the attention kernel itself (the cache rows are the ones pa_kv_append
  * writes).  Head sizes 96 and 256 (K and V alike, the same caches) run on instantiations of the same kernels with
  * these limits: the matrix kernel keeps to 16 query rows per wave, block-sparse prefill is not offered at 96, the u8 decode
