@@ -49,14 +49,32 @@ __device__ inline u4v nibbles_to_half_pairs(uint32_t w) {
     return u4v{w & 0x000f000fu, (w >> 8) & 0x000f000fu, (w >> 4) & 0x000f000fu, (w >> 12) & 0x000f000fu};
 }
 
-// The largest power of two not above `v` and its reciprocal, both kept within 2^+-100 (zero, subnormal and non-finite
-// values included).
-constexpr float VUNIT_MIN = 0x1p-100f;
-__device__ inline void power_of_two_below(float v, float& unit, float& inv) {
-    const uint32_t e = min(max(__builtin_bit_cast(uint32_t, v) & 0x7f800000u, 27u << 23), 227u << 23);
-    unit = __builtin_bit_cast(float, e);
-    inv = __builtin_bit_cast(float, (254u << 23) - e);
+// A pair of zero-extended codes (f16 subnormals, code * 2^-24) -> (code - c) * 2^-9, exactly, as normal f16 values: one packed
+// multiply-add with `neg_c` = (-c * 2^-9, -c * 2^-9).  The matrix pipe aligns its products by their operands' exponents before it
+// adds and truncates, and a subnormal operand counts there with the smallest normal exponent: a code of c bits gives away 10 - c
+// bits of every sum it is in.
+constexpr float CODE_UNIT_INV = 512.0f;
+__device__ inline uint32_t centred_codes(const uint32_t pair, const uint32_t neg_c) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, pair), h2{(_Float16)32768.0f, (_Float16)32768.0f},
+                                                                  __builtin_bit_cast(h2, neg_c)));
 }
+// u4: c = 8 for every row
+constexpr float U4_CENTRE = 8.0f;
+constexpr uint32_t U4_NEG_CENTRE = 0xa400a400u;  // -2^-6, twice
+
+// The largest power of two not above `v`, kept within 2^-112 .. 2^126 (zero, subnormal and non-finite values included), and 2^UP
+// over it.
+constexpr float UNIT_MIN = 0x1p-112f;
+template <int UP>
+__device__ inline void power_of_two_below(float v, float& unit, float& inv) {
+    const uint32_t e = min(max(__builtin_bit_cast(uint32_t, v) & 0x7f800000u, 15u << 23), 253u << 23);
+    unit = __builtin_bit_cast(float, e);
+    inv = __builtin_bit_cast(float, ((254u + UP) << 23) - e);
+}
+// u4: the weights are f16 pairs below 2^(WEIGHT_UP + 1), so that the pair carries 22 bits of a weight down to 2^-17 of the
+// largest V scale and some of it down to 2^-38
+constexpr int WEIGHT_UP = 14;
 
 // bytes of a wave's staging slot: a tile of K or V, or (u4, whose tiles are smaller) its share of the merge's
 // accumulators, eight heads' rows
@@ -123,19 +141,24 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
 
 // U4: rows of `f32 scale | f32 zero-point | D / 2 bytes` (element 2 i in the high nibble of byte i).  Everything up to the
 // operands is the u8 kernel's; what differs:
-//   * QK: four masks of a 32-bit word give four pairs of f16 subnormals (elements 1,5 | 3,7 | 0,4 | 2,6 of the eight), and
+//   * codes enter the matrix instructions less 8 and as normal values (`centred_codes`): what a subnormal operand costs shows
+//     here, where a code has four bits and the zero-point term is of the size of the code sums.  Over f16 queries (32 / 8
+//     heads, D = 128) plain subnormal codes missed the correctly rounded result in 63 % of the outputs (error 2.98e-4 against
+//     64 bits, 8.2e-4 at 32768 positions), these in 0.2 % (1.995e-4, 1.980e-4: f16's own rounding); the shape-generic kernel's
+//     f32 sums miss it in 1.4 - 2.7 %.  (Rows with every outlier on one side, zero-points near 1 or 14, gain nothing from the 8:
+//     0.10 % against 0.05 % there.)  The four packed instructions per word cost 4 % of the launch.
+//   * QK: four masks of a 32-bit word give four pairs of codes (elements 1,5 | 3,7 | 0,4 | 2,6 of the eight), and
 //     the query operand is permuted to match.  bf16 queries are brought below 2 by a power of two per head before they
-//     become f16 operands, so that nothing of their range is lost.
+//     become f16 operands: elements below 2^-17 of the head's largest are rounded to a multiple of 2^-24 of it, what f32
+//     sums that hold the largest would leave of them too.
 //   * PV: the weights are relative to the largest V scale seen so far (a power of two, `vunit`), so that small or large
 //     values of V neither underflow nor overflow f16; a tile's products are formed from zero and added to the running
-//     sums in f32 with one rounding per tile (the matrix pipe truncates as it accumulates, and with sixteen levels
-//     the zero-point term is of the size of the code sums themselves).
+//     sums in f32 with one rounding per tile (the matrix pipe truncates as it accumulates).
 //   * scores: the scaled logits go to `logits` in f32 and become scores in a kernel of their own, as for the
 //     shape-generic path that serves the other u4 steps; no probability is rounded to 16 bits on the way.
 // Bound by vector instructions (at 186 registers two waves a SIMD; capped at 168 for three the kernel spills and takes 56
-// instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 32 us, the fold of
-// its four splits included, where the shape-generic kernel, one lane to a row, took 149 + 17 us and an append launch of 5; 64 sequences of
-// 4096 tokens in 65 us = 4.6 TB/s.
+// instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 45 us per layer of a
+// step through the Python binding, where the shape-generic kernel, one lane to a row, took 178 (149 + 17 us and an append launch of 5).
 // COLS: 0 for sequences of one token each, whose group's heads are the columns of the matrix products.  1 or 2: sequences of a
 // few tokens (the validation step of speculative decoding or prompt lookup), up to 16 * COLS (token, head) columns that share
 // every cache byte; a column sees the positions up to its own token.  The append has run before, there are no scores.  A tile's
@@ -263,7 +286,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 for (int e = 0; e < 4; ++e)
                     mx = fmaxf(mx, fmaxf(fabsf(__builtin_bit_cast(float, w[e] << 16)), fabsf(__builtin_bit_cast(float, w[e] & 0xffff0000u))));
             }
-            power_of_two_below(xor_reduce_max_g(mx), qunit, inv_unit);
+            power_of_two_below<0>(xor_reduce_max_g(mx), qunit, inv_unit);
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -314,11 +337,12 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             for (int e = 0; e < 8; ++e) qsum[gi] += (float)qreg[gi][s][e];
         qsum[gi] = xor_reduce_sum_g(qsum[gi]);
     }
-    const float scl24 = st.scale * LOG2E * TWO24 * qunit;  // logits are kept in the log2 domain
+    constexpr float CODE_INV = U4 ? CODE_UNIT_INV : TWO24;  // the matrix operands hold the codes (u4: less 8) over this
+    const float scl24 = st.scale * LOG2E * CODE_INV * qunit;  // logits are kept in the log2 domain
     float qsum24[NG], m_run[NG], l_part[NG], z_part[NG];
 #pragma unroll
     for (int gi = 0; gi < NG; ++gi) {
-        qsum24[gi] = qsum[gi] * (1.0f / TWO24);
+        qsum24[gi] = qsum[gi] * (1.0f / CODE_INV);
         m_run[gi] = -INFINITY;
         l_part[gi] = 0.0f;
         z_part[gi] = 0.0f;
@@ -327,7 +351,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // token)
     const int free_lo = COLS && st.sliding_window > 0 ? max(0, kv_len - st.sliding_window) : first;
     const int free_hi = COLS ? kv_len - dsc->nq + 1 : kv_len;
-    float vunit = VUNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
+    float vunit = UNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
     f4 acc[NG][RT];
 #pragma unroll
     for (int gi = 0; gi < NG; ++gi)
@@ -356,6 +380,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 const uint32_t w1 = *reinterpret_cast<const uint32_t*>(slot + ROW * (16 + n) + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
                 a0 = nibbles_to_half_pairs(w0);
                 a1 = nibbles_to_half_pairs(w1);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a0[e] = centred_codes(a0[e], U4_NEG_CENTRE);
+                    a1[e] = centred_codes(a1[e], U4_NEG_CENTRE);
+                }
             } else {
                 const uint2 w0 = *reinterpret_cast<const uint2*>(slot + ROW * n + 8 + 32 * s + 8 * g);
                 const uint2 w1 = *reinterpret_cast<const uint2*>(slot + ROW * (16 + n) + 8 + 32 * s + 8 * g);
@@ -408,8 +437,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 for (int j = 0; j < 8; ++j) {
                     const float raw = (j < 4) ? sc0[gi][j & 3] : sc1[gi][j & 3];
                     const int pos = pos0 + 16 * (j >> 2) + 4 * g + (j & 3);
-                    // scale * sc_k * (q . codes - zp_k * sum(q)), the code products still carrying their 2^-24
-                    float v = (hk[j].x * scl24) * __builtin_fmaf(-hk[j].y, qsum24[gi], raw);
+                    // scale * sc_k * (q . codes - zp_k * sum(q)), the code products still carrying their 2^-24 (2^-9)
+                    float v = (hk[j].x * scl24) * __builtin_fmaf(U4 ? U4_CENTRE - hk[j].y : -hk[j].y, qsum24[gi], raw);
                     seen[gi][j] = !EDGE || (pos < vis_hi && pos >= vis_lo);
                     v = seen[gi][j] ? v : -INFINITY;
                     x[gi][j] = v;
@@ -437,8 +466,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
 #pragma unroll
                 for (int j = 0; j < 8; ++j) top = fmaxf(top, seen[gi][j] ? hv[j].x : 0.0f);
                 float unit, inv;
-                power_of_two_below(fmaxf(xor_reduce_max_g(top), vunit), unit, inv);
-                acc_corr[gi] = corr[gi] * (vunit * inv);
+                power_of_two_below<WEIGHT_UP>(fmaxf(xor_reduce_max_g(top), vunit), unit, inv);
+                acc_corr[gi] = corr[gi] * (vunit * inv * (1.0f / (1 << WEIGHT_UP)));
                 vunit = unit;
                 inv_vunit = inv;
             }
@@ -447,7 +476,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 const float p = __builtin_amdgcn_exp2f(x[gi][j] - m_new[gi]);
                 wf[j] = seen[gi][j] ? p * hv[j].x : 0.0f;
                 psum += p;
-                if constexpr (U4) zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
+                if constexpr (U4) zsum += seen[gi][j] ? wf[j] * (hv[j].y - U4_CENTRE) : 0.0f;
                 if constexpr (U4) wf[j] *= inv_vunit;  // (a power of two)
                 pb[gi][j] = (_Float16)wf[j];
                 ph[j] = (_Float16)p;
@@ -544,7 +573,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             const uint32_t sel = 0x0c000c00u | (uint32_t)byte | ((uint32_t)(4 + byte) << 16);
             u4v av;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
+            for (int p = 0; p < 4; ++p) {
+                av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
+                if constexpr (U4) av[p] = centred_codes(av[p], U4_NEG_CENTRE);
+            }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
                 if constexpr (FRESH) {
@@ -570,7 +602,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // (lanes n < G) in LDS; after one barrier each thread folds the waves for two channels of one head.
     if constexpr (U4) {
 #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[0][r] *= vunit;
+        for (int r = 0; r < RT; ++r) acc[0][r] *= vunit * (1.0f / (1 << WEIGHT_UP));
     }
     constexpr int NCOL = 16 * NG;
     __syncthreads();  // staging slots are dead from here on
@@ -640,7 +672,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 v0 += v.x * f[w];
                 v1 += v.y * f[w];
             }
-            const float o0 = v0 * TWO24 - Z, o1 = v1 * TWO24 - Z;
+            const float o0 = v0 * CODE_INV - Z, o1 = v1 * CODE_INV - Z;
             const long prow = orow * nsplit + split;
             if (final_out) {
                 const float inv_l = L > 0.0f ? 1.0f / L : 0.0f;

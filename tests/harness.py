@@ -126,3 +126,36 @@ def run_case_on_gpu(pkg, case, device, want_scores=True, op=None):
     return dict(key_cache=kc.cpu().numpy(), value_cache=vc.cpu().numpy(),
                 out=out.float().cpu().numpy(), out16=out.view(torch.int16).cpu().numpy().view(np.uint16),
                 scores=scores.cpu().numpy() if want_scores else None, op=op)
+
+
+def quantised_rows_f64(cache, levels, D):
+    """Rows of a u8 (levels 255) or u4 (15) cache as the binary64 values they stand for."""
+    hdr = np.ascontiguousarray(cache[..., :8]).view(np.float32).astype(np.float64)
+    codes = cache[..., 8:]
+    if levels == 15:
+        codes = np.stack([codes >> 4, codes & 15], -1).reshape(cache.shape[:-1] + (D,))
+    return (codes - hdr[..., 1:]) * hdr[..., :1]
+
+
+def attention_f64(query, key_cache, value_cache, levels, past, sb, bib, table, Hq, Hkv, D, bs):
+    """Causal attention in binary64 over quantised caches that hold the step's rows already; query [T, Hq * D] values."""
+    out = np.zeros((int(sb[-1]), Hq, D))
+    q = np.asarray(query, np.float64).reshape(-1, Hkv, Hq // Hkv, D)
+    for b in range(len(past)):
+        n = int(past[b] + sb[b + 1] - sb[b])
+        ids = table[bib[b]:bib[b + 1]]
+        k, v = (quantised_rows_f64(c[ids], levels, D).transpose(1, 0, 2, 3).reshape(Hkv, -1, D)[:, :n] for c in (key_cache, value_cache))
+        for t in range(int(sb[b]), int(sb[b + 1])):
+            m = int(past[b]) + t - int(sb[b]) + 1
+            x = q[t] @ k[:, :m].transpose(0, 2, 1) / np.sqrt(D)
+            p = np.exp(x - x.max(-1, keepdims=True))
+            out[t] = (p @ v[:, :m] / p.sum(-1, keepdims=True)).reshape(Hq, D)
+    return out.reshape(len(out), Hq * D)
+
+
+def misrounded(got, exact, q_dtype):
+    """How many outputs are not the binary64 result rounded to the query's type.  A result whose error before that last rounding
+    is e units in the last place misses with probability e, so the count tells errors apart that the rounding hides."""
+    import torch
+    want = torch.from_numpy(exact).to(_torch_dtype(torch, q_dtype)).float().numpy()
+    return int((np.asarray(got, np.float32) != want).sum())

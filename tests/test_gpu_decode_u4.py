@@ -20,9 +20,11 @@ CASES = [
 ]
 
 
-def _run(pkg, torch, c, qd, D, bs, Hq, Hkv, sw, scores_too, forward=True):
+def _run(pkg, torch, c, qd, D, bs, Hq, Hkv, sw, scores_too, forward=True, slopes=None):
     dev = torch.device("cuda:0")
     op = pkg.PagedAttention(Hq, Hkv, D, bs, qd, "u4", 1, 0, torch.cuda.current_stream(dev))
+    if slopes is not None:
+        op.set_alibi_slopes(slopes)
     q, k, v = (H.to_device_16(torch, c[n], qd, dev) for n in ("q", "k", "v"))
     kc, vc = torch.from_numpy(c["kc"]).to(dev), torch.from_numpy(c["vc"]).to(dev)
     out = torch.zeros_like(q)
@@ -87,3 +89,33 @@ def test_decode_u4_magnitudes(pkg, vmul, qmul):
     # every scaling above is exact: the same roundings at every place, so only a subnormal product could tell them apart
     assert np.abs(got[0] / np.float32(vmul) - plain[0]).max() <= 2.0 ** -8 * np.abs(plain[0]).max()
     assert np.abs(got[1] - plain[1]).max() <= 1e-5 * Hq
+
+
+@pytest.mark.parametrize("qd,D,bs,Hq,Hkv,past,far", [
+    ("f16", 128, 32, 8, 2, [4000, 700], False), ("f16", 64, 16, 16, 4, [2000, 31], False), ("f16", 256, 32, 4, 2, [1500], False),
+    ("bf16", 128, 32, 16, 2, [4000, 700], False), ("f16", 128, 32, 8, 2, [2500], True), ("bf16", 128, 64, 16, 2, [2500], True),
+])
+def test_decode_u4_error_against_64_bits(pkg, qd, D, bs, Hq, Hkv, past, far):
+    """The matrix instructions are no further from the binary64 result than the shape-generic kernel's binary32 arithmetic, which
+    ALiBi slopes too small to move any logit keep the same step on.  far: one V row 2^12 times the others, under a key that no
+    query attends to (its weight is far below 2^-12, the others' weights are that far below the largest V scale)."""
+    import torch
+    print(f"case decode u4 error {qd} D{D} bs{bs} {Hq}/{Hkv} past {past} far {far}", flush=True)
+    c = _case(np.random.default_rng(D + Hq), qd, D, D, "u4", "u4", bs, Hq, Hkv, past, [1] * len(past))
+    if far:
+        at = (c["table"][c["bib"][:-1]], slice(None), 5)  # token 5 of every sequence
+        keys = -3.0 * O.from_bits(c["q"], c["qdt"]).reshape(len(past), Hkv, Hq // Hkv, D).sum(2)
+        lo, hi = keys.min(-1, keepdims=True), keys.max(-1, keepdims=True)
+        codes = np.rint((keys - lo) / (hi - lo) * 15).astype(np.uint8)
+        scale = ((hi - lo) / 15).astype(np.float32)
+        c["kc"][at] = np.concatenate([scale.view(np.uint8), (-lo / scale).astype(np.float32).view(np.uint8),
+                                      codes[..., 0::2] << 4 | codes[..., 1::2]], -1)
+        v = c["vc"][at]
+        v[..., :4] = (np.ascontiguousarray(v[..., :4]).view(np.float32) * np.float32(4096)).view(np.uint8)
+        c["vc"][at] = v
+    out, _, kc, vc = _run(pkg, torch, c, qd, D, bs, Hq, Hkv, 0, False)
+    generic = _run(pkg, torch, c, qd, D, bs, Hq, Hkv, 0, False, slopes=np.full(Hq, 1e-30, np.float32))[0]
+    exact = H.attention_f64(O.from_bits(c["q"], c["qdt"]), kc, vc, 15, c["past"], c["sb"], c["bib"], c["table"], Hq, Hkv, D, bs)
+    ours, theirs = H.misrounded(out, exact, qd), H.misrounded(generic, exact, qd)
+    print(f"misrounded {ours} against {theirs} of {out.size}", flush=True)
+    assert ours <= theirs + 4 * np.sqrt(theirs + 1)  # (counts of rare independent events: four standard deviations)
