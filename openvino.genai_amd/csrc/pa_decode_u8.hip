@@ -59,9 +59,9 @@ __device__ inline uint32_t centred_codes(const uint32_t pair, const uint32_t neg
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, pair), h2{(_Float16)32768.0f, (_Float16)32768.0f},
                                                                   __builtin_bit_cast(h2, neg_c)));
 }
-// u4: c = 8 for every row
-constexpr float U4_CENTRE = 8.0f;
-constexpr uint32_t U4_NEG_CENTRE = 0xa400a400u;  // -2^-6, twice
+// c = 8 for every u4 row, 128 for every u8 row
+constexpr float U4_CENTRE = 8.0f, U8_CENTRE = 128.0f;
+constexpr uint32_t U4_NEG_CENTRE = 0xa400a400u, U8_NEG_CENTRE = 0xb400b400u;  // -2^-6 and -2^-2, twice
 
 // The largest power of two not above `v`, kept within 2^-112 .. 2^126 (zero, subnormal and non-finite values included), and 2^UP
 // over it.
@@ -72,9 +72,10 @@ __device__ inline void power_of_two_below(float v, float& unit, float& inv) {
     unit = __builtin_bit_cast(float, e);
     inv = __builtin_bit_cast(float, ((254u + UP) << 23) - e);
 }
-// u4: the weights are f16 pairs below 2^(WEIGHT_UP + 1), so that the pair carries 22 bits of a weight down to 2^-17 of the
-// largest V scale and some of it down to 2^-38
-constexpr int WEIGHT_UP = 14;
+// The weights are f16 pairs.  Relative to the largest V scale so far (u4 rows, and u8 rows of bf16 values) they are kept below
+// 2^(WEIGHT_UP + 1): the pair carries 22 bits of a weight down to 2^-17 of that scale and some of it down to 2^-38.  u8 rows
+// of f16 values have scales up to 131008 / 255 = 514, which leaves room for 2^WEIGHT_UP_F16 without looking.
+constexpr int WEIGHT_UP = 14, WEIGHT_UP_F16 = 6;
 
 // bytes of a wave's staging slot: a tile of K or V, or (u4, whose tiles are smaller) its share of the merge's
 // accumulators, eight heads' rows
@@ -161,9 +162,11 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
 // step through the Python binding, where the shape-generic kernel, one lane to a row, took 178 (149 + 17 us and an append launch of 5).
 // COLS: 0 for sequences of one token each, whose group's heads are the columns of the matrix products.  1 or 2: sequences of a
 // few tokens (the validation step of speculative decoding or prompt lookup), up to 16 * COLS (token, head) columns that share
-// every cache byte; a column sees the positions up to its own token.  The append has run before, there are no scores.  A tile's
-// products are formed from zero and added to the running sums in f32: the matrix kernel, which takes these sequences when
-// scores are wanted, centres the codes for the same reason (the matrix pipe truncates as it accumulates).
+// every cache byte; a column sees the positions up to its own token.  The append has run before, there are no scores.  Codes are
+// centred (128) and normal, weights scaled up and a tile's products added to the running sums in f32, as over u4 rows: the matrix
+// kernel, which takes these sequences when scores are wanted, centres each row's codes (as subnormals) and is no closer.  Five
+// tokens behind 500 - 4000 over f16 queries miss the correctly rounded result in 0.25 % of the outputs, on the matrix kernel in
+// 3.0 %, with plain subnormal codes in 9.7 %; behind 32000 in 0.3, 7.4 and 24 %.  A centre per row: 0.19 %, but 10 % slower.
 // 16 sequences of 500 - 4000 tokens x 5 new ones (32 / 8 heads, D = 128): 31.7 us in 4 parts (78 MB: 2.5 TB/s, bound by the
 // vector instructions of two softmaxes per tile); the matrix kernel took 51 + 5 us of merge.
 template <int D, int QDT, int WAVES, int BS, bool U4, int COLS>
@@ -190,7 +193,10 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     constexpr int ROW_LANES = D / EPL;     // lanes a new row spreads over (D = 96: 48, the others repeat lanes 32 - 47)
     constexpr int DEPTH = COLS == 2 && D == 128 ? 1 : 2;  // tiles a wave keeps in flight (the second of 32 columns would spill)
     constexpr int NG = COLS ? COLS : 1;    // groups of 16 columns
-    constexpr bool FRESH = U4 || COLS > 0; // a tile's products start from zero
+    constexpr bool FRESH = U4 || COLS > 0; // a tile's products start from zero, codes are centred, weights scaled up
+    constexpr bool UNIT = U4 || (COLS > 0 && QDT == DT_BF16);  // ... relative to the largest V scale so far
+    constexpr float CENTRE = U4 ? U4_CENTRE : U8_CENTRE;
+    constexpr uint32_t NEG_CENTRE = U4 ? U4_NEG_CENTRE : U8_NEG_CENTRE;
     static_assert(COLS == 0 || !U4, "sequences of several tokens over u4 rows are the shape-generic kernel's");
     // Channel of row m of output tile r (the lane with n = m reads that channel's byte of each of its token rows): a
     // lane's VB consecutive channels, except that with 6 bytes per lane (D = 96) the lanes take four consecutive
@@ -337,7 +343,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             for (int e = 0; e < 8; ++e) qsum[gi] += (float)qreg[gi][s][e];
         qsum[gi] = xor_reduce_sum_g(qsum[gi]);
     }
-    constexpr float CODE_INV = U4 ? CODE_UNIT_INV : TWO24;  // the matrix operands hold the codes (u4: less 8) over this
+    constexpr float CODE_INV = FRESH ? CODE_UNIT_INV : TWO24;  // the matrix operands hold the codes over this
     const float scl24 = st.scale * LOG2E * CODE_INV * qunit;  // logits are kept in the log2 domain
     float qsum24[NG], m_run[NG], l_part[NG], z_part[NG];
 #pragma unroll
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // token)
     const int free_lo = COLS && st.sliding_window > 0 ? max(0, kv_len - st.sliding_window) : first;
     const int free_hi = COLS ? kv_len - dsc->nq + 1 : kv_len;
-    float vunit = UNIT_MIN;  // u4: the power of two the weights in the accumulators are relative to
+    float vunit = UNIT_MIN;  // UNIT: the power of two the weights in the accumulators are relative to
     f4 acc[NG][RT];
 #pragma unroll
     for (int gi = 0; gi < NG; ++gi)
@@ -380,11 +386,6 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 const uint32_t w1 = *reinterpret_cast<const uint32_t*>(slot + ROW * (16 + n) + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
                 a0 = nibbles_to_half_pairs(w0);
                 a1 = nibbles_to_half_pairs(w1);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    a0[e] = centred_codes(a0[e], U4_NEG_CENTRE);
-                    a1[e] = centred_codes(a1[e], U4_NEG_CENTRE);
-                }
             } else {
                 const uint2 w0 = *reinterpret_cast<const uint2*>(slot + ROW * n + 8 + 32 * s + 8 * g);
                 const uint2 w1 = *reinterpret_cast<const uint2*>(slot + ROW * (16 + n) + 8 + 32 * s + 8 * g);
@@ -393,6 +394,13 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 bytes_to_half_pairs(w0.y, x0, x1); a0[2] = x0; a0[3] = x1;
                 bytes_to_half_pairs(w1.x, x0, x1); a1[0] = x0; a1[1] = x1;
                 bytes_to_half_pairs(w1.y, x0, x1); a1[2] = x0; a1[3] = x1;
+            }
+            if constexpr (FRESH) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a0[e] = centred_codes(a0[e], NEG_CENTRE);
+                    a1[e] = centred_codes(a1[e], NEG_CENTRE);
+                }
             }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
@@ -422,7 +430,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         // Rows outside [first, kv_len) may hold anything, headers included: blocks that reach beyond either end
         // mask them (EDGE); the blocks in between, nearly all of a long context, skip the tests and selects.
         h8 pb[NG], pl[NG];
-        float acc_corr[NG];  // FRESH: what the running sums are multiplied by when the tile's are added
+        float acc_corr[NG];  // FRESH: what the running sums are multiplied by when the tile's are added (the zero-points' too)
         auto softmax = [&](auto edge_tag) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge_tag)::value;
             float x[NG][8], m_new[NG], corr[NG];
@@ -438,7 +446,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                     const float raw = (j < 4) ? sc0[gi][j & 3] : sc1[gi][j & 3];
                     const int pos = pos0 + 16 * (j >> 2) + 4 * g + (j & 3);
                     // scale * sc_k * (q . codes - zp_k * sum(q)), the code products still carrying their 2^-24 (2^-9)
-                    float v = (hk[j].x * scl24) * __builtin_fmaf(U4 ? U4_CENTRE - hk[j].y : -hk[j].y, qsum24[gi], raw);
+                    float v = (hk[j].x * scl24) * __builtin_fmaf(FRESH ? CENTRE - hk[j].y : -hk[j].y, qsum24[gi], raw);
                     seen[gi][j] = !EDGE || (pos < vis_hi && pos >= vis_lo);
                     v = seen[gi][j] ? v : -INFINITY;
                     x[gi][j] = v;
@@ -455,29 +463,34 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 hv[j] = *reinterpret_cast<const float2*>(slot + ROW * (16 * (j >> 2) + 4 * g + (j & 3)));
+            if constexpr (FRESH) {
+                float inv_vunit = (float)(1 << WEIGHT_UP_F16), sums = 1.0f;
+                if constexpr (UNIT) {
+                    float top = 0.0f, unit;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int pos = pos0 + 16 * (j >> 2) + 4 * g + (j & 3);
+                        top = fmaxf(top, !EDGE || (pos < kv_len && pos >= first) ? hv[j].x : 0.0f);
+                    }
+                    power_of_two_below<WEIGHT_UP>(fmaxf(xor_reduce_max_g(top), vunit), unit, inv_vunit);
+                    sums = vunit * inv_vunit * (1.0f / (1 << WEIGHT_UP));
+                    vunit = unit;
+                }
+#pragma unroll
+                for (int gi = 0; gi < NG; ++gi) acc_corr[gi] = corr[gi] * sums;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) hv[j] = make_float2(hv[j].x * inv_vunit, hv[j].y - CENTRE);  // (by a power of two)
+            }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
             float psum = 0.0f, zsum = 0.0f;
             _Float16 ph[8];
             float wf[8];
-            float inv_vunit = 1.0f;
-            if constexpr (U4) {
-                float top = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) top = fmaxf(top, seen[gi][j] ? hv[j].x : 0.0f);
-                float unit, inv;
-                power_of_two_below<WEIGHT_UP>(fmaxf(xor_reduce_max_g(top), vunit), unit, inv);
-                acc_corr[gi] = corr[gi] * (vunit * inv * (1.0f / (1 << WEIGHT_UP)));
-                vunit = unit;
-                inv_vunit = inv;
-            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float p = __builtin_amdgcn_exp2f(x[gi][j] - m_new[gi]);
                 wf[j] = seen[gi][j] ? p * hv[j].x : 0.0f;
                 psum += p;
-                if constexpr (U4) zsum += seen[gi][j] ? wf[j] * (hv[j].y - U4_CENTRE) : 0.0f;
-                if constexpr (U4) wf[j] *= inv_vunit;  // (a power of two)
                 pb[gi][j] = (_Float16)wf[j];
                 ph[j] = (_Float16)p;
             }
@@ -500,10 +513,9 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if constexpr (!U4) zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
+                zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
             l_part[gi] = l_part[gi] * corr[gi] + psum;
-            z_part[gi] = z_part[gi] * corr[gi] + zsum;
-            if constexpr (COLS > 0) acc_corr[gi] = corr[gi];
+            z_part[gi] = z_part[gi] * (FRESH ? acc_corr[gi] : corr[gi]) + zsum;
             if constexpr (!FRESH) {
                 if (__any(corr[gi] != 1.0f)) {
 #pragma unroll
@@ -575,7 +587,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
-                if constexpr (U4) av[p] = centred_codes(av[p], U4_NEG_CENTRE);
+                if constexpr (FRESH) av[p] = centred_codes(av[p], NEG_CENTRE);
             }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
@@ -600,9 +612,14 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // ---- merge the waves ---------------------------------------------------------------------------
     // Every wave leaves (max, denominator, zero-point sum) per head and its raw accumulators of the group's heads
     // (lanes n < G) in LDS; after one barrier each thread folds the waves for two channels of one head.
-    if constexpr (U4) {
+    if constexpr (FRESH) {
+        const float unit = UNIT ? vunit * (1.0f / (1 << WEIGHT_UP)) : 1.0f / (1 << WEIGHT_UP_F16);
 #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[0][r] *= vunit * (1.0f / (1 << WEIGHT_UP));
+        for (int gi = 0; gi < NG; ++gi) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) acc[gi][r] *= unit;
+            z_part[gi] *= unit;
+        }
     }
     constexpr int NCOL = 16 * NG;
     __syncthreads();  // staging slots are dead from here on

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import harness as H
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +56,37 @@ def test_decode_few_beside_xattention(pkg):
         op.forward(q, k, v, kc, vc, out)
         op.synchronize()
         H.assert_close(out.float().cpu().numpy(), ref["out"], "f16", order)
+
+
+@pytest.mark.parametrize("qd,Hq,Hkv,D,past,new", [("f16", 16, 4, 128, [3000, 700], [5, 4]), ("f16", 16, 4, 128, [4000], [3]),
+                                                  ("f16", 16, 4, 64, [2000, 100], [8, 2]), ("bf16", 32, 8, 128, [3000, 700], [5, 4]),
+                                                  ("bf16", 32, 8, 64, [3000, 700], [4, 3])])
+def test_decode_few_error_against_64_bits(pkg, qd, Hq, Hkv, D, past, new):
+    """No further from the binary64 result than the matrix kernel, which the same step's call with scores runs on."""
+    import torch
+    dev = torch.device("cuda:0")
+    print(f"case decode few error {qd} {Hq}/{Hkv} D{D} past {past} new {new}", flush=True)
+    case = H.build_case(H.case_from_lens("few", Hq, Hkv, D, 32, qd, "u8", past, new), seed=D + Hq, outliers=True)
+    few = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
+    matrix = H.run_case_on_gpu(pkg, case, dev, op=few["op"])
+    exact = H.attention_f64(O.from_bits(case["query"], H.DT[qd]), few["key_cache"], few["value_cache"], 255, case["past_lens"],
+                            case["subsequence_begins"], case["block_indices_begins"], case["block_indices"], Hq, Hkv, D, 32)
+    ours, theirs = H.misrounded(few["out"], exact, qd), H.misrounded(matrix["out"], exact, qd)
+    print(f"misrounded {ours} against {theirs} of {exact.size}", flush=True)
+    assert ours <= theirs + 4 * np.sqrt(theirs + 1)  # (counts of rare independent events: four standard deviations)
+
+
+@pytest.mark.parametrize("vmul", [2.0 ** -60, 2.0 ** 14, 2.0 ** 60])
+def test_decode_few_magnitudes(pkg, vmul):
+    """bf16 values far outside f16's range: the rows' V scales times a power of two give outputs times it."""
+    import torch
+    dev = torch.device("cuda:0")
+    print(f"case decode few magnitudes V x {vmul}", flush=True)
+    case = H.build_case(H.case_from_lens("few", 8, 2, 128, 32, "bf16", "u8", [640, 77], [3, 5]), seed=5)
+    plain = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
+    vc = case["value_cache0"].copy()
+    vc[..., :4] = (np.ascontiguousarray(vc[..., :4]).view(np.float32) * np.float32(vmul)).view(np.uint8)
+    value = O.to_bits(O.from_bits(case["value"], H.DT["bf16"]) * np.float32(vmul), H.DT["bf16"])
+    got = H.run_case_on_gpu(pkg, dict(case, value_cache0=vc, value=value), dev, want_scores=False)
+    # every scaling is exact and each sum goes along with it: only a tile's unit can differ
+    assert np.abs(got["out"] / np.float32(vmul) - plain["out"]).max() <= 2.0 ** -8 * np.abs(plain["out"]).max()
