@@ -196,7 +196,6 @@ struct pa_ctx {
     DecPlan few_plan;
     int32_t few_cols = 1;        // 16-column groups of the decode kernel's few-token variant
     size_t few_off = 0;          // its descriptors within a table's buffer
-    std::vector<char> table_few; // per table: whether they are in there
     // the step's host arrays (packed metadata, work items, lists, block tables with their descriptors) pass through
     // this pinned area on their way to the device: pieces are handed out front to back, their copies are queued and not
     // waited for, and pa_step_begin starts over at the front once it has waited for the stream
@@ -766,9 +765,11 @@ void plan_items(pa_ctx* ctx) {
     }
     // Steps whose sequences schedule a few tokens each (the validation step of speculative decoding): with at most 32 (token,
     // head) rows per kv head they are the decode kernel's work, not the matrix kernel's, whose workgroups hold 128 rows and
-    // all widen codes for the one wave that has any.  Taken by calls without scores; the items above serve the others.
+    // all widen codes for the one wave that has any.  Taken by calls without scores in steps without block-sparse sequences; the
+    // items above serve the others.  (Planned whether or not there are any: thresholds may be set and taken back between the
+    // uploads of a step's tables, whose layout is one for the whole step.)
     ctx->h_few.clear();
-    if (T > B && B <= 65535 && decode_u8_shape(ctx) && (ctx->cfg.head_size == 64 || ctx->cfg.head_size == 128) && ctx->n_sparse == 0) {
+    if (T > B && B <= 65535 && decode_u8_shape(ctx) && (ctx->cfg.head_size == 64 || ctx->cfg.head_size == 128)) {
         int32_t rows = 0;
         for (int32_t b = 0; b < B; ++b) rows = std::max(rows, std::min(sb[b + 1] - sb[b], 33) * G);
         if (rows <= 32) {
@@ -924,7 +925,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         }
         return ctx->side;
     };
-    if (!ctx->h_few.empty() && !io->scores && !static_ws && ctx->table_few[ctx->shared_table ? 0 : (size_t)layer]) {
+    if (!ctx->h_few.empty() && !io->scores && !static_ws && ctx->n_sparse == 0) {
         pa::DecodeArgs a{};
         a.st = ctx->dev;
         a.sh = shape_of(c);
@@ -1350,7 +1351,6 @@ void shape_tables(pa_ctx* ctx, bool shared) {
         ctx->table_ptr.assign(n, nullptr);
         ctx->table_count.assign(n, -1);
         ctx->table_bound.assign(n, 0);
-        ctx->table_few.assign(n, 0);
     }
 }
 
@@ -1405,7 +1405,6 @@ int32_t pa_set_block_indices(pa_ctx* ctx, int32_t layer, const int32_t* ids, int
         ctx->table_ptr[idx] = ctx->tables[idx].p;
         ctx->table_count[idx] = count;
         ctx->table_bound[idx] = bound;
-        ctx->table_few[idx] = !ctx->h_few.empty();
     });
 }
 
@@ -1454,8 +1453,7 @@ int32_t pa_set_block_indices_layers(pa_ctx* ctx, int32_t first_layer, int32_t nu
             ctx->table_ptr[idx] = dst + (size_t)l * stride;
             ctx->table_count[idx] = count;
             ctx->table_bound[idx] = bound[(size_t)l];
-            ctx->table_few[idx] = !ctx->h_few.empty();
-        }
+            }
     });
 }
 

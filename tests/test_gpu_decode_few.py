@@ -58,6 +58,33 @@ def test_decode_few_beside_xattention(pkg):
         H.assert_close(out.float().cpu().numpy(), ref["out"], "f16", order)
 
 
+def test_decode_few_layer_tables_beside_xattention(pkg):
+    """Per-layer tables uploaded in several calls with thresholds set and taken back between them: every layer keeps its own."""
+    import torch
+    dev = torch.device("cuda:0")
+    layers = 6
+    case = H.build_case(H.case_from_lens("few", 8, 2, 128, 32, "f16", "u8", [300, 70, 2000], [4, 3, 2]), seed=9)
+    ref = H.run_case_on_checker(case, want_scores=False)
+    op = pkg.PagedAttention(8, 2, 128, 32, "f16", "u8", layers, 0, torch.cuda.current_stream(dev))
+    q, k, v = (H.to_device_16(torch, case[n], "f16", dev) for n in ("query", "key", "value"))
+    ids, n_blocks = case["block_indices"], case["num_blocks"]
+    rng = np.random.default_rng(0)
+    moved = [rng.permutation(n_blocks) for _ in range(layers)]  # layer l holds block i of the case as block moved[l][i]
+    for order in ((True, False), (False, True)):
+        op.step_begin(case["past_lens"], case["subsequence_begins"], case["block_indices_begins"], 2002, None, 0, case["scale"])
+        for half, on in zip((0, 3), order):
+            op.set_xattention(np.ones(3, np.float32) if on else None, 64, 8)  # (a threshold of 1 keeps every block)
+            op.set_block_indices_per_layer([moved[l][ids] for l in range(half, half + 3)], n_blocks, half)
+        for l in range(layers):
+            kc, vc = (torch.zeros(case[n].shape, dtype=torch.uint8, device=dev) for n in ("key_cache0", "value_cache0"))
+            at = torch.from_numpy(moved[l]).to(dev)
+            kc[at], vc[at] = (torch.from_numpy(case[n]).to(dev) for n in ("key_cache0", "value_cache0"))
+            out = torch.zeros_like(q)
+            op.forward(q, k, v, kc, vc, out, layer=l)
+            op.synchronize()
+            H.assert_close(out.float().cpu().numpy(), ref["out"], "f16", f"layer {l} {order}")
+
+
 @pytest.mark.parametrize("qd,Hq,Hkv,D,past,new", [("f16", 16, 4, 128, [3000, 700], [5, 4]), ("f16", 16, 4, 128, [4000], [3]),
                                                   ("f16", 16, 4, 64, [2000, 100], [8, 2]), ("bf16", 32, 8, 128, [3000, 700], [5, 4]),
                                                   ("bf16", 32, 8, 64, [3000, 700], [4, 3])])
