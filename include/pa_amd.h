@@ -194,6 +194,12 @@ int32_t pa_attention_static(pa_ctx* ctx, int32_t layer, const pa_layer_io* io);
 int32_t pa_synchronize(pa_ctx* ctx);
 /* Number of split-K partitions of the last attention call (diagnostics). */
 int32_t pa_get_num_splits(const pa_ctx* ctx);
+/* Which kernels the last attention call launched (diagnostics): PA_RAN_* bits.  FOLD: a decode launch of several splits
+ * folds their partials itself (else a launch behind it does); SIDE_STREAM: decode and matrix kernel side by side. */
+enum {
+    PA_RAN_GENERIC = 1, PA_RAN_DECODE = 2, PA_RAN_DECODE_FEW = 4, PA_RAN_MATRIX = 8, PA_RAN_FOLD = 16, PA_RAN_SIDE_STREAM = 32
+};
+int32_t pa_get_kernels_run(const pa_ctx* ctx);
 /* Per-op timing.  The reference times the whole infer() with a host timer (ManualTimer, model_runner.hpp:951-954)
  * and has no per-op figure; here, when enabled, the dominant attention kernel of each pa_attention / pa_forward call
  * is bracketed by HIP events on the context's stream.  pa_last_kernel_ms waits for that kernel and returns its

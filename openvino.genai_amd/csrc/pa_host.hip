@@ -191,6 +191,7 @@ struct pa_ctx {
     // per-(sequence, split) descriptors of both plans
     struct DecPlan { int32_t nsplit = 1, max_tiles = 1, waves = 4; } dec_plan[2];
     size_t desc_off[2] = {0, 0};       // byte offsets of the two descriptor arrays in a table's buffer
+    int32_t kernels_run = 0;     // PA_RAN_* of the last attention call
     bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams (else one after the other)
     std::vector<int32_t> h_few;  // every sequence of a step of few-token sequences, longest context first (else empty)
     DecPlan few_plan;
@@ -910,6 +911,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
                    PA_NOT_IMPLEMENTED,
                    "pa_attention_static serves steps in which every sequence schedules one token, over a u8 cache or a "
                    "16-bit cache of the query's type (block size 16 to 256, a power of two; head size 64, 96, 128 or 256 -- over u8 with 16-token blocks not 256 --, K and V alike; at most 16 heads per kv head)");
+    ctx->kernels_run = 0;
     // the timed kernel: the matrix kernel when there is prefill work, else the decode kernel
     hipEvent_t ev0 = ctx->profiling ? ctx->ev0 : nullptr, ev1 = ctx->profiling ? ctx->ev1 : nullptr;
     // fork: what is launched on the returned stream starts behind what the context's stream holds so far and runs
@@ -927,6 +929,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             HIP_CHECK(hipEventRecord(ctx->ev_fork, ctx->stream));
             HIP_CHECK(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
             forked = true;
+            ctx->kernels_run |= PA_RAN_SIDE_STREAM;
         }
         return ctx->side;
     };
@@ -951,6 +954,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.part_ml = ws.part_ml;
         a.final_ml = ws.final_ml;
         if (a.nsplit > 1 && 16 * ctx->few_cols * a.nsplit <= pa::FOLD_MAX_PAIRS) a.arrived = ctx->arrived.as<int32_t>();
+        ctx->kernels_run |= PA_RAN_DECODE_FEW | (a.arrived ? PA_RAN_FOLD : 0);
         HIP_CHECK(pa::launch_decode_few(ctx->stream, a, c.query_dtype, ctx->few_cols, ev0, ev1));
         ctx->timed = ctx->profiling;
         return;
@@ -985,6 +989,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
         a.arrived = fold_counters(ctx, a, use_u4);
+        ctx->kernels_run |= PA_RAN_DECODE | (a.arrived ? PA_RAN_FOLD : 0);
         if (use_u4) {
             if (io->scores) {
                 ctx->logits.reserve((size_t)c.num_heads * ctx->total_scores * sizeof(float));
@@ -1029,11 +1034,13 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
         a.arrived = fold_counters(ctx, a, false);
+        ctx->kernels_run |= PA_RAN_DECODE | (a.arrived ? PA_RAN_FOLD : 0);
         HIP_CHECK(pa::launch_decode16(side_by_side ? fork_side() : ctx->stream, a, c.query_dtype, io->scores, ctx->max_kv,
                                       mfma_left ? nullptr : ev0, mfma_left ? nullptr : ev1));
         ctx->timed = ctx->profiling;
     }
     if (mfma_left) {
+        ctx->kernels_run |= PA_RAN_MATRIX;
         pa::PrefillArgs a{};
         a.skip_single = use_decode16 ? 1 : 0;
         a.st = ctx->dev;
@@ -1135,6 +1142,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         HIP_CHECK(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
     }
     if (use_decode || use_mfma) return;  // (use_decode16 implies use_mfma)
+    ctx->kernels_run = PA_RAN_GENERIC;
     ctx->nsplit = ctx->generic_nsplit;
     ctx->part_acc.reserve(rows * ctx->nsplit * v_head(c) * sizeof(float));
     ctx->part_ml.reserve(rows * ctx->nsplit * 2 * sizeof(float));
@@ -1661,6 +1669,7 @@ int32_t pa_synchronize(pa_ctx* ctx) {
 }
 
 int32_t pa_get_num_splits(const pa_ctx* ctx) { return ctx ? ctx->nsplit : 0; }
+int32_t pa_get_kernels_run(const pa_ctx* ctx) { return ctx ? ctx->kernels_run : 0; }
 
 int32_t pa_set_profiling(pa_ctx* ctx, int32_t enable) {
     if (!ctx) return PA_INVALID_C_PARAM;

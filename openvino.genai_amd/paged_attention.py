@@ -186,6 +186,12 @@ class PagedAttention:
     def num_splits(self):
         return int(L.lib().pa_get_num_splits(self._h))
 
+    @property
+    def kernels_run(self):
+        """Names of the kernels the last attention call launched (diagnostics)."""
+        bits = int(L.lib().pa_get_kernels_run(self._h))
+        return {n for i, n in enumerate(("generic", "decode", "decode_few", "matrix", "fold", "side_stream")) if bits >> i & 1}
+
 
 def pack_step(processed, evicted, skipped_blocks, scheduled, num_blocks, block_size):
     """Integer part of ModelRunner::forward: returns past_lens, subsequence_begins, block_indices_begins, max_context_len."""

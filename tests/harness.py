@@ -128,6 +128,18 @@ def run_case_on_gpu(pkg, case, device, want_scores=True, op=None):
                 scores=scores.cpu().numpy() if want_scores else None, op=op)
 
 
+def spoil_rows_beyond_the_context(c):
+    """All-ones bytes -- NaN headers over u8 and u4 rows -- in every cache row behind a sequence's last token, its own blocks'
+    included and blocks of no sequence."""
+    bs = c["bs"]
+    keep = np.zeros((c["num_blocks"], bs), bool)
+    for b, (past, new) in enumerate(zip(c["past_lens"], c["new_lens"])):
+        pos = np.arange(past + new)
+        keep[c["block_indices"][c["block_indices_begins"][b] + pos // bs], pos % bs] = True
+    for cache in (c["key_cache0"], c["value_cache0"]):
+        cache.transpose(0, 2, 1, 3)[~keep] = 0xFF
+
+
 def quantised_rows_f64(cache, levels, D):
     """Rows of a u8 (levels 255) or u4 (15) cache as the binary64 values they stand for."""
     hdr = np.ascontiguousarray(cache[..., :8]).view(np.float32).astype(np.float64)

@@ -28,8 +28,11 @@ def test_decode_few(pkg, qd, bs, Hq, Hkv, D, past, new, sw):
     ref = H.run_case_on_checker(case)
     got = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
     assert np.array_equal(got["key_cache"], ref["key_cache"]) and np.array_equal(got["value_cache"], ref["value_cache"])
+    few = D in (64, 128) and max(new) * Hq // Hkv <= 32
+    assert got["op"].kernels_run - {"fold"} == ({"decode_few"} if few else {"matrix"} if 1 not in new else {"matrix", "decode", "side_stream"})
     H.assert_close(got["out"], ref["out"], qd)
     scored = H.run_case_on_gpu(pkg, case, dev, op=got["op"])
+    assert "matrix" in scored["op"].kernels_run and "decode_few" not in scored["op"].kernels_run
     H.assert_close(scored["out"], ref["out"], qd)
     H.assert_close(scored["scores"], ref["scores"], "f16", "scores")
     again = H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=got["op"])
@@ -55,6 +58,7 @@ def test_decode_few_beside_xattention(pkg):
                 op.set_xattention(np.ones(2, np.float32) if what == "set" else None, 64, 8)
         op.forward(q, k, v, kc, vc, out)
         op.synchronize()
+        assert op.kernels_run - {"fold"} == ({"matrix"} if order.endswith("set") or order == "set table" else {"decode_few"})
         H.assert_close(out.float().cpu().numpy(), ref["out"], "f16", order)
 
 
@@ -95,12 +99,28 @@ def test_decode_few_error_against_64_bits(pkg, qd, Hq, Hkv, D, past, new):
     print(f"case decode few error {qd} {Hq}/{Hkv} D{D} past {past} new {new}", flush=True)
     case = H.build_case(H.case_from_lens("few", Hq, Hkv, D, 32, qd, "u8", past, new), seed=D + Hq, outliers=True)
     few = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
+    assert few["op"].kernels_run - {"fold"} == {"decode_few"}
     matrix = H.run_case_on_gpu(pkg, case, dev, op=few["op"])
+    assert "matrix" in matrix["op"].kernels_run
     exact = H.attention_f64(O.from_bits(case["query"], H.DT[qd]), few["key_cache"], few["value_cache"], 255, case["past_lens"],
                             case["subsequence_begins"], case["block_indices_begins"], case["block_indices"], Hq, Hkv, D, 32)
     ours, theirs = H.misrounded(few["out"], exact, qd), H.misrounded(matrix["out"], exact, qd)
     print(f"misrounded {ours} against {theirs} of {exact.size}", flush=True)
     assert ours <= theirs + 4 * np.sqrt(theirs + 1)  # (counts of rare independent events: four standard deviations)
+
+
+@pytest.mark.parametrize("qd,D,bs,new", [("f16", 128, 32, [4, 2, 1]), ("bf16", 64, 16, [3, 8, 2])])
+def test_decode_few_ignores_garbage_beyond_the_context(pkg, qd, D, bs, new):
+    """Rows behind a sequence's last token may hold anything, NaN headers included."""
+    import torch
+    past = [40, 90, 2001]
+    print(f"case decode few garbage {qd} D{D} bs{bs}", flush=True)
+    case = H.build_case(H.case_from_lens("few", 8, 2, D, bs, qd, "u8", past, new), seed=6)
+    ref = H.run_case_on_checker(case, want_scores=False)
+    H.spoil_rows_beyond_the_context(case)
+    got = H.run_case_on_gpu(pkg, case, torch.device("cuda:0"), want_scores=False)
+    assert got["op"].kernels_run - {"fold"} == {"decode_few"}
+    H.assert_close(got["out"], ref["out"], qd)
 
 
 @pytest.mark.parametrize("vmul", [2.0 ** -60, 2.0 ** 14, 2.0 ** 60])

@@ -20,6 +20,9 @@ CASES = [
 ]
 
 
+KERNELS = []  # of the last call
+
+
 def _run(pkg, torch, c, qd, D, bs, Hq, Hkv, sw, scores_too, forward=True, slopes=None):
     dev = torch.device("cuda:0")
     op = pkg.PagedAttention(Hq, Hkv, D, bs, qd, "u4", 1, 0, torch.cuda.current_stream(dev))
@@ -37,6 +40,7 @@ def _run(pkg, torch, c, qd, D, bs, Hq, Hkv, sw, scores_too, forward=True, slopes
         op.kv_append(k, v, kc, vc)
         op.attention(q, kc, vc, out, scores)
     op.synchronize()
+    KERNELS[:] = [op.kernels_run - {"fold"}]
     return out.float().cpu().numpy(), scores.cpu().numpy() if scores_too else None, kc.cpu().numpy(), vc.cpu().numpy()
 
 
@@ -57,10 +61,26 @@ def test_decode_u4(pkg, qd, D, bs, Hq, Hkv, past, sw):
     ref = _checked(c, D, bs, Hq, Hkv, sw)
     for scores_too, forward in ((True, True), (False, True), (True, False)):
         got = _run(pkg, torch, c, qd, D, bs, Hq, Hkv, sw, scores_too, forward)
+        assert KERNELS == [{"generic"} if (D, bs) == (256, 16) or D == 96 or Hq > 16 * Hkv else {"decode"}]
         assert np.array_equal(got[2], ref[2]) and np.array_equal(got[3], ref[3]), "cache bytes differ"
         H.assert_close(got[0], ref[0], qd)
         if scores_too:  # (no rounding to 16 bits on the way: sums of at most Hq probabilities in binary32)
             assert np.abs(got[1] - ref[1]).max() <= 1e-5 * Hq
+
+
+@pytest.mark.parametrize("qd,D,bs", [("f16", 128, 32), ("bf16", 64, 16), ("bf16", 256, 64)])
+def test_decode_u4_ignores_garbage_beyond_the_context(pkg, qd, D, bs):
+    """Rows behind a sequence's last token may hold anything, NaN headers included."""
+    import torch
+    print(f"case decode u4 garbage {qd} D{D} bs{bs}", flush=True)
+    c = _case(np.random.default_rng(8), qd, D, D, "u4", "u4", bs, 8, 2, [40, 90, 2001], [1, 1, 1])
+    ref = _checked(c, D, bs, 8, 2, 0)
+    H.spoil_rows_beyond_the_context(dict(bs=bs, num_blocks=c["pool"], past_lens=c["past"], new_lens=c["new"], block_indices=c["table"],
+                                         block_indices_begins=c["bib"], key_cache0=c["kc"], value_cache0=c["vc"]))
+    got = _run(pkg, torch, c, qd, D, bs, 8, 2, 0, True)
+    assert KERNELS == [{"decode"}]
+    H.assert_close(got[0], ref[0], qd)
+    assert np.abs(got[1] - ref[1]).max() <= 1e-5 * 8
 
 
 @pytest.mark.parametrize("vmul,qmul", [(2.0 ** -40, 1.0), (2.0 ** 30, 1.0), (1.0, 2.0 ** 20), (1.0, 2.0 ** -30)])
@@ -114,7 +134,9 @@ def test_decode_u4_error_against_64_bits(pkg, qd, D, bs, Hq, Hkv, past, far):
         v[..., :4] = (np.ascontiguousarray(v[..., :4]).view(np.float32) * np.float32(4096)).view(np.uint8)
         c["vc"][at] = v
     out, _, kc, vc = _run(pkg, torch, c, qd, D, bs, Hq, Hkv, 0, False)
+    assert KERNELS == [{"decode"}]
     generic = _run(pkg, torch, c, qd, D, bs, Hq, Hkv, 0, False, slopes=np.full(Hq, 1e-30, np.float32))[0]
+    assert KERNELS == [{"generic"}]
     exact = H.attention_f64(O.from_bits(c["q"], c["qdt"]), kc, vc, 15, c["past"], c["sb"], c["bib"], c["table"], Hq, Hkv, D, bs)
     ours, theirs = H.misrounded(out, exact, qd), H.misrounded(generic, exact, qd)
     print(f"misrounded {ours} against {theirs} of {out.size}", flush=True)

@@ -43,9 +43,12 @@ def test_mixed_step_equals_separate_steps(pkg, qd, heads, past, new):
         for _ in range(3):  # (later calls of the step next to the tail of earlier ones)
             op.forward(qi, ki, vi, kc, vc, out)
         op.synchronize()
+        ran.append(op.kernels_run - {"fold"})
         return out.float().cpu().numpy()
 
+    ran = []
     together = step(list(range(B)))
+    assert ran == [{"decode", "matrix", "side_stream"} if new[0] >= 800 else {"decode", "matrix"}]
     n0 = int(new[0])
     # outputs of the same arithmetic cut into other ranges: both sides within the tolerance of the exact result
     H.assert_close(together[:n0], step([0]), qd)
