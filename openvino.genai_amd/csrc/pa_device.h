@@ -286,8 +286,22 @@ struct DecodeArgs {
     _Float16* p_split;            // nsplit > 1: [Hq, p_split_stride(total_scores, B)] probabilities relative to the
                                   // split maximum; a sequence's run starts at p_split_offset (16-byte aligned)
 };
-// Most (head, split) pairs of a kv head whose maxima and denominators the folding workgroup stages in LDS (8 KB).
-constexpr int FOLD_MAX_PAIRS = 1024;
+// Whether a decode launch of `nsplit` splits folds its own partials, `rows` (token, head) rows per kv head.  One workgroup folds all
+// rows of a (sequence, kv head): 256 pairs of channels at a time, eight splits' loads in flight, each such trip a latency past the
+// L2s that a merge launch, a wave to a row, does not have in a chain.  us per layer, fold / merge launch, one sequence unless stated:
+//   one pass over the channels: 1 - 4 trips 0.81 - 1.02 of the merge (llama's heads (32 / 8, D = 128), 4000 tokens over u8 in 32
+//   splits 17.9 / 19.6), 7 and 8 trips 0.98 - 1.03 (32 / 4, D = 64, 8000 over f16 in 63: 21.4 / 20.7);
+//   two: 1 trip 0.84 - 0.99, 2 trips 1.00 - 1.07 (28 / 4, D = 128, 4 x 8000 over u4 in 16: 23.3 / 21.8), 7 trips 1.14 - 1.19 (1 x 32768);
+//   four: 1 trip 0.84 - 1.05 (32 / 2, D = 128, 16 x 3000 over u8 in 8: 24.7 / 23.7), 8 trips 1.75 (1 x 8000 in 63: 39.1 / 22.3);
+//   eight: 1 trip 1.20 - 1.25, 8 trips 2.5 (16 / 1, D = 256, 1 x 8000 in 63: 63.2 / 25.5);
+//   few-token launches alike: five passes, 3 trips (32 / 8, D = 128, five tokens behind 8000) 37.9 / 29.4.
+__host__ __device__ constexpr bool fold_pays(int rows, int D, int nsplit) {
+    const int passes = (rows * (D / 2) + 255) / 256, trips = (nsplit + 7) / 8;
+    return passes == 1 ? trips <= 4 : passes * trips <= 3;
+}
+// ... and the most (row, split) pairs that rule lets through, whose maxima and denominators the folding workgroup stages in LDS:
+// eight rows of head size 64 in 32 splits.
+constexpr int FOLD_MAX_PAIRS = 256;
 #if defined(__HIPCC__)
 // Split partials of a decode launch that another workgroup of the same launch folds.  They cross from one XCD's L2 to
 // another's, which plain stores and loads do not reach inside a launch; a device-scope fence would (it writes back and
@@ -310,9 +324,8 @@ __device__ __forceinline__ float2 load_partial(const float* p) {
 // the last workgroup's loads are issued after its count came back, so it sees every split's partials.  The counter is zero
 // again when the launch ends.  Nobody waits: the other workgroups leave.
 // `lds`: FOLD_MAX_PAIRS float2 of LDS that no thread reads or writes any more behind the first barrier; `flag`: another word.
-// One sequence of 1118 tokens (12 splits, D = 128, 8 kv heads): 8.5 us per layer in a stream of layers against 9.9 with the merge
-// as a launch of its own (kernels 6.7 + 4.1 us), and 2.2 us less on the host; 32 such layers through the Python binding, which the
-// host bounds, 482 -> 386 us; 16 sequences of 64 - 2048 tokens over f16 (D = 64, 22 layers) 373 -> 308 us.
+// What it saves is a launch: one sequence of 1000 tokens (8 splits, 32 / 8 heads, D = 128, u8) through the Python binding, which the
+// host bounds, 16.3 us per layer against 19.8 with the merge as a launch of its own; 4 x 8000 26.5 against 28.0.
 template <int D, int QDT, int NT>
 __device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, const int hkv, const int rows, const long counter,
                                              float2* lds, int32_t* flag) {

@@ -195,7 +195,8 @@ struct pa_ctx {
     bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams (else one after the other)
     std::vector<int32_t> h_few;  // every sequence of a step of few-token sequences, longest context first (else empty)
     DecPlan few_plan;
-    int32_t few_cols = 1;        // 16-column groups of the decode kernel's few-token variant
+    int32_t few_rows = 0;        // most (token, head) rows of one per kv head
+    int32_t few_cols = 1;        // ... in this many 16-column groups of the decode kernel's few-token variant
     size_t few_off = 0;          // its descriptors within a table's buffer
     // the step's host arrays (packed metadata, work items, lists, block tables with their descriptors) pass through
     // this pinned area on their way to the device: pieces are handed out front to back, their copies are queued and not
@@ -510,10 +511,12 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
                 const int64_t full = w_run / slots, rem = w_run % slots;
                 // (a cut that fills its rounds exactly is preferred over one that does not at equal estimates: the
                 // estimate of a partly filled round is the less certain one -- 8 x 32769 runs 2 % faster in 8 than in 7)
-                // (launches that fold their own splits: what counts of a short workgroup are its waves' rounds -- nine tiles
-                // take four waves as long as twelve.  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17
-                // 12.6; of 1117 over f16 in 18 parts 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3)
-                const double steps = sc ? per : (per + 3) / 4 * 4;
+                // (without scores what counts of a short workgroup are its waves' rounds -- nine tiles take four waves as long as
+                // twelve.  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17 12.6; of 1117 over f16 in 18 parts
+                // 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3; with scores from logits eight of 2000 over u4
+                // (32 / 4, D = 64) in 7 23.3, in 8 21.3.  Longer ones keep the memory busy while a wave is late: one of 131072 over
+                // f16 (16 / 1, D = 256) in 64 parts of 65 tiles 87.6, in 61 of 68 90.8; of 32768 in 61 36.0, in 52 37.4)
+                const double steps = (sc && !u4) || per > 16 ? per : (per + 3) / 4 * 4;
                 const double t = ((double)full * steps * t_tile(slots) + (rem > 0 ? steps * t_tile(rem) : 0.0)) *
                                      (n > 1 && rem > 0 ? 1.02 : 1.0) +
                                  (n > 1 ? post_a + post_b * (double)w : 0.0);
@@ -781,6 +784,7 @@ void plan_items(pa_ctx* ctx) {
         if (rows <= 32) {
             for (int32_t b = 0; b < B; ++b) ctx->h_few.push_back(b);
             std::stable_sort(ctx->h_few.begin(), ctx->h_few.end(), [&](int32_t x, int32_t y) { return past[x] > past[y]; });
+            ctx->few_rows = rows;
             ctx->few_cols = rows <= 16 ? 1 : 2;
             plan_decode_u8(ctx, false, &ctx->few_plan.nsplit, &ctx->few_plan.max_tiles, &ctx->h_few);
         }
@@ -884,9 +888,9 @@ DecodeWs decode_workspace(pa_ctx* ctx, size_t rows, int32_t nsplit, bool want_sc
 
 // The counters with which a decode launch of several splits folds its own partials (null: it does not).  With scores the
 // merge is part of the score launch, which needs the splits' factors anyway (u4: its scores come from logits and final
-// values).  Contexts cut into more (head, split) pairs than the fold stages keep the merge launch.
+// values).  Wide groups cut into many splits keep the merge launch (`fold_pays`).
 int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, bool u4) {
-    if (a.nsplit <= 1 || (a.want_scores && !u4) || a.G * a.nsplit > pa::FOLD_MAX_PAIRS) return nullptr;
+    if (a.nsplit <= 1 || (a.want_scores && !u4) || !pa::fold_pays(a.G, ctx->cfg.head_size, a.nsplit)) return nullptr;
     return ctx->arrived.as<int32_t>();
 }
 
@@ -953,7 +957,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.part_acc = ws.part_acc;
         a.part_ml = ws.part_ml;
         a.final_ml = ws.final_ml;
-        if (a.nsplit > 1 && 16 * ctx->few_cols * a.nsplit <= pa::FOLD_MAX_PAIRS) a.arrived = ctx->arrived.as<int32_t>();
+        if (a.nsplit > 1 && pa::fold_pays(ctx->few_rows, c.head_size, a.nsplit)) a.arrived = ctx->arrived.as<int32_t>();
         ctx->kernels_run |= PA_RAN_DECODE_FEW | (a.arrived ? PA_RAN_FOLD : 0);
         HIP_CHECK(pa::launch_decode_few(ctx->stream, a, c.query_dtype, ctx->few_cols, ev0, ev1));
         ctx->timed = ctx->profiling;

@@ -12,7 +12,8 @@ CASES = [
     ("f16", "u8", 32, 8, 2, 128, [1117], 0), ("bf16", "u8", 16, 4, 4, 64, [900, 33, 0], 0), ("f16", "u8", 64, 12, 4, 96, [2000, 64], 0),
     ("bf16", "u8", 32, 16, 1, 256, [3000], 700), ("f16", "f16", 32, 14, 2, 128, [1500, 5], 0), ("bf16", "bf16", 16, 8, 8, 64, [64, 1030], 0),
     ("f16", "f16", 32, 16, 8, 256, [2500], 0), ("bf16", "bf16", 256, 6, 2, 96, [700, 701, 1], 600),
-    ("f16", "u8", 32, 16, 1, 128, [40000], 0),  # as many (head, split) pairs as the fold takes
+    ("f16", "u8", 32, 8, 1, 64, [4000], 0), ("bf16", "bf16", 32, 12, 1, 128, [1000, 40], 0),  # the most rows and splits a launch folds
+    ("f16", "u8", 32, 16, 1, 128, [40000], 0), ("f16", "f16", 32, 7, 1, 128, [1990], 0),      # too many for that: a merge launch
 ]
 
 
@@ -24,12 +25,17 @@ def test_split_fold(pkg, qd, kd, bs, Hq, Hkv, D, past, sw):
     case = H.build_case(H.case_from_lens("fold", Hq, Hkv, D, bs, qd, kd, past, [1] * len(past), sw), seed=D + bs)
     ref = H.run_case_on_checker(case, want_scores=False)
     got = H.run_case_on_gpu(pkg, case, dev, want_scores=False)
-    assert got["op"].num_splits > 1
+    ns = got["op"].num_splits
+    assert ns > 1
+    # one workgroup's trips to the partials: 256 pairs of channels, eight splits each
+    passes, trips = -(-(Hq // Hkv) * D // 512), -(-ns // 8)
+    assert ("fold" in got["op"].kernels_run) == (trips <= 4 if passes == 1 else passes * trips <= 3), (ns, passes, trips)
     H.assert_close(got["out"], ref["out"], qd)
     again = H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=got["op"])
     assert np.array_equal(got["out16"], again["out16"])
     # with scores (the merge is then part of the score launch) and without, in turn on one context
     scored = H.run_case_on_gpu(pkg, case, dev, want_scores=True, op=got["op"])
+    assert "fold" not in scored["op"].kernels_run
     H.assert_close(scored["out"], ref["out"], qd)
     assert np.array_equal(H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=got["op"])["out16"], got["out16"])
 
