@@ -639,15 +639,26 @@ void plan_items(pa_ctx* ctx) {
     // Fork and join cost four runtime calls and two waits between queues, 10 - 25 us per layer.  Sixteen mixed steps (4 to 60
     // single tokens beside 250 - 4096 chunk tokens), us per layer one after the other / side by side -- 16-bit caches: 68 / 72
     // at 4 GFLOP of chunk work, 141 / 169 at 9, 162 / 190 and (D = 64) 108 / 120 at 25, 211 / 209 at 63, 355 / 349 at 125:
-    // side by side from 45 GFLOP on.  Over u8, whose decode kernel leaves more of a CU to its neighbour, 75 / 75 at 4 GFLOP
+    // side by side from 45 GFLOP on.  And where a long context among short ones ends the decode launch on few CUs: 450 steps of
+    // 1 - 60 single tokens at 100 - 32768 positions beside 64 - 2048 chunk tokens (0.5 - 45 GFLOP) run 6 % faster one after the other
+    // in the mean, but 8 x 1000 - 26667 beside 256 tokens 259 / 222 us per layer, 16 x 500 - 8000 126 / 115.  With
+    // contexts of 4000 and more whose mean is below 0.75 of the longest side by side, one of them loses more than 4 % against side by
+    // side always (4.4 %), without that clause 27 (up to 17 %).  Over u8, whose decode kernel leaves more of a CU to its neighbour, 75 / 75 at 4 GFLOP
     // beside 55 MB of single tokens' rows, 126 / 119 at 10 beside 187 MB, 274 / 270 at 84: always.
     {
-        double flops = 0;
+        double flops = 0, positions = 0;
+        int32_t longest = 0, singles = 0;
         for (int32_t b = 0; b < B; ++b) {
             const int32_t q_len = sb[b + 1] - sb[b], kv = past[b] + q_len, vis = sw > 0 ? std::min(kv, sw) : kv;
-            if (q_len > 1) flops += 4.0 * ctx->cfg.num_heads * ctx->cfg.head_size * (double)q_len * std::max(vis - q_len / 2, 1);
+            if (q_len > 1) {
+                flops += 4.0 * ctx->cfg.num_heads * ctx->cfg.head_size * (double)q_len * std::max(vis - q_len / 2, 1);
+            } else {
+                longest = std::max(longest, vis);
+                positions += vis;
+                ++singles;
+            }
         }
-        ctx->fork_pays = !narrow_all || flops >= 45e9;
+        ctx->fork_pays = !narrow_all || flops >= 45e9 || (longest >= 4000 && positions < 0.75 * longest * singles);
     }
     size_t planned_tiles = 0;
     for (int32_t b = 0; b < B; ++b) {

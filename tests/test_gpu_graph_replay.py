@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
                                          ("bf16", [300, 40, 0], [1, 1, 70]),              # matrix kernel, mixed step
                                          ("u8", [300, 40, 0], [1, 1, 70]),                # decode kernel on the second stream beside the matrix kernel
                                          ("bf16", [700, 64, 1300, 31], [1, 1, 1, 1]),     # 16-bit decode kernel (appends too)
-                                         ("bf16", [9000, 20], [1, 1])])                   # the same with several splits
+                                         ("bf16", [9000, 20], [1, 1]),                    # the same with several splits
+                                         ("bf16", [6000, 40, 0], [1, 1, 70])])            # on the second stream beside the matrix kernel
 def test_graph_replays_equal_eager(pkg, kv, past, new):
     import torch
     dev = torch.device("cuda:0")
@@ -37,6 +38,7 @@ def test_graph_replays_equal_eager(pkg, kv, past, new):
                 op.forward(qd, kd, vd, kc[l], vc[l], outs[l], scores[l], layer=l)
 
         step()  # eager: also sizes every workspace
+        assert ("side_stream" in op.kernels_run) == (max(new) > 1 and (kv == "u8" or past[0] == 6000))
         s.synchronize()
         want_out = [o.clone() for o in outs]
         want_sc = [x.clone() for x in scores]
