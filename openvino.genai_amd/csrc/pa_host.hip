@@ -515,8 +515,9 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
                 // twelve.  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17 12.6; of 1117 over f16 in 18 parts
                 // 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3; with scores from logits eight of 2000 over u4
                 // (32 / 4, D = 64) in 7 23.3, in 8 21.3.  Longer ones keep the memory busy while a wave is late: one of 131072 over
-                // f16 (16 / 1, D = 256) in 64 parts of 65 tiles 87.6, in 61 of 68 90.8; of 32768 in 61 36.0, in 52 37.4)
-                const double steps = (sc && !u4) || per > 16 ? per : (per + 3) / 4 * 4;
+                // f16 (16 / 1, D = 256) in 64 parts of 65 tiles 87.6, in 61 of 68 90.8; but four of 500 - 8000 over f16 in 9 parts of 28 31.4, in 10
+                // of 25 29.6)
+                const double steps = (sc && !u4) || per > 32 ? per : (per + 3) / 4 * 4;
                 const double t = ((double)full * steps * t_tile(slots) + (rem > 0 ? steps * t_tile(rem) : 0.0)) *
                                      (n > 1 && rem > 0 ? 1.02 : 1.0) +
                                  (n > 1 ? post_a + post_b * (double)w : 0.0);
