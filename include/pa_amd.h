@@ -187,7 +187,9 @@ int32_t pa_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io);
  * step arrays and block tables are uploaded -- and their buffers grown -- by pa_step_begin / pa_set_block_indices,
  * as for pa_attention.)  Every call on a GPU shares that GPU's array: calls that overlap on one GPU race, also from
  * different contexts; calls in stream order on one stream do not.  Nothing in it needs clearing between calls: each
- * call writes every element it later reads. */
+ * call writes every element it later reads.  (The counters with which a launch of several splits without scores folds them belong to
+ * the context and its step, as the step arrays do: a captured call is replayed before the context's next pa_step_begin, and not
+ * beside another call of the context.) */
 #define PA_STATIC_SCRATCH_BYTES (40u << 20)
 int32_t pa_attention_static(pa_ctx* ctx, int32_t layer, const pa_layer_io* io);
 /* Blocks until everything launched on the context's stream has finished. */

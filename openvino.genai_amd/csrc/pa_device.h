@@ -335,9 +335,8 @@ __device__ __forceinline__ void fold_if_last(const DecodeArgs& a, const int t, c
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        const int32_t before = __hip_atomic_fetch_add(a.arrived + counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before == ns - 1) __hip_atomic_store(a.arrived + counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *flag = before == ns - 1;
+        // (one wrapping increment: launches that overlap by mistake spoil each other's results, but not the count)
+        *flag = atomicInc(reinterpret_cast<unsigned int*>(a.arrived + counter), (unsigned)(ns - 1)) == (unsigned)(ns - 1);
     }
     __syncthreads();
     if (!*flag) return;  // (uniform)

@@ -168,7 +168,7 @@ struct pa_ctx {
     DevBuf dec16_list;
     std::vector<int32_t> h_multi;     // sequences that schedule more than one token
     DevBuf multi_list;
-    DevBuf arrived;    // decode launches that fold their own splits: per (listed sequence, kv head) a count, zero between launches
+    size_t arrived_off = 0;  // in `items`: decode launches that fold their own splits count here, per (listed sequence, kv head)
     DevBuf tile_max;   // per (head, 32-token tile) maxima of single-token sequences handled by the matrix kernel
     bool dec_in_order = false, dec16_in_order = false;  // the lists hold 0 .. B-1 in order: every sequence, none moved
     bool stash_ok = false;  // the step's single-token items are short enough to keep their probabilities in LDS
@@ -806,7 +806,8 @@ void plan_items(pa_ctx* ctx) {
     ctx->max_split = max_split;
     const size_t item_bytes = items.size() * sizeof(pa::PrefillItem);
     // one upload: items | split count per token | single-token index per sequence (-1 for the others) | the tokens
-    // whose rows the merge kernel has to fold
+    // whose rows the merge kernel has to fold | zeros, the counters of decode launches that fold their splits (they leave them at
+    // zero; a step starts there whatever became of the last one)
     ctx->n_merge = 0;
     for (int32_t t = 0; t < T; ++t) ctx->n_merge += tok_ns[t] > 1;
     tok_ns.insert(tok_ns.end(), single_idx.begin(), single_idx.end());
@@ -814,6 +815,8 @@ void plan_items(pa_ctx* ctx) {
         if (tok_ns[t] > 1) tok_ns.push_back(t);
     ctx->single_idx_off = item_bytes + (size_t)T * sizeof(int32_t);
     ctx->merge_tok_off = ctx->single_idx_off + (size_t)B * sizeof(int32_t);
+    ctx->arrived_off = item_bytes + tok_ns.size() * sizeof(int32_t);
+    tok_ns.resize(tok_ns.size() + std::max({ctx->h_dec.size(), ctx->h_dec16.size(), ctx->h_few.size()}) * (size_t)ctx->cfg.num_kv_heads, 0);
     ctx->items.reserve(item_bytes + tok_ns.size() * sizeof(int32_t));
     stage_upload(ctx, ctx->items.p, items.data(), item_bytes);
     stage_upload(ctx, static_cast<uint8_t*>(ctx->items.p) + item_bytes, tok_ns.data(), tok_ns.size() * sizeof(int32_t));
@@ -834,12 +837,6 @@ void plan_items(pa_ctx* ctx) {
     if (!ctx->h_dec.empty()) {
         ctx->dec_list.reserve(ctx->h_dec.size() * sizeof(int32_t));
         stage_upload(ctx, ctx->dec_list.p, ctx->h_dec.data(), ctx->h_dec.size() * sizeof(int32_t));
-    }
-    // (the launches leave the counters at zero; an enlarged buffer starts there)
-    const size_t counters = std::max({ctx->h_dec.size(), ctx->h_dec16.size(), ctx->h_few.size()}) * (size_t)ctx->cfg.num_kv_heads * sizeof(int32_t);
-    if (counters > ctx->arrived.cap) {
-        ctx->arrived.reserve(counters);
-        HIP_CHECK(hipMemsetAsync(ctx->arrived.p, 0, ctx->arrived.cap, ctx->stream));
     }
     ctx->tok_nsplit_off = item_bytes;
     if (split_off_decode && !ctx->h_dec.empty())
@@ -901,9 +898,9 @@ DecodeWs decode_workspace(pa_ctx* ctx, size_t rows, int32_t nsplit, bool want_sc
 // The counters with which a decode launch of several splits folds its own partials (null: it does not).  With scores the
 // merge is part of the score launch, which needs the splits' factors anyway (u4: its scores come from logits and final
 // values).  Wide groups cut into many splits keep the merge launch (`fold_pays`).
-int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, bool u4) {
-    if (a.nsplit <= 1 || (a.want_scores && !u4) || !pa::fold_pays(a.G, ctx->cfg.head_size, a.nsplit)) return nullptr;
-    return ctx->arrived.as<int32_t>();
+int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, int32_t rows, bool u4) {
+    if (a.nsplit <= 1 || (a.want_scores && !u4) || !pa::fold_pays(rows, ctx->cfg.head_size, a.nsplit)) return nullptr;
+    return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(ctx->items.p) + ctx->arrived_off);
 }
 
 // fuse_append: the call is the attention half of pa_forward in a step whose sequences all go to one decode kernel (the
@@ -969,7 +966,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.part_acc = ws.part_acc;
         a.part_ml = ws.part_ml;
         a.final_ml = ws.final_ml;
-        if (a.nsplit > 1 && pa::fold_pays(ctx->few_rows, c.head_size, a.nsplit)) a.arrived = ctx->arrived.as<int32_t>();
+        a.arrived = fold_counters(ctx, a, ctx->few_rows, false);
         ctx->kernels_run |= PA_RAN_DECODE_FEW | (a.arrived ? PA_RAN_FOLD : 0);
         HIP_CHECK(pa::launch_decode_few(ctx->stream, a, c.query_dtype, ctx->few_cols, ev0, ev1));
         ctx->timed = ctx->profiling;
@@ -1004,7 +1001,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.final_ml = ws.final_ml;
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
-        a.arrived = fold_counters(ctx, a, use_u4);
+        a.arrived = fold_counters(ctx, a, a.G, use_u4);
         ctx->kernels_run |= PA_RAN_DECODE | (a.arrived ? PA_RAN_FOLD : 0);
         if (use_u4) {
             if (io->scores) {
@@ -1049,7 +1046,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.final_ml = ws.final_ml;
         a.group_scores = ws.group_scores;
         a.p_split = ws.p_split;
-        a.arrived = fold_counters(ctx, a, false);
+        a.arrived = fold_counters(ctx, a, a.G, false);
         ctx->kernels_run |= PA_RAN_DECODE | (a.arrived ? PA_RAN_FOLD : 0);
         HIP_CHECK(pa::launch_decode16(side_by_side ? fork_side() : ctx->stream, a, c.query_dtype, io->scores, ctx->max_kv,
                                       mfma_left ? nullptr : ev0, mfma_left ? nullptr : ev1));
@@ -1222,7 +1219,6 @@ void pa_destroy(pa_ctx* ctx) {
     ctx->dec16_list.release();
     ctx->multi_list.release();
     ctx->tile_max.release();
-    ctx->arrived.release();
     ctx->trig_lut.release();
     ctx->rot_args.release();
     ctx->div_seqs.release();

@@ -66,3 +66,38 @@ def test_split_fold_in_a_graph(pkg):
             torch.cuda.synchronize(dev)
             for o in out:
                 assert np.array_equal(o.view(torch.int16).cpu().numpy().view(np.uint16), eager["out16"]), i
+
+
+def test_split_fold_after_overlapping_launches(pkg):
+    """Calls of one context must not overlap; ones that did (here a graph replayed on two streams, every launch the same values in
+    the same places) leave the counters of the fold whole: what runs afterwards, alone, is right."""
+    import torch
+    dev = torch.device("cuda:0")
+    case = H.build_case(H.case_from_lens("fold", 32, 8, 128, 32, "f16", "u8", [1117, 300], [1, 1]), seed=4)
+    stream, other = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    with torch.cuda.stream(stream):
+        op = pkg.PagedAttention(32, 8, 128, 32, "f16", "u8", 1, 0, stream)
+        eager = H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=op)
+        assert "fold" in op.kernels_run
+        q = H.to_device_16(torch, case["query"], "f16", dev)
+        kc, vc = (torch.from_numpy(eager[n]).to(dev) for n in ("key_cache", "value_cache"))  # (the step's rows in place)
+        out = torch.zeros_like(q)
+        torch.cuda.synchronize(dev)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            for _ in range(20):
+                op.attention(q, kc, vc, out)
+        second = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(second, stream=stream):
+            for _ in range(20):
+                op.attention(q, kc, vc, out)
+        for _ in range(5):
+            graph.replay()
+            with torch.cuda.stream(other):
+                second.replay()
+            torch.cuda.synchronize(dev)
+        for _ in range(3):
+            out.zero_()
+            op.attention(q, kc, vc, out)
+            torch.cuda.synchronize(dev)
+            assert np.array_equal(out.view(torch.int16).cpu().numpy().view(np.uint16), eager["out16"])
