@@ -93,8 +93,8 @@ class PagedAttention:
     def _io(self, query, key, value, key_cache, value_cache, out, scores):
         # (one per layer call, and a small step's time is this host's: built in one go rather than field by field)
         return L.pa_layer_io(None if query is None else query.data_ptr(), None if key is None else key.data_ptr(),
-                             None if value is None else value.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
-                             key_cache.shape[0], None if out is None else out.data_ptr(),
+                             None if value is None else value.data_ptr(), key_cache.data_ptr(),
+                             None if value_cache is None else value_cache.data_ptr(), key_cache.shape[0], None if out is None else out.data_ptr(),
                              None if scores is None else scores.data_ptr())
 
     def kv_append(self, key, value, key_cache, value_cache, layer=0):

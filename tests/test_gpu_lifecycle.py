@@ -124,3 +124,20 @@ def test_two_host_threads_each_with_contexts_and_a_stream_of_their_own(pkg):
     for t in threads:
         t.join()
     assert not problems, problems[:5]
+
+
+def test_missing_tensors_are_errors_of_the_library(pkg):
+    """A layer call without one of its tensors is the library's error (its status and message), whichever tensor is missing."""
+    import torch
+    dev = torch.device("cuda:0")
+    op = pkg.PagedAttention(8, 2, 128, 32, "f16", "u8", 1, 0, torch.cuda.current_stream(dev))
+    op.step_begin([3], [0, 1], [0, 1])
+    op.set_block_indices([0], 1)
+    q, k = torch.zeros(1, 8 * 128, dtype=torch.float16, device=dev), torch.zeros(1, 2 * 128, dtype=torch.float16, device=dev)
+    cache = torch.zeros(1, 2, 32, 136, dtype=torch.uint8, device=dev)
+    for call in (lambda: op.forward(q, k, k, cache, None, q), lambda: op.attention(q, cache, None, q), lambda: op.kv_append(k, k, cache, None),
+                 lambda: op.forward(None, k, k, cache, cache, q), lambda: op.forward(q, None, k, cache, cache, q),
+                 lambda: op.forward(q, k, k, cache, cache, None)):
+        with pytest.raises(pkg.PaError) as e:
+            call()
+        assert e.value.status == -14, e.value
