@@ -90,7 +90,7 @@ __device__ __forceinline__ void load_row(uint32_t (&w)[E / 2], const uint16_t* s
 // four rows per wave.  A wave
 // takes four consecutive tokens of one kv head, so that what it writes is one run of cache bytes wherever the
 // tokens share a block.  Minimum and maximum of a row are reduced over its 16 lanes with four
-// cross-lane (DPP) steps; the arithmetic per element is that of quantize_row_u8, so the bytes are the same.
+// cross-lane (DPP) steps; the arithmetic per element is that of quantize_row, so the bytes are the same.
 template <int QDT, int KVDT, int E>
 __global__ __launch_bounds__(256) void kv_append_kernel(StepDev st, Shape sh, const uint16_t* __restrict__ key,
                                                         const uint16_t* __restrict__ value,

@@ -8,7 +8,7 @@
 //     through a wave-private LDS slot to re-shape them into MFMA operand layout;
 //   * u8 codes become fp16 operands in registers with one byte-permute per code pair: the
 //     zero-extended byte IS the fp16 subnormal code * 2^-24, which the gfx950 matrix cores take
-//     without flushing; scale / zero-point are applied to the 16x16 accumulator tiles instead
+//     without flushing (the variants below make normal values of them, see `centred_codes`); scale / zero-point are applied to the 16x16 accumulator tiles instead
 //     of to the D-wide rows:
 //         logit  = scale * sc_k * (q . codes - zp_k * sum(q))
 //         out    = sum_t p_t sc_v (codes_t - zp_v) = sum_t w_t codes_t - sum_t w_t zp_v
@@ -225,8 +225,8 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     // LDS carve-up
     uint8_t* slot = smem + wv * SLOT;                                  // wave-private staging
     float* wave_mlz = reinterpret_cast<float*>(smem + WAVES * SLOT);   // [WAVES][16][4]
-    float* msnap = wave_mlz + WAVES * 16 * NG * 4;                          // [max_tiles][16]
-    _Float16* ptile = reinterpret_cast<_Float16*>(msnap + (a.want_scores ? a.max_tiles * 16 : 0));  // (u4: neither)  // [G][max_tiles*TOK]
+    float* msnap = wave_mlz + WAVES * 16 * NG * 4;                     // [max_tiles][16] (not over u4, nor with several tokens)
+    _Float16* ptile = reinterpret_cast<_Float16*>(msnap + (a.want_scores ? a.max_tiles * 16 : 0));  // [G][max_tiles*TOK] (nor these)
     const int pstride = a.max_tiles * TOK;
 
     // The step's new K / V row of this (sequence, kv head) goes into the caches here when the step's append is fused
@@ -311,27 +311,27 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     } else {
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
-        const int c = 16 * gi + n;
-        const uint16_t* qp = a.query + ((long)(COLS ? t + c / G : t) * Hq + hkv * G + (COLS ? c % G : n)) * D + 8 * g;
+            const int c = 16 * gi + n;
+            const uint16_t* qp = a.query + ((long)(COLS ? t + c / G : t) * Hq + hkv * G + (COLS ? c % G : n)) * D + 8 * g;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if (c < R) {
-                const uint4 v = *reinterpret_cast<const uint4*>(qp + 32 * s);
-                if (QDT == DT_F16) {
-                    qreg[gi][s] = __builtin_bit_cast(h8, v);
-                } else {
-                    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+            for (int s = 0; s < KS; ++s) {
+                if (c < R) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(qp + 32 * s);
+                    if (QDT == DT_F16) {
+                        qreg[gi][s] = __builtin_bit_cast(h8, v);
+                    } else {
+                        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        qreg[gi][s][2 * e] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] & 0xffff));
-                        qreg[gi][s][2 * e + 1] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] >> 16));
+                        for (int e = 0; e < 4; ++e) {
+                            qreg[gi][s][2 * e] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] & 0xffff));
+                            qreg[gi][s][2 * e + 1] = (_Float16)bf16_bits_to_float((uint16_t)(w[e] >> 16));
+                        }
                     }
-                }
-            } else {
+                } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qreg[gi][s][e] = (_Float16)0.0f;
+                    for (int e = 0; e < 8; ++e) qreg[gi][s][e] = (_Float16)0.0f;
+                }
             }
-        }
         }
     }
 #pragma unroll
@@ -483,63 +483,63 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
-            float psum = 0.0f, zsum = 0.0f;
-            _Float16 ph[8];
-            float wf[8];
+                float psum = 0.0f, zsum = 0.0f;
+                _Float16 ph[8];
+                float wf[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float p = __builtin_amdgcn_exp2f(x[gi][j] - m_new[gi]);
-                wf[j] = seen[gi][j] ? p * hv[j].x : 0.0f;
-                psum += p;
-                pb[gi][j] = (_Float16)wf[j];
-                ph[j] = (_Float16)p;
-            }
-            // The weights are pinned in their registers: the compiler may otherwise form the f16 value twice (from the
-            // f32 product, and with a mixed-precision multiply), and the two differ by one f16 step at a tie
-            asm volatile("" : "+v"(pb[gi]));
-            // what the rounding to f16 dropped goes through the matrix pipe as a second operand: with 11 bits alone a
-            // row that leans on a few tokens with large V values of opposite sign can miss the tolerance
-            {
-                const u4v hi = __builtin_bit_cast(u4v, pb[gi]);
-                u4v lo;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t h = hi[j];
-                    lo[j] = residual_f16x2(h, wf[2 * j], wf[2 * j + 1]);
+                for (int j = 0; j < 8; ++j) {
+                    const float p = __builtin_amdgcn_exp2f(x[gi][j] - m_new[gi]);
+                    wf[j] = seen[gi][j] ? p * hv[j].x : 0.0f;
+                    psum += p;
+                    pb[gi][j] = (_Float16)wf[j];
+                    ph[j] = (_Float16)p;
                 }
-                pl[gi] = __builtin_bit_cast(h8, lo);
-            }
-            // the zero-point term must see the weight the matrix product sees, or the rounding error is scaled by the
-            // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
+                // The weights are pinned in their registers: the compiler may otherwise form the f16 value twice (from the
+                // f32 product, and with a mixed-precision multiply), and the two differ by one f16 step at a tie
+                asm volatile("" : "+v"(pb[gi]));
+                // what the rounding to f16 dropped goes through the matrix pipe as a second operand: with 11 bits alone a
+                // row that leans on a few tokens with large V values of opposite sign can miss the tolerance
+                {
+                    const u4v hi = __builtin_bit_cast(u4v, pb[gi]);
+                    u4v lo;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
-            l_part[gi] = l_part[gi] * corr[gi] + psum;
-            z_part[gi] = z_part[gi] * (FRESH ? acc_corr[gi] : corr[gi]) + zsum;
-            if constexpr (!FRESH) {
-                if (__any(corr[gi] != 1.0f)) {
+                    for (int j = 0; j < 4; ++j) {
+                        const uint32_t h = hi[j];
+                        lo[j] = residual_f16x2(h, wf[2 * j], wf[2 * j + 1]);
+                    }
+                    pl[gi] = __builtin_bit_cast(h8, lo);
+                }
+                // the zero-point term must see the weight the matrix product sees, or the rounding error is scaled by the
+                // code instead of by (code - zp); the two halves together carry it to 2^-22, so the f32 weight serves
 #pragma unroll
-                    for (int r = 0; r < RT; ++r) acc[gi][r] *= corr[gi];
-                }
-            }
-            if constexpr (COLS > 0) {  // no scores
-            } else if constexpr (U4) {
-                if (a.want_scores && n < G) {
-                    float* dst = a.logits + (long)(hkv * G + n) * a.total_scores + dsc->score_off + pos0 + 4 * g;
+                for (int j = 0; j < 8; ++j)
+                    zsum += seen[gi][j] ? wf[j] * hv[j].y : 0.0f;
+                l_part[gi] = l_part[gi] * corr[gi] + psum;
+                z_part[gi] = z_part[gi] * (FRESH ? acc_corr[gi] : corr[gi]) + zsum;
+                if constexpr (!FRESH) {
+                    if (__any(corr[gi] != 1.0f)) {
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (seen[gi][j]) dst[16 * (j >> 2) + (j & 3)] = x[gi][j];
+                        for (int r = 0; r < RT; ++r) acc[gi][r] *= corr[gi];
+                    }
                 }
-            } else if (a.want_scores) {
-                const int lt = tile - tb;
-                if (n < G) {
-                    _Float16* dst = ptile + n * pstride + lt * TOK + 4 * g;
-                    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                    *reinterpret_cast<h4*>(dst) = h4{ph[0], ph[1], ph[2], ph[3]};
-                    *reinterpret_cast<h4*>(dst + 16) = h4{ph[4], ph[5], ph[6], ph[7]};
-                    if (g == 0) msnap[lt * 16 + n] = m_new[gi];
+                if constexpr (COLS > 0) {  // no scores
+                } else if constexpr (U4) {
+                    if (a.want_scores && n < G) {
+                        float* dst = a.logits + (long)(hkv * G + n) * a.total_scores + dsc->score_off + pos0 + 4 * g;
+#pragma unroll
+                        for (int j = 0; j < 8; ++j)
+                            if (seen[gi][j]) dst[16 * (j >> 2) + (j & 3)] = x[gi][j];
+                    }
+                } else if (a.want_scores) {
+                    const int lt = tile - tb;
+                    if (n < G) {
+                        _Float16* dst = ptile + n * pstride + lt * TOK + 4 * g;
+                        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                        *reinterpret_cast<h4*>(dst) = h4{ph[0], ph[1], ph[2], ph[3]};
+                        *reinterpret_cast<h4*>(dst + 16) = h4{ph[4], ph[5], ph[6], ph[7]};
+                        if (g == 0) msnap[lt * 16 + n] = m_new[gi];
+                    }
                 }
-            }
             }
         };
         if (tile * TOK < free_lo || tile * TOK + TOK > free_hi) softmax(std::true_type{});
@@ -654,53 +654,54 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     float* red = reinterpret_cast<float*>(smem);
     const bool final_out = nsplit == 1;
 #pragma unroll
-    for (int gi = 0; gi < NG; ++gi)
-    for (int n0 = 16 * gi; n0 < min(R, 16 * gi + 16); n0 += HC) {  // (n0, like `head` below: a column)
-        if (n0) __syncthreads();
-        if (16 * gi + n >= n0 && 16 * gi + n < min(R, n0 + HC)) {
-            float* dst = red + ((wv * HC + 16 * gi + n - n0) * D);
+    for (int gi = 0; gi < NG; ++gi) {
+        for (int n0 = 16 * gi; n0 < min(R, 16 * gi + 16); n0 += HC) {  // (n0, like `head` below: a column)
+            if (n0) __syncthreads();
+            if (16 * gi + n >= n0 && 16 * gi + n < min(R, n0 + HC)) {
+                float* dst = red + ((wv * HC + 16 * gi + n - n0) * D);
 #pragma unroll
-            for (int r = 0; r < RT; ++r)
+                for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) dst[chan(4 * g + i, r)] = acc[gi][r][i];  // lane (n, g), register i of tile r: row 4 g + i
-        }
-        __syncthreads();
-        if (!U4 && COLS == 0 && n0 == 0 && a.want_scores) {
-            // one factor per (block, head): exp2(snapshot - M) (/ L when this workgroup saw the whole context), written
-            // over the snapshot.  Entry e belongs to head e % 16 = this thread's n; the barrier before the score
-            // phase publishes the factors
-            float f[WAVES], M, L, Z;
-            fold_head(n, f, M, L, Z);
-            const float fl = final_out ? (L > 0.0f ? 1.0f / L : 0.0f) : 1.0f;
-            for (int e = tid; e < max(te - tb, 0) * 16; e += NT)
-                msnap[e] = n < G ? __builtin_amdgcn_exp2f(msnap[e] - M) * fl : 0.0f;
-        }
-        const int heads = min(R, n0 + HC) - n0;
-        for (int idx = tid; idx < heads * (D / 2); idx += NT) {
-            const int hl = idx / (D / 2), d = 2 * (idx % (D / 2));
-            const int head = n0 + hl;
-            const long orow = COLS ? (long)(t + head / G) * Hq + hkv * G + head % G : (long)t * Hq + hkv * G + head;
-            float f[WAVES], M, L, Z;
-            fold_head(head, f, M, L, Z);
-            float v0 = 0.0f, v1 = 0.0f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const float2 v = *reinterpret_cast<const float2*>(red + (w * HC + hl) * D + d);
-                v0 += v.x * f[w];
-                v1 += v.y * f[w];
+                    for (int i = 0; i < 4; ++i) dst[chan(4 * g + i, r)] = acc[gi][r][i];  // lane (n, g), register i of tile r: row 4 g + i
             }
-            const float o0 = v0 * CODE_INV - Z, o1 = v1 * CODE_INV - Z;
-            const long prow = orow * nsplit + split;
-            if (final_out) {
-                const float inv_l = L > 0.0f ? 1.0f / L : 0.0f;
-                *reinterpret_cast<uint32_t*>(a.out + orow * D + d) =
-                    (uint32_t)store16<QDT>(o0 * inv_l) | ((uint32_t)store16<QDT>(o1 * inv_l) << 16);
-            } else {
-                store_partial(a.part_acc + prow * D + d, o0, o1, a.arrived != nullptr);
+            __syncthreads();
+            if (!U4 && COLS == 0 && n0 == 0 && a.want_scores) {
+                // one factor per (block, head): exp2(snapshot - M) (/ L when this workgroup saw the whole context), written
+                // over the snapshot.  Entry e belongs to head e % 16 = this thread's n; the barrier before the score
+                // phase publishes the factors
+                float f[WAVES], M, L, Z;
+                fold_head(n, f, M, L, Z);
+                const float fl = final_out ? (L > 0.0f ? 1.0f / L : 0.0f) : 1.0f;
+                for (int e = tid; e < max(te - tb, 0) * 16; e += NT)
+                    msnap[e] = n < G ? __builtin_amdgcn_exp2f(msnap[e] - M) * fl : 0.0f;
             }
-            if (d == 0) {  // maxima stay in the log2 domain within this kernel family
-                if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * orow) = make_float2(M, L);
-                else store_partial(a.part_ml + 2 * prow, M, L, a.arrived != nullptr);
+            const int heads = min(R, n0 + HC) - n0;
+            for (int idx = tid; idx < heads * (D / 2); idx += NT) {
+                const int hl = idx / (D / 2), d = 2 * (idx % (D / 2));
+                const int head = n0 + hl;
+                const long orow = COLS ? (long)(t + head / G) * Hq + hkv * G + head % G : (long)t * Hq + hkv * G + head;
+                float f[WAVES], M, L, Z;
+                fold_head(head, f, M, L, Z);
+                float v0 = 0.0f, v1 = 0.0f;
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) {
+                    const float2 v = *reinterpret_cast<const float2*>(red + (w * HC + hl) * D + d);
+                    v0 += v.x * f[w];
+                    v1 += v.y * f[w];
+                }
+                const float o0 = v0 * CODE_INV - Z, o1 = v1 * CODE_INV - Z;
+                const long prow = orow * nsplit + split;
+                if (final_out) {
+                    const float inv_l = L > 0.0f ? 1.0f / L : 0.0f;
+                    *reinterpret_cast<uint32_t*>(a.out + orow * D + d) =
+                        (uint32_t)store16<QDT>(o0 * inv_l) | ((uint32_t)store16<QDT>(o1 * inv_l) << 16);
+                } else {
+                    store_partial(a.part_acc + prow * D + d, o0, o1, a.arrived != nullptr);
+                }
+                if (d == 0) {  // maxima stay in the log2 domain within this kernel family
+                    if (final_out) *reinterpret_cast<float2*>(a.final_ml + 2 * orow) = make_float2(M, L);
+                    else store_partial(a.part_ml + 2 * prow, M, L, a.arrived != nullptr);
+                }
             }
         }
     }

@@ -148,10 +148,6 @@ __device__ __forceinline__ void quantize_row(const uint16_t (&raw)[EPL], uint8_t
     else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(c) = (uint16_t)packed;
     else *c = (uint8_t)packed;
 }
-template <int QDT, int EPL>
-__device__ __forceinline__ void quantize_row_u8(const uint16_t (&raw)[EPL], uint8_t* dst, const int lane, const bool store = true) {
-    quantize_row<QDT, EPL, false>(raw, dst, lane, store);
-}
 // The lane's EPL consecutive elements of a row of 16-bit values.
 template <int EPL>
 __device__ __forceinline__ void load_row16(const uint16_t* src, uint16_t (&raw)[EPL]) {
@@ -280,7 +276,7 @@ struct DecodeArgs {
     float* part_ml;               // nsplit > 1: [T*Hq*nsplit, 2] (max in the log2 domain, denominator)
     float* final_ml;              // [T*Hq, 2]
     _Float16* group_scores;       // nsplit == 1: [Hkv, total_scores] per-kv-head score sums on their way to the score kernel
-    int32_t* arrived;             // nsplit > 1: [n_seqs * Hkv] zeros; the workgroup that finds itself the last of its
+    int32_t* arrived;             // nsplit > 1: [n_seqs * Hkv] counts, zero between launches; the workgroup that finds itself the last of its
                                   // (sequence, kv head) folds the split partials (null: a launch of its own does)
     float* logits;                // u4 with scores: [Hq, total_scores] scaled logits in the log2 domain
     _Float16* p_split;            // nsplit > 1: [Hq, p_split_stride(total_scores, B)] probabilities relative to the

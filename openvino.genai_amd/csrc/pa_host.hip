@@ -786,7 +786,7 @@ void plan_items(pa_ctx* ctx) {
     // one behind the other -- 63 x 4096 beside one of 5 tokens 122 / 141 / 134, 30 x 500 - 8000 beside 6 last tokens of a prompt
     // 84 / 98 / 91, 15 x 128 - 4000 beside one of 5 42 / 74 / 57, 3 x 1000 beside one of 5 33 / 74 / 39, 8 x 32768 beside one of 5
     // 155 / 223 / 149, 60 x 512 - 8192 beside four of 5 144 / 164 / 145 (22 such steps: always ahead of the second, of the third
-    // but for the last two).  Taken by calls without scores in steps without block-sparse sequences; the
+    // but for 8 x 32768).  Taken by calls without scores in steps without block-sparse sequences; the
     // items above serve the others.  (Planned whether or not there are any: thresholds may be set and taken back between the
     // uploads of a step's tables, whose layout is one for the whole step.)
     ctx->h_few.clear();
