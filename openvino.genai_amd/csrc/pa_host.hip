@@ -495,8 +495,16 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             const double tile_bytes = 2.0 * 32 * pa::row_bytes(c.head_size, c.kv_cache_dtype), bw = sc && !u4 ? 5.9e6 : 6.97e6;
             const double post_a = u8 ? (sc && !u4 ? 2.4 : 1.0) : (sc ? 4.2 : 2.8), post_b = few ? 0.02 : u4 ? 0.0105 : u8 ? (sc ? 0.0079 : 0.0066) : (sc ? 0.0050 : 0.0046);
             const double fill = (double)all_tiles / ((double)most * (double)(pairs / c.num_kv_heads));
-            auto t_tile = [&](int64_t w) {  // per tile, with w workgroups running at once
-                return std::max(w <= slots / 2 || slots == 256 ? t1 : t2, (double)w * tile_bytes / bw);
+            // `per` tiles, with w workgroups running at once.  What counts of a short workgroup alone on its CU are its waves' rounds:
+            // nine tiles take four waves as long as twelve, as long as they wait for latencies and not for the memory system
+            // (with scores the estimate goes without).  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17
+            // 12.6; of 1117 over f16 in 18 parts 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3; with scores from
+            // logits eight of 2000 over u4 (32 / 4, D = 64) in 7 23.3, in 8 21.3.  Rounds counted in every case cost 4 - 11 %: over f16
+            // 37 of 3437 in 3 instead of 6 parts 101.3 / 94.8, 12 of 4096 in 2 instead of 5 44.9 / 42.4, over 28 / 4 heads in 4 instead
+            // of 5 28.9 / 25.9, one of 131072 (16 / 1, D = 256) in 61 instead of 64 90.8 / 87.6.
+            auto t_run = [&](int32_t per, int64_t w) {
+                const bool rounds = (!sc || u4) && w <= 256 && per <= 32;
+                return std::max((rounds ? (per + 3) / 4 * 4 : per) * (w <= slots / 2 || slots == 256 ? t1 : t2), per * (double)w * tile_bytes / bw);
             };
             // Contexts of unequal length: every sequence is cut into the same number of parts, so its workgroups are
             // as much shorter than the longest one's as its context is; the launch then behaves like one of fewer
@@ -511,15 +519,7 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
                 const int64_t full = w_run / slots, rem = w_run % slots;
                 // (a cut that fills its rounds exactly is preferred over one that does not at equal estimates: the
                 // estimate of a partly filled round is the less certain one -- 8 x 32769 runs 2 % faster in 8 than in 7)
-                // (without scores what counts of a short workgroup are its waves' rounds -- nine tiles take four waves as long as
-                // twelve.  One sequence of 4096 tokens over u8 in 26 parts 13.7 us per layer, in 17 12.6; of 1117 over f16 in 18 parts
-                // 10.9, in 9 10.0; four of 2000 over u8 in 7 parts 13.6, in 8 12.3; with scores from logits eight of 2000 over u4
-                // (32 / 4, D = 64) in 7 23.3, in 8 21.3.  Longer ones keep the memory busy while a wave is late: one of 131072 over
-                // f16 (16 / 1, D = 256) in 64 parts of 65 tiles 87.6, in 61 of 68 90.8; but four of 500 - 8000 over f16 in 9 parts of 28 31.4, in 10
-                // of 25 29.6)
-                const double steps = (sc && !u4) || per > 32 ? per : (per + 3) / 4 * 4;
-                const double t = ((double)full * steps * t_tile(slots) + (rem > 0 ? steps * t_tile(rem) : 0.0)) *
-                                     (n > 1 && rem > 0 ? 1.02 : 1.0) +
+                const double t = ((double)full * t_run(per, slots) + (rem > 0 ? t_run(per, rem) : 0.0)) * (n > 1 && rem > 0 ? 1.02 : 1.0) +
                                  (n > 1 ? post_a + post_b * (double)w : 0.0);
                 if (best_n == 0 || t < best_t) {
                     best_n = n;
@@ -897,9 +897,15 @@ DecodeWs decode_workspace(pa_ctx* ctx, size_t rows, int32_t nsplit, bool want_sc
 
 // The counters with which a decode launch of several splits folds its own partials (null: it does not).  With scores the
 // merge is part of the score launch, which needs the splits' factors anyway (u4: its scores come from logits and final
-// values).  Wide groups cut into many splits keep the merge launch (`fold_pays`).
+// values).  Wide groups cut into many splits keep the merge launch (`fold_pays`), and so do launches of more workgroups than
+// run at once: there a workgroup that folds, or waits for its partials to arrive, keeps the next one from starting (over f16,
+// 32 / 8 heads, D = 128, 33 sequences of 5000 tokens in 8 splits 131.2 us per layer, with the merge launch 123.5; 37 of 1000 in 4
+// 41.7 / 38.0; 28 / 4 heads, 70 of 2500 in 5 80.1 / 73.7; over u8 up to 2 %; but over u4, whose workgroups wait for the vector unit,
+// 24 of 100 - 4000 in 4 30.1 / 31.6).
 int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, int32_t rows, bool u4) {
+    const int64_t slots = ctx->cfg.head_size > 128 ? 256 : 512;
     if (a.nsplit <= 1 || (a.want_scores && !u4) || !pa::fold_pays(rows, ctx->cfg.head_size, a.nsplit)) return nullptr;
+    if (!u4 && (int64_t)a.n_seqs * ctx->cfg.num_kv_heads * a.nsplit > slots) return nullptr;
     return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(ctx->items.p) + ctx->arrived_off);
 }
 

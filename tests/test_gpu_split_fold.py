@@ -14,6 +14,7 @@ CASES = [
     ("f16", "f16", 32, 16, 8, 256, [2500], 0), ("bf16", "bf16", 256, 6, 2, 96, [700, 701, 1], 600),
     ("f16", "u8", 32, 8, 1, 64, [4000], 0), ("bf16", "bf16", 32, 12, 1, 128, [1000, 40], 0),  # the most rows and splits a launch folds
     ("f16", "u8", 32, 16, 1, 128, [40000], 0), ("f16", "f16", 32, 7, 1, 128, [1990], 0),      # too many for that: a merge launch
+    ("f16", "f16", 32, 16, 8, 128, [1000] * 37, 0),                                            # ... and of more than a round of workgroups
 ]
 
 
@@ -29,7 +30,8 @@ def test_split_fold(pkg, qd, kd, bs, Hq, Hkv, D, past, sw):
     assert ns > 1
     # one workgroup's trips to the partials: 256 pairs of channels, eight splits each
     passes, trips = -(-(Hq // Hkv) * D // 512), -(-ns // 8)
-    assert ("fold" in got["op"].kernels_run) == (trips <= 4 if passes == 1 else passes * trips <= 3), (ns, passes, trips)
+    one_round = len(past) * Hkv * ns <= (256 if D > 128 else 512)
+    assert ("fold" in got["op"].kernels_run) == (one_round and (trips <= 4 if passes == 1 else passes * trips <= 3)), (ns, passes, trips)
     H.assert_close(got["out"], ref["out"], qd)
     again = H.run_case_on_gpu(pkg, case, dev, want_scores=False, op=got["op"])
     assert np.array_equal(got["out16"], again["out16"])
