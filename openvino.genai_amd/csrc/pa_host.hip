@@ -192,7 +192,8 @@ struct pa_ctx {
     struct DecPlan { int32_t nsplit = 1, max_tiles = 1, waves = 4; } dec_plan[2];
     size_t desc_off[2] = {0, 0};       // byte offsets of the two descriptor arrays in a table's buffer
     int32_t kernels_run = 0;     // PA_RAN_* of the last attention call
-    bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams (else one after the other)
+    bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams also in calls without scores
+                                 // (else one after the other)
     std::vector<int32_t> h_few;  // every sequence of a step of few-token sequences, longest context first (else empty)
     DecPlan few_plan;
     int32_t few_rows = 0;        // most (token, head) rows of one per kv head
@@ -644,7 +645,9 @@ void plan_items(pa_ctx* ctx) {
     // 1 - 60 single tokens at 100 - 32768 positions beside 64 - 2048 chunk tokens (0.5 - 45 GFLOP) run 6 % faster one after the other
     // in the mean, but 8 x 1000 - 26667 beside 256 tokens 259 / 222 us per layer, 16 x 500 - 8000 126 / 115.  With
     // contexts of 4000 and more whose mean is below 0.75 of the longest side by side, one of them loses more than 4 % against side by
-    // side always (4.4 %), without that clause 27 (up to 17 %).  Over u8, whose decode kernel leaves more of a CU to its neighbour, 75 / 75 at 4 GFLOP
+    // side always (4.4 %), without that clause 27 (up to 17 %).  With scores, whose kernels lie between the two then, 422 such steps
+    // are no faster one after the other (0.95 - 1.03 of the time by head shape) and 109 of them more than 4 % and up to 20 % slower:
+    // side by side always.  Over u8, whose decode kernel leaves more of a CU to its neighbour, 75 / 75 at 4 GFLOP
     // beside 55 MB of single tokens' rows, 126 / 119 at 10 beside 187 MB, 274 / 270 at 84: always.
     {
         double flops = 0, positions = 0;
@@ -938,7 +941,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     // (a step whose two kernels are too short for that, see plan_items: the same kernels one after the other)
     bool forked = false;
     auto fork_side = [&]() -> hipStream_t {
-        if (!ctx->fork_pays) return ctx->stream;
+        if (!ctx->fork_pays && !io->scores) return ctx->stream;
         if (!ctx->side) {
             HIP_CHECK(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
             HIP_CHECK(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));

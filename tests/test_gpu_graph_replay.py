@@ -10,11 +10,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kv,past,new", [("u8", [700, 64, 1300, 31], [1, 1, 1, 1]),       # decode kernel, one split
                                          ("u8", [9000], [1]),                             # several splits + merge
-                                         ("bf16", [300, 40, 0], [1, 1, 70]),              # matrix kernel, mixed step
+                                         ("bf16", [300, 40, 0], [1, 1, 70]),              # 16-bit decode kernel on the second stream beside the matrix kernel
                                          ("u8", [300, 40, 0], [1, 1, 70]),                # decode kernel on the second stream beside the matrix kernel
                                          ("bf16", [700, 64, 1300, 31], [1, 1, 1, 1]),     # 16-bit decode kernel (appends too)
                                          ("bf16", [9000, 20], [1, 1]),                    # the same with several splits
-                                         ("bf16", [6000, 40, 0], [1, 1, 70])])            # on the second stream beside the matrix kernel
+                                         ("bf16", [6000, 40, 0], [1, 1, 70])])            # the same, several splits
 def test_graph_replays_equal_eager(pkg, kv, past, new):
     import torch
     dev = torch.device("cuda:0")
@@ -38,7 +38,7 @@ def test_graph_replays_equal_eager(pkg, kv, past, new):
                 op.forward(qd, kd, vd, kc[l], vc[l], outs[l], scores[l], layer=l)
 
         step()  # eager: also sizes every workspace
-        assert ("side_stream" in op.kernels_run) == (max(new) > 1 and (kv == "u8" or past[0] == 6000))
+        assert ("side_stream" in op.kernels_run) == (max(new) > 1)  # (with scores: every mixed step)
         s.synchronize()
         want_out = [o.clone() for o in outs]
         want_sc = [x.clone() for x in scores]
