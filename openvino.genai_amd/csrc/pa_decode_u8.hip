@@ -158,17 +158,17 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
 //   * scores: the scaled logits go to `logits` in f32 and become scores in a kernel of their own, as for the
 //     shape-generic path that serves the other u4 steps; no probability is rounded to 16 bits on the way.
 // Bound by vector instructions (at 186 registers two waves a SIMD; capped at 168 for three the kernel spills and takes 56
-// instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 45 us per layer of a
-// step through the Python binding, where the shape-generic kernel, one lane to a row, took 178 (149 + 17 us and an append launch of 5).
+// instead of 28 us): 32 sequences of 256 - 4096 tokens (32 / 8 heads, D = 128, bf16 queries, 75 MB of rows) in 34 us, the fold
+// of its four splits included, where the shape-generic kernel, one lane to a row, took 149 + 17 us and an append launch of 5.
 // COLS: 0 for sequences of one token each, whose group's heads are the columns of the matrix products.  1 or 2: sequences of a
 // few tokens (the validation step of speculative decoding or prompt lookup), up to 16 * COLS (token, head) columns that share
 // every cache byte; a column sees the positions up to its own token.  The append has run before, there are no scores.  Codes are
 // centred (128) and normal, weights scaled up and a tile's products added to the running sums in f32, as over u4 rows: the matrix
 // kernel, which takes these sequences when scores are wanted, centres each row's codes (as subnormals) and is no closer.  Five
 // tokens behind 500 - 4000 over f16 queries miss the correctly rounded result in 0.25 % of the outputs, on the matrix kernel in
-// 3.0 %, with plain subnormal codes in 9.7 %; behind 32000 in 0.3, 7.4 and 24 %.  A centre per row: 0.19 %, but 10 % slower.
-// 16 sequences of 500 - 4000 tokens x 5 new ones (32 / 8 heads, D = 128): 31.7 us in 4 parts (78 MB: 2.5 TB/s, bound by the
-// vector instructions of two softmaxes per tile); the matrix kernel took 51 + 5 us of merge.
+// 3.0 %, with plain subnormal codes in 9.7 %; behind 32000 in 0.3, 7.4 and 24 %.  A centre per row: 0.19 %, but 4 - 10 % slower.
+// 16 sequences of 500 - 4000 tokens x 5 new ones (32 / 8 heads, D = 128): 30 us in 4 parts and 5 of merge (78 MB: 2.6 TB/s, bound by
+// the vector instructions of two softmaxes per tile); the matrix kernel took 51 + 5 us.
 template <int D, int QDT, int WAVES, int BS, bool U4, int COLS>
 // (head size 256: one workgroup per CU, whose waves may then use the accumulation registers as well -- 16 KB blocks,
 // two of them in flight, 64 accumulators and 32 query registers do not fit 256 registers)

@@ -486,11 +486,12 @@ void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, in
             // (u4 rows, counts of 1 - 32 forced over batches of 1 - 128 sequences and contexts of 512 - 32768 tokens: 0.33 and
             // 0.49 us per tile -- vector instructions, whatever the bytes -- and 0.0105 us per further workgroup; the counts
             // these give are within 5 % of the best forced one, 14 % for 128 sequences of 128 - 8000 tokens.  With the u8
-            // figures 32 sequences of 256 - 4096 tokens were cut in 2 instead of 4: 49.3 against 41.9 us per layer)
+            // figures 32 sequences of 256 - 4096 tokens were cut in 2 instead of 4: 49.3 against 41.9 us per layer; before the codes
+            // were centred, which adds 4 %)
             // (few-token sequences, counts of 1 - 24 forced over batches of 1 - 64 sequences: the partial rows of up to 32 columns
             // make a further workgroup as dear as three of the single-token kernel, and a second round of them never
             // paid: 16 sequences of 500 - 4000 tokens x 5 in 1 / 2 / 3 / 4 / 5 / 8 parts 61.0 / 47.4 / 48.2 / 41.7 / 51.5 /
-            // 55.0 us per layer, 64 of 4096 x 4 in 1 / 2 / 3 parts 110 / 127 / 142)
+            // 55.0 us per layer, 64 of 4096 x 4 in 1 / 2 / 3 parts 110 / 127 / 142; before the codes were centred, which adds 2 - 6 %)
             const double t2 = few ? 0.40 * dscale : u4 ? 0.49 * dscale : (u8 ? (sc ? 0.525 : 0.468) : (sc ? 1.104 : 1.064)) * dscale;
             const double t1 = slots == 256 ? t2 / 2 : few ? 0.38 * dscale : u4 ? 0.33 * dscale : (u8 ? (sc ? 0.316 : 0.276) : (sc ? 0.495 : 0.478)) * dscale;
             const double tile_bytes = 2.0 * 32 * pa::row_bytes(c.head_size, c.kv_cache_dtype), bw = sc && !u4 ? 5.9e6 : 6.97e6;
