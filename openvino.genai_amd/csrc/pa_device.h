@@ -460,6 +460,7 @@ struct PrefillArgs {
     int32_t n_merge;
     int32_t n_items;
     int32_t n_wide;               // the first n_wide items have more than 16 query rows, the others at most 16
+    int32_t widened;              // u8 caches: the n_wide items are the straight-to-LDS kernel's, over widened rows
     int32_t G;                    // query heads per kv head
     int32_t max_split;            // stride of the partial buffers
     uint16_t* out;
@@ -482,6 +483,27 @@ struct PrefillArgs {
     // nothing is left (the score replay serves those sequences).
     _Float16* p_out;              // [tiles][Hq][32]: a sequence's tiles start at tile_max_offset(score offset, b)
     float* tile_max;              // [tiles][Hq]
+    // u8 rows widened for the straight-to-LDS kernel (pa_prefill_dense.hip), whose key_cache and value_cache they are
+    const uint8_t *wide_k, *wide_v;  // [widened tiles][Hkv][32][128] f16
+    const float* wide_hdr;        // [widened tiles][Hkv][4][32]
+    const int32_t* wide_tile0;    // [B]: a sequence's widened tile t is number wide_tile0 + t
+};
+// u8 rows of the listed sequences as f16 integers for the straight-to-LDS kernel (pa_prefill_dense.hip): blocks lo .. hi - 1 of
+// sequence b become the widened tiles tile0 + lo .. tile0 + hi - 1.
+constexpr size_t WIDE_TILE_BYTES = 32 * 128 * 2;                            // of K or V of a (block, kv head)
+constexpr size_t WIDE_BLOCK_BYTES = 2 * WIDE_TILE_BYTES + 4 * 32 * 4;       // ... of both and the headers
+struct WidenSeq {
+    int32_t b, lo, hi, tile0;
+};
+struct WidenArgs {
+    StepDev st;
+    Shape sh;
+    const uint8_t *key_cache, *value_cache;
+    const int32_t* block_indices;
+    const WidenSeq* seqs;         // [n_seqs]
+    int32_t n_seqs, max_tiles;    // most blocks of one
+    uint8_t *wide_k, *wide_v;     // [tiles][Hkv][32][D] f16
+    float* wide_hdr;              // [tiles][Hkv][4][32]
 };
 // What an item of a single-token sequence may keep in LDS: 64 G bytes of probabilities and 4 G of maxima per tile.
 constexpr int SINGLE_STASH_BYTES = 20480;
@@ -729,6 +751,8 @@ __device__ __forceinline__ void single_scores_rows(const StepDev& st, const Shap
 }
 #endif
 // merge_later: the fold of the rows cut into ranges is left to the caller (`launch_scores_replay` takes it along).
+hipError_t launch_widen(hipStream_t s, const WidenArgs& a);
+hipError_t launch_prefill_dense(hipStream_t s, const PrefillArgs& a, int q_dtype, bool widened);
 hipError_t launch_prefill16(hipStream_t s, const PrefillArgs& a, int q_dtype, int kv_dtype, hipEvent_t ev0,
                             hipEvent_t ev1, bool merge_later = false);
 

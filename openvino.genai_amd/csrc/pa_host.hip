@@ -50,6 +50,23 @@ struct DevBuf {
         HIP_CHECK(hipMalloc(&p, want));
         cap = want;
     }
+    // ... for what the step can do without: false, with nothing held, if there is no memory for it
+    bool try_reserve(size_t bytes) {
+        if (bytes <= cap) return true;
+        if (p) {
+            HIP_CHECK(hipDeviceSynchronize());
+            HIP_CHECK(hipFree(p));
+        }
+        p = nullptr;
+        cap = 0;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        cap = bytes;
+        return true;
+    }
     void release() {
         if (p) (void)hipFree(p);
         p = nullptr;
@@ -117,6 +134,9 @@ bool kv_alike(const pa_config& c) {
 constexpr size_t STATIC_SCRATCH_BYTES = PA_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) uint8_t scratch[STATIC_SCRATCH_BYTES];
 
+// Most a context keeps of widened u8 rows (16.5 KB per 32 tokens and kv head: half a million tokens of eight kv heads)
+constexpr size_t MAX_WIDE_BYTES = (size_t)2 << 30;
+
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mutex;
 void* g_scratch_ptr[MAX_DEVICES] = {};
@@ -166,6 +186,8 @@ struct pa_ctx {
     std::vector<int32_t> h_dec;
     std::vector<int32_t> h_dec16;     // single-token sequences of a 16-bit-cache step (also listed as matrix-kernel items)
     DevBuf dec16_list;
+    std::vector<pa::WidenSeq> h_wide;
+    std::vector<int32_t> h_wide_tile0;
     std::vector<int32_t> h_multi;     // sequences that schedule more than one token
     DevBuf multi_list;
     size_t arrived_off = 0;  // in `items`: decode launches that fold their own splits count here, per (listed sequence, kv head)
@@ -173,6 +195,10 @@ struct pa_ctx {
     bool dec_in_order = false, dec16_in_order = false;  // the lists hold 0 .. B-1 in order: every sequence, none moved
     bool stash_ok = false;  // the step's single-token items are short enough to keep their probabilities in LDS
     int32_t n_items = 0, n_wide = 0, max_split = 1;
+    // u8 caches: the rows that the step's dense chunks see, widened for the straight-to-LDS matrix kernel
+    DevBuf wide;                      // K rows | V rows | headers of the widened tiles
+    size_t wide_blocks = 0, wide_seqs_off = 0, wide_tile0_off = 0;
+    int32_t n_wide_seqs = 0, wide_max_tiles = 0;
     size_t tok_nsplit_off = 0;
     // single-token sequences the matrix kernel may take (16-bit caches): their work items, and behind the split
     // counts a per-sequence flag array (for the call that hands them to the decode kernel instead)
@@ -605,6 +631,40 @@ void stage_upload(pa_ctx* ctx, void* dst, const void* src, size_t bytes) {
     HIP_CHECK(hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, ctx->stream));
 }
 
+// u8 caches, head size 128: which sequences' rows are widened to f16 integers ahead of the matrix kernel (n_wide_seqs, all of
+// the step's dense chunks, or none).  The kernel that walks widened rows saves about 0.75 ns per (query tile, KV block, kv head)
+// over the one that widens them on their way to LDS; widening takes about 1.7 ns per (KV block, kv head), once, and 3 us for the
+// launch.  us per layer as a step, widened / not: 32 / 8 heads, 512 tokens behind 1000 65.6 / 72.4, behind 8000 175 / 202, 2048
+// behind 8000 526 / 644, 128 behind 8000 99.6 / 100, 33 behind 8000 79.8 / 74.2; 28 / 4 heads, 256 behind 1000 54.6 / 51.6, behind
+// 8000 111 / 121; 32 heads without grouping, 512 behind 1000 78 / 74, 2048 behind 1000 183 / 197.
+void plan_widen(pa_ctx* ctx) {
+    const pa_config& c = ctx->cfg;
+    const int32_t B = ctx->B, G = c.num_heads / c.num_kv_heads, QT = std::max(1, 128 / G), sw = ctx->sliding_window;
+    const int32_t *past = ctx->h_past.data(), *sb = ctx->h_sb.data();
+    ctx->n_wide_seqs = 0;
+    ctx->h_wide.clear();
+    if (c.head_size != 128 || c.kv_cache_dtype != PA_U8 || !mfma_shape(ctx)) return;
+    ctx->h_wide_tile0.assign(B, 0);
+    ctx->wide_max_tiles = 0;
+    int64_t blocks = 0, tiles = 0;  // KV blocks to widen, and such blocks walked by the query tiles
+    for (int32_t b = 0; b < B; ++b) {
+        const int32_t q_len = sb[b + 1] - sb[b];
+        if (q_len * G <= 16 || q_len == 1 || xatt_seq_index(ctx, b) >= 0) continue;
+        const int32_t lo = (sw > 0 ? std::max(0, past[b] + 1 - sw) : 0) / 32, hi = (past[b] + q_len + 31) / 32;
+        ctx->h_wide_tile0[b] = (int32_t)blocks - lo;
+        ctx->h_wide.push_back({b, lo, hi, (int32_t)blocks - lo});
+        ctx->wide_max_tiles = std::max(ctx->wide_max_tiles, hi - lo);
+        blocks += hi - lo;
+        for (int32_t q0 = 0; q0 < q_len; q0 += QT)
+            tiles += (past[b] + std::min(q0 + QT, q_len) - 1) / 32 + 1 - (sw > 0 ? std::max(0, past[b] + q0 + 1 - sw) : 0) / 32;
+    }
+    if (tiles * c.num_kv_heads < 3500 + 2.3 * blocks * c.num_kv_heads) return;
+    const size_t bytes = (size_t)blocks * c.num_kv_heads * pa::WIDE_BLOCK_BYTES;
+    if (ctx->h_wide.empty() || bytes > MAX_WIDE_BYTES || !ctx->wide.try_reserve(bytes)) return;
+    ctx->wide_blocks = (size_t)blocks;
+    ctx->n_wide_seqs = (int32_t)ctx->h_wide.size();
+}
+
 void plan_items(pa_ctx* ctx) {
     const int32_t B = ctx->B, T = ctx->T;
     const int32_t* past = ctx->h_past.data();
@@ -665,6 +725,7 @@ void plan_items(pa_ctx* ctx) {
         }
         ctx->fork_pays = !narrow_all || flops >= 45e9 || (longest >= 4000 && positions < 0.75 * longest * singles);
     }
+    plan_widen(ctx);
     size_t planned_tiles = 0;
     for (int32_t b = 0; b < B; ++b) {
         const int32_t q_len = sb[b + 1] - sb[b];
@@ -729,6 +790,8 @@ void plan_items(pa_ctx* ctx) {
         for (int32_t i = 0; i < t.nq; ++i) tok_ns[sb[t.b] + t.q0 + i] = ns;
         max_split = std::max(max_split, ns);
     }
+    for (const pa::PrefillItem& it : items)  // (the LDS table of the straight-to-LDS kernel)
+        PA_REQUIRE(it.te - it.tb <= 128, PA_UNKNOWN_EXCEPTION, "a matrix work item walks more than 128 KV blocks");
     // Workgroups start in list order and a CU slot works through two or three of them in a launch: the dense items of
     // multi-token sequences are listed longest first (within the wide and the narrow group), so that no long item
     // starts last and finishes alone.
@@ -817,6 +880,13 @@ void plan_items(pa_ctx* ctx) {
     tok_ns.insert(tok_ns.end(), single_idx.begin(), single_idx.end());
     for (int32_t t = 0; t < T; ++t)
         if (tok_ns[t] > 1) tok_ns.push_back(t);
+    if (ctx->n_wide_seqs > 0) {
+        ctx->wide_tile0_off = item_bytes + tok_ns.size() * sizeof(int32_t);
+        tok_ns.insert(tok_ns.end(), ctx->h_wide_tile0.begin(), ctx->h_wide_tile0.end());
+        ctx->wide_seqs_off = item_bytes + tok_ns.size() * sizeof(int32_t);
+        const int32_t* ws = reinterpret_cast<const int32_t*>(ctx->h_wide.data());
+        tok_ns.insert(tok_ns.end(), ws, ws + 4 * ctx->h_wide.size());
+    }
     ctx->single_idx_off = item_bytes + (size_t)T * sizeof(int32_t);
     ctx->merge_tok_off = ctx->single_idx_off + (size_t)B * sizeof(int32_t);
     ctx->arrived_off = item_bytes + tok_ns.size() * sizeof(int32_t);
@@ -1076,6 +1146,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.tok_nsplit = reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(ctx->items.p) + ctx->tok_nsplit_off);
         a.n_items = ctx->n_items;
         a.n_wide = ctx->n_wide;
+        a.widened = ctx->n_wide_seqs > 0 ? 1 : 0;
         a.G = c.num_heads / c.num_kv_heads;
         a.max_split = ctx->max_split;
         a.out = static_cast<uint16_t*>(io->out);
@@ -1124,6 +1195,27 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         // Single-token sequences that are work items of this launch (16-bit caches, next to dense chunks): with scores
         // wanted the kernel leaves their probabilities for a small score kernel, instead of a replay that reads all
         // their K rows once more.
+        if (ctx->n_wide_seqs > 0) {  // u8 rows of the dense chunks as f16 integers
+            const size_t slots = ctx->wide_blocks * c.num_kv_heads;
+            const uint8_t* lists = static_cast<const uint8_t*>(ctx->items.p);
+            pa::WidenArgs w{};
+            w.st = ctx->dev;
+            w.sh = a.sh;
+            w.key_cache = a.key_cache;
+            w.value_cache = a.value_cache;
+            w.block_indices = table;
+            w.seqs = reinterpret_cast<const pa::WidenSeq*>(lists + ctx->wide_seqs_off);
+            w.n_seqs = ctx->n_wide_seqs;
+            w.max_tiles = ctx->wide_max_tiles;
+            w.wide_k = ctx->wide.as<uint8_t>();
+            w.wide_v = w.wide_k + slots * pa::WIDE_TILE_BYTES;
+            w.wide_hdr = reinterpret_cast<float*>(w.wide_v + slots * pa::WIDE_TILE_BYTES);
+            HIP_CHECK(pa::launch_widen(ctx->stream, w));
+            a.wide_k = w.wide_k;
+            a.wide_v = w.wide_v;
+            a.wide_hdr = w.wide_hdr;
+            a.wide_tile0 = reinterpret_cast<const int32_t*>(lists + ctx->wide_tile0_off);
+        }
         const bool hand_over = io->scores && ctx->stash_ok && !use_decode16 && ctx->n_single > 0;
         if (hand_over) {
             const size_t tiles = (size_t)pa::tile_max_count(ctx->total_scores, ctx->B);
@@ -1240,6 +1332,7 @@ void pa_destroy(pa_ctx* ctx) {
     ctx->x_sums.release();
     ctx->x_mask.release();
     ctx->x_item_keep.release();
+    ctx->wide.release();
     if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);

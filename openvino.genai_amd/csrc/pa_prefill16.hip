@@ -12,7 +12,7 @@
 // items stay comparable in length; their partial (max, denominator, accumulator) rows are merged
 // by a second kernel.
 // KV blocks (32 tokens) travel global -> registers (two or three blocks in flight per thread) -> LDS (two K
-// slots, four V slots, one barrier per block), or straight into LDS; K rows are read back as MFMA A operands with
+// slots, four V slots, one barrier per block); K rows are read back as MFMA A operands with
 // ds_read_b128, V rows through the LDS transpose read (ds_read_b64_tr_b16), which hands each lane
 // four consecutive tokens of one channel.  A block is worked through in one go: QK, softmax, rescale, PV.
 //   S^T[token][row] = K . Q^T          v_mfma_f32_16x16x32_{f16,bf16}
@@ -26,7 +26,7 @@
 // it kept instead of its whole range.
 //
 // Roofline: dense MFMA.  Flops per (query row, visible position): 4 * D.
-#include "pa_device.h"
+#include "pa_prefill.h"
 
 #include <climits>
 #include <type_traits>
@@ -34,86 +34,8 @@
 namespace pa {
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef short s8v __attribute__((ext_vector_type(8)));
-typedef short s4v __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-
-constexpr int TOK = 32;
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float LN2 = 0.6931471805599453f;
-
-template <int DT>
-__device__ __forceinline__ f4 mma(const s8v& a, const s8v& b, const f4& c) {
-    if (DT == DT_F16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ s4v lds_read_tr16(const uint8_t* p) {
-    typedef s4v __attribute__((address_space(3))) * lds_ptr;
-    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p);
-}
-
-// Reductions over the four 16-lane groups of a wave with the gfx950 lane-swap instructions (no LDS round trip):
-// v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of the second,
-// v_permlane32_swap the upper half of the first with the lower half of the second.  With both operands holding
-// the same value the pair afterwards holds, per lane, the values of the two rows (halves) being combined.
-__device__ __forceinline__ void swap_rows16(float& a, float& b) {
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-__device__ __forceinline__ void swap_halves32(float& a, float& b) {
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-// (the maxima as instructions of their own: behind the lane swaps the compiler no longer knows its operands to be
-// ordinary numbers and puts a quieting `v_max x, x, x` in front of every fmaxf)
-__device__ __forceinline__ float max_raw(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float xor_max_g(float v) {
-    float a = v, b = v;
-    swap_rows16(a, b);
-    a = b = max_raw(a, b);
-    swap_halves32(a, b);
-    return max_raw(a, b);
-}
-__device__ __forceinline__ float xor_sum_g(float v) {
-    float a = v, b = v;
-    swap_rows16(a, b);
-    a = b = a + b;
-    swap_halves32(a, b);
-    return a + b;
-}
-
-// acc + the two 16-bit floats of `w` (one instruction: a dot product with (1, 1))
-template <int DT>
-__device__ __forceinline__ float add_pair(uint32_t w, float acc) {
-    if (DT == DT_F16) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, w), __builtin_bit_cast(h2, 0x3c003c00u), acc, false);
-    }
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, w), __builtin_bit_cast(b2, 0x3f803f80u), acc, false);
-}
-
-// f32 -> cache-type bits, two values at a time
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if (DT == DT_F16) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
-    }
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
-}
-
 // ---- KV block fetches -------------------------------------------------------------------------------------
-// Through registers (u8 caches, whose rows are transformed on the way to LDS; block-sparse items; head size 64):
-// ordinary loads into three register sets, three blocks in flight per thread; the compiler counts the outstanding
+// Through registers: ordinary loads into three register sets, three blocks in flight per thread; the compiler counts the outstanding
 // loads itself (it waits for the oldest set only).  Every step issues the same loads per thread: tile indices are
 // clamped rather than skipped.
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
@@ -140,79 +62,42 @@ __device__ __forceinline__ void kv_issue(KvRegs<true>& r, const uint8_t* krow, c
     r.vh = *reinterpret_cast<const u2v*>(vrow);
 }
 
-// Straight into LDS (dense items over 16-bit caches, head size 128): one instruction moves 64 x 16 bytes from
-// per-lane global addresses to 1024 consecutive bytes of LDS at a wave-uniform address; no registers, no LDS stores.
-__device__ __forceinline__ void dma16(const uint8_t* src, uint8_t* lds_dst) {
-    typedef __attribute__((address_space(3))) void* lds_p;
-    typedef const __attribute__((address_space(1))) void* glb_p;
-    __builtin_amdgcn_global_load_lds((glb_p)src, (lds_p)lds_dst, 16, 0, 0);
-}
-// Waits until at most N of the wave's vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14; the other counters left at their maxima).
-// Workgroup barrier for LDS traffic only.  __syncthreads() (and a workgroup fence of any kind) makes the compiler wait
-// for every copy into LDS that is in flight, the prefetched blocks included; here the wave waits for its own LDS
-// operations, meets the others, and the copies it must have finished are named by the caller (wait_vmem).  The
-// barrier instruction and the empty asm statements keep the compiler from moving LDS accesses across.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); vmcnt and expcnt at their maxima
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-    __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | 0x0f70);
-}
-
 // DT: type of the MFMA operands and of the rows staged in LDS; QDT: type of query and output; U8: the cache holds
 // `f32 scale | f32 zero-point | D codes` rows; codes go to LDS as 16-bit words, headers to a small table beside them.
 // NG: 16-row groups per wave.  1 = up to 128 query rows per 512-thread workgroup, the variant for mixed steps over
 // 16-bit caches and for work items with few rows (single-token sequences: G rows), where a second group would only cost
-// arithmetic; it fits four waves per SIMD over 16-bit caches.  2 = 32 rows per wave (the 256-thread variants below).
+// arithmetic; it fits four waves per SIMD over 16-bit caches.  2 = 32 rows per wave (the 256-thread variant below).
 // A block is worked through in one go: QK, softmax, rescale, PV.
 // XATT: the work items belong to block-sparse sequences.
 // HALF: 256-thread workgroups of 128 rows whose KV blocks go through registers, two load units per thread (u8 caches,
 // whose codes are widened on the way to LDS): two such workgroups share a CU and fill in for each other at the
 // barriers.  (One 512-thread workgroup of 256 rows per CU, with a three-block software pipeline inside each wave, took
 // 0.296 ms for what this variant does in 0.255 ms: a third of the launch had neither pipe busy.)
-// DMA: 256-thread workgroups whose KV blocks go straight from global memory into LDS (four K and four V slots, three
-// blocks in flight behind the one being worked on).  Rows sit in LDS unpadded; instead the 16-byte pieces of a row are
-// permuted: K row r keeps piece p at position p ^ (r & 15) (16 lanes read one piece of 16 rows), V row r at
-// p ^ 2 (r & 7) (the transpose read takes 32 bytes of each of four consecutive rows), which keeps both operand reads
-// free of bank conflicts -- the permutation is applied on the global side of the copy, each lane fetching the piece
-// that belongs at its LDS position.  With no
-// staging registers the kernel fits three waves per SIMD at two 16-row groups per wave: half the LDS operand traffic
-// per matrix instruction of the one-group variant.
-template <int D, int DT, int QDT, bool U8, int NG, bool XATT, bool DMA, bool HALF = false>
-__global__ __launch_bounds__((DMA || HALF) ? 256 : 512, D > 128 ? 1 : (DMA || HALF) ? 2 : U8 ? 2 : (XATT && DT == DT_F16 && D == 128) ? 3 : 4)
+// Dense chunks at head size 128 over 16-bit caches, and the long ones over u8 caches, are pa_prefill_dense.hip's.
+template <int D, int DT, int QDT, bool U8, int NG, bool XATT, bool HALF = false>
+__global__ __launch_bounds__(HALF ? 256 : 512, D > 128 ? 1 : HALF ? 2 : U8 ? 2 : (XATT && DT == DT_F16 && D == 128) ? 3 : 4)
 void pa_prefill16_kernel(PrefillArgs a) {
     static_assert(!U8 || DT == DT_F16, "u8 codes are multiplied as f16");
     static_assert(U8 || DT == QDT, "16-bit caches are used in the query's type");
-    static_assert(!DMA || (!U8 && !XATT && D == 128), "the straight-to-LDS variant: dense items, 16-bit caches, head size 128");
-    static_assert(!(DMA && HALF) && (!HALF || (NG == 2 && !XATT)), "the register variant of 256 threads: dense items, two row groups per wave");
-    constexpr int NT = (DMA || HALF) ? 256 : 512;
+    static_assert(!HALF || (NG == 2 && !XATT), "the register variant of 256 threads: dense items, two row groups per wave");
+    constexpr int NT = HALF ? 256 : 512;
     constexpr int NCH = TOK * (D * 2 / 16);  // 16-byte chunks (eight codes of a u8 row) per block and tensor: 512 (D = 128) or 256 (D = 64)
     constexpr int UPT = (NCH + NT - 1) / NT;  // load units (a chunk, or eight codes and a row header) per thread and tensor
     constexpr int ROWB = D * 2;            // bytes of a row as staged in LDS
     constexpr int CROWB = U8 ? D + 8 : D * 2;  // bytes of a row in the cache
-    constexpr int LROWK = DMA ? ROWB : ROWB + 16;  // LDS row strides chosen so that the operand reads are bank-conflict free:
-    constexpr int LROWV = DMA ? ROWB : ROWB + 32;  // K rows are read 16 B per lane, V rows 32 B per 4 lanes (transpose read)
+    constexpr int LROWK = ROWB + 16;  // LDS row strides chosen so that the operand reads are bank-conflict free:
+    constexpr int LROWV = ROWB + 32;  // K rows are read 16 B per lane, V rows 32 B per 4 lanes (transpose read)
     constexpr int TILEK = TOK * LROWK, TILEV = TOK * LROWV;
-    constexpr int NKS = DMA ? 4 : 2, NVS = 4;  // K and V slots
+    constexpr int NKS = 2, NVS = 4;  // K and V slots
     constexpr int KS = D / 32;
     constexpr int RT = D / 16;
     constexpr int CPR = ROWB / 16;         // 16-byte chunks per row
-    static_assert(DMA || NCH <= NT * UPT, "one chunk per load unit");
+    static_assert(NCH <= NT * UPT, "one chunk per load unit");
     constexpr int HDRB = U8 ? 4 * TOK * 4 : 0;  // per buffer: sc_k * scl | zp_k * sc_k | sc_v | zp_v, one f32 per token each
     constexpr float CODE_UNIT = 16777216.0f;    // a code byte read as f16 is code * 2^-24
     // Block t+1 is read while block t+2 is written: two K slots; the V and header slots are indexed modulo four.
     constexpr int OFF_V = NKS * TILEK, OFF_H = NKS * TILEK + NVS * TILEV;
-    __shared__ __align__(16) uint8_t smem[DMA ? 16 : NKS * TILEK + NVS * TILEV + 4 * HDRB];  // K slots | V slots | headers[4]
-    // DMA: every slot is an LDS object of its own, so that the compiler can tell a copy into one slot from the operand
-    // reads of another (it orders reads after the copies that may have written what they read; with one array for all
-    // slots that would be every copy in flight, the prefetched blocks included)
-    __shared__ __align__(16) uint8_t dk0[DMA ? TILEK : 16], dk1[DMA ? TILEK : 16], dk2[DMA ? TILEK : 16], dk3[DMA ? TILEK : 16];
-    __shared__ __align__(16) uint8_t dv0[DMA ? TILEV : 16], dv1[DMA ? TILEV : 16], dv2[DMA ? TILEV : 16], dv3[DMA ? TILEV : 16];
+    __shared__ __align__(16) uint8_t smem[NKS * TILEK + NVS * TILEV + 4 * HDRB];  // K slots | V slots | headers[4]
     auto kslot = [](int j) { return (j & 1); };
     auto vslot = [](int j) { return (j & (NVS - 1)); };
 
@@ -434,7 +319,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
     // and the workgroup writes them out behind the loop.  (A store inside the loop would make every wait for a block
     // fetch a wait for all of them: loads and stores share a counter and complete out of order with respect to each
     // other.)  The host keeps such items at single_item_max_tiles(G) tiles.
-    constexpr bool STASH = !U8 && !XATT && !DMA && NG == 1;
+    constexpr bool STASH = !U8 && !XATT && NG == 1;
     __shared__ __align__(16) uint8_t pkeep[STASH ? SINGLE_STASH_BYTES : 16];
     bool emit = false;
     if constexpr (STASH) emit = a.p_out != nullptr && a.single_idx[b] >= 0;
@@ -448,8 +333,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
     // V operands come through the LDS transpose read: source lane (e = n >> 2, q = n & 3) of a 16-lane group
     // supplies 4 channels of token 16 h + 4 g + e; lane n receives channel 16 r + n of tokens 16 h + 4 g + 0..3.
     auto load_v = [&](const uint8_t* vb, int r) __attribute__((always_inline)) {
-        const uint8_t* p0 = DMA ? vb + (4 * g + (n >> 2)) * LROWV + (((2 * r + ((n & 3) >> 1)) ^ (((4 * g + (n >> 2)) & 7) << 1)) << 4) + 8 * (n & 1)
-                                : vb + (4 * g + (n >> 2)) * LROWV + (16 * r + 4 * (n & 3)) * 2;
+        const uint8_t* p0 = vb + (4 * g + (n >> 2)) * LROWV + (16 * r + 4 * (n & 3)) * 2;
         const s4v v0 = lds_read_tr16(p0);
         const s4v v1 = lds_read_tr16(p0 + 16 * LROWV);
         return s8v{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
@@ -466,8 +350,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
             if (do_qk && s < KS) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const s8v kop = DMA ? *reinterpret_cast<const s8v*>(kb + (16 * u + n) * LROWK + (((4 * s + g) ^ n) << 4))
-                                        : *reinterpret_cast<const s8v*>(kb + (16 * u + n) * LROWK + (32 * s + 8 * g) * 2);
+                    const s8v kop = *reinterpret_cast<const s8v*>(kb + (16 * u + n) * LROWK + (32 * s + 8 * g) * 2);
 #pragma unroll
                     for (int gi = 0; gi < NG; ++gi) sc[gi][u] = mma<DT>(kop, qreg[gi][s], sc[gi][u]);
                 }
@@ -753,80 +636,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
         whole_at(j, smem + kslot(j) * TILEK, smem + OFF_V + vslot(j) * TILEV);
     };
 
-    if constexpr (DMA) {
-        // Block number j lives in K slot and V slot j % 4.  A wave moves rows 8 wv .. 8 wv + 7 of a block: lane l of
-        // its two instructions per tensor takes row 8 wv + 4 i + l / 16, LDS piece position l % 16, i.e. the row's
-        // piece (l % 16) ^ (row & 15) of K, (l % 16) ^ 2 (row & 7) of V.  Every step issues the same four copies per
-        // wave (indices clamped), so that "at most eight outstanding" always means: everything but the two youngest
-        // blocks has landed.
-        const int wvs = __builtin_amdgcn_readfirstlane(wv);
-        const int my_row = 8 * wvs + (lane >> 4);         // + 4 for the second instruction
-        // per-lane byte offsets within a block (32 bits, added to a wave-uniform block address)
-        const uint32_t off_k0 = my_row * ROWB + (((lane & 15) ^ (my_row & 15)) << 4);
-        const uint32_t off_k1 = (my_row + 4) * ROWB + (((lane & 15) ^ ((my_row + 4) & 15)) << 4);
-        const uint32_t off_v0 = my_row * ROWB + (((lane & 15) ^ ((my_row & 7) << 1)) << 4);
-        const uint32_t off_v1 = (my_row + 4) * ROWB + (((lane & 15) ^ (((my_row + 4) & 7) << 1)) << 4);
-        const bool upper_half = wvs >= (NT / 64) / 2;  // this wave moves rows 16 - 31
-        // The table entry of a copy's block is read one step before the copy goes out, and nothing is computed from it
-        // until then: a scalar load that is waited for right behind its issue stalls the wave at every step.
-        auto table_index = [&](int tile) __attribute__((always_inline)) {
-            return bs16 ? min(2 * tile + (upper_half ? 1 : 0), last_block16) : tile >> sub_shift;
-        };
-        int id_next = table[table_index(tile_at(0))];
-        auto copy_in = [&](int j, uint8_t* kslot_base, uint8_t* vslot_base) __attribute__((always_inline)) {
-            const int tile = tile_at(j);
-            // (what tile_base gives for this wave's half of the tile, from the entry read a step ago)
-            const long blk = bs16 ? ((long)id_next * Hkv + hkv) * (16 * CROWB) - (upper_half ? 16 * CROWB : 0)
-                                  : ((long)id_next * Hkv + hkv) * ((long)a.sh.bs * CROWB) + (long)(tile & sub_mask) * (TOK * CROWB);
-            id_next = table[table_index(tile_at(j + 1))];
-            const uint8_t* kg = a.key_cache + blk;
-            const uint8_t* vg = a.value_cache + blk;
-            uint8_t* kd = kslot_base + wvs * 2048;
-            uint8_t* vd = vslot_base + wvs * 2048;
-            dma16(kg + off_k0, kd);
-            dma16(kg + off_k1, kd + 1024);
-            dma16(vg + off_v0, vd);
-            dma16(vg + off_v1, vd + 1024);
-        };
-        // The wait in front of a step's barrier names how many of the wave's vector-memory operations may still be
-        // outstanding: the copies of the two youngest blocks.  It is only right while a step issues exactly this many
-        // copies per wave and nothing else that counts (the table reads above are scalar loads; the build fails on
-        // spills, whose scratch traffic would count).
-        constexpr int COPIES_PER_STEP = 4;
-        static_assert(COPIES_PER_STEP == 2 * (TOK * ROWB / 1024) / (NT / 64), "copy_in issues one 1024-byte copy per 8 rows of K and of V for each wave");
-        copy_in(0, dk0, dv0);
-        copy_in(1, dk1, dv1);
-        copy_in(2, dk2, dv2);
-        // the query loads (issued above, tracked by the compiler) are waited for here, not inside the loop
-#pragma unroll
-        for (int gi = 0; gi < NG; ++gi)
-#pragma unroll
-            for (int s = 0; s < KS; ++s) asm volatile("" ::"v"(qreg[gi][s]));
-        // step j: block j sits in slot j % 4 (kc, vc); the slot of block j - 1 (kn, vn) takes block j + 3
-#define PA_DMA_STEP(kc, vc, kn, vn)                                                                      \
-        {                                                                                                \
-            if (j >= cnt) break;                                                                         \
-            wait_vmem<2 * COPIES_PER_STEP>();  /* this wave's part of block j has landed (blocks j + 1, j + 2 may be on their way) */ \
-            lds_barrier();   /* so has everyone else's, and block j - 1 is done with */                  \
-            copy_in(j + 3, kn, vn);                                                                      \
-            const int tile = tile_at(j);                                                                 \
-            if (tile * TOK + TOK > kv_len) { /* (uniform) the sequence's last block: clear the V rows beyond its tokens */ \
-                for (int c = tid; c < (TOK - (kv_len - tile * TOK)) * CPR; c += NT)                       \
-                    *reinterpret_cast<u4v*>(vc + (kv_len - tile * TOK) * LROWV + c * 16) = u4v{0u, 0u, 0u, 0u}; \
-                lds_barrier();                                                                           \
-            }                                                                                            \
-            if (active) whole_at(j, kc, vc);                                                             \
-            ++j;                                                                                         \
-        }
-        for (int j = 0;;) {
-            PA_DMA_STEP(dk0, dv0, dk3, dv3)
-            PA_DMA_STEP(dk1, dv1, dk0, dv0)
-            PA_DMA_STEP(dk2, dv2, dk1, dv1)
-            PA_DMA_STEP(dk3, dv3, dk2, dv2)
-        }
-#undef PA_DMA_STEP
-        wait_vmem<0>();  // the clamped copies of the last three steps still target this workgroup's LDS
-    } else if constexpr (HALF) {
+    if constexpr (HALF) {
         // Two register sets: block j + 2 goes from its set to LDS at the start of step j and the set takes block j + 4
         // right behind it (the same two steps between a fetch and its use as with three sets, 16 registers fewer).
         fetch(set[0], 0);
@@ -973,7 +783,14 @@ static hipError_t launch_prefill16_typed(hipStream_t s, const PrefillArgs& a, hi
         if (a.n_wide > 0) {  // u8 caches: the items with more than 16 query rows (up to 128) come first in the list
             PrefillArgs w = a;
             w.n_items = a.n_wide;
-            hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 2, false, false, true>), dim3((unsigned)w.n_items * a.sh.Hkv), dim3(256), 0, s, w);
+            if (a.widened) {
+                w.key_cache = a.wide_k;
+                w.value_cache = a.wide_v;
+                const hipError_t e = launch_prefill_dense(s, w, QDT, true);
+                if (e != hipSuccess) return e;
+            } else {
+                hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 2, false, true>), dim3((unsigned)w.n_items * a.sh.Hkv), dim3(256), 0, s, w);
+            }
         }
     } else if (a.n_wide > 0) {
         return hipErrorInvalidValue;  // (16-bit caches list no such group)
@@ -989,11 +806,13 @@ static hipError_t launch_prefill16_typed(hipStream_t s, const PrefillArgs& a, hi
         bool straight = false;
         if constexpr (!U8 && D == 128) straight = a.n_single == 0 || a.skip_single;
         if constexpr (!U8 && D == 128) {
-            if (straight)
-                hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 2, false, true>), dim3((unsigned)nrw.n_items * a.sh.Hkv), dim3(256), 0, s, nrw);
+            if (straight) {
+                const hipError_t e = launch_prefill_dense(s, nrw, QDT, false);
+                if (e != hipSuccess) return e;
+            }
         }
         if (!straight)
-            hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 1, false, false>), dim3((unsigned)nrw.n_items * a.sh.Hkv), dim3(512), 0, s, nrw);
+            hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 1, false>), dim3((unsigned)nrw.n_items * a.sh.Hkv), dim3(512), 0, s, nrw);
     }
     if (a.n_sparse > 0) {  // the items of block-sparse sequences come last
         PrefillArgs sp = a;
@@ -1001,7 +820,7 @@ static hipError_t launch_prefill16_typed(hipStream_t s, const PrefillArgs& a, hi
         sp.n_items = a.n_sparse;
         // 128 query rows per workgroup whatever the cache: the fewer tokens share a work item, the fewer KV blocks
         // it has to walk for rows that did not keep them
-        hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 1, true, false>), dim3((unsigned)sp.n_items * a.sh.Hkv), dim3(512), 0, s, sp);
+        hipLaunchKernelGGL((pa_prefill16_kernel<D, DT, QDT, U8, 1, true>), dim3((unsigned)sp.n_items * a.sh.Hkv), dim3(512), 0, s, sp);
     }
     if (ev1) (void)hipEventRecord(ev1, s);
     if (a.n_merge > 0 && !merge_later) {
