@@ -167,9 +167,8 @@ struct pa_ctx {
     int32_t sliding_window = 0;
     float scale = 0.0f;
     std::vector<int32_t> h_past, h_sb, h_bib;
-    DevBuf meta;  // past | sb | bib | window | score_off | token_seq
-    DevBuf items;     // work items of the MFMA kernel, then the per-token split counts
-    DevBuf dec_list;  // single-token sequences (for the u8 decode kernel)
+    DevBuf items;     // work items of the MFMA kernel, then the per-token split counts, the lists below and the step's arrays
+    const int32_t* dec_list = nullptr;  // single-token sequences (for the u8 decode kernel)
     DevBuf trig_lut, rot_args;  // cache rotation: [rows, head_size] table; block ids + deltas of one call
     DevBuf div_seqs, div_stats, div_mean, div_colsum;  // block diversity: per-call sequence list and workspace
     // block-sparse prefill (XAttention) of the current step
@@ -185,11 +184,11 @@ struct pa_ctx {
     int32_t trig_rows = 0;
     std::vector<int32_t> h_dec;
     std::vector<int32_t> h_dec16;     // single-token sequences of a 16-bit-cache step (also listed as matrix-kernel items)
-    DevBuf dec16_list;
+    const int32_t* dec16_list = nullptr;
     std::vector<pa::WidenSeq> h_wide;
     std::vector<int32_t> h_wide_tile0;
     std::vector<int32_t> h_multi;     // sequences that schedule more than one token
-    DevBuf multi_list;
+    const int32_t* multi_list = nullptr;
     size_t arrived_off = 0;  // in `items`: decode launches that fold their own splits count here, per (listed sequence, kv head)
     DevBuf tile_max;   // per (head, 32-token tile) maxima of single-token sequences handled by the matrix kernel
     bool dec_in_order = false, dec16_in_order = false;  // the lists hold 0 .. B-1 in order: every sequence, none moved
@@ -226,10 +225,15 @@ struct pa_ctx {
     int32_t few_cols = 1;        // ... in this many 16-column groups of the decode kernel's few-token variant
     size_t few_off = 0;          // its descriptors within a table's buffer
     // the step's host arrays (packed metadata, work items, lists, block tables with their descriptors) pass through
-    // this pinned area on their way to the device: pieces are handed out front to back, their copies are queued and not
-    // waited for, and pa_step_begin starts over at the front once it has waited for the stream
-    PinnedBuf step_staging;
-    size_t step_staged = 0;
+    // a pinned area on their way to the device: pieces are handed out front to back, their copies are queued and not
+    // waited for.  Its two halves take turns: pa_step_begin goes over to the other one, from its front, once everything queued
+    // up to the begin of the step before is done (`half_free`), so a step is prepared while the one before it still runs.
+    PinnedBuf staging;
+    size_t staged = 0;      // bytes handed out of the half in use
+    int half = 0;
+    hipEvent_t half_free[2] = {nullptr, nullptr};
+    bool half_pending[2] = {false, false};
+    std::vector<int32_t> h_meta;  // past | sb | bib | window | score_off | token_seq | token tiles of the generic kernel
     bool shared_table = true;
     // workspace
     DevBuf part_acc, part_ml, final_ml, logits, group_scores, p_split, pf_part_acc, pf_part_ml;
@@ -612,14 +616,31 @@ pa::XattDev xatt_dev(const pa_ctx* ctx) {
 // until a whole step's pieces fit, up to 32 MiB -- beyond that a step pays such a wait now and then).
 uint8_t* stage_piece(pa_ctx* ctx, size_t bytes) {
     const size_t need = (std::max<size_t>(bytes, 1) + 63) & ~(size_t)63;
-    if (ctx->step_staged + need > ctx->step_staging.cap) {
-        HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        ctx->step_staged = 0;
-        ctx->step_staging.reserve(std::max<size_t>({need, (size_t)1 << 16, std::min<size_t>(2 * ctx->step_staging.cap, (size_t)32 << 20)}));
+    if (ctx->staged + need > ctx->staging.cap / 128 * 64) {
+        HIP_CHECK(hipStreamSynchronize(ctx->stream));  // (neither half is read any more)
+        ctx->half_pending[0] = ctx->half_pending[1] = false;
+        ctx->staged = 0;
+        const size_t half_cap = ctx->staging.cap / 2;
+        ctx->staging.reserve(2 * std::max<size_t>({need, (size_t)1 << 16, std::min<size_t>(2 * half_cap, (size_t)32 << 20)}));
     }
-    uint8_t* at = ctx->step_staging.as<uint8_t>() + ctx->step_staged;
-    ctx->step_staged += need;
+    uint8_t* at = ctx->staging.as<uint8_t>() + ctx->half * (ctx->staging.cap / 128 * 64) + ctx->staged;
+    ctx->staged += need;
     return at;
+}
+
+// A new step's staging: the other half, when what was queued from it (two steps ago) has left it.
+void turn_staging(pa_ctx* ctx) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capturing));
+    if (capturing != hipStreamCaptureStatusNone) HIP_CHECK(hipErrorStreamCaptureUnsupported);  // (a step's uploads are no part of a graph)
+    hipEvent_t& now_free = ctx->half_free[ctx->half];
+    if (!now_free) HIP_CHECK(hipEventCreateWithFlags(&now_free, hipEventDisableTiming));
+    HIP_CHECK(hipEventRecord(now_free, ctx->stream));
+    ctx->half_pending[ctx->half] = true;
+    ctx->half ^= 1;
+    if (ctx->half_pending[ctx->half]) HIP_CHECK(hipEventSynchronize(ctx->half_free[ctx->half]));
+    ctx->half_pending[ctx->half] = false;
+    ctx->staged = 0;
 }
 
 // Queues a copy of `bytes` of host memory to `dst` on the context's stream through the staging area (from a pageable
@@ -874,7 +895,7 @@ void plan_items(pa_ctx* ctx) {
     const size_t item_bytes = items.size() * sizeof(pa::PrefillItem);
     // one upload: items | split count per token | single-token index per sequence (-1 for the others) | the tokens
     // whose rows the merge kernel has to fold | zeros, the counters of decode launches that fold their splits (they leave them at
-    // zero; a step starts there whatever became of the last one)
+    // zero; a step starts there whatever became of the last one) | the lists of sequences | the step's arrays
     ctx->n_merge = 0;
     for (int32_t t = 0; t < T; ++t) ctx->n_merge += tok_ns[t] > 1;
     tok_ns.insert(tok_ns.end(), single_idx.begin(), single_idx.end());
@@ -891,27 +912,35 @@ void plan_items(pa_ctx* ctx) {
     ctx->merge_tok_off = ctx->single_idx_off + (size_t)B * sizeof(int32_t);
     ctx->arrived_off = item_bytes + tok_ns.size() * sizeof(int32_t);
     tok_ns.resize(tok_ns.size() + std::max({ctx->h_dec.size(), ctx->h_dec16.size(), ctx->h_few.size()}) * (size_t)ctx->cfg.num_kv_heads, 0);
-    ctx->items.reserve(item_bytes + tok_ns.size() * sizeof(int32_t));
-    stage_upload(ctx, ctx->items.p, items.data(), item_bytes);
-    stage_upload(ctx, static_cast<uint8_t*>(ctx->items.p) + item_bytes, tok_ns.data(), tok_ns.size() * sizeof(int32_t));
     // the sequences a score replay has rows for: those with more than one token, longest context first
     ctx->h_multi.clear();
     for (int32_t b = 0; b < B; ++b)
         if (sb[b + 1] - sb[b] > 1) ctx->h_multi.push_back(b);
     std::stable_sort(ctx->h_multi.begin(), ctx->h_multi.end(),
                      [&](int32_t x, int32_t y) { return past[x] + sb[x + 1] - sb[x] > past[y] + sb[y + 1] - sb[y]; });
-    if (!ctx->h_multi.empty()) {
-        ctx->multi_list.reserve(ctx->h_multi.size() * sizeof(int32_t));
-        stage_upload(ctx, ctx->multi_list.p, ctx->h_multi.data(), ctx->h_multi.size() * sizeof(int32_t));
+    const std::vector<int32_t>* parts[] = {&tok_ns, &ctx->h_multi, &ctx->h_dec16, &ctx->h_dec, &ctx->h_meta};
+    size_t at[6] = {item_bytes};
+    for (int i = 0; i < 5; ++i) at[i + 1] = at[i] + parts[i]->size() * sizeof(int32_t);
+    ctx->items.reserve(at[5]);
+    {
+        uint8_t* stage = stage_piece(ctx, at[5]);
+        if (item_bytes) std::memcpy(stage, items.data(), item_bytes);
+        for (int i = 0; i < 5; ++i)
+            if (!parts[i]->empty()) std::memcpy(stage + at[i], parts[i]->data(), at[i + 1] - at[i]);
+        HIP_CHECK(hipMemcpyAsync(ctx->items.p, stage, at[5], hipMemcpyHostToDevice, ctx->stream));
     }
-    if (!ctx->h_dec16.empty()) {
-        ctx->dec16_list.reserve(ctx->h_dec16.size() * sizeof(int32_t));
-        stage_upload(ctx, ctx->dec16_list.p, ctx->h_dec16.data(), ctx->h_dec16.size() * sizeof(int32_t));
-    }
-    if (!ctx->h_dec.empty()) {
-        ctx->dec_list.reserve(ctx->h_dec.size() * sizeof(int32_t));
-        stage_upload(ctx, ctx->dec_list.p, ctx->h_dec.data(), ctx->h_dec.size() * sizeof(int32_t));
-    }
+    const uint8_t* up = static_cast<const uint8_t*>(ctx->items.p);
+    ctx->multi_list = reinterpret_cast<const int32_t*>(up + at[1]);
+    ctx->dec16_list = reinterpret_cast<const int32_t*>(up + at[2]);
+    ctx->dec_list = reinterpret_cast<const int32_t*>(up + at[3]);
+    const int32_t* d = reinterpret_cast<const int32_t*>(up + at[4]);
+    ctx->dev.past_lens = d;
+    ctx->dev.subsequence_begins = d + B;
+    ctx->dev.block_indices_begins = d + B + (B + 1);
+    ctx->dev.score_window = d + B + 2 * (B + 1);
+    ctx->dev.score_offsets = d + 2 * B + 2 * (B + 1);
+    ctx->dev.token_seq = d + 2 * B + 3 * (B + 1);
+    ctx->dev.gtiles = ctx->dev.token_seq + T;
     ctx->tok_nsplit_off = item_bytes;
     if (split_off_decode && !ctx->h_dec.empty())
         for (int w = 0; w < 2; ++w)
@@ -1068,7 +1097,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.value = static_cast<const uint16_t*>(io->value);
         a.fuse_append = fuse_append ? 1 : 0;
         a.n_seqs = (int32_t)ctx->h_dec.size();
-        a.seq_list = ctx->dec_in_order ? nullptr : ctx->dec_list.as<int32_t>();
+        a.seq_list = ctx->dec_in_order ? nullptr : ctx->dec_list;
         ctx->nsplit = a.nsplit;
         const DecodeWs ws = decode_workspace(ctx, rows, a.nsplit, io->scores != nullptr && !use_u4, static_ws);
         a.query = static_cast<const uint16_t*>(io->query);
@@ -1113,7 +1142,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.value = static_cast<const uint16_t*>(io->value);
         a.fuse_append = fuse_append ? 1 : 0;
         a.n_seqs = (int32_t)ctx->h_dec16.size();
-        a.seq_list = ctx->dec16_in_order ? nullptr : ctx->dec16_list.as<int32_t>();
+        a.seq_list = ctx->dec16_in_order ? nullptr : ctx->dec16_list;
         ctx->nsplit = a.nsplit;
         const DecodeWs ws = decode_workspace(ctx, rows, a.nsplit, io->scores != nullptr, static_ws);
         a.query = static_cast<const uint16_t*>(io->query);
@@ -1234,7 +1263,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         if (score_launch && hand_over) {
             ss.p_out = a.p_out;
             ss.tile_max = a.tile_max;
-            ss.seq_list = ctx->dec16_list.as<int32_t>();
+            ss.seq_list = ctx->dec16_list;
             ss.n_seqs = (int32_t)ctx->h_dec16.size();
         }
         // (without the single-token sequences the launch has rows for the listed multi-token sequences only)
@@ -1248,7 +1277,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             if (merge_later) mg = pa::merge_rows_of(a);
             HIP_CHECK(pa::launch_scores_replay(ctx->stream, ctx->dev, a.sh, c.query_dtype, c.kv_cache_dtype, io->query,
                                                io->key_cache, table, a.final_ml, io->scores, ctx->max_kv,
-                                               singles_too ? nullptr : ctx->multi_list.as<int32_t>(), replay_seqs,
+                                               singles_too ? nullptr : ctx->multi_list, replay_seqs,
                                                a.xatt, ss, mg));
         }
     }
@@ -1303,12 +1332,13 @@ void pa_destroy(pa_ctx* ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->cfg.device);
     (void)hipStreamSynchronize(ctx->stream);
-    ctx->meta.release();
     ctx->items.release();
     for (auto& t : ctx->tables) t.release();
     ctx->table_pool.release();
     ctx->alibi.release();
-    ctx->step_staging.release();
+    ctx->staging.release();
+    for (hipEvent_t e : ctx->half_free)
+        if (e) (void)hipEventDestroy(e);
     ctx->part_acc.release();
     ctx->part_ml.release();
     ctx->final_ml.release();
@@ -1317,9 +1347,6 @@ void pa_destroy(pa_ctx* ctx) {
     ctx->p_split.release();
     ctx->pf_part_acc.release();
     ctx->pf_part_ml.release();
-    ctx->dec_list.release();
-    ctx->dec16_list.release();
-    ctx->multi_list.release();
     ctx->tile_max.release();
     ctx->trig_lut.release();
     ctx->rot_args.release();
@@ -1379,7 +1406,8 @@ int32_t pa_step_begin(pa_ctx* ctx, const pa_step_meta* m) {
         // pack the device copy: past | sb | bib | window | score_off | token_seq | token tiles of the generic kernel
         const pa::GenericShape gsh = generic_shape_of(ctx->cfg);
         const pa::GenericPlan gplan = pa::generic_plan(gsh, T > B);
-        std::vector<int32_t> h((size_t)B + (B + 1) + (B + 1) + B + (B + 1) + T + T);
+        std::vector<int32_t>& h = ctx->h_meta;
+        h.resize((size_t)B + (B + 1) + (B + 1) + B + (B + 1) + T + T);
         int32_t* past = h.data();
         int32_t* sb = past + B;
         int32_t* bib = sb + B + 1;
@@ -1406,20 +1434,7 @@ int32_t pa_step_begin(pa_ctx* ctx, const pa_step_meta* m) {
                 gtiles[n_gtiles++] = t * 8 + (std::min(gplan.tokens, sb[b + 1] - t) - 1);
 
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
-        // the previous step's kernels may still read the old copy
-        HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        ctx->meta.reserve(h.size() * sizeof(int32_t));
-        ctx->step_staged = 0;
-        stage_upload(ctx, ctx->meta.p, h.data(), h.size() * sizeof(int32_t));
-
-        int32_t* d = ctx->meta.as<int32_t>();
-        ctx->dev.past_lens = d;
-        ctx->dev.subsequence_begins = d + B;
-        ctx->dev.block_indices_begins = d + B + (B + 1);
-        ctx->dev.score_window = d + B + 2 * (B + 1);
-        ctx->dev.score_offsets = d + 2 * B + 2 * (B + 1);
-        ctx->dev.token_seq = d + 2 * B + 3 * (B + 1);
-        ctx->dev.gtiles = ctx->dev.token_seq + T;
+        turn_staging(ctx);  // (the arrays themselves go up with the plan, behind what the previous step has queued)
         ctx->dev.n_gtiles = n_gtiles;
         ctx->dev.B = B;
         ctx->dev.T = T;
@@ -1657,7 +1672,7 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         }
         PA_REQUIRE(logit_off * 4 <= ((int64_t)4 << 30), PA_NOT_ALLOCATED,
                    "block-sparse prefill: the strided logits of this step exceed 4 GiB (larger stride or shorter chunks)");
-        // (pa_step_begin has waited for the previous step's kernels, which read the old plan; the copies are queued)
+        // (the copies are queued behind the previous step's kernels, which read the old plan)
         const size_t seq_bytes = seqs.size() * sizeof(pa::XattSeq), tile_bytes = tiles.size() * sizeof(pa::XattTile);
         ctx->x_tiles_off = seq_bytes;
         ctx->x_seq_of_off = seq_bytes + tile_bytes;

@@ -68,7 +68,7 @@ class PagedAttention:
         m.score_aggregation_window = _p32(saw) if saw is not None else None
         m.max_context_len, m.sliding_window, m.scale = int(max_context_len), int(sliding_window), float(scale)
         self._ck(L.lib().pa_step_begin(self._h, C.byref(m)))
-        self.total_scores = int(np.sum(past.astype(np.int64)) + sb[-1])
+        self.total_scores = int(past.sum(dtype=np.int64)) + int(sb[-1])
         self.num_tokens = int(sb[-1])
 
     def set_block_indices(self, block_indices, num_blocks, layer=-1):
