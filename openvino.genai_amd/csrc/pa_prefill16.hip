@@ -205,9 +205,9 @@ void pa_prefill16_kernel(PrefillArgs a) {
         free_lo = sw > 0 ? max(low, 0) : 0;
     }
 
-    float m_run[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.0f, 0.0f};
-    // 16-bit caches keep the running maximum negated (NO_MAX while the row has seen nothing), ready for the exponent's
-    // multiply-add, and the level (log2, relative to the running maximum) a block's largest probability must stay
+    float l_part[2] = {0.0f, 0.0f};
+    // The running maximum is kept negated (NO_MAX while the row has seen nothing), ready for the exponent's
+    // multiply-add; 16-bit caches also keep the level (log2, relative to the running maximum) a block's largest probability must stay
     // under for the block to do without the second, low-half product: log2(LO_SHARE x the row's denominator when
     // last looked at).
     constexpr float NO_MAX = 1e30f;
@@ -380,82 +380,100 @@ void pa_prefill16_kernel(PrefillArgs a) {
             }
         }
     };
-    // u8 caches: masks + online softmax of block `tile` (number j): weights as MFMA operands, rescale factors.
-    // The running maximum is only raised when a block exceeds it by more than 2^4: probabilities then stay
-    // below 16 and the accumulators are rescaled a few times per row instead of once per block.
-    auto softmax = [&](auto masked_c, const f4 (&sc)[2][2], int tile, int j, u4v (&pb)[2], u4v (&pl)[2],
-                       float (&corr)[2], const bool (&kept)[2]) __attribute__((always_inline)) {
+    // The running maximum is only raised when a block exceeds it by more than 2^4: probabilities then stay below 16 and the
+    // accumulators are rescaled a few times per row instead of once per block.  Whether any row of the wave has to be is
+    // asked lane by lane; the maximum over a row's four lanes is formed only then.  mx: the lane's maximum of the block
+    // (log2 domain); d: what the running maximum moves by (0 for a row that stays; -NO_MAX for one that held nothing).
+    auto raise_to = [&](int gi, float mx, float& d) __attribute__((always_inline)) {
+        mx = xor_max_g(mx);
+        const float m_old = -neg_m[gi], m_new = mx + neg_m[gi] > 4.0f ? mx : m_old;
+        d = m_old - m_new;
+        const float corr = __builtin_amdgcn_exp2f(d);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[gi][r] *= corr;
+        l_part[gi] *= corr;
+        zsum[gi] *= corr;
+        neg_m[gi] = -m_new;
+    };
+    // u8 caches: masks + online softmax of block `tile` (number j): weights as MFMA operands.  sc: raw products, then logits
+    // (log2 domain) over CODE_UNIT, which the exponent's multiply-add puts back.
+    auto softmax = [&](auto masked_c, f4 (&sc)[2][2], int tile, int j, u4v (&pb)[2], u4v (&pl)[2],
+                       const bool (&kept)[2]) __attribute__((always_inline)) {
         constexpr bool MASKED = decltype(masked_c)::value;
         const int pos0 = tile * TOK + 4 * g;
-        f4 h_sck[2], h_zpk[2], h_scv[2], h_zpv[2];  // headers of this lane's 8 tokens (16 u + 4 g + i)
-        if (U8) {
-            const float* hdr = reinterpret_cast<const float*>(smem + OFF_H + (j & 3) * HDRB);
+        const float* hdr = reinterpret_cast<const float*>(smem + OFF_H + (j & 3) * HDRB) + 4 * g;  // of this lane's 8 tokens (16 u + 4 g + i)
+        float mx[2];
+        bool raise = false;
+        {
+            f4 h_sck[2], h_zpk[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                h_sck[u] = *reinterpret_cast<const f4*>(hdr + 16 * u + 4 * g);
-                h_zpk[u] = *reinterpret_cast<const f4*>(hdr + TOK + 16 * u + 4 * g);
-                h_scv[u] = *reinterpret_cast<const f4*>(hdr + 2 * TOK + 16 * u + 4 * g);
-                h_zpv[u] = *reinterpret_cast<const f4*>(hdr + 3 * TOK + 16 * u + 4 * g);
+                h_sck[u] = *reinterpret_cast<const f4*>(hdr + 16 * u);
+                h_zpk[u] = *reinterpret_cast<const f4*>(hdr + TOK + 16 * u);
             }
-        }
 #pragma unroll
-        for (int gi = 0; gi < NG; ++gi) {
-            float x[8];  // logits (log2 domain) over CODE_UNIT, which the exponent's multiply-add puts back
-            float mx = -INFINITY;
-            if (U8) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        x[4 * u + i] = fmaf(sc[gi][u][i], h_sck[u][i], -h_zpk[u][i] * qsum[gi]);
-            }
-            if (MASKED) {
+            for (int gi = 0; gi < NG; ++gi) {
+                mx[gi] = -INFINITY;
                 const int lim = row_pos[gi];
                 const int low = sw > 0 ? max(0, lim + 1 - sw) : 0;
 #pragma unroll
                 for (int jj = 0; jj < 8; ++jj) {
-                    const int pos = pos0 + 16 * (jj >> 2) + (jj & 3);
-                    x[jj] = (pos <= lim && pos >= low && kept[gi]) ? x[jj] : -INFINITY;
+                    float x = fmaf(sc[gi][jj >> 2][jj & 3], h_sck[jj >> 2][jj & 3], -h_zpk[jj >> 2][jj & 3] * qsum[gi]);
+                    if (MASKED) {
+                        const int pos = pos0 + 16 * (jj >> 2) + (jj & 3);
+                        x = (pos <= lim && pos >= low && kept[gi]) ? x : -INFINITY;
+                    }
+                    sc[gi][jj >> 2][jj & 3] = x;
+                    mx[gi] = fmaxf(mx[gi], x);
                 }
+                mx[gi] *= CODE_UNIT;
+                raise |= mx[gi] + neg_m[gi] > 4.0f;
             }
+        }
+        if (__any(raise)) {
 #pragma unroll
-            for (int jj = 0; jj < 8; ++jj) mx = fmaxf(mx, x[jj]);
-            mx = xor_max_g(mx) * CODE_UNIT;
-            const float m_new = mx > m_run[gi] + 4.0f ? mx : m_run[gi];
-            const float m_safe = m_new == -INFINITY ? 0.0f : m_new;
-            corr[gi] = __builtin_amdgcn_exp2f(m_run[gi] - m_safe);
+            for (int gi = 0; gi < NG; ++gi) {
+                float d;
+                raise_to(gi, mx[gi], d);
+            }
+        }
+        f4 h_scv[2], h_zpv[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            h_scv[u] = *reinterpret_cast<const f4*>(hdr + 2 * TOK + 16 * u);
+            h_zpv[u] = *reinterpret_cast<const f4*>(hdr + 3 * TOK + 16 * u);
+        }
+#pragma unroll
+        for (int gi = 0; gi < NG; ++gi) {
             float p[8];
             float psum = 0.0f;
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) {
-                p[jj] = __builtin_amdgcn_exp2f(fmaf(x[jj], CODE_UNIT, -m_safe));
+                p[jj] = __builtin_amdgcn_exp2f(fmaf(sc[gi][jj >> 2][jj & 3], CODE_UNIT, neg_m[gi]));
                 psum += p[jj];
             }
-            if (U8) {
-                // Weights carry the V row's scale.  They go to the matrix pipe as an f16 value plus what that
-                // rounding dropped (a second f16), like the probabilities of the 16-bit caches: with 11 bits alone
-                // a row that leans on a few tokens with large, opposite V values misses the tolerance now and then.
-                // The zero-point term takes the f32 weight, which the two halves reproduce to 2^-23.
-                float zs = 0.0f;
+            // Weights carry the V row's scale.  They go to the matrix pipe as an f16 value plus what that
+            // rounding dropped (a second f16), like the probabilities of the 16-bit caches: with 11 bits alone
+            // a row that leans on a few tokens with large, opposite V values misses the tolerance now and then.
+            // The zero-point term takes the f32 weight, which the two halves reproduce to 2^-23.
+            float zs = 0.0f;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) {
-                    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-                    const float w0 = p[2 * jj] * h_scv[jj >> 1][(2 * jj) & 3];
-                    const float w1 = p[2 * jj + 1] * h_scv[jj >> 1][(2 * jj + 1) & 3];
-                    uint32_t wb = __builtin_bit_cast(uint32_t, h2{(_Float16)w0, (_Float16)w1});
-                    // one rounded value for both uses below: left alone, the compiler forms the f16 weight twice, once
-                    // from the f32 product (two roundings) and once with a mixed-precision multiply (one rounding); at
-                    // a tie the two differ by one f16 step, and the low half would belong to another high half
-                    asm volatile("" : "+v"(wb));
-                    pb[gi][jj] = wb;
-                    pl[gi][jj] = residual_f16x2(wb, w0, w1);
-                    zs = fmaf(w0, h_zpv[jj >> 1][(2 * jj) & 3], zs);
-                    zs = fmaf(w1, h_zpv[jj >> 1][(2 * jj + 1) & 3], zs);
-                }
-                zsum[gi] = zsum[gi] * corr[gi] + zs;
+            for (int jj = 0; jj < 4; ++jj) {
+                typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+                const float w0 = p[2 * jj] * h_scv[jj >> 1][(2 * jj) & 3];
+                const float w1 = p[2 * jj + 1] * h_scv[jj >> 1][(2 * jj + 1) & 3];
+                uint32_t wb = __builtin_bit_cast(uint32_t, h2{(_Float16)w0, (_Float16)w1});
+                // one rounded value for both uses below: left alone, the compiler forms the f16 weight twice, once
+                // from the f32 product (two roundings) and once with a mixed-precision multiply (one rounding); at
+                // a tie the two differ by one f16 step, and the low half would belong to another high half
+                asm volatile("" : "+v"(wb));
+                pb[gi][jj] = wb;
+                pl[gi][jj] = residual_f16x2(wb, w0, w1);
+                zs = fmaf(w0, h_zpv[jj >> 1][(2 * jj) & 3], zs);
+                zs = fmaf(w1, h_zpv[jj >> 1][(2 * jj + 1) & 3], zs);
             }
-            l_part[gi] = l_part[gi] * corr[gi] + psum;
-            m_run[gi] = m_new;
+            zsum[gi] += zs;
+            l_part[gi] += psum;
         }
     };
 
@@ -478,7 +496,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
                          const bool (&kept)[2]) __attribute__((always_inline)) -> bool {
         constexpr bool MASKED = decltype(masked_c)::value;
         const int pos0 = tile * TOK + 4 * g;
-        float x[2][8], mxs[2], rel[2];  // rel: the block's maximum relative to the running one (huge while there is none)
+        float x[2][8], mxs[2];  // mxs: the lane's maximum of the block
         bool raise = false;
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
@@ -496,24 +514,15 @@ void pa_prefill16_kernel(PrefillArgs a) {
             float mx = -INFINITY;
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) mx = fmaxf(mx, x[gi][jj]);
-            mxs[gi] = xor_max_g(mx) * scl;
-            rel[gi] = mxs[gi] + neg_m[gi];  // (-inf for a row that sees nothing of this block)
-            raise |= rel[gi] > 4.0f;
+            mxs[gi] = mx * scl;
+            raise |= mxs[gi] + neg_m[gi] > 4.0f;
         }
-        // The running maximum is only raised when a block exceeds it by more than 2^4: probabilities then stay below
-        // 16 and the accumulators are rescaled a few times per row instead of once per block.
         if (__any(raise)) {
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
-                const float m_new = rel[gi] > 4.0f ? mxs[gi] : -neg_m[gi];
-                const float d = -neg_m[gi] - m_new;  // 0 for a row that stays; -NO_MAX for one that held nothing (zeros)
-                const float corr = __builtin_amdgcn_exp2f(d);
-#pragma unroll
-                for (int r = 0; r < RT; ++r) acc[gi][r] *= corr;
-                l_part[gi] *= corr;
+                float d;
+                raise_to(gi, mxs[gi], d);
                 lo_at[gi] += d;
-                neg_m[gi] = -m_new;
-                rel[gi] = mxs[gi] + neg_m[gi];
             }
         }
         bool need = false;
@@ -544,7 +553,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
                     }
                 }
             }
-            need |= rel[gi] > lo_at[gi];
+            need |= mxs[gi] + neg_m[gi] > lo_at[gi];
         }
         if constexpr (LO_ALWAYS) return true;
         if (!__any(need)) return false;
@@ -554,7 +563,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
             lo_at[gi] = __log2f(xor_sum_g(l_part[gi])) + LO_SHARE_LOG2;
-            need |= rel[gi] > lo_at[gi];
+            need |= mxs[gi] + neg_m[gi] > lo_at[gi];
         }
         return __any(need);
     };
@@ -592,16 +601,8 @@ void pa_prefill16_kernel(PrefillArgs a) {
         f4 sc[2][2];
         u4v pb[2], pl[2];
         if constexpr (U8) {
-            float corr[2];
             qk_pv_at(true, kb, sc, false, vb, pb, pl);
-            softmax(masked_c, sc, tile_at(j), j, pb, pl, corr, kept);
-#pragma unroll
-            for (int gi = 0; gi < NG; ++gi) {
-                if (__any(corr[gi] != 1.0f)) {
-#pragma unroll
-                    for (int r = 0; r < RT; ++r) acc[gi][r] *= corr[gi];
-                }
-            }
+            softmax(masked_c, sc, tile_at(j), j, pb, pl, kept);
             qk_pv_at(false, kb, sc, true, vb, pb, pl);
         } else {
             float p[2][8];
@@ -702,10 +703,9 @@ void pa_prefill16_kernel(PrefillArgs a) {
     }
 
     // ---- write the rows ------------------------------------------------------------------------------
-    if constexpr (!U8) {
+    float m_run[2];
 #pragma unroll
-        for (int gi = 0; gi < NG; ++gi) m_run[gi] = neg_m[gi] == NO_MAX ? -INFINITY : -neg_m[gi];
-    }
+    for (int gi = 0; gi < NG; ++gi) m_run[gi] = neg_m[gi] == NO_MAX ? -INFINITY : -neg_m[gi];
     const bool final_out = item.nsplit == 1;
     // the lane's group number again, from an opaque copy of the thread id: nothing inside the loop reads it, and kept
     // alive across the loop it costs the variants that sit at their register limit a spill
