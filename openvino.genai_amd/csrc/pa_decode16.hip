@@ -16,6 +16,8 @@
 // Scores as in the u8 decode kernel: the un-normalised probabilities of a workgroup's positions stay in LDS (fp16,
 // relative to the running maximum, which is snapshotted per block); once the final maximum and denominator are
 // known they are normalised, summed over the group's heads and written out.
+// A workgroup's first fetch depends on one descriptor (as in the u8 kernel) instead of a chain of four reads -- sequence list,
+// step arrays, table begin, table: 16 sequences of 64 - 2048 tokens (32 / 4 heads, D = 64, f16) 12.4 -> 11.4 us a launch.
 // Split partials, per-kv-head score sums and split probabilities have the layouts of the u8 decode kernel and are
 // folded by its merge and score kernels.
 //
@@ -86,21 +88,19 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
     constexpr int CPR = ROWB / 16;         // 16-byte pieces per row
     extern __shared__ __align__(16) uint8_t smem[];
 
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const StepDev& st = a.st;
     const int Hq = a.sh.Hq, Hkv = a.sh.Hkv, G = a.G, nsplit = a.nsplit;
     const int split = blockIdx.x % nsplit;
     const int hkv = (blockIdx.x / nsplit) % Hkv;
-    const int b = a.seq_list ? a.seq_list[blockIdx.x / (nsplit * Hkv)] : (int)(blockIdx.x / (nsplit * Hkv));
-    const int t = st.subsequence_begins[b];
-    const int kv_len = st.past_lens[b] + 1;
-    const int first = st.sliding_window > 0 ? max(0, kv_len - st.sliding_window) : 0;
-    const int tile_lo = first / TOK, tile_hi = (kv_len + TOK - 1) / TOK;
-    const int per = ceil_div(tile_hi - tile_lo, nsplit);
-    const int tb = tile_lo + split * per;
-    const int te = min(tile_hi, tb + per);
-    const int32_t* table = a.block_indices + st.block_indices_begins[b];
+    // everything the first block's fetch depends on sits in one descriptor (one scalar load)
+    const DecodeDesc* __restrict__ dsc = a.descs + ((long)(blockIdx.x / (nsplit * Hkv)) * nsplit + split);
+    const int b = dsc->b, t = dsc->t, kv_len = dsc->kv_len, first = dsc->first;
+    const int tb = dsc->tb, te = dsc->te;
+    const int tile_hi = (kv_len + TOK - 1) / TOK;
+    const int32_t* table = a.block_indices + dsc->table_off;
 
     uint8_t* slot = smem + wv * SLOT;                                  // this wave's V block
     float* wave_ml = reinterpret_cast<float*>(smem + WAVES * SLOT);    // [WAVES][16][2]
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
             const int piece = isv ? lane - CPR : lane, pos = kv_len - 1;
             const u4v row = *reinterpret_cast<const u4v*>(reinterpret_cast<const uint8_t*>(isv ? a.value : a.key) +
                                                           ((long)t * Hkv + hkv) * ROWB + piece * 16);
-            const long dst = (((long)table[pos / bsz] * Hkv + hkv) * bsz + pos % bsz) * ROWB + piece * 16;
+            const long dst = (((long)dsc->last_id * Hkv + hkv) * bsz + pos % bsz) * ROWB + piece * 16;
             *reinterpret_cast<u4v*>(const_cast<uint8_t*>(isv ? a.value_cache : a.key_cache) + dst) = row;
         }
     };
@@ -152,9 +152,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
         append_row();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    if (tile < te)
-        issue(ba, table[min((BPT * tile) >> sub_shift, last_block)], table[min((BPT * tile + BPT - 1) >> sub_shift, last_block)],
-              tile & sub_mask);
+    if (tile < te) issue(ba, dsc->ids[BPT * wv], dsc->ids[BPT * wv + BPT - 1], tile & sub_mask);
     if (owner && tile != tile_hi - 1) append_row();
     for (int i = tid; i < BPT * (te - tb); i += 64 * WAVES) tab[i] = table[min((BPT * tb + i) >> sub_shift, last_block)];
 
@@ -361,7 +359,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void pa_decode16_kernel(Decod
     const float* fac = msnap;
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     typedef _Float16 h4u __attribute__((ext_vector_type(4), aligned(2)));
-    const long soff = st.score_offsets[b];
+    const long soff = dsc->score_off;
     if (final_out) {
         // sum over the group's heads -> group_scores[hkv][position] (fp16, as in the u8 decode kernel), four positions
         // per thread; positions before the first block of the window get 0

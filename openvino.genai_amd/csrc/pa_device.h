@@ -259,7 +259,7 @@ struct DecodeArgs {
     const uint8_t* value_cache;
     const int32_t* block_indices;
     const int32_t* seq_list;      // sequences this launch covers (single-token ones); null = all B
-    const DecodeDesc* descs;      // u8 kernel: [n_seqs][nsplit]
+    const DecodeDesc* descs;      // [n_seqs][nsplit]
     const uint16_t* key;          // with fuse_append: the step's new K / V rows [T, Hkv*D], which the workgroup that
     const uint16_t* value;        // owns a sequence's last block writes (u8: quantises) into the caches itself
     int32_t fuse_append;

@@ -216,6 +216,8 @@ struct pa_ctx {
     // per-(sequence, split) descriptors of both plans
     struct DecPlan { int32_t nsplit = 1, max_tiles = 1, waves = 4; } dec_plan[2];
     size_t desc_off[2] = {0, 0};       // byte offsets of the two descriptor arrays in a table's buffer
+    DecPlan dec16_plan[2];             // ... and the 16-bit decode kernel's, for h_dec16
+    size_t desc16_off[2] = {0, 0};
     int32_t kernels_run = 0;     // PA_RAN_* of the last attention call
     bool fork_pays = true;       // mixed steps: matrix and decode kernel side by side on two streams also in calls without scores
                                  // (else one after the other)
@@ -342,8 +344,9 @@ void check_io(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool need_kv, b
 
 bool decode_u8_step(const pa_ctx* ctx);
 bool decode_u4_step(const pa_ctx* ctx);
+bool decode16_descs(const pa_ctx* ctx);
 
-// Descriptors of the u8 decode kernel's workgroups for one block table (host ids), both plans (and those of a step of
+// Descriptors of the decode kernels' workgroups for one block table (host ids), both plans (and those of a step of
 // few-token sequences), into the staging copy
 // of the table's buffer.
 void fill_decode_descs(const pa_ctx* ctx, const int32_t* ids, uint8_t* stage) {
@@ -384,6 +387,9 @@ void fill_decode_descs(const pa_ctx* ctx, const int32_t* ids, uint8_t* stage) {
     if (decode_u8_step(ctx) || decode_u4_step(ctx))
         for (int w = 0; w < 2; ++w)
             fill(ctx->h_dec, ctx->dec_plan[w].nsplit, reinterpret_cast<pa::DecodeDesc*>(stage + ctx->desc_off[w]));
+    if (decode16_descs(ctx))
+        for (int w = 0; w < 2; ++w)
+            fill(ctx->h_dec16, ctx->dec16_plan[w].nsplit, reinterpret_cast<pa::DecodeDesc*>(stage + ctx->desc16_off[w]));
     if (!ctx->h_few.empty()) fill(ctx->h_few, ctx->few_plan.nsplit, reinterpret_cast<pa::DecodeDesc*>(stage + ctx->few_off));
 }
 
@@ -462,6 +468,9 @@ bool decode_u8_step(const pa_ctx* ctx) {
 bool decode_u4_step(const pa_ctx* ctx) {
     return decode_u4_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B && ctx->B <= 65535;
 }
+
+// Whether the step's single-token sequences may run on the 16-bit decode kernel, whose descriptors its tables then carry.
+bool decode16_descs(const pa_ctx* ctx) { return decode16_shape(ctx) && !ctx->h_dec16.empty(); }
 
 // Split-K plan of the decode kernels: workgroups per (sequence, kv head) and the most blocks one walks.
 void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, int32_t* max_tiles_out,
@@ -942,6 +951,9 @@ void plan_items(pa_ctx* ctx) {
     ctx->dev.token_seq = d + 2 * B + 3 * (B + 1);
     ctx->dev.gtiles = ctx->dev.token_seq + T;
     ctx->tok_nsplit_off = item_bytes;
+    if (decode16_descs(ctx))
+        for (int w = 0; w < 2; ++w)
+            plan_decode_u8(ctx, w == 1, &ctx->dec16_plan[w].nsplit, &ctx->dec16_plan[w].max_tiles, &ctx->h_dec16);
     if (split_off_decode && !ctx->h_dec.empty())
         for (int w = 0; w < 2; ++w)
             plan_decode_u8(ctx, w == 1, &ctx->dec_plan[w].nsplit, &ctx->dec_plan[w].max_tiles, nullptr, &ctx->dec_plan[w].waves);
@@ -1136,7 +1148,10 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.G = c.num_heads / c.num_kv_heads;
         a.want_scores = io->scores ? 1 : 0;
         a.total_scores = ctx->total_scores;
-        plan_decode_u8(ctx, io->scores != nullptr, &a.nsplit, &a.max_tiles, &ctx->h_dec16);
+        const int wplan = io->scores ? 1 : 0;
+        a.nsplit = ctx->dec16_plan[wplan].nsplit;
+        a.max_tiles = ctx->dec16_plan[wplan].max_tiles;
+        a.descs = reinterpret_cast<const pa::DecodeDesc*>(reinterpret_cast<const uint8_t*>(table) + ctx->desc16_off[wplan]);
         a.waves = 4;
         a.key = static_cast<const uint16_t*>(io->key);
         a.value = static_cast<const uint16_t*>(io->value);
@@ -1502,12 +1517,17 @@ void shape_tables(pa_ctx* ctx, bool shared) {
 size_t table_upload_bytes(pa_ctx* ctx, int32_t count, size_t* id_bytes, bool* with_descs) {
     *id_bytes = std::max<size_t>(((size_t)count * sizeof(int32_t) + 127) & ~(size_t)127, 128);
     size_t total = *id_bytes;
-    const bool single = decode_u8_step(ctx) || decode_u4_step(ctx), few = !ctx->h_few.empty();
-    *with_descs = single || few;
+    const bool single = decode_u8_step(ctx) || decode_u4_step(ctx), single16 = decode16_descs(ctx), few = !ctx->h_few.empty();
+    *with_descs = single || single16 || few;
     if (single)
         for (int w = 0; w < 2; ++w) {
             ctx->desc_off[w] = total;
             total += ctx->h_dec.size() * ctx->dec_plan[w].nsplit * sizeof(pa::DecodeDesc);
+        }
+    if (single16)
+        for (int w = 0; w < 2; ++w) {
+            ctx->desc16_off[w] = total;
+            total += ctx->h_dec16.size() * ctx->dec16_plan[w].nsplit * sizeof(pa::DecodeDesc);
         }
     if (few) {
         ctx->few_off = total;
