@@ -43,22 +43,20 @@ __device__ inline void bytes_to_half_pairs(uint32_t w, uint32_t& p01, uint32_t& 
     p23 = perm(0u, w, 0x0c030c02u);
 }
 
-// the eight nibbles of `w` -> four dwords of fp16 pairs, zero-extended: with byte i holding element 2 i in its high nibble,
-// the pairs are the elements (1, 5), (3, 7), (0, 4), (2, 6)
-__device__ inline u4v nibbles_to_half_pairs(uint32_t w) {
-    return u4v{w & 0x000f000fu, (w >> 8) & 0x000f000fu, (w >> 4) & 0x000f000fu, (w >> 12) & 0x000f000fu};
-}
-
 // A pair of zero-extended codes (f16 subnormals, code * 2^-24) -> (code - c) * 2^-9, exactly, as normal f16 values: one packed
 // multiply-add with `neg_c` = (-c * 2^-9, -c * 2^-9).  The matrix pipe aligns its products by their operands' exponents before it
 // adds and truncates, and a subnormal operand counts there with the smallest normal exponent: a code of c bits gives away 10 - c
 // bits of every sum it is in.
 constexpr float CODE_UNIT_INV = 512.0f;
-__device__ inline uint32_t centred_codes(const uint32_t pair, const uint32_t neg_c) {
+__device__ inline uint32_t centred_codes(const uint32_t pair, const uint32_t neg_c, const float unit = 32768.0f) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, pair), h2{(_Float16)32768.0f, (_Float16)32768.0f},
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, pair), h2{(_Float16)unit, (_Float16)unit},
                                                                   __builtin_bit_cast(h2, neg_c)));
 }
+// The low (high) nibbles of the bytes 0 and 2 of `w`, centred: a high nibble is left where it is, 16 code * 2^-24, and multiplied
+// by a sixteenth.
+__device__ inline uint32_t centred_low_nibbles(const uint32_t w, const uint32_t neg_c) { return centred_codes(w & 0x000f000fu, neg_c); }
+__device__ inline uint32_t centred_high_nibbles(const uint32_t w, const uint32_t neg_c) { return centred_codes(w & 0x00f000f0u, neg_c, 2048.0f); }
 // c = 8 for every u4 row, 128 for every u8 row
 constexpr float U4_CENTRE = 8.0f, U8_CENTRE = 128.0f;
 constexpr uint32_t U4_NEG_CENTRE = 0xa400a400u, U8_NEG_CENTRE = 0xb400b400u;  // -2^-6 and -2^-2, twice
@@ -148,7 +146,8 @@ __device__ __forceinline__ void issue_block(const DecodeArgs& a, int phys0, int 
 //     64 bits, 8.2e-4 at 32768 positions), these in 0.2 % (1.995e-4, 1.980e-4: f16's own rounding); the shape-generic kernel's
 //     f32 sums miss it in 1.4 - 2.7 %.  (Rows with every outlier on one side, zero-points near 1 or 14, gain nothing from the 8:
 //     0.10 % against 0.05 % there.)  The four packed instructions per word cost 4 % of the launch.
-//   * QK: four masks of a 32-bit word give four pairs of codes (elements 1,5 | 3,7 | 0,4 | 2,6 of the eight), and
+//   * QK: four masks of a 32-bit word and of the word shifted by a byte give four pairs of codes (elements 1,5 | 3,7 | 0,4 |
+//     2,6 of the eight; high nibbles stay where they are and are scaled by a sixteenth), and
 //     the query operand is permuted to match.  bf16 queries are brought below 2 by a power of two per head before they
 //     become f16 operands: elements below 2^-17 of the head's largest are rounded to a multiple of 2^-24 of it, what f32
 //     sums that hold the largest would leave of them too.
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
     constexpr int KS = D / 32;             // k-steps of the QK contraction
     constexpr int RT = D / 16;             // 16-row output tiles of PV
     constexpr int VB = D / 16;             // V channels per lane per token row
-    constexpr int NW = (VB + 3) / 4;       // ... held in this many 32-bit words
+    constexpr int NW = U4 ? (VB + 7) / 8 : (VB + 3) / 4;  // ... held in this many 32-bit words
     constexpr int SLOT = decode_slot_bytes(D, U4);  // a wave's LDS staging slot: a K block, then a V block
     constexpr int EPL = U4 && D == 64 ? 2 : (D + 63) / 64;  // elements per lane of a new K / V row
     constexpr int ROW_LANES = D / EPL;     // lanes a new row spreads over (D = 96: 48, the others repeat lanes 32 - 47)
@@ -384,8 +383,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             if constexpr (U4) {
                 const uint32_t w0 = *reinterpret_cast<const uint32_t*>(slot + ROW * n + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
                 const uint32_t w1 = *reinterpret_cast<const uint32_t*>(slot + ROW * (16 + n) + 8 + 32 * (s >> 1) + 8 * g + 4 * (s & 1));
-                a0 = nibbles_to_half_pairs(w0);
-                a1 = nibbles_to_half_pairs(w1);
+                // (with byte i holding element 2 i in its high nibble, the pairs are the elements (1, 5), (3, 7), (0, 4), (2, 6))
+                a0 = u4v{centred_low_nibbles(w0, NEG_CENTRE), centred_low_nibbles(w0 >> 8, NEG_CENTRE),
+                         centred_high_nibbles(w0, NEG_CENTRE), centred_high_nibbles(w0 >> 8, NEG_CENTRE)};
+                a1 = u4v{centred_low_nibbles(w1, NEG_CENTRE), centred_low_nibbles(w1 >> 8, NEG_CENTRE),
+                         centred_high_nibbles(w1, NEG_CENTRE), centred_high_nibbles(w1 >> 8, NEG_CENTRE)};
             } else {
                 const uint2 w0 = *reinterpret_cast<const uint2*>(slot + ROW * n + 8 + 32 * s + 8 * g);
                 const uint2 w1 = *reinterpret_cast<const uint2*>(slot + ROW * (16 + n) + 8 + 32 * s + 8 * g);
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
                 bytes_to_half_pairs(w1.x, x0, x1); a1[0] = x0; a1[1] = x1;
                 bytes_to_half_pairs(w1.y, x0, x1); a1[2] = x0; a1[3] = x1;
             }
-            if constexpr (FRESH) {
+            if constexpr (FRESH && !U4) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     a0[e] = centred_codes(a0[e], NEG_CENTRE);
@@ -558,14 +560,11 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
             } else if constexpr (U4) {  // VB channels in VB / 2 bytes: channel VB n + r in nibble r, the even ones the high nibbles
                 if constexpr (VB == 16) {
                     const uint2 w = *reinterpret_cast<const uint2*>(p + 8 * n);
-                    vw[0][j] = (w.x >> 4) & 0x0f0f0f0fu, vw[1][j] = w.x & 0x0f0f0f0fu;
-                    vw[2][j] = (w.y >> 4) & 0x0f0f0f0fu, vw[3][j] = w.y & 0x0f0f0f0fu;
+                    vw[0][j] = w.x, vw[1][j] = w.y;
                 } else if constexpr (VB == 8) {
-                    const uint32_t w = *reinterpret_cast<const uint32_t*>(p + 4 * n);
-                    vw[0][j] = (w >> 4) & 0x0f0f0f0fu, vw[1][j] = w & 0x0f0f0f0fu;
-                } else {  // two bytes: both nibble sets in one word
-                    const uint32_t w = *reinterpret_cast<const uint16_t*>(p + 2 * n);
-                    vw[0][j] = ((w >> 4) & 0x0f0fu) | ((w & 0x0f0fu) << 16);
+                    vw[0][j] = *reinterpret_cast<const uint32_t*>(p + 4 * n);
+                } else {
+                    vw[0][j] = *reinterpret_cast<const uint16_t*>(p + 2 * n);
                 }
             } else if constexpr (VB == 8) {
                 const uint2 w = *reinterpret_cast<const uint2*>(p + 8 * n);
@@ -579,15 +578,16 @@ __global__ __launch_bounds__(64 * WAVES, D > 128 ? 1 : 2) void pa_decode_u8_kern
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            // the word and the byte within it that hold channel chan(., r): u4 words hold four channels of one parity
-            const int word = U4 ? (VB == 4 ? 0 : 2 * (r >> 3) + (r & 1)) : r >> 2;
-            const int byte = U4 ? (VB == 4 ? 2 * (r & 1) + (r >> 1) : (r >> 1) & 3) : r & 3;
+            // the word and the byte within it that hold channel chan(., r) (u4: two channels, the even one in the high nibble)
+            const int word = U4 ? r >> 3 : r >> 2;
+            const int byte = U4 ? (r >> 1) & 3 : r & 3;
             const uint32_t sel = 0x0c000c00u | (uint32_t)byte | ((uint32_t)(4 + byte) << 16);
             u4v av;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 av[p] = perm(vw[word][2 * p + 1], vw[word][2 * p], sel);
-                if constexpr (FRESH) av[p] = centred_codes(av[p], NEG_CENTRE);
+                if constexpr (U4) av[p] = r & 1 ? centred_low_nibbles(av[p], NEG_CENTRE) : centred_high_nibbles(av[p], NEG_CENTRE);
+                else if constexpr (FRESH) av[p] = centred_codes(av[p], NEG_CENTRE);
             }
 #pragma unroll
             for (int gi = 0; gi < NG; ++gi) {
