@@ -156,7 +156,7 @@ typedef struct pa_layer_io {
  * kernels, correct but far from the tuned ones' speed -- except steps of single-token sequences over u4 K and V rows of head
  * size 64, 128 or (block size 32 up) 256 with at most 16 heads per kv head, which have a tuned kernel too.  In a step whose sequences all schedule one token, over a cache
  * the tuned kernels serve, the append is done by the attention kernel itself (the cache rows are the ones pa_kv_append
- * writes).  Head sizes 96 and 256 (K and V alike, the same caches) run on instantiations of the same kernels with
+ * writes); so it is in a step of few-token sequences over u8 whose blocks with new rows stand in the table once only.  Head sizes 96 and 256 (K and V alike, the same caches) run on instantiations of the same kernels with
  * these limits: the matrix kernel keeps to 16 query rows per wave, block-sparse prefill is not offered at 96, the u8 decode
  * kernel does not take head size 256 with 16-token blocks (such steps run on the shape-generic kernel). */
 int32_t pa_forward(pa_ctx* ctx, int32_t layer, const pa_layer_io* io);

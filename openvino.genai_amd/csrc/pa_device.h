@@ -148,6 +148,45 @@ __device__ __forceinline__ void quantize_row(const uint16_t (&raw)[EPL], uint8_t
     else if constexpr (EPL == 2) *reinterpret_cast<uint16_t*>(c) = (uint16_t)packed;
     else *c = (uint8_t)packed;
 }
+// The same over u8 with sixteen lanes to a row (four rows per wave; the same bytes): lane l16 holds D / 16 consecutive elements.
+template <int QDT, int D>
+__device__ __forceinline__ void quantize_row16(const uint16_t* src, uint8_t* dst, const int l16) {
+#pragma clang fp contract(off)
+    constexpr int EPL = D / 16;
+    static_assert(EPL == 4 || EPL == 8, "one load and one store per lane");
+    float x[EPL];
+    uint32_t w[EPL / 2];
+    if constexpr (EPL == 8) {
+        const uint4 v = *reinterpret_cast<const uint4*>(src + 8 * l16);
+        w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
+    } else {
+        const uint2 v = *reinterpret_cast<const uint2*>(src + 4 * l16);
+        w[0] = v.x, w[1] = v.y;
+    }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) x[e] = load16<QDT>((uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+    float mn = x[0], mx = x[0];
+#pragma unroll
+    for (int e = 1; e < EPL; ++e) { mn = fminf(mn, x[e]); mx = fmaxf(mx, x[e]); }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+        mn = fminf(mn, __shfl_xor(mn, o, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, o, 16));
+    }
+    float scale = (mx - mn) / 255.0f;
+    if (scale == 0.0f) scale = 0.0001f;
+    const float zp = -mn / scale;
+    const float inv = 1.0f / scale;
+    uint32_t packed[EPL / 4];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+        const float v = fminf(fmaxf(rintf(__fmaf_rn(x[e], inv, zp)), 0.0f), 255.0f);
+        packed[e >> 2] = (e & 3 ? packed[e >> 2] : 0u) | (uint32_t)(int)v << (8 * (e & 3));
+    }
+    if (l16 == 0) *reinterpret_cast<float2*>(dst) = make_float2(scale, zp);
+    if constexpr (EPL == 8) *reinterpret_cast<uint2*>(dst + 8 + 8 * l16) = make_uint2(packed[0], packed[1]);
+    else *reinterpret_cast<uint32_t*>(dst + 8 + 4 * l16) = packed[0];
+}
 // The lane's EPL consecutive elements of a row of 16-bit values.
 template <int EPL>
 __device__ __forceinline__ void load_row16(const uint16_t* src, uint16_t (&raw)[EPL]) {

@@ -211,6 +211,7 @@ struct pa_ctx {
     std::vector<const void*> table_ptr;  // where each table lives: its own buffer, or a slice of table_pool
     DevBuf table_pool;                   // the tables of a whole-model call, one after the other
     std::vector<int32_t> table_count;
+    std::vector<uint8_t> table_apart;  // of a step of few-token sequences: rows_apart() of each table
     std::vector<int64_t> table_bound;  // largest block id of each table + 1: the smallest cache it may be used with
     // u8 decode kernel: its split-K plan without / with scores (fixed per step) and, behind every table, the
     // per-(sequence, split) descriptors of both plans
@@ -1024,8 +1025,17 @@ int32_t* fold_counters(const pa_ctx* ctx, const pa::DecodeArgs& a, int32_t rows,
     return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(ctx->items.p) + ctx->arrived_off);
 }
 
+// Whether a layer call of the planned step runs on the few-token variant of the u8 decode kernel.
+bool few_call(const pa_ctx* ctx, const pa_layer_io* io) { return !ctx->h_few.empty() && !io->scores && ctx->n_sparse == 0; }
+
+// (of the layer's table; check_io and table_for refuse a layer or a table that is not there)
+bool few_apart(const pa_ctx* ctx, int32_t layer) {
+    const size_t idx = ctx->shared_table ? 0 : (size_t)layer;
+    return layer >= 0 && idx < ctx->table_apart.size() && ctx->table_apart[idx];
+}
+
 // fuse_append: the call is the attention half of pa_forward in a step whose sequences all go to one decode kernel (the
-// u8 one or the 16-bit one), and no append kernel has run: the decode kernel writes the step's K / V rows itself.
+// u8 one, its few-token variant or the 16-bit one), and no append kernel has run: the decode kernel writes the step's K / V rows itself.
 void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static_ws = false, bool fuse_append = false) {
     check_io(ctx, layer, io, false, true);
     const int32_t* table = table_for(ctx, layer);
@@ -1067,8 +1077,11 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         }
         return ctx->side;
     };
-    if (!ctx->h_few.empty() && !io->scores && !static_ws && ctx->n_sparse == 0) {
+    if (few_call(ctx, io) && !static_ws) {
         pa::DecodeArgs a{};
+        a.key = static_cast<const uint16_t*>(io->key);
+        a.value = static_cast<const uint16_t*>(io->value);
+        a.fuse_append = fuse_append ? 1 : 0;
         a.st = ctx->dev;
         a.sh = shape_of(c);
         a.G = c.num_heads / c.num_kv_heads;
@@ -1497,6 +1510,25 @@ int64_t checked_bound(const int32_t* ids, int32_t count, int64_t num_blocks) {
     return count == 0 ? 0 : (int64_t)id_hi + 1;
 }
 
+// Whether every block that takes a new row of the step stands in the table once only.  (A sequence whose past holds a block that
+// another one writes in the same step reads the new rows if all of them are in place before any sequence is attended to: such a
+// step keeps its append launch.)  A 64 Kbit map of the written ids' low bits passes over nearly all others: 1000 ids take 1 us.
+bool rows_apart(const pa_ctx* ctx, const int32_t* ids, int32_t count) {
+    std::vector<int32_t> written;
+    const int32_t bs = ctx->cfg.block_size;
+    for (int32_t b = 0; b < ctx->B; ++b) {
+        const int32_t kv = ctx->h_past[b] + ctx->h_sb[b + 1] - ctx->h_sb[b];
+        for (int32_t j = ctx->h_past[b] / bs; j < (kv + bs - 1) / bs; ++j) written.push_back(ids[ctx->h_bib[b] + j]);
+    }
+    std::sort(written.begin(), written.end());
+    uint64_t map[1024] = {};
+    for (const int32_t id : written) map[(id & 0xffff) >> 6] |= 1ull << (id & 63);
+    size_t found = 0;
+    for (int32_t i = 0; i < count; ++i)
+        if (map[(ids[i] & 0xffff) >> 6] >> (ids[i] & 63) & 1) found += std::binary_search(written.begin(), written.end(), ids[i]);
+    return found == written.size() && std::adjacent_find(written.begin(), written.end()) == written.end();
+}
+
 // Switches the context between one table for all layers and a table per layer.
 void shape_tables(pa_ctx* ctx, bool shared) {
     if (!ctx->tables.empty() && shared == ctx->shared_table) return;
@@ -1509,6 +1541,7 @@ void shape_tables(pa_ctx* ctx, bool shared) {
         ctx->table_ptr.assign(n, nullptr);
         ctx->table_count.assign(n, -1);
         ctx->table_bound.assign(n, 0);
+        ctx->table_apart.assign(n, 0);
     }
 }
 
@@ -1568,6 +1601,7 @@ int32_t pa_set_block_indices(pa_ctx* ctx, int32_t layer, const int32_t* ids, int
         ctx->table_ptr[idx] = ctx->tables[idx].p;
         ctx->table_count[idx] = count;
         ctx->table_bound[idx] = bound;
+        ctx->table_apart[idx] = !ctx->h_few.empty() && rows_apart(ctx, ids, count);
     });
 }
 
@@ -1590,10 +1624,12 @@ int32_t pa_set_block_indices_layers(pa_ctx* ctx, int32_t first_layer, int32_t nu
         // area (a table is read once, while it is in the core's cache; memory-bound host work); nothing of the
         // context changes before every layer has passed.
         std::vector<int64_t> bound((size_t)num_layers, 0);
+        std::vector<uint8_t> apart((size_t)num_layers, 0);
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
         uint8_t* stage = stage_piece(ctx, stride * (size_t)num_layers);
         pa::parallel_items((size_t)num_layers, std::min<size_t>(8, (size_t)num_layers * (size_t)count / 131072 + 1), [&](size_t l) {
             bound[l] = checked_bound(ids_per_layer[l], count, num_blocks);
+            apart[l] = !ctx->h_few.empty() && rows_apart(ctx, ids_per_layer[l], count);
             fill_table_stage(ctx, ids_per_layer[l], count, id_bytes, with_descs, stage + l * stride);
         });
         if (ctx->table_pool.cap < stride * (size_t)ctx->cfg.num_layers) {
@@ -1616,6 +1652,7 @@ int32_t pa_set_block_indices_layers(pa_ctx* ctx, int32_t first_layer, int32_t nu
             ctx->table_ptr[idx] = dst + (size_t)l * stride;
             ctx->table_count[idx] = count;
             ctx->table_bound[idx] = bound[(size_t)l];
+            ctx->table_apart[idx] = apart[(size_t)l];
             }
     });
 }
@@ -1799,11 +1836,13 @@ int32_t pa_forward(pa_ctx* ctx, int32_t layer, const pa_layer_io* io) {
     if (!ctx) return PA_INVALID_C_PARAM;
     return guarded(ctx, [&] {
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
-        // a step of single-token sequences that all go to one of the decode kernels: it appends the new rows itself
+        // a step of single-token sequences that all go to one of the decode kernels, or one of few-token sequences on the u8 kernel's
+        // variant for them that write into blocks of their own: the kernel appends the new rows itself
         const bool fuse = ctx->step_ready &&
                           ((decode_u8_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B) || decode_u4_step(ctx) ||
                            (mfma_shape(ctx) && decode16_shape(ctx) && (int32_t)ctx->h_dec16.size() == ctx->B &&
-                            ctx->n_sparse == 0 && ctx->n_single == ctx->n_items));
+                            ctx->n_sparse == 0 && ctx->n_single == ctx->n_items) ||
+                           (io && few_call(ctx, io) && few_apart(ctx, layer)));
         if (fuse) check_io(ctx, layer, io, true, false);
         else do_kv_append(ctx, layer, io);
         do_attention(ctx, layer, io, false, fuse);

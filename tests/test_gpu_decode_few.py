@@ -137,3 +137,37 @@ def test_decode_few_magnitudes(pkg, vmul):
     got = H.run_case_on_gpu(pkg, dict(case, value_cache0=vc, value=value), dev, want_scores=False)
     # every scaling is exact and each sum goes along with it: only a tile's unit can differ
     assert np.abs(got["out"] / np.float32(vmul) - plain["out"]).max() <= 2.0 ** -8 * np.abs(plain["out"]).max()
+
+
+@pytest.mark.parametrize("qd,bs,Hq,Hkv,D,past,new,sw", [
+    ("f16", 32, 32, 8, 128, [4000, 30, 0, 95], [5, 5, 5, 1], 0), ("bf16", 16, 8, 2, 64, [15, 700], [8, 3], 0),
+    ("f16", 64, 4, 4, 64, [31, 4000], [32, 1], 40), ("bf16", 256, 4, 1, 128, [254, 9000], [4, 4], 0)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_append_in_the_few_token_kernel(pkg, qd, bs, Hq, Hkv, D, past, new, sw, shared):
+    """pa_forward against its two halves, bit for bit; `shared`: a sequence more whose past is the first one's context, the rows that
+    the same step writes included (its own new rows go behind them or into a block of its own)."""
+    import torch
+    dev = torch.device("cuda:0")
+    case = H.build_case(H.case_from_lens("few", Hq, Hkv, D, bs, qd, "u8", past + [past[0] + new[0]] * shared, new + [2] * shared, sw), seed=bs)
+    ids, bib = case["block_indices"].copy(), case["block_indices_begins"]
+    if shared:
+        n = -(-(past[0] + new[0]) // bs)
+        ids[bib[-2]:bib[-2] + n] = ids[:n]
+    q, k, v = (H.to_device_16(torch, case[x], qd, dev) for x in ("query", "key", "value"))
+    got = []
+    for halves in (False, True):
+        op = pkg.PagedAttention(Hq, Hkv, D, bs, qd, "u8", 1, 0, torch.cuda.current_stream(dev))
+        kc, vc = (torch.from_numpy(case[x]).to(dev) for x in ("key_cache0", "value_cache0"))
+        out = torch.zeros_like(q)
+        op.step_begin(case["past_lens"], case["subsequence_begins"], bib, int((case["past_lens"] + case["new_lens"]).max()), None, sw, case["scale"])
+        op.set_block_indices(ids, case["num_blocks"])
+        if halves:
+            op.kv_append(k, v, kc, vc)
+            op.attention(q, kc, vc, out)
+        else:
+            op.forward(q, k, v, kc, vc, out)
+        op.synchronize()
+        assert "decode_few" in op.kernels_run
+        got.append((out.view(torch.int16).cpu(), kc.cpu(), vc.cpu()))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
