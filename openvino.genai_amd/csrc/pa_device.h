@@ -436,7 +436,7 @@ hipError_t launch_scores_from_logits(hipStream_t s, const StepDev& st, int Hq, f
 // ---- block-sparse prefill (XAttention) -----------------------------------------------------------
 // Blocks and strided groups are counted by absolute position: query / key block I covers positions
 // [I * xb, (I + 1) * xb), strided group i covers [i * S, (i + 1) * S); xb and S are powers of two, S <= 32 <= xb.
-constexpr int XATT_KEY_TILE = 64;   // strided key groups one workgroup of the logits kernel covers (rows of logits are padded to 128)
+constexpr int XATT_KEY_TILE = 64;   // strided key groups one workgroup of the u8 logits kernel covers (rows of logits are padded to 128)
 struct XattSeq {            // one sequence of the step that runs block-sparse
     int32_t b;              // sequence
     int32_t qb0, nqb;       // first query block of the chunk and how many it touches
@@ -796,9 +796,10 @@ hipError_t launch_prefill16(hipStream_t s, const PrefillArgs& a, int q_dtype, in
                             hipEvent_t ev1, bool merge_later = false);
 
 // ---- block-sparse prefill (XAttention): the estimate's launch ---------------------------------
-struct XattTile {           // one workgroup-sized piece of the strided logits: 32 query groups x 128 key groups
+struct XattTile {           // one workgroup-sized piece of the strided logits
     int32_t x;              // index into the XattSeq list
-    int32_t it, jc;         // query groups [32 it, 32 it + 32) of the chunk, key groups [128 jc, 128 jc + 128)
+    int32_t it, jc;         // u8: query groups [32 it, 32 it + 32) of the chunk, key groups [64 jc, 64 jc + 64); 16-bit: (query
+                            // group, head) rows and key groups, `tile16` of each
     int32_t pad;
 };
 struct XattArgs {
@@ -811,6 +812,7 @@ struct XattArgs {
     const int32_t* seq_of;      // [B]: index into seqs, -1 for a dense sequence
     const XattTile* tiles;
     int32_t nseq, ntiles;
+    int32_t tile16;             // 16-bit caches: 64 or 128
     int32_t max_nqs, max_nqb, max_nkb;
     int32_t xb_shift, s_shift;  // log2 of the block size and of the stride
     float* logits;

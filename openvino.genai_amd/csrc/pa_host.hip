@@ -182,7 +182,7 @@ struct pa_ctx {
     std::vector<pa::PrefillItem> h_items;
     int32_t xatt_block = 0, xatt_stride = 0;
     bool x_ran = false;               // a layer call of this step has produced block sums and masks
-    int32_t n_sparse = 0, x_ntiles = 0, x_keep_words = 1, x_max_nqs = 0, x_max_nqb = 0, x_max_nkb = 0;
+    int32_t n_sparse = 0, x_ntiles = 0, x_tile16 = 128, x_keep_words = 1, x_max_nqs = 0, x_max_nqb = 0, x_max_nkb = 0;
     size_t x_tiles_off = 0, x_seq_of_off = 0;
     DevBuf x_plan;                    // XattSeq list | tiles of the estimate | sequence -> list index
     DevBuf x_logits, x_sums, x_mask, x_item_keep;
@@ -1239,6 +1239,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             x.tiles = reinterpret_cast<const pa::XattTile*>(static_cast<const uint8_t*>(ctx->x_plan.p) + ctx->x_tiles_off);
             x.nseq = (int32_t)ctx->h_xseq.size();
             x.ntiles = ctx->x_ntiles;
+            x.tile16 = ctx->x_tile16;
             x.max_nqs = ctx->x_max_nqs;
             x.max_nqb = ctx->x_max_nqb;
             x.max_nkb = ctx->x_max_nkb;
@@ -1725,13 +1726,29 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
             logit_off += (int64_t)Hq * rows * xs.ld;
             sum_off += (int64_t)Hq * xs.nqb * xs.nkb;
             mask_off += (int64_t)Hq * xs.nqb * xs.words;
-            for (int32_t it = 0; it < rows / 32; ++it) {
-                const int32_t last = xs.qs0 + std::min(32 * it + 31, xs.nqs - 1);  // last strided query group of the tile
-                for (int32_t jc = 0; pa::XATT_KEY_TILE * jc <= last; ++jc) tiles.push_back({(int32_t)x, it, jc, 0});
-            }
             max_nqs = std::max(max_nqs, xs.nqs);
             max_nqb = std::max(max_nqb, xs.nqb);
             max_nkb = std::max(max_nkb, xs.nkb);
+        }
+        // 16-bit caches: tiles of 128 x 128 logits where they give three quarters of the CUs one each, else of 64 x 64, of which four
+        // buffers fit.  us per layer as a step, 64 / 128 / (the kernel before, 32 groups x 64 keys x 4 heads): 28 / 4 heads of 128, 144
+        // large tiles 78 / 83 / 85, 224: 105 / 103 / 106, 900: 264 / 237 / 256; 32 / 8 heads, 120: 142 / 147 / 146, 432: 124 / 119 / 121.
+        const int32_t G = Hq / c.num_kv_heads;
+        int32_t tile16 = 128;
+        auto list_tiles = [&](int32_t q_rows, int32_t heads, int32_t keys) {  // q_rows: (query group, head) rows, `heads` to a group
+            tiles.clear();
+            for (size_t x = 0; x < seqs.size(); ++x) {
+                const int32_t last = seqs[x].nqs - 1;  // (the last query group of a tile is the last key group it needs)
+                for (int32_t it = 0; (int64_t)q_rows * it < (int64_t)seqs[x].nqs * heads; ++it)
+                    for (int32_t jc = 0; keys * jc <= seqs[x].qs0 + std::min((q_rows * it + q_rows - 1) / heads, last); ++jc)
+                        tiles.push_back({(int32_t)x, it, jc, 0});
+            }
+        };
+        if (c.kv_cache_dtype == PA_U8) {
+            list_tiles(32, 1, pa::XATT_KEY_TILE);
+        } else {
+            list_tiles(128, G, 128);
+            if ((int64_t)tiles.size() * c.num_kv_heads < 192) list_tiles(tile16 = 64, G, 64);
         }
         PA_REQUIRE(logit_off * 4 <= ((int64_t)4 << 30), PA_NOT_ALLOCATED,
                    "block-sparse prefill: the strided logits of this step exceed 4 GiB (larger stride or shorter chunks)");
@@ -1752,6 +1769,7 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         ctx->xatt_block = block_size;
         ctx->xatt_stride = stride;
         ctx->x_ntiles = (int32_t)tiles.size();
+        ctx->x_tile16 = tile16;
         ctx->x_max_nqs = max_nqs;
         ctx->x_max_nqb = max_nqb;
         ctx->x_max_nkb = max_nkb;

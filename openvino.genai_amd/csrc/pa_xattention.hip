@@ -14,34 +14,20 @@
 //
 // Roofline: step 1 is dense MFMA work, 2 D / S flops per (query position, key position, head) -- 1 / (2 S) of the
 // attention it prunes; the other steps touch a few hundred KB.
-#include "pa_device.h"
+#include "pa_prefill.h"
 
 #include <algorithm>
 
 namespace pa {
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef short s8v __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-
-constexpr float LOG2E = 1.4426950408889634f;
-
-template <int DT>
-__device__ __forceinline__ f4 mma(const s8v& a, const s8v& b, const f4& c) {
-    if (DT == DT_F16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
-}
 
 __device__ __forceinline__ uint32_t f16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
 }
 
-// ---- 1. strided logits ---------------------------------------------------------------------------------------
+// ---- 1. strided logits, u8 caches ----------------------------------------------------------------------------
 // A workgroup (four waves) = 32 strided query groups of up to four query heads that share a kv head x 64 strided
 // key groups (XATT_KEY_TILE); wave w takes head w of the four: two 16-column tiles of queries (B operands) against
 // four 16-row tiles of keys (A operands).  (With 128 key groups per workgroup -- half as many workgroups, 64
@@ -55,17 +41,16 @@ __device__ __forceinline__ uint32_t f16x2(float a, float b) {
 // into operand layout -- sixteen rows per instruction, every lane in a cache line of its own -- the address unit set
 // the pace).  Within a stage lane (n, g) supplies channels 16 g .. 16 g + 15 of row n as the k-slices of two matrix
 // instructions (which channel sits in which k-slice is free as long as both operands agree).
-template <int D, int DT, int QDT, bool U8>
-__global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
-    static_assert(!U8 || DT == DT_F16, "u8 codes are multiplied as f16");
-    constexpr int CROWB = U8 ? D + 8 : D * 2;
+template <int D, int QDT>
+__global__ __launch_bounds__(256, 2) void xatt_logits_u8_kernel(XattArgs a) {
+    constexpr int CROWB = D + 8;
     constexpr int DP = D / 64;             // stages per slot
     constexpr int KST = 128;               // LDS bytes per key or query row of a stage; the row's 16-byte piece p sits at
                                            // p ^ ((row >> 1) & 7): stores (eight or four lanes to a row) and operand
                                            // reads (sixteen rows at one piece) both touch every bank once
     constexpr int KT = XATT_KEY_TILE;      // strided key groups per workgroup
     constexpr int NJ = KT / 16;
-    constexpr int RPP = U8 ? 64 : 32;      // key rows one pass of the 256 threads covers
+    constexpr int RPP = 64;                // key rows one pass of the 256 threads covers
     constexpr int KCH = KT / RPP;          // 16-byte pieces of the cache a thread moves per stage
     __shared__ __align__(16) uint8_t kbuf[2][KT * KST];
     __shared__ __align__(16) uint8_t qbuf[2][4][32 * KST];   // per wave: its head's 32 query rows of a stage
@@ -95,7 +80,7 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
     const int bs_shift = 31 - __builtin_clz(a.sh.bs);  // cache blocks of 32 tokens or more (a power of two)
 
     // this thread's share of a stage's key rows: rows kr0 + RPP * k, the piece `kpart` of each
-    const int kr0 = U8 ? tid >> 2 : tid >> 3, kpart = U8 ? tid & 3 : tid & 7;
+    const int kr0 = tid >> 2, kpart = tid & 3;
     int k_pos0[KCH];
     const uint8_t* k_blk[KCH];
 #pragma unroll
@@ -108,19 +93,15 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
     // group's last token) of this lane's row in the first load, relative to the chunk
     const int qrow = lane >> 3, qpart = lane & 7;
     const int q_rel0 = ((xs.qs0 + 32 * tl.it + qrow) << a.s_shift) + S - 1 - past;
-    struct KSet { u4v c[KCH]; uint2 hd[KCH]; };   // hd: u8 row headers
+    struct KSet { u4v c[KCH]; uint2 hd[KCH]; };   // hd: row headers
     struct QSet { u4v q[4]; };
     auto load_k = [&](KSet& ks, int u) __attribute__((always_inline)) {
         const int s = u / DP, ch = (u % DP) * 64;
 #pragma unroll
         for (int k = 0; k < KCH; ++k) {
             const uint8_t* row = k_blk[k] + (min(k_pos0[k] + s, kv_len - 1) & (a.sh.bs - 1)) * CROWB;
-            if (U8) {
-                ks.c[k] = *reinterpret_cast<const u4v*>(row + 8 + ch + 16 * kpart);
-                ks.hd[k] = *reinterpret_cast<const uint2*>(row);
-            } else {
-                ks.c[k] = *reinterpret_cast<const u4v*>(row + ch * 2 + 16 * kpart);
-            }
+            ks.c[k] = *reinterpret_cast<const u4v*>(row + 8 + ch + 16 * kpart);
+            ks.hd[k] = *reinterpret_cast<const uint2*>(row);
         }
     };
     auto store_k = [&](const KSet& ks, int u) __attribute__((always_inline)) {
@@ -131,21 +112,17 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
             const bool ok = k_pos0[k] + s < kv_len;
             const int krow = kr0 + RPP * k, ksw = (krow >> 1) & 7;
             uint8_t* dst = buf + krow * KST;
-            if (U8) {
-                const float sc = ok ? __builtin_bit_cast(float, ks.hd[k].x) : 0.0f;
-                const float nz = ok ? -__builtin_bit_cast(float, ks.hd[k].y) * sc : 0.0f;
-                u4v v[2];
+            const float sc = ok ? __builtin_bit_cast(float, ks.hd[k].x) : 0.0f;
+            const float nz = ok ? -__builtin_bit_cast(float, ks.hd[k].y) * sc : 0.0f;
+            u4v v[2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t w = ks.c[k][e];
-                    v[e >> 1][2 * (e & 1)] = f16x2(fmaf((float)(w & 0xffu), sc, nz), fmaf((float)((w >> 8) & 0xffu), sc, nz));
-                    v[e >> 1][2 * (e & 1) + 1] = f16x2(fmaf((float)((w >> 16) & 0xffu), sc, nz), fmaf((float)(w >> 24), sc, nz));
-                }
-                *reinterpret_cast<u4v*>(dst + 16 * ((2 * kpart) ^ ksw)) = v[0];
-                *reinterpret_cast<u4v*>(dst + 16 * ((2 * kpart + 1) ^ ksw)) = v[1];
-            } else {
-                *reinterpret_cast<u4v*>(dst + 16 * (kpart ^ ksw)) = ok ? ks.c[k] : u4v{0u, 0u, 0u, 0u};
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t w = ks.c[k][e];
+                v[e >> 1][2 * (e & 1)] = f16x2(fmaf((float)(w & 0xffu), sc, nz), fmaf((float)((w >> 8) & 0xffu), sc, nz));
+                v[e >> 1][2 * (e & 1) + 1] = f16x2(fmaf((float)((w >> 16) & 0xffu), sc, nz), fmaf((float)(w >> 24), sc, nz));
             }
+            *reinterpret_cast<u4v*>(dst + 16 * ((2 * kpart) ^ ksw)) = v[0];
+            *reinterpret_cast<u4v*>(dst + 16 * ((2 * kpart + 1) ^ ksw)) = v[1];
         }
     };
     auto load_q = [&](QSet& qs, int u) __attribute__((always_inline)) {
@@ -164,7 +141,7 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
         for (int c = 0; c < 4; ++c) {
             const int rel = q_rel0 + ((8 * c) << a.s_shift) - s;
             u4v v = (rel >= 0 && rel < q_len) ? qs.q[c] : u4v{0u, 0u, 0u, 0u};
-            if (QDT != DT) {
+            if (QDT != DT_F16) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     v[e] = f16x2(__builtin_bit_cast(float, v[e] << 16), __builtin_bit_cast(float, v[e] & 0xffff0000u));
@@ -191,7 +168,7 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
             for (int nj = 0; nj < NJ; ++nj) {
                 const s8v kop = *reinterpret_cast<const s8v*>(buf + (16 * nj + n) * KST + 16 * ((2 * g + kk) ^ ((n >> 1) & 7)));
 #pragma unroll
-                for (int mi = 0; mi < 2; ++mi) acc[mi][nj] = mma<DT>(kop, qop[mi], acc[mi][nj]);
+                for (int mi = 0; mi < 2; ++mi) acc[mi][nj] = mma<DT_F16>(kop, qop[mi], acc[mi][nj]);
             }
         }
     };
@@ -241,6 +218,141 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_kernel(XattArgs a) {
         float* out = a.logits + xs.logit_off + ((long)hq * rows + 32 * tl.it + 16 * mi + n) * xs.ld + KT * tl.jc + 4 * g;
 #pragma unroll
         for (int nj = 0; nj < NJ; ++nj) *reinterpret_cast<f4*>(out + 16 * nj) = acc[mi][nj] * scl;
+    }
+}
+
+// ---- 1. strided logits, 16-bit caches ------------------------------------------------------------------------
+// A product of (strided group, head) rows and strided key groups per kv head, in tiles of MT x MT, four waves of a quarter each.  The
+// rows of a kv head's heads are numbered through (row = query group * G + head), so a group of seven heads fills its tiles as
+// one of eight does.  A stage is 64 channels of one slot: 128 bytes of MT + MT rows, copied from memory straight into LDS while
+// earlier stages are multiplied: two buffers of 32 KB at MT = 128, where two workgroups per CU cover for each other, four of 16 KB
+// at MT = 64, for steps too small to fill the chip with the large tiles.  Pieces of 16 bytes are placed as in the u8 kernel, by the
+// address each lane reads; lanes whose row is outside the chunk or beyond the context read zeros.  Same products in the same
+// order as there: the same logits bit for bit.
+// Bound by LDS: a 64-channel stage of a large tile takes 128 operand reads of 1 KB and 32 KB of copies beside 510 cycles of the
+// matrix pipe.  2048 tokens behind 14011 (28 / 4 heads, D = 128, stride 8): 71 us a launch with 32 groups x 64 keys x 4 heads
+// per workgroup and operands through registers, 53 us (525 TFLOP/s) so; as a step of two layers 514 -> 480 us, 16 / 8 heads of 256
+// behind 12000 534 -> 435, 128 tokens from scratch 98 -> 90.  Four buffers of large tiles, one workgroup per CU: 543 for 483 us.
+__device__ const u4v xatt_zeros = {0u, 0u, 0u, 0u};
+
+template <int D, int DT, int MT>
+__global__ __launch_bounds__(256, 2) void xatt_logits16_kernel(XattArgs a) {
+    constexpr int KST = 128, DP = D / 64, CROWB = 2 * D, STAGE = MT * KST;
+    constexpr int NBUF = MT == 128 ? 2 : 4;  // stages in LDS
+    constexpr int NC = MT / 32;              // copies of each operand per wave and stage
+    constexpr int NI = MT / 32;              // 16-row operands of each kind per wave
+    // (every buffer an LDS object of its own: operand reads wait for copies that may write what they read)
+    __shared__ __align__(16) uint8_t k0[STAGE], k1[STAGE], k2[NBUF > 2 ? STAGE : 16], k3[NBUF > 2 ? STAGE : 16];
+    __shared__ __align__(16) uint8_t q0[STAGE], q1[STAGE], q2[NBUF > 2 ? STAGE : 16], q3[NBUF > 2 ? STAGE : 16];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int Hq = a.sh.Hq, Hkv = a.sh.Hkv, G = a.G;
+    // (a contiguous eighth of the numbering per XCD, as in the u8 kernel)
+    const int total = gridDim.x, xcd = blockIdx.x & 7;
+    const int work = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
+    const int hkv = work / a.ntiles;
+    const XattTile tl = a.tiles[work % a.ntiles];
+    const XattSeq xs = a.seqs[tl.x];
+    const int t0 = a.st.subsequence_begins[xs.b];
+    const int q_len = a.st.subsequence_begins[xs.b + 1] - t0;
+    const int past = a.st.past_lens[xs.b];
+    const int kv_len = past + q_len;
+    const int S = 1 << a.s_shift;
+    const int32_t* table = a.block_indices + a.st.block_indices_begins[xs.b];
+    const int bs_shift = 31 - __builtin_clz(a.sh.bs);
+
+    // Wave w copies rows 8 NC w .. of both operands, eight rows per instruction and eight lanes to a row; this lane's rows are
+    // 8 NC w + 8 c + lane / 8.  Key row of slot s: k_at + s rows, for s < k_cnt; query row: q_at - s tokens, for
+    // 0 <= q_rel - s < q_len.
+    const uint8_t* const zeros = reinterpret_cast<const uint8_t*>(&xatt_zeros);
+    const uint8_t* k_at[NC];
+    uint64_t q_at[NC];
+    int k_cnt[NC], q_rel[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int row = 8 * NC * wv + 8 * c + (lane >> 3), piece = 16 * ((lane & 7) ^ ((row >> 1) & 7));
+        const int pos0 = (MT * tl.jc + row) << a.s_shift, pos = min(pos0, kv_len - 1);
+        k_cnt[c] = kv_len - pos0;
+        k_at[c] = a.key_cache + (((long)table[pos >> bs_shift] * Hkv + hkv) * a.sh.bs + (pos & (a.sh.bs - 1))) * CROWB + piece;
+        const int r = MT * tl.it + row, qg = r / G;
+        q_rel[c] = qg < xs.nqs ? ((xs.qs0 + qg) << a.s_shift) + S - 1 - past : -1;
+        q_at[c] = reinterpret_cast<uint64_t>(a.query) + ((long)(t0 + q_rel[c]) * Hq + hkv * G + r % G) * (D * 2) + piece;
+    }
+    auto copy = [&](int u, uint8_t* kb, uint8_t* qb) __attribute__((always_inline)) {
+        const int s = u / DP, ch = (u % DP) * 128;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) dma16(s < k_cnt[c] ? k_at[c] + s * CROWB + ch : zeros, kb + 1024 * (NC * wv + c));
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int rel = q_rel[c] - s;
+            dma16(rel >= 0 && rel < q_len ? reinterpret_cast<const uint8_t*>(q_at[c] - (uint64_t)((long)s * Hq * D * 2) + ch) : zeros,
+                  qb + 1024 * (NC * wv + c));
+        }
+    };
+    const int wk = MT / 2 * (wv & 1), wq = MT / 2 * (wv >> 1);  // the wave's quarter: keys (A operands) and queries (B operands)
+    f4 acc[NI][NI];
+#pragma unroll
+    for (int mi = 0; mi < NI; ++mi)
+#pragma unroll
+        for (int nj = 0; nj < NI; ++nj) acc[mi][nj] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](const uint8_t* kb, const uint8_t* qb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int at = n * KST + 16 * ((2 * g + kk) ^ ((n >> 1) & 7));
+            s8v qop[NI], kop[NI];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                qop[i] = *reinterpret_cast<const s8v*>(qb + (wq + 16 * i) * KST + at);
+                kop[i] = *reinterpret_cast<const s8v*>(kb + (wk + 16 * i) * KST + at);
+            }
+#pragma unroll
+            for (int nj = 0; nj < NI; ++nj)
+#pragma unroll
+                for (int mi = 0; mi < NI; ++mi) acc[mi][nj] = mma<DT>(kop[nj], qop[mi], acc[mi][nj]);
+        }
+    };
+    // Stage u: every wave waits for its own copies of it and meets the others, who are then through with stage u - 1 as well, whose
+    // buffers take stage u + NBUF - 1 while stage u is multiplied (behind the last stage it once more: the count of copies under way
+    // stays the same).
+    const int NU = S * DP;
+    copy(0, k0, q0);
+    if (NBUF > 2) {
+        copy(min(1, NU - 1), k1, q1);
+        copy(min(2, NU - 1), k2, q2);
+    }
+#define PA_XSTEP(KC, QC, KN, QN)                             \
+    {                                                        \
+        wait_vmem<2 * NC * (NBUF - 2)>();                    \
+        lds_barrier();                                       \
+        if (NBUF > 2) copy(min(u + NBUF - 1, NU - 1), KN, QN); \
+        else if (u + 1 < NU) copy(u + 1, KN, QN);            \
+        compute(KC, QC);                                     \
+        if (++u == NU) break;                                \
+    }
+    for (int u = 0;;) {
+        if constexpr (NBUF == 2) {
+            PA_XSTEP(k0, q0, k1, q1)
+            PA_XSTEP(k1, q1, k0, q0)
+        } else {
+            PA_XSTEP(k0, q0, k3, q3)
+            PA_XSTEP(k1, q1, k0, q0)
+            PA_XSTEP(k2, q2, k1, q1)
+            PA_XSTEP(k3, q3, k2, q2)
+        }
+    }
+    wait_vmem<0>();  // (the copies behind the last stage still target this workgroup's LDS)
+#undef PA_XSTEP
+
+    // lane (n, g), register i of tile (mi, nj): row wq + 16 mi + n, key group wk + 16 nj + 4 g + i
+    const float scl = a.st.scale * LOG2E / (float)S;
+    const int rows = (xs.nqs + 31) & ~31;
+#pragma unroll
+    for (int mi = 0; mi < NI; ++mi) {
+        const int r = MT * tl.it + wq + 16 * mi + n, qg = r / G;
+        if (qg >= xs.nqs) continue;
+        float* out = a.logits + xs.logit_off + ((long)(hkv * G + r % G) * rows + qg) * xs.ld + MT * tl.jc + wk + 4 * g;
+#pragma unroll
+        for (int nj = 0; nj < NI; ++nj) *reinterpret_cast<f4*>(out + 16 * nj) = acc[mi][nj] * scl;
     }
 }
 
@@ -431,24 +543,31 @@ __global__ __launch_bounds__(64) void xatt_item_keep_kernel(XattArgs a) {
 
 hipError_t launch_xattention(hipStream_t s, const XattArgs& a, int q_dtype, int kv_dtype) {
     if (a.nseq == 0) return hipSuccess;
-    const dim3 lgrid((unsigned)(a.ntiles * a.sh.Hkv * ceil_div(a.G, 4)));
-#define PA_XLOGITS(DD, DT, Q, U8) \
-    hipLaunchKernelGGL((xatt_logits_kernel<DD, DT, Q, U8>), lgrid, dim3(256), 0, s, a)
     const bool f16q = q_dtype == DT_F16;
     // (a stage is 64 channels of a slot: head sizes that are multiples of 64)
     if (a.sh.bs < 32 || a.sh.bs > 256 || (a.sh.bs & (a.sh.bs - 1)) || (a.sh.D != 64 && a.sh.D != 128 && a.sh.D != 256)) return hipErrorInvalidValue;
     if (kv_dtype == DT_U8) {
-        if (a.sh.D == 64) { if (f16q) PA_XLOGITS(64, DT_F16, DT_F16, true); else PA_XLOGITS(64, DT_F16, DT_BF16, true); }
-        else if (a.sh.D == 128) { if (f16q) PA_XLOGITS(128, DT_F16, DT_F16, true); else PA_XLOGITS(128, DT_F16, DT_BF16, true); }
-        else { if (f16q) PA_XLOGITS(256, DT_F16, DT_F16, true); else PA_XLOGITS(256, DT_F16, DT_BF16, true); }
+        const dim3 grid((unsigned)(a.ntiles * a.sh.Hkv * ceil_div(a.G, 4)));
+#define PA_XLOGITS(DD, Q) hipLaunchKernelGGL((xatt_logits_u8_kernel<DD, Q>), grid, dim3(256), 0, s, a)
+        if (a.sh.D == 64) { if (f16q) PA_XLOGITS(64, DT_F16); else PA_XLOGITS(64, DT_BF16); }
+        else if (a.sh.D == 128) { if (f16q) PA_XLOGITS(128, DT_F16); else PA_XLOGITS(128, DT_BF16); }
+        else { if (f16q) PA_XLOGITS(256, DT_F16); else PA_XLOGITS(256, DT_BF16); }
+#undef PA_XLOGITS
     } else if (kv_dtype == q_dtype) {
-        if (a.sh.D == 64) { if (f16q) PA_XLOGITS(64, DT_F16, DT_F16, false); else PA_XLOGITS(64, DT_BF16, DT_BF16, false); }
-        else if (a.sh.D == 128) { if (f16q) PA_XLOGITS(128, DT_F16, DT_F16, false); else PA_XLOGITS(128, DT_BF16, DT_BF16, false); }
-        else { if (f16q) PA_XLOGITS(256, DT_F16, DT_F16, false); else PA_XLOGITS(256, DT_BF16, DT_BF16, false); }
+        const dim3 grid((unsigned)(a.ntiles * a.sh.Hkv));
+        if (a.tile16 != 64 && a.tile16 != 128) return hipErrorInvalidValue;
+#define PA_XLOGITS(DD, Q)                                                                                  \
+    {                                                                                                      \
+        if (a.tile16 == 64) hipLaunchKernelGGL((xatt_logits16_kernel<DD, Q, 64>), grid, dim3(256), 0, s, a); \
+        else hipLaunchKernelGGL((xatt_logits16_kernel<DD, Q, 128>), grid, dim3(256), 0, s, a);             \
+    }
+        if (a.sh.D == 64) { if (f16q) PA_XLOGITS(64, DT_F16) else PA_XLOGITS(64, DT_BF16) }
+        else if (a.sh.D == 128) { if (f16q) PA_XLOGITS(128, DT_F16) else PA_XLOGITS(128, DT_BF16) }
+        else { if (f16q) PA_XLOGITS(256, DT_F16) else PA_XLOGITS(256, DT_BF16) }
+#undef PA_XLOGITS
     } else {
         return hipErrorInvalidValue;
     }
-#undef PA_XLOGITS
     const int R = 1 << (a.xb_shift - a.s_shift);
     const size_t lds = (size_t)a.max_nkb * 16 + 256 * 8 + (size_t)R * 8 + (size_t)ceil_div(a.max_nkb, 32) * 4;
     hipLaunchKernelGGL(xatt_select_kernel, dim3((unsigned)a.max_nqb, (unsigned)a.sh.Hq, (unsigned)a.nseq), dim3(256), lds,

@@ -128,6 +128,19 @@ def test_sparse_prefill(env, name, Hq, Hkv, D, qd, kd, past, new, xb, S, mult, t
     assert kept.mean() < 1.0  # something was left out, or the case says nothing about masking
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,dt,past,new,S", [
+    # rows (query groups x heads of a kv head) and key groups one short of, at and one beyond 128 and 256
+    (16, 1, 64, "f16", [120], [8], 1), (16, 1, 64, "bf16", [120], [9], 1), (1, 1, 128, "bf16", [0], [127], 1), (2, 2, 128, "f16", [1], [128], 1),
+    (1, 1, 64, "f16", [128], [129], 1), (7, 1, 128, "bf16", [1021], [146], 8), (5, 1, 128, "f16", [2040, 7], [209, 2], 8),
+    (6, 2, 256, "bf16", [1013], [43], 4),
+    # steps large enough for the tiles of 128 x 128: whole tiles and remainders of both kinds, two sequences
+    (16, 1, 64, "f16", [600], [424], 1), (20, 4, 128, "bf16", [1021, 30], [517, 129], 2), (12, 6, 256, "f16", [400], [385], 1)])
+def test_edges_of_the_16_bit_estimate(env, Hq, Hkv, D, dt, past, new, S):
+    pkg, dev = env
+    c = H.build_case(H.case_from_lens("edges", Hq, Hkv, D, 32, dt, dt, past, new, scale=4.0 / np.sqrt(D)), Hq + D + S)
+    _check(pkg, dev, c, np.full(len(past), 0.7, np.float32), 32, S, min_decided=0.0)
+
+
 def test_mixed_step(env):
     """Sparse chunks, a dense chunk (threshold 0) and single-token sequences in one step, with a sliding window."""
     pkg, dev = env
