@@ -151,7 +151,7 @@ typedef struct pa_layer_io {
 
 /* One layer's PagedAttention: KV append (+ u8 / u4 quantisation), attention, optional scores.  Tuned
  * kernels serve block_size 16, 32, 64, 128 and 256 with head size 64 or 128, K and V alike, over a u8 cache or an f16 /
- * bf16 cache of the query's type; every other combination pa_create accepts (other head sizes, a value head size or
+ * bf16 cache of the query's type, and at most 128 query heads per kv head; every other combination pa_create accepts (other head sizes, a value head size or
  * value precision of its own, u4 rows, a 16-bit cache of the other 16-bit type, other block sizes) runs on shape-generic
  * kernels, correct but far from the tuned ones' speed -- except steps of single-token sequences over u4 K and V rows of head
  * size 64, 128 or (block size 32 up) 256 with at most 16 heads per kv head, which have a tuned kernel too.  In a step whose sequences all schedule one token, over a cache
@@ -287,8 +287,8 @@ float pa_xattention_threshold(float configured_threshold, uint64_t num_last_dens
  *     its groups; tokens outside the chunk count as zero vectors;
  *   - per (query head, I): key blocks 0 and I are kept, then the others in descending importance until the kept sum
  *     reaches threshold * the row's sum; a query row then sees a key position only if its block pair was kept.
- * Needs a cache block_size of 32, 64, 128 or 256, head_size 64 / 128 / 256 (K and V alike), a u8 cache or one of the query's
- * type; xattention_block_size a power of two >= 32, xattention_stride a power of two <= 32 (PA_NOT_IMPLEMENTED
+ * Needs a cache block_size of 32, 64, 128 or 256, head_size 64 / 128 / 256 (K and V alike), at most 128 query heads per kv
+ * head, a u8 cache or one of the query's type; xattention_block_size a power of two >= 32, xattention_stride a power of two <= 32 (PA_NOT_IMPLEMENTED
  * otherwise). */
 int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t xattention_block_size,
                           int32_t xattention_stride);

@@ -475,6 +475,10 @@ hipError_t launch_decode_merge(hipStream_t s, const DecodeArgs& a, int q_dtype);
 hipError_t launch_decode_scores(hipStream_t s, const DecodeArgs& a, float* scores, int max_kv_len);
 hipError_t launch_decode_post(hipStream_t s, const DecodeArgs& a, int q_dtype, float* scores, int max_kv_len);
 
+// Query rows (token, head of the kv head's group) a workgroup of the matrix kernels holds: 4 waves x 32 or 8 x 16.  No row beyond
+// them is computed, so a group of more heads is not theirs.
+constexpr int PREFILL_ROWS = 128;
+
 // One work item of the 16-bit-cache MFMA kernel: a tile of query tokens against a range of KV blocks.
 struct PrefillItem {
     int32_t b;        // sequence

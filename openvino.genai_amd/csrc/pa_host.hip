@@ -431,14 +431,15 @@ bool decode_u4_shape(const pa_config& c) {
 }
 
 // Shapes the MFMA kernel is built for: 16-bit caches of the query's type, or u8 caches (dequantised on the way to
-// LDS).  It takes every sequence the decode kernel does not.
+// LDS).  It takes every sequence the decode kernel does not.  A work item holds at least one token, so a kv head's group
+// has to fit a workgroup's rows: wider ones run on the shape-generic kernel.
 // (head sizes 96 and 256: its one-row-group variants only -- at 256 one workgroup per CU, two blocks of LDS slots fill
 // 103 of its 160 KB; the 16-bit decode kernel, the straight-to-LDS variant and the block-sparse estimate are built for
 // 64 and 128)
 bool narrow_only(const pa_config& c) { return c.head_size == 96 || c.head_size == 256; }
 bool mfma_shape(const pa_config& c) {
     return kv_alike(c) && (c.kv_cache_dtype == PA_U8 || c.kv_cache_dtype == c.query_dtype) && tuned_block_size(c.block_size) &&
-           (c.head_size == 64 || c.head_size == 128 || narrow_only(c)) && c.num_heads / c.num_kv_heads <= 256;
+           (c.head_size == 64 || c.head_size == 128 || narrow_only(c)) && c.num_heads / c.num_kv_heads <= pa::PREFILL_ROWS;
 }
 
 // Shapes the 16-bit decode kernel is built for (single-token sequences of a call that asks for no scores).
@@ -623,7 +624,7 @@ pa::XattDev xatt_dev(const pa_ctx* ctx) {
     return d;
 }
 
-// Work items of the MFMA kernel: tiles of QT query tokens (QT x G <= 128 rows) against ranges of KV blocks sized so
+// Work items of the MFMA kernel: tiles of QT query tokens (QT x G <= 128 rows, PREFILL_ROWS) against ranges of KV blocks sized so
 // that the launch has several hundred workgroups of comparable length.  Listed as: items with more than 16 query
 // rows (u8 caches), the other dense ones, then the items of block-sparse sequences.
 // A piece of the pinned staging area for an upload of `bytes` that the caller fills and queues on the context's stream.
@@ -675,7 +676,7 @@ void stage_upload(pa_ctx* ctx, void* dst, const void* src, size_t bytes) {
 // 8000 111 / 121; 32 heads without grouping, 512 behind 1000 78 / 74, 2048 behind 1000 183 / 197.
 void plan_widen(pa_ctx* ctx) {
     const pa_config& c = ctx->cfg;
-    const int32_t B = ctx->B, G = c.num_heads / c.num_kv_heads, QT = std::max(1, 128 / G), sw = ctx->sliding_window;
+    const int32_t B = ctx->B, G = c.num_heads / c.num_kv_heads, QT = std::max(1, pa::PREFILL_ROWS / G), sw = ctx->sliding_window;
     const int32_t *past = ctx->h_past.data(), *sb = ctx->h_sb.data();
     ctx->n_wide_seqs = 0;
     ctx->h_wide.clear();
@@ -712,7 +713,7 @@ void plan_items(pa_ctx* ctx) {
     // (32 rows per wave, two waves per SIMD) and are listed first
     const bool narrow_all = ctx->cfg.kv_cache_dtype != PA_U8;
     const bool no_wide = narrow_all || narrow_only(ctx->cfg);  // (the 32-rows-per-wave u8 variant: head size 64 / 128)
-    const int32_t QT = std::max(1, 128 / G), QTX = std::max(1, 128 / G), sw = ctx->sliding_window;
+    const int32_t QT = std::max(1, pa::PREFILL_ROWS / G), QTX = QT, sw = ctx->sliding_window;
     struct Tile { int32_t b, q0, nq, lo, hi, kind; };  // kind 0: more than 16 rows, 1: the rest, 2: single-token sequences, 3: block-sparse
     std::vector<int32_t> single_idx(B, -1);
     int32_t n_single_seqs = 0;
@@ -1697,8 +1698,8 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         }
         PA_REQUIRE(!ctx->has_alibi, PA_NOT_IMPLEMENTED, "block-sparse prefill is not available with ALiBi slopes");
         PA_REQUIRE(mfma_shape(c) && c.head_size != 96 && c.block_size >= 32, PA_NOT_IMPLEMENTED,
-                   "block-sparse prefill needs a block_size of 32 to 256 (a power of two), head_size 64, 128 or 256 and a u8 cache "
-                   "or one of the query's type");
+                   "block-sparse prefill needs a block_size of 32 to 256 (a power of two), head_size 64, 128 or 256, at most 128 query "
+                   "heads per kv head and a u8 cache or one of the query's type");
         auto pow2 = [](int32_t v) { return v > 0 && (v & (v - 1)) == 0; };
         PA_REQUIRE(pow2(block_size) && block_size >= 32, PA_NOT_IMPLEMENTED,
                    "xattention_block_size must be a power of two, at least 32");

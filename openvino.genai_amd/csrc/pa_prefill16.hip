@@ -81,6 +81,7 @@ void pa_prefill16_kernel(PrefillArgs a) {
     static_assert(U8 || DT == QDT, "16-bit caches are used in the query's type");
     static_assert(!HALF || (NG == 2 && !XATT), "the register variant of 256 threads: dense items, two row groups per wave");
     constexpr int NT = HALF ? 256 : 512;
+    static_assert(NT / 64 * 16 * NG == PREFILL_ROWS, "rows of a work item");
     constexpr int NCH = TOK * (D * 2 / 16);  // 16-byte chunks (eight codes of a u8 row) per block and tensor: 512 (D = 128) or 256 (D = 64)
     constexpr int UPT = (NCH + NT - 1) / NT;  // load units (a chunk, or eight codes and a row header) per thread and tensor
     constexpr int ROWB = D * 2;            // bytes of a row as staged in LDS
@@ -844,6 +845,7 @@ static hipError_t launch_prefill16_d(hipStream_t s, const PrefillArgs& a, int q_
 hipError_t launch_prefill16(hipStream_t s, const PrefillArgs& a, int q_dtype, int kv_dtype, hipEvent_t ev0,
                             hipEvent_t ev1, bool merge_later) {
     if (a.n_items == 0) return hipSuccess;
+    if (a.G > PREFILL_ROWS) return hipErrorInvalidValue;
     if (a.sh.D == 128) return launch_prefill16_d<128>(s, a, q_dtype, kv_dtype, ev0, ev1, merge_later);
     if (a.sh.D == 64) return launch_prefill16_d<64>(s, a, q_dtype, kv_dtype, ev0, ev1, merge_later);
     if (a.sh.D == 96) return launch_prefill16_d<96>(s, a, q_dtype, kv_dtype, ev0, ev1, merge_later);

@@ -34,6 +34,7 @@ constexpr int KS = HD / 32;         // k-steps of QK
 constexpr int RT = HD / 16;         // 16-channel tiles of PV
 constexpr int NW = 4;               // waves
 constexpr int NG = 2;               // 16-row groups per wave
+static_assert(16 * NG * NW == PREFILL_ROWS, "rows of a work item");
 constexpr int MAX_RANGE = 128;      // KV blocks an item walks at most
 constexpr int HDRB = 4 * TOK * 4;   // header bytes of a widened (block, kv head)
 
@@ -563,7 +564,7 @@ hipError_t launch_widen(hipStream_t s, const WidenArgs& a) {
 }
 
 hipError_t launch_prefill_dense(hipStream_t s, const PrefillArgs& a, int q_dtype, bool widened) {
-    if (a.sh.D != HD) return hipErrorInvalidValue;
+    if (a.sh.D != HD || a.G > PREFILL_ROWS) return hipErrorInvalidValue;
     const dim3 grid((unsigned)a.n_items * a.sh.Hkv);
     if (widened) {
         if (q_dtype == DT_F16) hipLaunchKernelGGL((pa_prefill_dense_kernel<DT_F16, DT_F16, true>), grid, dim3(64 * NW), 0, s, a);

@@ -156,3 +156,23 @@ def test_alibi_slopes(pkg, qd, Dk, Dv, kd, vd, bs, Hq, Hkv, kind):
     assert np.array_equal(before[0], after[0])
     with pytest.raises(pkg.PaError):   # one slope per query head
         op.set_alibi_slopes(slopes[:-1])
+
+
+@pytest.mark.parametrize("qd,kd,D,Hq,Hkv", [("f16", "u8", 128, 160, 1), ("bf16", "bf16", 64, 258, 2), ("f16", "f16", 128, 256, 1),
+                                            ("bf16", "u8", 64, 128, 1), ("f16", "f16", 128, 128, 1)])
+@pytest.mark.parametrize("new", [[1, 1], [37, 1], [5, 70]])
+def test_groups_wider_than_a_matrix_work_item(pkg, qd, kd, D, Hq, Hkv, new):
+    """A work item of the matrix kernels holds 128 rows: with more query heads per kv head every row comes from the shape-generic
+    kernel, and block-sparse prefill, which has no other kernel, is refused."""
+    import torch
+    print(f"case wide groups {qd}/{kd} D{D} {Hq}/{Hkv} new {new}", flush=True)
+    case = H.build_case(H.case_from_lens("wide", Hq, Hkv, D, 32, qd, kd, [100, 33], new), seed=Hq + new[0])
+    ref = H.run_case_on_checker(case)
+    got = H.run_case_on_gpu(pkg, case, torch.device("cuda:0"))
+    assert got["op"].kernels_run == ({"generic"} if Hq // Hkv > 128 else {"matrix"})
+    H.assert_close(got["out"], ref["out"], qd)
+    H.assert_close(got["scores"], ref["scores"], "f16", "scores")
+    if Hq // Hkv > 128 and max(new) > 1:
+        with pytest.raises(pkg.PaError) as e:
+            got["op"].set_xattention([0.9, 0.9], 64, 8)
+        assert e.value.status == -2
