@@ -50,27 +50,31 @@ struct DevBuf {
         HIP_CHECK(hipMalloc(&p, want));
         cap = want;
     }
-    // ... for what the step can do without: false, with nothing held, if there is no memory for it.  It grows to twice its size, up
-    // to `most`: chunk after chunk of one prompt asks for a little more each time, and each growth waits for the device (16384 tokens
-    // in chunks of 512, four layers over u8: 31 - 33 ms grown to what is asked for, 22.7 so).
+    // ... for what the step can do without: false, and the buffer as it was, if there is no memory for the larger one.  It grows to
+    // twice its size, up to `most`: chunk after chunk of one prompt asks for a little more each time, and each growth waits for the
+    // device (16384 tokens in chunks of 512, four layers over u8: 31 - 33 ms grown to what is asked for, 22.7 so).
     bool try_reserve(size_t bytes, size_t most) {
         if (bytes <= cap) return true;
         const size_t ample = std::max(bytes, std::min(2 * cap, most));
-        if (p) {
-            HIP_CHECK(hipDeviceSynchronize());
-            HIP_CHECK(hipFree(p));
-        }
-        p = nullptr;
-        cap = 0;
-        for (const size_t want : {ample, bytes}) {
-            if (hipMalloc(&p, want) == hipSuccess) {
-                cap = want;
-                return true;
-            }
+        void* larger = nullptr;
+        size_t got = ample;
+        if (hipMalloc(&larger, got) != hipSuccess) {
             (void)hipGetLastError();
-            p = nullptr;
+            got = bytes;
+            if (ample == bytes || hipMalloc(&larger, got) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
         }
-        return false;
+        const size_t held = cap;
+        void* const old = p;
+        p = larger;
+        cap = got;
+        if (held) {  // work in flight may still use the old buffer
+            HIP_CHECK(hipDeviceSynchronize());
+            HIP_CHECK(hipFree(old));
+        }
+        return true;
     }
     void release() {
         if (p) (void)hipFree(p);
@@ -141,6 +145,8 @@ static __device__ __align__(256) uint8_t scratch[STATIC_SCRATCH_BYTES];
 
 // Most a context keeps of widened u8 rows (16.5 KB per 32 tokens and kv head: half a million tokens of eight kv heads)
 constexpr size_t MAX_WIDE_BYTES = (size_t)2 << 30;
+// ... and for how many steps that want more it goes without, once there was no memory for it
+constexpr int32_t WIDE_RETRY_STEPS = 256;
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mutex;
@@ -203,6 +209,7 @@ struct pa_ctx {
     DevBuf wide;                      // K rows | V rows | headers of the widened tiles
     size_t wide_blocks = 0, wide_seqs_off = 0, wide_tile0_off = 0;
     int32_t n_wide_seqs = 0, wide_max_tiles = 0;
+    int32_t wide_wait = 0;            // steps to go without asking for a larger one, after there was no memory for it
     size_t tok_nsplit_off = 0;
     // single-token sequences the matrix kernel may take (16-bit caches): their work items, and behind the split
     // counts a per-sequence flag array (for the call that hands them to the decode kernel instead)
@@ -698,7 +705,14 @@ void plan_widen(pa_ctx* ctx) {
     if (tiles * c.num_kv_heads < 3500 + 2.3 * blocks * c.num_kv_heads) return;
     const size_t bytes = (size_t)blocks * c.num_kv_heads * pa::WIDE_BLOCK_BYTES;
     if (ctx->h_wide.empty() || ctx->h_wide.size() > 65535 /* (a grid's z) */ || bytes > MAX_WIDE_BYTES) return;
-    if (!ctx->wide.try_reserve(bytes, MAX_WIDE_BYTES)) return;
+    if (bytes > ctx->wide.cap && ctx->wide_wait > 0) {
+        --ctx->wide_wait;
+        return;
+    }
+    if (!ctx->wide.try_reserve(bytes, MAX_WIDE_BYTES)) {
+        ctx->wide_wait = WIDE_RETRY_STEPS;
+        return;
+    }
     ctx->wide_blocks = (size_t)blocks;
     ctx->n_wide_seqs = (int32_t)ctx->h_wide.size();
 }

@@ -1,0 +1,80 @@
+"""What the library's host side does between the runtime calls: memory that runs out, copies that are still queued.  The library
+runs in a process of its own on a stand-in for the HIP runtime (fake_hip.cpp), which launches nothing and logs what it was asked."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+TESTS = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+rt = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+rt.fake_log.restype = ctypes.c_char_p
+rt.fake_used.restype = ctypes.c_size_t
+rt.fake_late_copies.restype = rt.fake_malloc_failures.restype = rt.fake_pending.restype = ctypes.c_long
+rt.fake_set_budget.argtypes = [ctypes.c_size_t]
+rt.fake_fail_sizes.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+import __graft_entry__ as entry
+pkg = entry.load_package()
+
+class T:  # a tensor as the binding sees one: nothing reads it here
+    def __init__(self, *shape):
+        self.shape = shape
+    def data_ptr(self):
+        return 1 << 40
+
+def ran():
+    return [l.split()[2] for l in rt.fake_log().decode().splitlines() if l.startswith("run")]
+
+def begin(op, past, new, bs=32, **kw):
+    past, new = np.asarray(past, np.int32), np.asarray(new, np.int32)
+    bib = np.concatenate([[0], np.cumsum((past + new + bs - 1) // bs)]).astype(np.int32)
+    op.step_begin(past, np.concatenate([[0], np.cumsum(new)]), bib, **kw)
+    op.set_block_indices(np.arange(bib[-1]) % 1000, 1000)
+
+def forward(op, scores=None):
+    rt.fake_clear_log()
+    op.forward(T(1), T(1), T(1), T(1000), T(1000), T(1), scores)
+    return ran()
+WIDE = 16896  # bytes of a widened (32-token block, kv head)
+"""
+
+
+@pytest.fixture(scope="module")
+def on_fake(tmp_path_factory, pkg):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(TESTS, "fake_hip.cpp"), "-o", so], check=True)
+
+    def run(script):
+        head = PRELUDE.format(root=os.path.dirname(TESTS), fake=so)
+        r = subprocess.run([sys.executable, "-c", head + textwrap.dedent(script)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_widened_rows_outlive_a_failed_growth(on_fake):
+    """No memory for more widened rows: the step goes without, the rows held serve the steps that fit them, and a long row of such
+    steps does not ask the runtime again and again."""
+    on_fake("""
+        op = pkg.PagedAttention(16, 1, 128, 32, "f16", "u8")
+        begin(op, [0], [1400])
+        assert any("widen" in k for k in forward(op))
+        blocks = (8000 + 3000 + 31) // 32
+        rt.fake_fail_sizes(blocks * WIDE, blocks * WIDE)
+        for i in range(20):
+            begin(op, [8000], [3000])
+            assert not any("widen" in k for k in forward(op))
+            begin(op, [0], [1400])
+            assert any("widen" in k for k in forward(op)), i
+        assert rt.fake_malloc_failures() == 1, rt.fake_malloc_failures()
+        rt.fake_fail_sizes(1, 0)
+        for i in range(300):
+            begin(op, [8000], [3000])
+        assert any("widen" in k for k in forward(op))  # (after a while it asks again)
+    """)
