@@ -92,7 +92,12 @@ typedef struct pa_config {
     int32_t value_cache_dtype_p1;   /* 0 = kv_cache_dtype, else 1 + (PA_U8 | PA_U4 | PA_F16 | PA_BF16) */
 } pa_config;
 
-/* Replaces Core::compile_model + create_infer_request for this op (pipeline_impl.cpp:182,193). */
+/* Replaces Core::compile_model + create_infer_request for this op (pipeline_impl.cpp:182,193).
+ * Device memory of a context, allocated by its calls as they need it and kept until pa_destroy: split partials, maxima and score
+ * staging of the largest step so far, the step arrays and block tables -- and, over u8 caches at head size 128, up to 2 GiB for the
+ * rows of long prompt chunks widened to f16 (16.5 KiB per 32 tokens of context and kv head, for one layer at a time), which speed a
+ * step up and which it can do without: they are taken only where there is memory for them, and given back when a call of the
+ * context finds none for what it cannot do without (PA_NOT_ALLOCATED only if that was not enough). */
 int32_t pa_create(const pa_config* cfg, pa_ctx** out);
 void pa_destroy(pa_ctx* ctx);
 const char* pa_last_error(const pa_ctx* ctx);

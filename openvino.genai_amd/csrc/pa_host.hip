@@ -46,8 +46,13 @@ struct DevBuf {
         }
         p = nullptr;
         cap = 0;
-        size_t want = std::max<size_t>(bytes, 256);
-        HIP_CHECK(hipMalloc(&p, want));
+        const size_t want = std::max<size_t>(bytes, 256);
+        if (const hipError_t e = hipMalloc(&p, want)) {
+            p = nullptr;
+            (void)hipGetLastError();  // (or the next launch would report it as its own)
+            throw StatusError(e == hipErrorOutOfMemory ? PA_NOT_ALLOCATED : PA_GENERAL_ERROR,
+                              "hipMalloc of " + std::to_string(want) + " bytes: " + hipGetErrorString(e));
+        }
         cap = want;
     }
     // ... for what the step can do without: false, and the buffer as it was, if there is no memory for the larger one.  It grows to
@@ -145,7 +150,7 @@ static __device__ __align__(256) uint8_t scratch[STATIC_SCRATCH_BYTES];
 
 // Most a context keeps of widened u8 rows (16.5 KB per 32 tokens and kv head: half a million tokens of eight kv heads)
 constexpr size_t MAX_WIDE_BYTES = (size_t)2 << 30;
-// ... and for how many steps that want more it goes without, once there was no memory for it
+// ... and for how many steps that want more it goes without, once there was no memory or it had to be given back
 constexpr int32_t WIDE_RETRY_STEPS = 256;
 
 constexpr int MAX_DEVICES = 64;
@@ -316,6 +321,21 @@ int32_t guarded(Obj* obj, Fn&& fn) {
 }
 
 struct NoObj { std::string error; };
+
+// Memory a call cannot do without.  Where there is none left, the widened u8 rows, which a step can do without at any point before
+// their launch (its work items are the same), are given back first.
+void need(pa_ctx* ctx, DevBuf& buf, size_t bytes) {
+    try {
+        buf.reserve(bytes);
+    } catch (const StatusError& e) {
+        if (e.code != PA_NOT_ALLOCATED || !ctx->wide.p) throw;
+        HIP_CHECK(hipDeviceSynchronize());  // (earlier layers' kernels may still read them)
+        ctx->wide.release();
+        ctx->n_wide_seqs = 0;
+        ctx->wide_wait = WIDE_RETRY_STEPS;
+        buf.reserve(bytes);
+    }
+}
 
 pa::Shape shape_of(const pa_config& c) { return pa::Shape{c.num_heads, c.num_kv_heads, c.head_size, c.block_size}; }
 pa::GenericShape generic_shape_of(const pa_config& c) {
@@ -952,7 +972,7 @@ void plan_items(pa_ctx* ctx) {
     const std::vector<int32_t>* parts[] = {&tok_ns, &ctx->h_multi, &ctx->h_dec16, &ctx->h_dec, &ctx->h_meta};
     size_t at[6] = {item_bytes};
     for (int i = 0; i < 5; ++i) at[i + 1] = at[i] + parts[i]->size() * sizeof(int32_t);
-    ctx->items.reserve(at[5]);
+    need(ctx, ctx->items, at[5]);
     {
         uint8_t* stage = stage_piece(ctx, at[5]);
         if (item_bytes) std::memcpy(stage, items.data(), item_bytes);
@@ -1019,11 +1039,11 @@ DecodeWs decode_workspace(pa_ctx* ctx, size_t rows, int32_t nsplit, bool want_sc
         w.p_split = reinterpret_cast<_Float16*>(base + o_psplit);
         return w;
     }
-    ctx->final_ml.reserve(b_final);
-    if (b_acc) ctx->part_acc.reserve(b_acc);
-    if (b_ml) ctx->part_ml.reserve(b_ml);
-    if (b_group) ctx->group_scores.reserve(b_group);
-    if (b_psplit) ctx->p_split.reserve(b_psplit);
+    need(ctx, ctx->final_ml, b_final);
+    if (b_acc) need(ctx, ctx->part_acc, b_acc);
+    if (b_ml) need(ctx, ctx->part_ml, b_ml);
+    if (b_group) need(ctx, ctx->group_scores, b_group);
+    if (b_psplit) need(ctx, ctx->p_split, b_psplit);
     w.final_ml = ctx->final_ml.as<float>();
     w.part_acc = ctx->part_acc.as<float>();
     w.part_ml = ctx->part_ml.as<float>();
@@ -1160,7 +1180,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         ctx->kernels_run |= PA_RAN_DECODE | (a.arrived ? PA_RAN_FOLD : 0);
         if (use_u4) {
             if (io->scores) {
-                ctx->logits.reserve((size_t)c.num_heads * ctx->total_scores * sizeof(float));
+                need(ctx, ctx->logits, (size_t)c.num_heads * ctx->total_scores * sizeof(float));
                 a.logits = ctx->logits.as<float>();
             }
             HIP_CHECK(pa::launch_decode_u4(ctx->stream, a, c.query_dtype, ev0, ev1));
@@ -1224,15 +1244,14 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         a.tok_nsplit = reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(ctx->items.p) + ctx->tok_nsplit_off);
         a.n_items = ctx->n_items;
         a.n_wide = ctx->n_wide;
-        a.widened = ctx->n_wide_seqs > 0 ? 1 : 0;
         a.G = c.num_heads / c.num_kv_heads;
         a.max_split = ctx->max_split;
         a.out = static_cast<uint16_t*>(io->out);
-        ctx->final_ml.reserve(rows * 2 * sizeof(float));
+        need(ctx, ctx->final_ml, rows * 2 * sizeof(float));
         a.final_ml = ctx->final_ml.as<float>();
         if (ctx->max_split > 1) {
-            ctx->pf_part_acc.reserve(rows * ctx->max_split * c.head_size * sizeof(float));
-            ctx->pf_part_ml.reserve(rows * ctx->max_split * 2 * sizeof(float));
+            need(ctx, ctx->pf_part_acc, rows * ctx->max_split * c.head_size * sizeof(float));
+            need(ctx, ctx->pf_part_ml, rows * ctx->max_split * 2 * sizeof(float));
         }
         a.part_acc = ctx->pf_part_acc.as<float>();
         a.part_ml = ctx->pf_part_ml.as<float>();
@@ -1274,7 +1293,15 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
         // Single-token sequences that are work items of this launch (16-bit caches, next to dense chunks): with scores
         // wanted the kernel leaves their probabilities for a small score kernel, instead of a replay that reads all
         // their K rows once more.
-        if (ctx->n_wide_seqs > 0) {  // u8 rows of the dense chunks as f16 integers
+        const bool hand_over = io->scores && ctx->stash_ok && !use_decode16 && ctx->n_single > 0;
+        if (hand_over) {
+            const size_t tiles = (size_t)pa::tile_max_count(ctx->total_scores, ctx->B);
+            need(ctx, ctx->p_split, tiles * c.num_heads * 32 * sizeof(uint16_t));
+            need(ctx, ctx->tile_max, tiles * c.num_heads * sizeof(float));
+            a.p_out = ctx->p_split.as<_Float16>();
+            a.tile_max = ctx->tile_max.as<float>();
+        }
+        if (ctx->n_wide_seqs > 0) {  // u8 rows of the dense chunks as f16 integers (all memory of this call is in hand: see need())
             const size_t slots = ctx->wide_blocks * c.num_kv_heads;
             const uint8_t* lists = static_cast<const uint8_t*>(ctx->items.p);
             pa::WidenArgs w{};
@@ -1290,18 +1317,11 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             w.wide_v = w.wide_k + slots * pa::WIDE_TILE_BYTES;
             w.wide_hdr = reinterpret_cast<float*>(w.wide_v + slots * pa::WIDE_TILE_BYTES);
             HIP_CHECK(pa::launch_widen(ctx->stream, w));
+            a.widened = 1;
             a.wide_k = w.wide_k;
             a.wide_v = w.wide_v;
             a.wide_hdr = w.wide_hdr;
             a.wide_tile0 = reinterpret_cast<const int32_t*>(lists + ctx->wide_tile0_off);
-        }
-        const bool hand_over = io->scores && ctx->stash_ok && !use_decode16 && ctx->n_single > 0;
-        if (hand_over) {
-            const size_t tiles = (size_t)pa::tile_max_count(ctx->total_scores, ctx->B);
-            ctx->p_split.reserve(tiles * c.num_heads * 32 * sizeof(uint16_t));
-            ctx->tile_max.reserve(tiles * c.num_heads * sizeof(float));
-            a.p_out = ctx->p_split.as<_Float16>();
-            a.tile_max = ctx->tile_max.as<float>();
         }
         if (!use_decode && !use_decode16) ctx->nsplit = ctx->max_split;
         // scores of the multi-token sequences (and of single-token ones that were work items of this kernel and kept
@@ -1338,10 +1358,10 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     if (use_decode || use_mfma) return;  // (use_decode16 implies use_mfma)
     ctx->kernels_run = PA_RAN_GENERIC;
     ctx->nsplit = ctx->generic_nsplit;
-    ctx->part_acc.reserve(rows * ctx->nsplit * v_head(c) * sizeof(float));
-    ctx->part_ml.reserve(rows * ctx->nsplit * 2 * sizeof(float));
-    ctx->final_ml.reserve(rows * 2 * sizeof(float));
-    if (io->scores) ctx->logits.reserve((size_t)c.num_heads * ctx->total_scores * sizeof(float));
+    need(ctx, ctx->part_acc, rows * ctx->nsplit * v_head(c) * sizeof(float));
+    need(ctx, ctx->part_ml, rows * ctx->nsplit * 2 * sizeof(float));
+    need(ctx, ctx->final_ml, rows * 2 * sizeof(float));
+    if (io->scores) need(ctx, ctx->logits, (size_t)c.num_heads * ctx->total_scores * sizeof(float));
     pa::AttnWorkspace ws{ctx->part_acc.as<float>(), ctx->part_ml.as<float>(), ctx->final_ml.as<float>(),
                          ctx->logits.as<float>(), ctx->nsplit, ctx->total_scores,
                          ctx->has_alibi ? ctx->alibi.as<float>() : nullptr};
@@ -1615,7 +1635,7 @@ int32_t pa_set_block_indices(pa_ctx* ctx, int32_t layer, const int32_t* ids, int
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
         if (ctx->tables[idx].cap < total) {  // kernels in flight may still read the buffer this would free
             HIP_CHECK(hipStreamSynchronize(ctx->stream));
-            ctx->tables[idx].reserve(total);
+            need(ctx, ctx->tables[idx], total);
         }
         uint8_t* stage = stage_piece(ctx, total);
         fill_table_stage(ctx, ids, count, id_bytes, with_descs, stage);
@@ -1665,7 +1685,7 @@ int32_t pa_set_block_indices_layers(pa_ctx* ctx, int32_t first_layer, int32_t nu
                     ctx->table_count[i] = -1;
                 }
             }
-            ctx->table_pool.reserve(stride * (size_t)ctx->cfg.num_layers);
+            need(ctx, ctx->table_pool, stride * (size_t)ctx->cfg.num_layers);
         }
         uint8_t* dst = ctx->table_pool.as<uint8_t>() + (size_t)first_layer * stride;
         HIP_CHECK(hipMemcpyAsync(dst, stage, stride * (size_t)num_layers, hipMemcpyHostToDevice, ctx->stream));
@@ -1771,14 +1791,14 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         const size_t seq_bytes = seqs.size() * sizeof(pa::XattSeq), tile_bytes = tiles.size() * sizeof(pa::XattTile);
         ctx->x_tiles_off = seq_bytes;
         ctx->x_seq_of_off = seq_bytes + tile_bytes;
-        ctx->x_plan.reserve(seq_bytes + tile_bytes + (size_t)B * sizeof(int32_t));
+        need(ctx, ctx->x_plan, seq_bytes + tile_bytes + (size_t)B * sizeof(int32_t));
         uint8_t* d = static_cast<uint8_t*>(ctx->x_plan.p);
         stage_upload(ctx, d, seqs.data(), seq_bytes);
         stage_upload(ctx, d + seq_bytes, tiles.data(), tile_bytes);
         stage_upload(ctx, d + seq_bytes + tile_bytes, seq_of.data(), (size_t)B * sizeof(int32_t));
-        ctx->x_logits.reserve((size_t)logit_off * sizeof(float));
-        ctx->x_sums.reserve((size_t)sum_off * sizeof(float));
-        ctx->x_mask.reserve((size_t)mask_off * sizeof(uint32_t));
+        need(ctx, ctx->x_logits, (size_t)logit_off * sizeof(float));
+        need(ctx, ctx->x_sums, (size_t)sum_off * sizeof(float));
+        need(ctx, ctx->x_mask, (size_t)mask_off * sizeof(uint32_t));
         ctx->h_xseq = seqs;
         ctx->h_xseq_of = seq_of;
         ctx->xatt_block = block_size;
@@ -1789,7 +1809,7 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         ctx->x_max_nqb = max_nqb;
         ctx->x_max_nkb = max_nkb;
         plan_items(ctx);
-        ctx->x_item_keep.reserve((size_t)std::max(1, ctx->n_sparse) * c.num_kv_heads * ctx->x_keep_words * sizeof(int32_t));
+        need(ctx, ctx->x_item_keep, (size_t)std::max(1, ctx->n_sparse) * c.num_kv_heads * ctx->x_keep_words * sizeof(int32_t));
     });
 }
 
@@ -2008,7 +2028,7 @@ int32_t pa_set_alibi_slopes(pa_ctx* ctx, const float* slopes, int32_t count) {
         HIP_CHECK(hipStreamSynchronize(ctx->stream));  // earlier launches may still read the old slopes
         if (any) {
             const size_t bytes = (size_t)count * sizeof(float);
-            ctx->alibi.reserve(bytes);
+            need(ctx, ctx->alibi, bytes);
             HIP_CHECK(hipMemcpyAsync(ctx->alibi.p, slopes, bytes, hipMemcpyHostToDevice, ctx->stream));
             HIP_CHECK(hipStreamSynchronize(ctx->stream));  // `slopes` is the caller's, pageable
         }
@@ -2025,7 +2045,7 @@ int32_t pa_set_rotation_trig_lut(pa_ctx* ctx, const float* lut, int32_t rows) {
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
         HIP_CHECK(hipStreamSynchronize(ctx->stream));  // an earlier rotation may still read the old table
         const size_t bytes = (size_t)rows * ctx->cfg.head_size * sizeof(float);
-        ctx->trig_lut.reserve(bytes);
+        need(ctx, ctx->trig_lut, bytes);
         HIP_CHECK(hipMemcpyAsync(ctx->trig_lut.p, lut, bytes, hipMemcpyHostToDevice, ctx->stream));
         HIP_CHECK(hipStreamSynchronize(ctx->stream));  // `lut` is the caller's, pageable
         ctx->trig_rows = rows;
@@ -2056,7 +2076,7 @@ int32_t pa_rotate_cache(pa_ctx* ctx, void* key_cache, int64_t num_blocks, const 
         HIP_CHECK(hipSetDevice(c.device));
         // (the previous call's kernel may still read the arguments: the copies below are ordered behind it on the
         // stream, and a buffer that has to grow is freed by a call that waits for the device)
-        ctx->rot_args.reserve((num_rotated + n_delta) * sizeof(int32_t));
+        need(ctx, ctx->rot_args, (num_rotated + n_delta) * sizeof(int32_t));
         int32_t* d_idx = ctx->rot_args.as<int32_t>();
         int32_t* d_delta = d_idx + num_rotated;
         stage_upload(ctx, d_idx, rotated_block_indices, num_rotated * sizeof(int32_t));
@@ -2118,10 +2138,10 @@ int32_t pa_adaptive_rkv_diversity(pa_ctx* ctx, int32_t layer, const void* key_ca
         // (the previous call's kernels may still read the sequence list and the work buffers: this call's copy and
         // kernels are ordered behind them on the stream, and a buffer that has to grow is freed by a call that waits)
         const int chunks = pa::rkv_diversity_chunks(ev_max);
-        ctx->div_seqs.reserve(seqs.size() * sizeof(pa::RkvDivSeq));
-        ctx->div_stats.reserve((size_t)c.num_kv_heads * tok_total * sizeof(float4));
-        ctx->div_mean.reserve((size_t)c.num_kv_heads * tok_total * sizeof(float));
-        ctx->div_colsum.reserve(seqs.size() * c.num_kv_heads * (chunks + 1) * c.head_size * sizeof(float));
+        need(ctx, ctx->div_seqs, seqs.size() * sizeof(pa::RkvDivSeq));
+        need(ctx, ctx->div_stats, (size_t)c.num_kv_heads * tok_total * sizeof(float4));
+        need(ctx, ctx->div_mean, (size_t)c.num_kv_heads * tok_total * sizeof(float));
+        need(ctx, ctx->div_colsum, seqs.size() * c.num_kv_heads * (chunks + 1) * c.head_size * sizeof(float));
         stage_upload(ctx, ctx->div_seqs.p, seqs.data(), seqs.size() * sizeof(pa::RkvDivSeq));
         pa::RkvDivArgs a{};
         a.key_cache = static_cast<const uint8_t*>(key_cache);

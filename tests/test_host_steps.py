@@ -58,6 +58,44 @@ def on_fake(tmp_path_factory, pkg):
     return run
 
 
+def test_mandatory_memory_before_widened_rows(on_fake):
+    """A prompt step over u8 whose workspaces do not fit beside its widened rows gives those back and runs without them."""
+    on_fake("""
+        op = pkg.PagedAttention(16, 1, 128, 32, "f16", "u8")
+        begin(op, [300], [1101])
+        before = rt.fake_used()
+        assert any("widen" in k for k in forward(op))
+        workspaces = rt.fake_used() - before
+        del op
+        wide = 44 * WIDE
+        for short in (1, wide // 2, wide):
+            op = pkg.PagedAttention(16, 1, 128, 32, "f16", "u8")
+            begin(op, [300], [1101])
+            held = rt.fake_used()
+            rt.fake_set_budget(held + workspaces - short)
+            for layer in range(2):
+                names = forward(op)
+                assert not any("widen" in k or "dense" in k for k in names) and any("pa_prefill16_kernel" in k for k in names), names
+            assert rt.fake_used() == held - wide + workspaces
+            rt.fake_set_budget(rt.fake_used() + 4096)
+            begin(op, [0], [1])  # (a launch behind the failed allocation is not taken for it)
+            forward(op)
+            del op
+            rt.fake_set_budget(1 << 62)
+        # what does not fit without them either is still the library's error
+        op = pkg.PagedAttention(16, 1, 128, 32, "f16", "u8")
+        begin(op, [300], [1101])
+        rt.fake_set_budget(rt.fake_used() + workspaces - wide - 1)
+        try:
+            forward(op)
+            assert False
+        except pkg.PaError as e:
+            assert e.status == -10, e
+        rt.fake_set_budget(1 << 62)
+        assert any("pa_prefill16_kernel" in k for k in forward(op))
+    """)
+
+
 def test_widened_rows_outlive_a_failed_growth(on_fake):
     """No memory for more widened rows: the step goes without, the rows held serve the steps that fit them, and a long row of such
     steps does not ask the runtime again and again."""
