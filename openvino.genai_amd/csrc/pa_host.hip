@@ -1727,7 +1727,9 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         if (seqs.empty()) {
             ctx->h_xseq.clear();
             ctx->h_xseq_of.clear();
+            ctx->step_ready = !had;
             if (had) plan_items(ctx);
+            ctx->step_ready = true;
             return;
         }
         PA_REQUIRE(!ctx->has_alibi, PA_NOT_IMPLEMENTED, "block-sparse prefill is not available with ALiBi slopes");
@@ -1787,6 +1789,8 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         }
         PA_REQUIRE(logit_off * 4 <= ((int64_t)4 << 30), PA_NOT_ALLOCATED,
                    "block-sparse prefill: the strided logits of this step exceed 4 GiB (larger stride or shorter chunks)");
+        // (from here on a failure leaves a plan and buffers of two settings: the step has to begin again)
+        ctx->step_ready = false;
         // (the copies are queued behind the previous step's kernels, which read the old plan)
         const size_t seq_bytes = seqs.size() * sizeof(pa::XattSeq), tile_bytes = tiles.size() * sizeof(pa::XattTile);
         ctx->x_tiles_off = seq_bytes;
@@ -1810,6 +1814,7 @@ int32_t pa_set_xattention(pa_ctx* ctx, const float* thresholds, int32_t block_si
         ctx->x_max_nkb = max_nkb;
         plan_items(ctx);
         need(ctx, ctx->x_item_keep, (size_t)std::max(1, ctx->n_sparse) * c.num_kv_heads * ctx->x_keep_words * sizeof(int32_t));
+        ctx->step_ready = true;
     });
 }
 
@@ -2045,6 +2050,7 @@ int32_t pa_set_rotation_trig_lut(pa_ctx* ctx, const float* lut, int32_t rows) {
         HIP_CHECK(hipSetDevice(ctx->cfg.device));
         HIP_CHECK(hipStreamSynchronize(ctx->stream));  // an earlier rotation may still read the old table
         const size_t bytes = (size_t)rows * ctx->cfg.head_size * sizeof(float);
+        ctx->trig_rows = 0;  // (no table, should this one find no memory)
         need(ctx, ctx->trig_lut, bytes);
         HIP_CHECK(hipMemcpyAsync(ctx->trig_lut.p, lut, bytes, hipMemcpyHostToDevice, ctx->stream));
         HIP_CHECK(hipStreamSynchronize(ctx->stream));  // `lut` is the caller's, pageable

@@ -116,3 +116,37 @@ def test_widened_rows_outlive_a_failed_growth(on_fake):
             begin(op, [8000], [3000])
         assert any("widen" in k for k in forward(op))  # (after a while it asks again)
     """)
+
+
+def test_a_call_without_memory_leaves_no_freed_buffer_in_use(on_fake):
+    """Larger thresholds' plans or trig tables that find no memory: what they replaced is gone, and calls that need it are refused."""
+    on_fake("""
+        def refused(status, fn, *args):
+            try:
+                fn(*args)
+            except pkg.PaError as e:
+                assert e.status == status, e
+            else:
+                assert False
+        op = pkg.PagedAttention(8, 2, 128, 32, "f16", "f16")
+        begin(op, [3000], [500])
+        op.set_xattention([0.9], 64, 16)
+        assert any("xatt" in k for k in forward(op))
+        for lo, hi in ((1 << 24, 1 << 40), (40000, 1 << 17)):  # (the logits; the block sums)
+            rt.fake_fail_sizes(lo, hi)
+            refused(-10, op.set_xattention, [0.9], 32, 1)
+            rt.fake_fail_sizes(1, 0)
+            refused(-4, forward, op)
+            begin(op, [3000], [500])
+            forward(op)
+            op.set_xattention([0.9], 64, 16)
+            forward(op)
+        op.set_rotation_trig_lut(np.ones((8, 128), np.float32))
+        op.rotate_cache(T(1000), [3], [7])
+        rt.fake_fail_sizes(64 * 512, 64 * 512)
+        refused(-10, op.set_rotation_trig_lut, np.ones((64, 128), np.float32))
+        refused(-10, op.rotate_cache, T(1000), [3], [7])
+        rt.fake_fail_sizes(1, 0)
+        op.set_rotation_trig_lut(np.ones((64, 128), np.float32))
+        op.rotate_cache(T(1000), [3], [63])
+    """)
