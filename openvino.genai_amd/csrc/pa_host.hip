@@ -1102,7 +1102,19 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     // fork: what is launched on the returned stream starts behind what the context's stream holds so far and runs
     // next to what follows on it, until the join at the end of this call
     // (a step whose two kernels are too short for that, see plan_items: the same kernels one after the other)
-    bool forked = false;
+    // (also where something fails in between: what the other stream runs then still reads and writes the caller's tensors)
+    struct Fork {
+        pa_ctx* ctx;
+        bool open;
+        void join() {
+            open = false;
+            HIP_CHECK(hipEventRecord(ctx->ev_join, ctx->side));
+            HIP_CHECK(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
+        }
+        ~Fork() {
+            if (open && hipEventRecord(ctx->ev_join, ctx->side) == hipSuccess) (void)hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0);
+        }
+    } fork{ctx, false};
     auto fork_side = [&]() -> hipStream_t {
         if (!ctx->fork_pays && !io->scores) return ctx->stream;
         if (!ctx->side) {
@@ -1110,10 +1122,10 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             HIP_CHECK(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));
             HIP_CHECK(hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming));
         }
-        if (!forked) {
+        if (!fork.open) {
             HIP_CHECK(hipEventRecord(ctx->ev_fork, ctx->stream));
             HIP_CHECK(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-            forked = true;
+            fork.open = true;
             ctx->kernels_run |= PA_RAN_SIDE_STREAM;
         }
         return ctx->side;
@@ -1351,10 +1363,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
                                                a.xatt, ss, mg));
         }
     }
-    if (forked) {  // join
-        HIP_CHECK(hipEventRecord(ctx->ev_join, ctx->side));
-        HIP_CHECK(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
-    }
+    if (fork.open) fork.join();
     if (use_decode || use_mfma) return;  // (use_decode16 implies use_mfma)
     ctx->kernels_run = PA_RAN_GENERIC;
     ctx->nsplit = ctx->generic_nsplit;

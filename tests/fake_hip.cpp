@@ -75,6 +75,7 @@ hipError_t hipMalloc(void** p, size_t n) {
         return g_last = hipErrorOutOfMemory;
     }
     if (posix_memalign(p, 256, n ? n : 1)) return g_last = hipErrorOutOfMemory;
+    g_log += "malloc " + std::to_string(n) + "\n";
     g_device[*p] = n;
     g_used += n;
     return hipSuccess;

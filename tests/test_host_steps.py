@@ -150,3 +150,31 @@ def test_a_call_without_memory_leaves_no_freed_buffer_in_use(on_fake):
         op.set_rotation_trig_lut(np.ones((64, 128), np.float32))
         op.rotate_cache(T(1000), [3], [63])
     """)
+
+
+def test_a_failed_mixed_step_joins_its_second_stream(on_fake):
+    """A mixed step that finds no memory for the chunk's partials has its decode kernel on the second stream already: the context's
+    stream waits for it all the same."""
+    on_fake("""
+        def step():
+            op = pkg.PagedAttention(32, 8, 128, 32, "f16", "u8")
+            begin(op, [4000, 3000, 2000, 9000], [1, 1, 1, 40])
+            return op
+        op = step()
+        names = forward(op)
+        log = rt.fake_log().decode().splitlines()
+        forked = [i for i, l in enumerate(log) if l.startswith("run 100") and "decode" in l]
+        late = [int(l.split()[1]) for l in log[forked[0]:] if l.startswith("malloc")]
+        assert late, log
+        op = step()
+        rt.fake_fail_sizes(late[0], late[0])
+        try:
+            forward(op)
+            assert False
+        except pkg.PaError as e:
+            assert e.status == -10
+        log = rt.fake_log().decode().splitlines()
+        side = [l.split()[1] for l in log if l.startswith("run") and "decode" in l]
+        assert side and side[0] != "0", log
+        assert log[-1] == "wait 0 " + side[0], log
+    """)
