@@ -83,15 +83,13 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
 }
 
-// Straight into LDS (dense items over 16-bit caches, head size 128): one instruction moves 64 x 16 bytes from
+// Straight into LDS: one instruction moves 64 x 16 bytes from
 // per-lane global addresses to 1024 consecutive bytes of LDS at a wave-uniform address; no registers, no LDS stores.
 __device__ __forceinline__ void dma16(const uint8_t* src, uint8_t* lds_dst) {
     typedef __attribute__((address_space(3))) void* lds_p;
     typedef const __attribute__((address_space(1))) void* glb_p;
     __builtin_amdgcn_global_load_lds((glb_p)src, (lds_p)lds_dst, 16, 0, 0);
 }
-// Waits until at most N of the wave's vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14; the other counters left at their maxima).
 // Workgroup barrier for LDS traffic only.  __syncthreads() (and a workgroup fence of any kind) makes the compiler wait
 // for every copy into LDS that is in flight, the prefetched blocks included; here the wave waits for its own LDS
 // operations, meets the others, and the copies it must have finished are named by the caller (wait_vmem).  The
@@ -102,6 +100,8 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
+// Waits until at most N of the wave's vector-memory operations are outstanding (gfx9 encoding: vmcnt in bits 3:0 and
+// 15:14; the other counters left at their maxima).
 template <int N>
 __device__ __forceinline__ void wait_vmem() {
     __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | 0x0f70);

@@ -410,15 +410,6 @@ __global__ __launch_bounds__(64 * NW, 2) void pa_prefill_dense_kernel(PrefillArg
     };
 
     // ---- the walk -----------------------------------------------------------------------------------------------
-    // Step j of a wave: barrier | copies of a later block go out, matrix phase: S^T of block j, O^T of block j - 1 | its share
-    // of what step j + 1 reads has landed | barrier | vector phase: softmax of block j.  Steps 0 .. cnt; the first half of the
-    // workgroup meets the second half's barriers one phase apart, so the halves are always in different phases.  Block j
-    // lives in slot j % 4 of K, V and (u8) headers.  Copies of step j: headers of block j + 2, K of j + 3, V of j + 2; their slots
-    // were last read in the vector phase of step j - 2, the matrix phases of steps j - 1 and j - 1 (V of block j - 2): all of them
-    // behind a barrier for both halves.  A wave's operations complete in order: behind the matrix phase of step j everything but
-    // the newest 2 + COPIES (headers go out first) or, without headers, 2 COPIES has landed, that is all that step j + 1's matrix
-    // phase and (headers) vector phase read -- for the other half too, which is there one barrier later.
-    // ---- the walk -----------------------------------------------------------------------------------------------
     // Step j: barrier | copies of later blocks go out | S^T of block j, O^T of block j - 1 | the wave's share of what step j + 1
     // reads has landed | softmax of block j.  Block j lives in slot j % 4 of K, V and (u8) headers.
     // Slots: step j copies K of block j + 3 over block j - 1, V of j + 2 and headers of j + 2 over j - 2: what was read from there was
@@ -426,7 +417,9 @@ __global__ __launch_bounds__(64 * NW, 2) void pa_prefill_dense_kernel(PrefillArg
     // Waits: a wave's copies land in order; at the end of step j only its newest COPIES may be outstanding, those of this step, so
     // that K up to block j + 2, V and headers up to j + 1 are there.  This is only right while a step issues exactly this many
     // copies and nothing else that counts (the build fails on spills, whose scratch traffic would).
-    constexpr int COPIES = (U8 ? 1 : 0) + 4;
+    constexpr int COPIES_PER_TENSOR = TILEB / (NW * 64 * 16);  // dma16 moves 64 x 16 bytes
+    static_assert(COPIES_PER_TENSOR == 2 && HDRB == 2 * 64 * 4, "copy_k and copy_v issue two copies each, copy_h one");
+    constexpr int COPIES = 2 * COPIES_PER_TENSOR + (U8 ? 1 : 0);
     // The rows of a sequence's last block that lie behind its tokens repeat the last row; in V they are cleared, each wave its own
     // once they have landed: 0 * inf must not reach the accumulators where the last row's own weight does not.  (Widened: zeros.)
     const int tail_j = !U8 && te * TOK > kv_len ? cnt - 1 : -1;
