@@ -202,9 +202,12 @@ int32_t pa_synchronize(pa_ctx* ctx);
 /* Number of split-K partitions of the last attention call (diagnostics). */
 int32_t pa_get_num_splits(const pa_ctx* ctx);
 /* Which kernels the last attention call launched (diagnostics): PA_RAN_* bits.  FOLD: a decode launch of several splits
- * folds their partials itself (else a launch behind it does); SIDE_STREAM: decode and matrix kernel side by side. */
+ * folds their partials itself (else a launch behind it does); SIDE_STREAM: decode and matrix kernel side by side; WIDENED: the rows of
+ * long u8 chunks were widened ahead of the matrix kernel; APPEND: pa_forward ran an append launch of its own in front (else the
+ * attention kernel appended). */
 enum {
-    PA_RAN_GENERIC = 1, PA_RAN_DECODE = 2, PA_RAN_DECODE_FEW = 4, PA_RAN_MATRIX = 8, PA_RAN_FOLD = 16, PA_RAN_SIDE_STREAM = 32
+    PA_RAN_GENERIC = 1, PA_RAN_DECODE = 2, PA_RAN_DECODE_FEW = 4, PA_RAN_MATRIX = 8, PA_RAN_FOLD = 16, PA_RAN_SIDE_STREAM = 32,
+    PA_RAN_WIDENED = 64, PA_RAN_APPEND = 128
 };
 int32_t pa_get_kernels_run(const pa_ctx* ctx);
 /* Per-op timing.  The reference times the whole infer() with a host timer (ManualTimer, model_runner.hpp:951-954)

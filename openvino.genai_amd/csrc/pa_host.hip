@@ -1329,6 +1329,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
             w.wide_v = w.wide_k + slots * pa::WIDE_TILE_BYTES;
             w.wide_hdr = reinterpret_cast<float*>(w.wide_v + slots * pa::WIDE_TILE_BYTES);
             HIP_CHECK(pa::launch_widen(ctx->stream, w));
+            ctx->kernels_run |= PA_RAN_WIDENED;
             a.widened = 1;
             a.wide_k = w.wide_k;
             a.wide_v = w.wide_v;
@@ -1919,6 +1920,7 @@ int32_t pa_forward(pa_ctx* ctx, int32_t layer, const pa_layer_io* io) {
         if (fuse) check_io(ctx, layer, io, true, false);
         else do_kv_append(ctx, layer, io);
         do_attention(ctx, layer, io, false, fuse);
+        if (!fuse) ctx->kernels_run |= PA_RAN_APPEND;
     });
 }
 

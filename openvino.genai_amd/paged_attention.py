@@ -188,9 +188,15 @@ class PagedAttention:
 
     @property
     def kernels_run(self):
-        """Names of the kernels the last attention call launched (diagnostics)."""
+        """Names of the attention kernels the last call launched, and how (diagnostics)."""
         bits = int(L.lib().pa_get_kernels_run(self._h))
         return {n for i, n in enumerate(("generic", "decode", "decode_few", "matrix", "fold", "side_stream")) if bits >> i & 1}
+
+    @property
+    def launches_ahead(self):
+        """What the last call launched ahead of its attention kernels: "widen" (rows of long u8 chunks) and, for ``forward``, "append"."""
+        bits = int(L.lib().pa_get_kernels_run(self._h))
+        return {n for i, n in enumerate(("widen", "append"), 6) if bits >> i & 1}
 
 
 def pack_step(processed, evicted, skipped_blocks, scheduled, num_blocks, block_size):

@@ -167,7 +167,38 @@ def test_append_in_the_few_token_kernel(pkg, qd, bs, Hq, Hkv, D, past, new, sw, 
         else:
             op.forward(q, k, v, kc, vc, out)
         op.synchronize()
-        assert "decode_few" in op.kernels_run
+        assert "decode_few" in op.kernels_run and ("append" in op.launches_ahead) == (shared and not halves)
         got.append((out.view(torch.int16).cpu(), kc.cpu(), vc.cpu()))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_append_in_the_few_token_kernel_by_layer(pkg):
+    """A table per layer: only the layer in which one sequence reads a block that another one writes has an append launch."""
+    import torch
+    dev = torch.device("cuda:0")
+    print("case few append by layer", flush=True)
+    case = H.build_case(H.case_from_lens("few", 16, 4, 128, 32, "f16", "u8", [700, 705, 33], [5, 2, 1]), seed=2)
+    ids, bib = case["block_indices"], case["block_indices_begins"]
+    shared = ids.copy()
+    shared[bib[1]:bib[1] + 22] = ids[:22]  # (positions 0 .. 703; the first sequence's new rows start at 700)
+    q, k, v = (H.to_device_16(torch, case[x], "f16", dev) for x in ("query", "key", "value"))
+    got = []
+    for halves in (False, True):
+        op = pkg.PagedAttention(16, 4, 128, 32, "f16", "u8", 3, 0, torch.cuda.current_stream(dev))
+        op.step_begin(case["past_lens"], case["subsequence_begins"], bib, 707, None, 0, case["scale"])
+        op.set_block_indices_per_layer([ids, shared, ids], case["num_blocks"])
+        for layer in range(3):
+            kc, vc = (torch.from_numpy(case[x]).to(dev) for x in ("key_cache0", "value_cache0"))
+            out = torch.zeros_like(q)
+            if halves:
+                op.kv_append(k, v, kc, vc, layer)
+                op.attention(q, kc, vc, out, layer=layer)
+            else:
+                op.forward(q, k, v, kc, vc, out, layer=layer)
+                assert ("append" in op.launches_ahead) == (layer == 1)
+            op.synchronize()
+            assert "decode_few" in op.kernels_run
+            got.append((out.view(torch.int16).cpu(), kc.cpu(), vc.cpu()))
+    for a, b in zip(got[:3], got[3:]):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
