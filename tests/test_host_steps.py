@@ -178,3 +178,35 @@ def test_a_failed_mixed_step_joins_its_second_stream(on_fake):
         assert side and side[0] != "0", log
         assert log[-1] == "wait 0 " + side[0], log
     """)
+
+
+def test_copies_of_steps_queued_ahead(on_fake):
+    """Steps prepared one behind the other without a wait: no copy finds its part of the staging area written over, also where a step's
+    arrays do not fit it, with thresholds, with a table per layer and with rotations in between."""
+    on_fake("""
+        rng = np.random.default_rng(0)
+        op = pkg.PagedAttention(8, 2, 128, 32, "f16", "f16", num_layers=3)
+        op.set_rotation_trig_lut(np.ones((64, 128), np.float32))
+        ahead = 0
+        for i in range(60):
+            B = int(rng.integers(1, 6))
+            past, new = rng.integers(1, 4000, B).astype(np.int32), rng.integers(1, 900, B).astype(np.int32)
+            extra = 30000 if i in (20, 21, 40) else 0
+            bib = np.concatenate([[0], np.cumsum((past + new + 31) // 32 + extra)]).astype(np.int32)
+            op.step_begin(past, np.concatenate([[0], np.cumsum(new)]), bib)
+            ahead += rt.fake_pending(0) > 1  # (its own upload, and some of the step before)
+            if i % 3 == 0:
+                op.set_xattention(rng.random(B), 64, 8)
+            tables = rng.integers(0, 1000, (3, bib[-1]))
+            if i // 10 % 2:  # (going over from one table to one per layer waits)
+                op.set_block_indices_per_layer(tables, 1000)
+            else:
+                op.set_block_indices(tables[0], 1000)
+            if i % 5 == 0:
+                op.rotate_cache(T(1000), np.arange(7), np.arange(7))
+            for layer in range(3):
+                op.forward(T(1), T(1), T(1), T(1000), T(1000), T(1), layer=layer)
+        op.synchronize()
+        assert rt.fake_late_copies() == 0
+        assert ahead >= 30, ahead
+    """)
