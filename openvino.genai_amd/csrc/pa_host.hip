@@ -503,8 +503,12 @@ bool decode_u4_step(const pa_ctx* ctx) {
     return decode_u4_shape(ctx) && (int32_t)ctx->h_dec.size() == ctx->B && ctx->B <= 65535;
 }
 
-// Whether the step's single-token sequences may run on the 16-bit decode kernel, whose descriptors its tables then carry.
-bool decode16_descs(const pa_ctx* ctx) { return decode16_shape(ctx) && !ctx->h_dec16.empty(); }
+// Whether the step's single-token sequences may run on the 16-bit decode kernel, whose descriptors its tables then carry.  (Head
+// size 256 next to chunks: only where all of those are block-sparse, and thresholds may still be set behind the tables.)
+bool decode16_descs(const pa_ctx* ctx) {
+    const pa_config& c = ctx->cfg;
+    return decode16_shape(ctx) && !ctx->h_dec16.empty() && (ctx->T == ctx->B || c.head_size != 256 || c.block_size >= 32);
+}
 
 // Split-K plan of the decode kernels: workgroups per (sequence, kv head) and the most blocks one walks.
 void plan_decode_u8(const pa_ctx* ctx, bool want_scores, int32_t* nsplit_out, int32_t* max_tiles_out,
@@ -1088,7 +1092,7 @@ void do_attention(pa_ctx* ctx, int32_t layer, const pa_layer_io* io, bool static
     // dense chunks they stay work items of the matrix kernel: bandwidth-bound and matrix-bound items share the CUs
     // inside one launch, which two launches one after the other do not.)
     const bool side_by_side = ctx->split16 && !static_ws;
-    const bool use_decode16 = use_mfma && decode16_shape(ctx) && !ctx->h_dec16.empty() &&
+    const bool use_decode16 = use_mfma && decode16_descs(ctx) &&
                               (ctx->n_single + ctx->n_sparse == ctx->n_items || side_by_side);
     const bool mfma_left = use_mfma && !(use_decode16 && ctx->n_single == ctx->n_items);
     if (static_ws)

@@ -210,3 +210,20 @@ def test_copies_of_steps_queued_ahead(on_fake):
         assert rt.fake_late_copies() == 0
         assert ahead >= 30, ahead
     """)
+
+
+def test_tables_carry_the_descriptors_their_step_can_use(on_fake):
+    """Descriptors of the 16-bit decode kernel go up with a table only in steps that may run it."""
+    on_fake("""
+        def bytes_up(D, bs, new):
+            op = pkg.PagedAttention(8, 4, D, bs, "f16", "f16")
+            rt.fake_clear_log()
+            begin(op, [500, 900, 100, 300], new, bs)
+            return [int(l.split()[1]) for l in rt.fake_log().decode().splitlines() if l.startswith("malloc")][-1]
+        for D in (128, 256):
+            for bs in (16, 32):
+                for new in ([1, 1, 1, 1], [1, 1, 1, 64], [9, 9, 9, 64]):
+                    ids = sum(-(-(p + n) // bs) for p, n in zip([500, 900, 100, 300], new))
+                    plain = bytes_up(D, bs, new) == -(-4 * ids // 128) * 128
+                    assert plain == (1 not in new or (D == 256 and bs == 16 and max(new) > 1)), (D, bs, new)
+    """)
