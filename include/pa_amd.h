@@ -118,7 +118,9 @@ typedef struct pa_step_meta {
     float scale;
 } pa_step_meta;
 
-/* Replaces the set_tensor calls at the end of ModelRunner::forward (model_runner.hpp:907-948). */
+/* Replaces the set_tensor calls at the end of ModelRunner::forward (model_runner.hpp:907-948).  The arrays are copied before the
+ * call returns; their upload is queued on the context's stream behind what earlier steps have queued there.  The call waits for the
+ * step before the previous one only: it does not say that the previous step's outputs are there, nor that its inputs are free. */
 int32_t pa_step_begin(pa_ctx* ctx, const pa_step_meta* meta);
 
 /* `block_indices` (layer = -1: one table for all layers) or `block_indices.<layer>`

@@ -13,7 +13,7 @@
 //   * S^T of block j and O^T of block j - 1 are one run of matrix instructions, the softmax of block j follows them.
 // us per launch and layer, before (copies with scalar addresses and the row maximum per block; u8: codes widened by every
 // workgroup on their way to LDS) / now: bf16 28 / 4 heads 2048 tokens behind 30000 1386 / 1330 (0.91 TF of products, 1.36 with the
-// low halves, 1.02 PFLOP/s), f16 32 / 8 heads 1024 behind 8000 222 / 203; u8 32 / 8 heads 6143 tokens 700 / 558 in a kernel
+// low halves, 1.02 PFLOP/s; 3 - 5 % by card, as a step 1381 / 1311 to 1422 / 1381), f16 32 / 8 heads 1024 behind 8000 222 / 203; u8 32 / 8 heads 6143 tokens 700 / 558 in a kernel
 // trace, their rows widened in 8.
 // Also tried here: 32 x 32 x 16 products (5.7 cycles per vector instruction beside them, but loads and copies of another wave do
 // not issue at all while one is in flight), 512-thread workgroups whose halves alternate between matrix and vector work (the

@@ -231,8 +231,9 @@ __global__ __launch_bounds__(256, 2) void xatt_logits_u8_kernel(XattArgs a) {
 // order as there: the same logits bit for bit.
 // Bound by LDS: a 64-channel stage of a large tile takes 128 operand reads of 1 KB and 32 KB of copies beside 510 cycles of the
 // matrix pipe.  2048 tokens behind 14011 (28 / 4 heads, D = 128, stride 8): 74 us a launch with 32 groups x 64 keys x 4 heads
-// per workgroup and operands through registers, 53 us (525 TFLOP/s) so; as a step of two layers 514 -> 480 us, 16 / 8 heads of 256
-// behind 12000 534 -> 435, 128 tokens from scratch 98 -> 90.  Four buffers of large tiles, one workgroup per CU: 543 for 483 us.
+// per workgroup and operands through registers, 53 us (525 TFLOP/s) so; as a step of two layers 514 -> 480 us (on other cards
+// 574 -> 485 and 570 -> 451), 16 / 8 heads of 256 behind 12000 534 -> 435, 128 tokens from scratch 98 -> 90.  Four buffers of large
+// tiles, one workgroup per CU: 543 for 483 us.
 __device__ const u4v xatt_zeros = {0u, 0u, 0u, 0u};
 
 template <int D, int DT, int MT>
