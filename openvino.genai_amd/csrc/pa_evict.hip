@@ -50,9 +50,11 @@ struct StatusError : std::runtime_error {
 #define HIP_CHECK(expr)                                                                        \
     do {                                                                                       \
         hipError_t e_ = (expr);                                                                \
-        if (e_ != hipSuccess)                                                                  \
+        if (e_ != hipSuccess) {                                                                \
+            (void)hipGetLastError();  /* (or the next launch would report it as its own) */    \
             throw StatusError(e_ == hipErrorOutOfMemory ? PA_NOT_ALLOCATED : PA_GENERAL_ERROR, \
                               std::string(#expr) + ": " + hipGetErrorString(e_));              \
+        }                                                                                      \
     } while (0)
 
 enum : int32_t { RULE_SKIP = 0, RULE_INIT = 1, RULE_INIT_SNAPKV = 2, RULE_ADD = 3, RULE_ADD_SNAPKV = 4 };

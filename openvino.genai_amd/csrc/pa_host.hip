@@ -29,9 +29,11 @@ struct StatusError : std::runtime_error {
 #define HIP_CHECK(expr)                                                                               \
     do {                                                                                              \
         hipError_t e_ = (expr);                                                                       \
-        if (e_ != hipSuccess)                                                                         \
+        if (e_ != hipSuccess) {                                                                       \
+            (void)hipGetLastError();  /* (or the next launch would report it as its own) */           \
             throw StatusError(e_ == hipErrorOutOfMemory ? PA_NOT_ALLOCATED : PA_GENERAL_ERROR,        \
                               std::string(#expr) + ": " + hipGetErrorString(e_));                     \
+        }                                                                                             \
     } while (0)
 
 // Device buffer that only ever grows.
@@ -47,12 +49,9 @@ struct DevBuf {
         p = nullptr;
         cap = 0;
         const size_t want = std::max<size_t>(bytes, 256);
-        if (const hipError_t e = hipMalloc(&p, want)) {
-            p = nullptr;
-            (void)hipGetLastError();  // (or the next launch would report it as its own)
-            throw StatusError(e == hipErrorOutOfMemory ? PA_NOT_ALLOCATED : PA_GENERAL_ERROR,
-                              "hipMalloc of " + std::to_string(want) + " bytes: " + hipGetErrorString(e));
-        }
+        void* fresh = nullptr;
+        HIP_CHECK(hipMalloc(&fresh, want));
+        p = fresh;
         cap = want;
     }
     // ... for what the step can do without: false, and the buffer as it was, if there is no memory for the larger one.  It grows to

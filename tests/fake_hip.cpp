@@ -89,7 +89,11 @@ hipError_t hipFree(void* p) {
     std::free(p);
     return hipSuccess;
 }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return posix_memalign(p, 256, n ? n : 1) ? g_last = hipErrorOutOfMemory : hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    *p = nullptr;
+    if (n >= g_fail_lo && n <= g_fail_hi) return g_last = hipErrorOutOfMemory;
+    return posix_memalign(p, 256, n ? n : 1) ? g_last = hipErrorOutOfMemory : hipSuccess;
+}
 hipError_t hipHostFree(void* p) {
     drain_all();  // (as the runtime's does)
     return std::free(p), hipSuccess;

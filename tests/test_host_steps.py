@@ -41,6 +41,13 @@ def forward(op, scores=None):
     rt.fake_clear_log()
     op.forward(T(1), T(1), T(1), T(1000), T(1000), T(1), scores)
     return ran()
+def refused(status, fn, *args):
+    try:
+        fn(*args)
+    except pkg.PaError as e:
+        assert e.status == status, e
+    else:
+        assert False
 WIDE = 16896  # bytes of a widened (32-token block, kv head)
 """
 
@@ -121,13 +128,6 @@ def test_widened_rows_outlive_a_failed_growth(on_fake):
 def test_a_call_without_memory_leaves_no_freed_buffer_in_use(on_fake):
     """Larger thresholds' plans or trig tables that find no memory: what they replaced is gone, and calls that need it are refused."""
     on_fake("""
-        def refused(status, fn, *args):
-            try:
-                fn(*args)
-            except pkg.PaError as e:
-                assert e.status == status, e
-            else:
-                assert False
         op = pkg.PagedAttention(8, 2, 128, 32, "f16", "f16")
         begin(op, [3000], [500])
         op.set_xattention([0.9], 64, 16)
@@ -226,4 +226,30 @@ def test_tables_carry_the_descriptors_their_step_can_use(on_fake):
                     ids = sum(-(-(p + n) // bs) for p, n in zip([500, 900, 100, 300], new))
                     plain = bytes_up(D, bs, new) == -(-4 * ids // 128) * 128
                     assert plain == (1 not in new or (D == 256 and bs == 16 and max(new) > 1)), (D, bs, new)
+    """)
+
+
+def test_a_failed_call_is_not_reported_again(on_fake):
+    """The error of a runtime call that failed, pinned or device memory, belongs to the call it failed in, not to the next launch."""
+    on_fake("""
+        op = pkg.PagedAttention(8, 2, 128, 32, "f16", "f16")
+        rt.fake_fail_sizes(1, 1 << 40)
+        for _ in range(2):
+            refused(-10, begin, op, [30], [4])
+            rt.fake_fail_sizes(1, 0)
+            begin(op, [30], [4])
+            rt.fake_fail_sizes(1, 1 << 40)
+            refused(-10, forward, op)
+            rt.fake_fail_sizes(1, 0)
+            forward(op)
+            op = pkg.PagedAttention(8, 2, 128, 32, "f16", "f16")
+            rt.fake_fail_sizes(1, 1 << 40)
+        rt.fake_fail_sizes(1, 0)
+        from openvino_genai_amd.cache_eviction import AggregationMode, CacheEvictionConfig, Evictor
+        ev = Evictor(CacheEvictionConfig(32, 64, 192, AggregationMode.SUM, snapkv_window_size=0), 32, 2, 7, 1, 4096)
+        ev.register_new_token_scores([0], [1 << 40, 1 << 41], [0, 640])
+        rt.fake_fail_sizes(1, 1 << 40)
+        refused(-10, ev.block_scores, 0, 0)
+        rt.fake_fail_sizes(1, 0)
+        assert len(ev.block_scores(0, 0)) > 0
     """)
